@@ -311,6 +311,11 @@ struct Context {
   int x1_ra = 0, x1_rb = 0;
   DevBuf x1list;   // int32 nx1
   DevBuf st_x1;    // int32: index into x1list of the stick's i1
+  // LDS image of a z-plane (planes.hpp): rows held (a zero row last when x1_runs), the runs as the
+  // plane passes index them, the stick of each element (-1: zero) and the element of each stick
+  int pl_rows = 0, pl_ra = 0, pl_rb = 0;
+  DevBuf pl_src;   // int32 pl_rows·(ny + 1)
+  DevBuf st_off;   // int32 nsticks
 
   // effective potential (pwk_set_veff)
   bool have_v = false;
@@ -338,6 +343,8 @@ struct Context {
   DevBuf kin_pack64, kin_pack32, B_pack64, B_pack32, DBH_pack64, DBH_pack32;
   DevBuf band_tab;                  // int32 k-point per band of the last batch
   std::vector<int32_t> band_tab_host;
+
+  std::vector<double> dens_host;  // weights and list of the last density's live bands
 
   // workspaces
   DevBuf work_a, work_b;  // stick buffers / FFT scratch
@@ -412,6 +419,12 @@ void launch_hpsi(Context& c, int ik, int nb, const void* psi, void* hpsi, int pr
 // rho += Σ_b fw_b |ψ_b(r)|² (overwrite: rho = Σ ...)
 void launch_density(Context& c, int nb, const void* psi, const double* fw_host, void* rho, int precision,
                     bool overwrite = false);
+// z-inverse of nb bands into the stick buffer out[band][i3][stick] (list: device, the band of each of
+// the nb; null: the first nb)
+void launch_zinv(Context& c, int nb, const void* psi, void* out, int precision, const int* list);
+// density.hip: the band density on square grids of register-length lines (fw on the host)
+void launch_density_sticks(Context& c, int nb, const void* psi, const double* fw_host, void* rho, int precision,
+                           bool overwrite);
 void launch_hpsi_multi(Context& c, int nk, int nb, const void* psi, void* hpsi, int precision, const void* kin,
                        int nch, const void* B, const void* DBH, void* proj);
 // k × band batches with a band count per entry (bands of the entries packed back to back)

@@ -1,0 +1,230 @@
+// Band density on the sphere-pruned FFT (square grids): ρ(r) += Σ_b fw_b |ψ_b(r)|²
+// (src/scf/density.rs:59-97).
+//
+// Three launches: the z-inverse of the bands that carry weight (launch_zinv), the plane pass
+// k_plane_density on (z-plane, band group), and k_density_sum, which adds the groups' FP64 partial
+// sums in group order, so the result does not depend on scheduling.
+#include <algorithm>
+#include <vector>
+
+#include "common.hpp"
+#include "fft_sizes.hpp"
+#include "planes.hpp"
+
+namespace pwk {
+
+namespace {
+
+// Whether a thread keeps the FP64 sums of its x-line in registers: the line and its sums in at most
+// 280 32-bit registers; longer lines keep them in LDS.
+template <typename T, int N>
+constexpr bool acc_in_regs() {
+  return 2 * N * (int)(sizeof(T) / 4) + 2 * N <= 280;
+}
+template <typename T, int N>
+using DensityShape = PlaneShape<T, N, !acc_in_regs<T, N>()>;
+
+// One z-plane of `per` batches of SLOTS bands per workgroup: y- and x-inverse of each, then the sums
+// of fw·|ψ|² over the workgroup's bands to part[group][i3][i1][i2]. A thread owns one x-line of one
+// slot throughout, so its sums stay in registers over all its bands and are added across the slots
+// once, at the end.
+// Bound: vector arithmetic of the line transforms (a band's plane enters LDS once and never
+// returns). One workgroup per plane that loops over every band, as before, left 60 of 256 CUs with
+// one wave each.
+template <typename T, int N>
+__global__ void __launch_bounds__((DensityShape<T, N>::NT))
+    k_plane_density(const typename V2t<T>::t* __restrict__ tbuf, int nb, int per, const double* __restrict__ fw,
+                    double* __restrict__ part, int S, int nz, const int* __restrict__ src, int nsrc, int image,
+                    PlaneRows pr, int nx1, const int* __restrict__ x1list) {
+  using V2 = typename V2t<T>::t;
+  using Sh = DensityShape<T, N>;
+  constexpr int LD = Sh::LD, NT = Sh::NT, SLOTS = Sh::SLOTS;
+  constexpr bool REGS = acc_in_regs<T, N>();
+  constexpr int U = 16 / (int)(sizeof(T) / 4);
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
+  V2* P = reinterpret_cast<V2*>(smem_raw);
+  double* acc_lds = reinterpret_cast<double*>(smem_raw + (size_t)SLOTS * image * sizeof(V2));  // !REGS
+  const int i3 = blockIdx.x, g = blockIdx.y, t = threadIdx.x;
+  const int slot = t / N, i2 = t - slot * N;
+  double acc[REGS ? N : 1];
+#pragma unroll
+  for (int q = 0; q < (REGS ? N : 1); ++q) acc[q] = 0.0;
+  if (!REGS)
+    for (int i = t; i < SLOTS * N * N; i += NT) acc_lds[i] = 0.0;
+  const int b_end = min(nb, (g + 1) * per * SLOTS);
+  for (int b0 = g * per * SLOTS; b0 < b_end; b0 += SLOTS) {
+    const int nsl = min(SLOTS, b_end - b0);
+    plane_fill<T, N, NT, U>(P, image, tbuf + ((size_t)b0 * nz + i3) * S, (size_t)nz * S, nsl, src, nsrc);
+    __syncthreads();
+    plane_ylines<T, N, NT, 1>(P, image, nsl, nx1, x1list);
+    __syncthreads();
+    if (slot < nsl) {
+      const double f = fw[b0 + slot];
+      const V2* col = P + slot * image + i2;
+      T re[N], im[N];
+#pragma unroll
+      for (int j = 0; j < N; ++j) {
+        const V2 v = col[plane_row<N>(pr, j, nx1) * LD];
+        re[j] = v.x;
+        im[j] = v.y;
+      }
+      fft_dif<T, N, 1>(re, im);
+#pragma unroll
+      for (int q = 0; q < N; ++q) {
+        const double x = (double)re[FftOrder<N>::pos(q)], y = (double)im[FftOrder<N>::pos(q)];
+        if constexpr (REGS)
+          acc[q] += f * (x * x + y * y);
+        else
+          acc_lds[(slot * N + q) * N + i2] += f * (x * x + y * y);
+      }
+    }
+    __syncthreads();  // the image is filled again
+  }
+  // add the slots in order and write the plane
+  double* sum = REGS ? reinterpret_cast<double*>(smem_raw) : acc_lds;  // [N][N]
+  if constexpr (REGS) {
+    for (int p = 0; p < SLOTS; ++p) {
+      if (slot == p) {
+#pragma unroll
+        for (int q = 0; q < N; ++q) sum[q * N + i2] = p == 0 ? acc[q] : sum[q * N + i2] + acc[q];
+      }
+      __syncthreads();
+    }
+  }
+  double* out = part + ((size_t)g * nz + i3) * N * N;
+  for (int i = t; i < N * N; i += NT) {
+    double s = sum[i];
+    if (!REGS)
+      for (int p = 1; p < SLOTS; ++p) s += sum[p * N * N + i];
+    out[i] = s;
+  }
+}
+
+// rho[i1][i2][i3] (+)= Σ_g part[g][i3][i1][i2] in group order; a 32 × 32 (i2, i3) tile per workgroup
+// goes through LDS, so that both sides are read and written along their contiguous axis. Bound: the
+// partials' traffic (groups·N·8 bytes).
+__global__ void __launch_bounds__(256) k_density_sum(int ngroups, int nx, int ny, int nz, const double* __restrict__ part,
+                                                     double* __restrict__ rho, int overwrite) {
+  __shared__ double tile[32][33];
+  const int i1 = blockIdx.z, i20 = blockIdx.x * 32, i30 = blockIdx.y * 32;
+  const int c = threadIdx.x & 31, r = threadIdx.x >> 5;
+  const size_t n = (size_t)nx * ny * nz;
+  double s[4] = {0.0, 0.0, 0.0, 0.0};
+  const int i2 = min(i20 + c, ny - 1);
+  size_t o[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) o[k] = ((size_t)min(i30 + r + 8 * k, nz - 1) * nx + i1) * ny + i2;
+#pragma unroll 4
+  for (int g = 0; g < ngroups; ++g)
+#pragma unroll
+    for (int k = 0; k < 4; ++k) s[k] += part[(size_t)g * n + o[k]];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) tile[r + 8 * k][c] = s[k];
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const int y = i20 + r + 8 * k, z = i30 + c;
+    if (y < ny && z < nz) {
+      double* d = &rho[((size_t)i1 * ny + y) * nz + z];
+      const double v = tile[c][r + 8 * k];
+      *d = overwrite ? v : *d + v;
+    }
+  }
+}
+
+template <typename T, int N>
+void plane_density(Context& c, const void* tbuf, int nb, int per, int groups, const double* fw, double* part) {
+  using V2 = typename V2t<T>::t;
+  using Sh = DensityShape<T, N>;
+  const int image = c.pl_rows * Sh::LD;
+  size_t sh = (size_t)Sh::SLOTS * image * sizeof(V2);
+  if (acc_in_regs<T, N>())
+    sh = std::max(sh, (size_t)N * N * sizeof(double));
+  else
+    sh += (size_t)Sh::SLOTS * N * N * sizeof(double);
+  PWK_REQUIRE(sh <= 160 * 1024, PWK_E_UNSUPPORTED, "density plane exceeds the LDS");
+  ensure_lds_limit((const void*)k_plane_density<T, N>, sh);
+  const PlaneRows pr{c.pl_ra, c.pl_rb};
+  k_plane_density<T, N><<<dim3((unsigned)c.dims[2], (unsigned)groups), Sh::NT, sh, c.stream>>>(
+      (const V2*)tbuf, nb, per, fw, part, c.nsticks, c.dims[2], c.pl_src.as<int>(), image, image, pr, c.nx1,
+      c.x1_runs ? nullptr : c.x1list.as<int>());
+  PWK_HIP(hipGetLastError());
+}
+
+template <typename T>
+int plane_slots(int n) {
+  switch (n) {
+#define PWK_CASE(L) \
+  case L:           \
+    return DensityShape<T, L>::SLOTS;
+    PWK_FOR_EACH_FFT_SIZE(PWK_CASE)
+#undef PWK_CASE
+    default:
+      throw Error(PWK_E_UNSUPPORTED, "nx has no compiled kernel");
+  }
+}
+
+template <typename T>
+void density_sticks_t(Context& c, int nb, const void* psi, const double* fw_host, double* rho, bool overwrite) {
+  using V2 = typename V2t<T>::t;
+  // the bands that carry weight (src/scf/density.rs:14,72), their weights first
+  std::vector<double>& h = c.dens_host;
+  h.clear();
+  for (int b = 0; b < nb; ++b)
+    if (fw_host[b] >= 1e-15) h.push_back(fw_host[b]);
+  const int live = (int)h.size();
+  h.resize((size_t)live + (size_t)(live + 1) / 2);
+  {
+    int32_t* list = reinterpret_cast<int32_t*>(h.data() + live);
+    for (int b = 0, i = 0; b < nb; ++b)
+      if (fw_host[b] >= 1e-15) list[i++] = b;
+  }
+  const int nx = c.dims[0], ny = c.dims[1], nz = c.dims[2];
+  int groups = 0;
+  if (live > 0) {
+    c.work_b.ensure(h.size() * sizeof(double));
+    PWK_HIP(hipMemcpyAsync(c.work_b.p, h.data(), h.size() * sizeof(double), hipMemcpyHostToDevice, c.stream));
+    const double* fw = c.work_b.as<double>();
+    // about 1024 workgroups (four per CU): more only adds partial sums to store and read, fewer leave
+    // CUs idle. Measured with the groups' count that this gives: 60 planes × 144 bands in 16 groups.
+    const int slots = plane_slots<T>(nx);
+    const int batches = (live + slots - 1) / slots;
+    const int per = std::max(1, (int)(((long)batches * nz + 1023) / 1024));
+    groups = (batches + per - 1) / per;
+    // one z-inverse buffer for all live bands, then the groups' partial sums
+    const size_t tb = (((size_t)live * nz * c.nsticks * sizeof(V2)) + 255) & ~(size_t)255;
+    c.work_a.ensure(tb + (size_t)groups * c.N * sizeof(double));
+    double* part = reinterpret_cast<double*>(c.work_a.as<unsigned char>() + tb);
+    launch_zinv(c, live, psi, c.work_a.p, std::is_same<T, double>::value ? PWK_FP64 : PWK_FP32,
+                reinterpret_cast<const int*>(fw + live));
+    switch (nx) {
+#define PWK_CASE(L)                                                             \
+  case L:                                                                       \
+    plane_density<T, L>(c, c.work_a.p, live, per, groups, fw, part);            \
+    break;
+      PWK_FOR_EACH_FFT_SIZE(PWK_CASE)
+#undef PWK_CASE
+      default:
+        throw Error(PWK_E_UNSUPPORTED, "nx has no compiled kernel");
+    }
+    const dim3 gs(blocks_for((size_t)ny, 32), blocks_for((size_t)nz, 32), (unsigned)nx);
+    k_density_sum<<<gs, 256, 0, c.stream>>>(groups, nx, ny, nz, part, rho, overwrite ? 1 : 0);
+    PWK_HIP(hipGetLastError());
+  } else if (overwrite) {
+    const dim3 gs(blocks_for((size_t)ny, 32), blocks_for((size_t)nz, 32), (unsigned)nx);
+    k_density_sum<<<gs, 256, 0, c.stream>>>(0, nx, ny, nz, nullptr, rho, 1);
+    PWK_HIP(hipGetLastError());
+  }
+}
+
+}  // namespace
+
+void launch_density_sticks(Context& c, int nb, const void* psi, const double* fw_host, void* rho, int precision,
+                           bool overwrite) {
+  if (precision == PWK_FP64)
+    density_sticks_t<double>(c, nb, psi, fw_host, (double*)rho, overwrite);
+  else
+    density_sticks_t<float>(c, nb, psi, fw_host, (double*)rho, overwrite);
+}
+
+}  // namespace pwk

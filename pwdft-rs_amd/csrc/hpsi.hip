@@ -19,21 +19,11 @@
 #include "common.hpp"
 #include "fft_reg.hpp"
 #include "fft_sizes.hpp"
+#include "planes.hpp"
 
 namespace pwk {
 
 namespace {
-
-template <typename T>
-struct V2t;
-template <>
-struct V2t<double> {
-  using t = double2;
-};
-template <>
-struct V2t<float> {
-  using t = float2;
-};
 
 // index of n3 ≡ i3 (mod nz) inside a stick starting at n3 = lo, or >= cnt if absent
 __device__ __forceinline__ int stick_slot(int i3, int lo, int nz) {
@@ -47,12 +37,12 @@ template <typename T, int NZ>
 __global__ void __launch_bounds__(64) k_zinv(const typename V2t<T>::t* __restrict__ psi,
                                              typename V2t<T>::t* __restrict__ tbuf, int npw, int S,
                                              const int* __restrict__ st_pw0, const int* __restrict__ st_cnt,
-                                             const int* __restrict__ st_lo) {
+                                             const int* __restrict__ st_lo, const int* __restrict__ list) {
   int s = blockIdx.x * 64 + threadIdx.x;
   int b = blockIdx.y;
   if (s >= S) return;
   int pw0 = st_pw0[s], cnt = st_cnt[s], lo = st_lo[s];
-  const typename V2t<T>::t* src = psi + (size_t)b * npw + pw0;
+  const typename V2t<T>::t* src = psi + (size_t)(list ? list[b] : b) * npw + pw0;
   T re[NZ], im[NZ];
 #pragma unroll
   for (int i3 = 0; i3 < NZ; ++i3) {
@@ -205,59 +195,6 @@ __global__ void __launch_bounds__(64) k_plane_hpsi(typename V2t<T>::t* __restric
   for (int s = threadIdx.x; s < S; s += blockDim.x) {
     const int xy = st_xy[s];
     tp[s] = P[(COMPACT ? st_x1[s] : xy / NY) * LD + (xy % NY)];
-  }
-}
-
-// Density plane pass: one block per z-plane, loops over bands, accumulates
-// Σ_b fw_b |ψ_b(r)|² in an FP64 LDS plane, then adds it to rho (row-major grid).
-template <typename T, int NX, int NY>
-__global__ void __launch_bounds__(64) k_plane_density(const typename V2t<T>::t* __restrict__ tbuf, int nb,
-                                                      const double* __restrict__ fw, double* __restrict__ rho,
-                                                      int S, int nz, const int* __restrict__ st_xy, int nx1,
-                                                      const int* __restrict__ x1list) {
-  extern __shared__ unsigned char smem_raw[];
-  using V2 = typename V2t<T>::t;
-  constexpr int LD = NY + 1;
-  V2* P = reinterpret_cast<V2*>(smem_raw);
-  double* acc = reinterpret_cast<double*>(smem_raw + Plane<T, NX, NY>::bytes);
-  const int i3 = blockIdx.x;
-  for (int i = threadIdx.x; i < NX * NY; i += blockDim.x) acc[i] = 0.0;
-  for (int b = 0; b < nb; ++b) {
-    double f = fw[b];
-    if (f < 1e-15) continue;  // src/scf/density.rs:14,72
-    const V2* tp = tbuf + ((size_t)b * nz + i3) * S;
-    __syncthreads();
-    for (int i = threadIdx.x; i < NX * LD; i += blockDim.x) {
-      P[i].x = 0;
-      P[i].y = 0;
-    }
-    __syncthreads();
-    for (int s = threadIdx.x; s < S; s += blockDim.x) {
-      int xy = st_xy[s];
-      P[(xy / NY) * LD + (xy % NY)] = tp[s];
-    }
-    __syncthreads();
-    plane_rows<T, NY, 1>(P, nx1, x1list);
-    __syncthreads();
-    for (int i2 = threadIdx.x; i2 < NY; i2 += blockDim.x) {
-      T re[NX], im[NX];
-#pragma unroll
-      for (int j = 0; j < NX; ++j) {
-        re[j] = P[j * LD + i2].x;
-        im[j] = P[j * LD + i2].y;
-      }
-      fft_dif<T, NX, 1>(re, im);
-#pragma unroll
-      for (int q = 0; q < NX; ++q) {
-        double x = (double)re[FftOrder<NX>::pos(q)], y = (double)im[FftOrder<NX>::pos(q)];
-        acc[q * NY + i2] += f * (x * x + y * y);
-      }
-    }
-  }
-  __syncthreads();
-  for (int i = threadIdx.x; i < NX * NY; i += blockDim.x) {
-    int i1 = i / NY, i2 = i % NY;
-    rho[((size_t)i1 * NY + i2) * nz + i3] += acc[i];
   }
 }
 
@@ -415,6 +352,25 @@ void density_fullgrid(Context& c, int nb, const void* psi, const double* fw_host
 }
 
 // ---- dispatch ------------------------------------------------------------------
+template <typename T>
+void zinv_t(Context& c, int nb, const void* psi, typename V2t<T>::t* out, const int* list) {
+  using V2 = typename V2t<T>::t;
+  PWK_REQUIRE(nb <= 65535, PWK_E_UNSUPPORTED, "too many bands in one launch");
+  const dim3 gz(blocks_for((size_t)c.nsticks, 64), (unsigned)nb);
+  switch (c.dims[2]) {
+#define PWK_CASE(L)                                                                                             \
+  case L:                                                                                                       \
+    k_zinv<T, L><<<gz, 64, 0, c.stream>>>((const V2*)psi, out, c.npw, c.nsticks, c.st_pw0.as<int>(),            \
+                                          c.st_cnt.as<int>(), c.st_n3lo.as<int>(), list);                       \
+    break;
+    PWK_FOR_EACH_FFT_SIZE(PWK_CASE)
+#undef PWK_CASE
+    default:
+      throw Error(PWK_E_UNSUPPORTED, "nz has no compiled kernel");
+  }
+  PWK_HIP(hipGetLastError());
+}
+
 // Local part of H·ψ for nb bands; band b uses the kinetic diagonal kin + (b / nbk)·npw,
 // so consecutive groups of nbk bands may belong to different k-points.
 template <typename T>
@@ -434,18 +390,7 @@ void hpsi_local(Context& c, const T* kin, int nb, int nbk, const void* psi, void
   dim3 gz(blocks_for((size_t)c.nsticks, 64), (unsigned)nb);
   {
     TimedScope ts(c, "hpsi_zinv");
-    switch (nz) {
-#define PWK_CASE(L)                                                                                     \
-  case L:                                                                                               \
-    k_zinv<T, L><<<gz, 64, 0, c.stream>>>((const V2*)psi, T_, c.npw, c.nsticks, c.st_pw0.as<int>(),     \
-                                          c.st_cnt.as<int>(), c.st_n3lo.as<int>());                    \
-    break;
-      PWK_FOR_EACH_FFT_SIZE(PWK_CASE)
-#undef PWK_CASE
-      default:
-        throw Error(PWK_E_UNSUPPORTED, "nz has no compiled kernel");
-    }
-    PWK_HIP(hipGetLastError());
+    zinv_t<T>(c, nb, psi, T_, nullptr);
   }
   dim3 gp((unsigned)nz, (unsigned)nb);
   {
@@ -488,51 +433,6 @@ void hpsi_local(Context& c, const T* kin, int nb, int nbk, const void* psi, void
 #undef PWK_CASE
     default:
       throw Error(PWK_E_UNSUPPORTED, "nz has no compiled kernel");
-  }
-  PWK_HIP(hipGetLastError());
-}
-
-template <typename T>
-void density_t(Context& c, int nb, const void* psi, const double* fw_host, void* rho) {
-  using V2 = typename V2t<T>::t;
-  int nx = c.dims[0], nz = c.dims[2];
-  if (!stick_path_ok(c)) {
-    density_fullgrid<T>(c, nb, psi, fw_host, rho);
-    return;
-  }
-  size_t tb = (size_t)nb * nz * c.nsticks * sizeof(V2);
-  c.work_a.ensure(tb);
-  c.work_b.ensure((size_t)nb * sizeof(double));
-  PWK_HIP(hipMemcpyAsync(c.work_b.p, fw_host, (size_t)nb * sizeof(double), hipMemcpyHostToDevice, c.stream));
-  V2* T_ = c.work_a.as<V2>();
-  dim3 gz(blocks_for((size_t)c.nsticks, 64), (unsigned)nb);
-  switch (nz) {
-#define PWK_CASE(L)                                                                                     \
-  case L:                                                                                               \
-    k_zinv<T, L><<<gz, 64, 0, c.stream>>>((const V2*)psi, T_, c.npw, c.nsticks, c.st_pw0.as<int>(),     \
-                                          c.st_cnt.as<int>(), c.st_n3lo.as<int>());                    \
-    break;
-    PWK_FOR_EACH_FFT_SIZE(PWK_CASE)
-#undef PWK_CASE
-    default:
-      throw Error(PWK_E_UNSUPPORTED, "nz has no compiled kernel");
-  }
-  PWK_HIP(hipGetLastError());
-  switch (nx) {
-#define PWK_CASE(L)                                                                                      \
-  case L: {                                                                                              \
-    size_t sh = Plane<T, L, L>::bytes + (size_t)L * L * sizeof(double);                                  \
-    ensure_lds_limit((const void*)k_plane_density<T, L, L>, sh);                                        \
-    k_plane_density<T, L, L><<<(unsigned)nz, 64, sh, c.stream>>>(T_, nb, c.work_b.as<double>(),          \
-                                                                 (double*)rho, c.nsticks, nz,            \
-                                                                 c.st_xy.as<int>(), c.nx1,              \
-                                                                 c.x1list.as<int>());                   \
-    break;                                                                                               \
-  }
-    PWK_FOR_EACH_FFT_SIZE(PWK_CASE)
-#undef PWK_CASE
-    default:
-      throw Error(PWK_E_UNSUPPORTED, "nx has no compiled kernel");
   }
   PWK_HIP(hipGetLastError());
 }
@@ -588,6 +488,15 @@ void setup_basis(Context& c, int npw, const int32_t* m) {
     c.x1_ra = runs ? ra : 0;
     c.x1_rb = runs ? rb : 0;
   }
+  const int ld = ny + 1;
+  c.pl_rows = c.x1_runs ? c.nx1 + 1 : nx;
+  c.pl_ra = c.x1_runs ? c.x1_ra : nx;
+  c.pl_rb = c.x1_runs ? c.x1_rb : 0;
+  std::vector<int32_t> psrc((size_t)c.pl_rows * ld, -1), off;
+  for (size_t s = 0; s < xy.size(); ++s) {
+    off.push_back((c.x1_runs ? sx1[s] : xy[s] / ny) * ld + xy[s] % ny);
+    psrc[(size_t)off.back()] = (int32_t)s;
+  }
   auto up = [&](DevBuf& d, const void* h, size_t bytes) {
     d.ensure(bytes);
     PWK_HIP(hipMemcpyAsync(d.p, h, bytes, hipMemcpyHostToDevice, c.stream));
@@ -599,6 +508,8 @@ void setup_basis(Context& c, int npw, const int32_t* m) {
   up(c.st_n3lo, lo.data(), lo.size() * sizeof(int32_t));
   up(c.st_xy, xy.data(), xy.size() * sizeof(int32_t));
   up(c.x1list, x1list.data(), x1list.size() * sizeof(int32_t));
+  up(c.pl_src, psrc.data(), psrc.size() * sizeof(int32_t));
+  up(c.st_off, off.data(), off.size() * sizeof(int32_t));
   up(c.st_x1, sx1.data(), sx1.size() * sizeof(int32_t));
   c.sync();  // the host tables go out of scope here
 }
@@ -633,6 +544,13 @@ void set_veff_device(Context& c, const void* veff_g_dev, int slot, bool need_g) 
                                                          c.vrn32.as<float>() + o, c.dims[0], c.dims[1], c.dims[2]);
   PWK_HIP(hipGetLastError());
   if (slot == 0) c.have_v = true;
+}
+
+void launch_zinv(Context& c, int nb, const void* psi, void* out, int precision, const int* list) {
+  if (precision == PWK_FP64)
+    zinv_t<double>(c, nb, psi, (double2*)out, list);
+  else
+    zinv_t<float>(c, nb, psi, (float2*)out, list);
 }
 
 void launch_hpsi(Context& c, int ik, int nb, const void* psi, void* hpsi, int precision) {
@@ -811,11 +729,15 @@ void launch_density(Context& c, int nb, const void* psi, const double* fw_host, 
     launch_density_small(c, nb, psi, c.work_b.as<double>(), rho, dprec, overwrite);
     return;
   }
+  if (stick_path_ok(c)) {
+    launch_density_sticks(c, nb, psi, fw_host, rho, dprec, overwrite);
+    return;
+  }
   if (overwrite) PWK_HIP(hipMemsetAsync(rho, 0, c.N * sizeof(double), c.stream));
   if (precision == PWK_FP64)
-    density_t<double>(c, nb, psi, fw_host, rho);
+    density_fullgrid<double>(c, nb, psi, fw_host, rho);
   else
-    density_t<float>(c, nb, psi, fw_host, rho);
+    density_fullgrid<float>(c, nb, psi, fw_host, rho);
 }
 
 }  // namespace pwk

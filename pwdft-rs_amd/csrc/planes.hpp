@@ -1,0 +1,117 @@
+// One z-plane of the sphere-pruned FFT in LDS, shared by the H·ψ plane pass (hpsi.hip) and the band
+// density (density.hip).
+//
+// A workgroup works on SLOTS planes at once (the same i3 of SLOTS bands), so that the y-lines (only
+// the nx1 rows that carry sticks, about half of them) and the x-lines of a plane fill whole waves: a
+// 60-point plane alone has 29 y-lines for 64 lanes, two planes have 58.
+//
+// A plane's LDS image holds only the rows that carry sticks when these are the two runs i1 < ra and
+// i1 >= nx - rb (a sphere's columns), followed by a zero row that stands for every other row; grids
+// whose columns are not two such runs hold all rows (ra = nx, rb = 0). pl_src (setup_basis) gives the
+// stick of every element of that image, -1 for zeros: one pass of coalesced loads fills it, without
+// clearing it first and without a barrier in between.
+#pragma once
+
+#include "common.hpp"
+#include "fft_reg.hpp"
+
+namespace pwk {
+
+template <typename T>
+struct V2t;
+template <>
+struct V2t<double> {
+  using t = double2;
+};
+template <>
+struct V2t<float> {
+  using t = float2;
+};
+
+// Waves and planes per workgroup of a square N × N plane pass. Cost of a workgroup's passes in
+// wave-wide line transforms, per plane: ceil(SLOTS·N / 64) waves run x-lines, ceil(SLOTS·(N/2) / 64)
+// run y-lines; the cheapest of 1-4 waves is taken, fewer waves on a tie, whose planes fit 72 KB of
+// LDS (two workgroups per CU) with the rows of a sphere, and the 160 KB of a CU with all rows. ACC:
+// an FP64 sum per point and plane in LDS as well.
+template <typename T, int N, bool ACC = false>
+struct PlaneShape {
+  static constexpr int LD = N + 1;  // one element of padding against bank conflicts on row access
+  static constexpr int slots(int w) { return 64 * w / N; }
+  static constexpr size_t lds(int w, int rows) {
+    return (size_t)slots(w) * (rows * LD * sizeof(typename V2t<T>::t) + (ACC ? N * N * sizeof(double) : 0));
+  }
+  static constexpr int cost(int w) {  // in 1/720 of a wave-wide transform per plane (720: all slot counts divide)
+    return ((slots(w) * N + 63) / 64 + (slots(w) * (N / 2) + 63) / 64) * 720 / slots(w);
+  }
+  static constexpr int best() {
+    int w = (N + 63) / 64;
+    for (int v = w + 1; v <= 4; ++v)
+      if (lds(v, N / 2 + 3) <= 72 * 1024 && lds(v, N + 2) <= 160 * 1024 && cost(v) < cost(w)) w = v;
+    return w;
+  }
+  static constexpr int W = best(), NT = 64 * W, SLOTS = slots(W);
+};
+
+// the plane row j in the held image (`absent` for a row without sticks)
+struct PlaneRows {
+  int ra, rb;
+};
+template <int N>
+__device__ __forceinline__ int plane_row(const PlaneRows& pr, int j, int absent) {
+  return j < pr.ra ? j : (j >= N - pr.rb ? j - (N - pr.rb) + pr.ra : absent);
+}
+
+// fills `nsl` images (stride `image` elements) from the stick rows tp0 + p·band_stride; n elements each
+template <typename T, int N, int NT, int U>
+__device__ __forceinline__ void plane_fill(typename V2t<T>::t* P, int image,
+                                           const typename V2t<T>::t* __restrict__ tp0, size_t band_stride, int nsl,
+                                           const int* __restrict__ src, int n) {
+  using V2 = typename V2t<T>::t;
+  for (int e0 = threadIdx.x; e0 < n; e0 += U * NT) {
+    int s[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) s[u] = src[min(e0 + u * NT, n - 1)];
+    for (int p = 0; p < nsl; ++p) {
+      const V2* tp = tp0 + (size_t)p * band_stride;
+      V2 v[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) v[u] = tp[max(s[u], 0)];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int e = e0 + u * NT;
+        if (e < n) {
+          V2 x;
+          x.x = s[u] >= 0 ? v[u].x : (T)0;
+          x.y = s[u] >= 0 ? v[u].y : (T)0;
+          P[p * image + e] = x;
+        }
+      }
+    }
+  }
+}
+
+// the y-lines of the rows that carry sticks: row r of an image, or (x1list non-null: all rows held)
+// row x1list[r]
+template <typename T, int N, int NT, int SIGN>
+__device__ __forceinline__ void plane_ylines(typename V2t<T>::t* P, int image, int nsl, int nx1,
+                                             const int* __restrict__ x1list) {
+  constexpr int LD = N + 1;
+  for (int t = threadIdx.x; t < nsl * nx1; t += NT) {
+    const int p = t / nx1, r = t - p * nx1;
+    typename V2t<T>::t* row = P + p * image + (x1list ? x1list[r] : r) * LD;
+    T re[N], im[N];
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      re[j] = row[j].x;
+      im[j] = row[j].y;
+    }
+    fft_dif<T, N, SIGN>(re, im);
+#pragma unroll
+    for (int f = 0; f < N; ++f) {
+      row[f].x = re[FftOrder<N>::pos(f)];
+      row[f].y = im[FftOrder<N>::pos(f)];
+    }
+  }
+}
+
+}  // namespace pwk

@@ -1,0 +1,67 @@
+"""The z-plane passes of the sphere-pruned transforms (square grids) against numpy in 64 bits, at the
+sizes where their layout changes: planes per workgroup, sums in registers or LDS, bases whose columns
+are two runs of rows or every row, band counts around the planes per workgroup."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def sphere(dims, m):
+    """Miller indices with |n|² ≤ m² in n1 → n2 → n3 order, and their flat grid index."""
+    r = np.arange(-m, m + 1)
+    n = np.stack(np.meshgrid(r, r, r, indexing="ij"), -1).reshape(-1, 3)
+    n = n[(n * n).sum(1) <= m * m]
+    i = [n[:, d] % dims[d] for d in range(3)]
+    return n.astype(np.int32), (i[0] * dims[1] + i[1]) * dims[2] + i[2]
+
+
+def setup(acc, dims, m):
+    miller, idx = sphere(dims, m)
+    acc.prepare_buffers(dims, np.ones(int(np.prod(dims))))
+    acc.set_basis(miller)
+    acc.set_nk(1)
+    acc.set_kinetic(0, (miller.astype(float) ** 2).sum(1))
+    return miller, idx
+
+
+def bands(rng, nb, npw):
+    psi = rng.standard_normal((nb, npw)) + 1j * rng.standard_normal((nb, npw))
+    return psi / np.linalg.norm(psi, axis=1)[:, None]
+
+
+def to_grid(psi, idx, dims):
+    g = np.zeros((len(psi), int(np.prod(dims))), dtype=complex)
+    g[:, idx] = psi
+    return np.fft.ifftn(g.reshape((len(psi),) + tuple(dims)), axes=(1, 2, 3)) * np.prod(dims)
+
+
+# (grid, sphere radius): 15 with every row carrying sticks and 16 with all but one, 25 and 27 with
+# several planes per workgroup, 45 and 48 around the register limit of the FP64 sums, 64 and 72 with
+# sums in LDS, 81 the longest line
+PLANES = [((15, 15, 18), 7), ((16, 16, 12), 5), ((25, 25, 25), 6), ((27, 27, 27), 13), ((45, 45, 16), 7),
+          ((48, 48, 9), 4), ((60, 60, 10), 4), ((64, 64, 15), 7), ((72, 72, 8), 3), ((81, 81, 72), 3)]
+
+
+@pytest.mark.parametrize("dims,m", PLANES)
+@pytest.mark.parametrize("prec,tol", [("fp64", 1e-13), ("fp32", 4e-6)])
+def test_density_planes(gpu, dims, m, prec, tol):
+    # tolerance: three axes of log2(N) ≈ 6 roundings each on ψ, doubled by the square (FP32: 18 ·
+    # 6e-8 · 2 = 2.1e-6 of the largest value)
+    gpu.set_fused_hpsi(False)  # the plane passes also where a fused small-grid kernel exists
+    try:
+        miller, idx = setup(gpu, dims, m)
+        rng = np.random.default_rng(31)
+        for nb in (1, 2, 3, 11, 12):
+            psi = bands(rng, nb, len(miller))
+            fw = rng.uniform(0.1, 2.0, nb)
+            fw[nb // 2] = 0.0 if nb > 2 else fw[nb // 2]  # a band without weight is left out
+            rho0 = rng.uniform(0.0, 1e-3, int(np.prod(dims)))
+            print("density planes", dims, m, prec, "bands", nb, flush=True)
+            got = gpu.density(psi, fw, rho0, prec)
+            ref = rho0 + (fw[:, None] * np.abs(to_grid(psi, idx, dims).reshape(nb, -1)) ** 2).sum(0)
+            assert np.abs(got - ref).max() < tol * np.abs(ref).max()
+        psi[:] = np.nan  # bands without weight are not read
+        assert np.array_equal(gpu.density(psi, np.zeros(nb), rho0, prec), rho0)
+    finally:
+        gpu.set_fused_hpsi(True)
