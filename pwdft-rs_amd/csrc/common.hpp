@@ -316,6 +316,10 @@ struct Context {
   int pl_rows = 0, pl_ra = 0, pl_rb = 0;
   DevBuf pl_src;   // int32 pl_rows·(ny + 1)
   DevBuf st_off;   // int32 nsticks
+  // every plane wave within a quarter of each axis (planes.hpp, Quarter): the pruned passes run, with
+  // the stick of each held (row, column) and the image element of each stick
+  bool quarter = false;
+  DevBuf q_src, q_off;
 
   // effective potential (pwk_set_veff)
   bool have_v = false;
@@ -422,6 +426,13 @@ void launch_density(Context& c, int nb, const void* psi, const double* fw_host, 
 // z-inverse of nb bands into the stick buffer out[band][i3][stick] (list: device, the band of each of
 // the nb; null: the first nb)
 void launch_zinv(Context& c, int nb, const void* psi, void* out, int precision, const int* list);
+// hpsi_sphere.hip: the passes on spheres within a quarter of the axes (c.quarter)
+template <typename T>
+void sphere_zinv(Context& c, int nb, const void* psi, void* out, const int* list);
+template <typename T>
+void sphere_plane(Context& c, int nb, void* buf, const T* vr);
+template <typename T>
+void sphere_zfwd(Context& c, int nb, const void* buf, const T* kin, int nbk, const void* psi, void* hpsi);
 // density.hip: the band density on square grids of register-length lines (fw on the host)
 void launch_density_sticks(Context& c, int nb, const void* psi, const double* fw_host, void* rho, int precision,
                            bool overwrite);

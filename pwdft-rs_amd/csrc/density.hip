@@ -21,6 +21,10 @@ template <typename T, int N>
 constexpr bool acc_in_regs() {
   return 2 * N * (int)(sizeof(T) / 4) + 2 * N <= 280;
 }
+template <int N, bool QUARTER>
+struct LineTable : LineOrder<N> {};
+template <int N>
+struct LineTable<N, false> : FftOrder<N> {};
 template <typename T, int N>
 using DensityShape = PlaneShape<T, N, !acc_in_regs<T, N>()>;
 
@@ -31,10 +35,12 @@ using DensityShape = PlaneShape<T, N, !acc_in_regs<T, N>()>;
 // Bound: vector arithmetic of the line transforms (a band's plane enters LDS once and never
 // returns). One workgroup per plane that loops over every band, as before, left 60 of 256 CUs with
 // one wave each.
-template <typename T, int N>
+// QUARTER: a sphere within a quarter of the axes (planes.hpp); otherwise the held rows come from the
+// basis' tables.
+template <typename T, int N, bool QUARTER>
 __global__ void __launch_bounds__((DensityShape<T, N>::NT))
     k_plane_density(const typename V2t<T>::t* __restrict__ tbuf, int nb, int per, const double* __restrict__ fw,
-                    double* __restrict__ part, int S, int nz, const int* __restrict__ src, int nsrc, int image,
+                    double* __restrict__ part, int S, int nz, const int* __restrict__ src, int image,
                     PlaneRows pr, int nx1, const int* __restrict__ x1list) {
   using V2 = typename V2t<T>::t;
   using Sh = DensityShape<T, N>;
@@ -54,24 +60,36 @@ __global__ void __launch_bounds__((DensityShape<T, N>::NT))
   const int b_end = min(nb, (g + 1) * per * SLOTS);
   for (int b0 = g * per * SLOTS; b0 < b_end; b0 += SLOTS) {
     const int nsl = min(SLOTS, b_end - b0);
-    plane_fill<T, N, NT, U>(P, image, tbuf + ((size_t)b0 * nz + i3) * S, (size_t)nz * S, nsl, src, nsrc);
+    const V2* tp0 = tbuf + ((size_t)b0 * nz + i3) * S;
+    if constexpr (QUARTER)
+      quarter_fill<T, N, NT, U>(P, tp0, (size_t)nz * S, nsl, src);
+    else
+      plane_fill<T, N, NT, U>(P, image, tp0, (size_t)nz * S, nsl, src, image);
     __syncthreads();
-    plane_ylines<T, N, NT, 1>(P, image, nsl, nx1, x1list);
+    if constexpr (QUARTER)
+      quarter_ylines<T, N, NT, 1>(P, nsl);
+    else
+      plane_ylines<T, N, NT, 1>(P, image, nsl, nx1, x1list);
     __syncthreads();
     if (slot < nsl) {
       const double f = fw[b0 + slot];
       const V2* col = P + slot * image + i2;
       T re[N], im[N];
+      if constexpr (QUARTER) {
+        quarter_xline<T, N>(col, re, im);
+      } else {
 #pragma unroll
-      for (int j = 0; j < N; ++j) {
-        const V2 v = col[plane_row<N>(pr, j, nx1) * LD];
-        re[j] = v.x;
-        im[j] = v.y;
+        for (int j = 0; j < N; ++j) {
+          const V2 v = col[plane_row<N>(pr, j, nx1) * LD];
+          re[j] = v.x;
+          im[j] = v.y;
+        }
+        fft_dif<T, N, 1>(re, im);
       }
-      fft_dif<T, N, 1>(re, im);
 #pragma unroll
       for (int q = 0; q < N; ++q) {
-        const double x = (double)re[FftOrder<N>::pos(q)], y = (double)im[FftOrder<N>::pos(q)];
+        const int o = LineTable<N, QUARTER>::pos(q);
+        const double x = (double)re[o], y = (double)im[o];
         if constexpr (REGS)
           acc[q] += f * (x * x + y * y);
         else
@@ -132,22 +150,22 @@ __global__ void __launch_bounds__(256) k_density_sum(int ngroups, int nx, int ny
   }
 }
 
-template <typename T, int N>
+template <typename T, int N, bool QUARTER>
 void plane_density(Context& c, const void* tbuf, int nb, int per, int groups, const double* fw, double* part) {
   using V2 = typename V2t<T>::t;
   using Sh = DensityShape<T, N>;
-  const int image = c.pl_rows * Sh::LD;
+  const int image = QUARTER ? Quarter<N>::R * Quarter<N>::LD : c.pl_rows * Sh::LD;
   size_t sh = (size_t)Sh::SLOTS * image * sizeof(V2);
   if (acc_in_regs<T, N>())
     sh = std::max(sh, (size_t)N * N * sizeof(double));
   else
     sh += (size_t)Sh::SLOTS * N * N * sizeof(double);
   PWK_REQUIRE(sh <= 160 * 1024, PWK_E_UNSUPPORTED, "density plane exceeds the LDS");
-  ensure_lds_limit((const void*)k_plane_density<T, N>, sh);
+  ensure_lds_limit((const void*)k_plane_density<T, N, QUARTER>, sh);
   const PlaneRows pr{c.pl_ra, c.pl_rb};
-  k_plane_density<T, N><<<dim3((unsigned)c.dims[2], (unsigned)groups), Sh::NT, sh, c.stream>>>(
-      (const V2*)tbuf, nb, per, fw, part, c.nsticks, c.dims[2], c.pl_src.as<int>(), image, image, pr, c.nx1,
-      c.x1_runs ? nullptr : c.x1list.as<int>());
+  k_plane_density<T, N, QUARTER><<<dim3((unsigned)c.dims[2], (unsigned)groups), Sh::NT, sh, c.stream>>>(
+      (const V2*)tbuf, nb, per, fw, part, c.nsticks, c.dims[2], QUARTER ? c.q_src.as<int>() : c.pl_src.as<int>(), image,
+      pr, c.nx1, c.x1_runs ? nullptr : c.x1list.as<int>());
   PWK_HIP(hipGetLastError());
 }
 
@@ -200,7 +218,10 @@ void density_sticks_t(Context& c, int nb, const void* psi, const double* fw_host
     switch (nx) {
 #define PWK_CASE(L)                                                             \
   case L:                                                                       \
-    plane_density<T, L>(c, c.work_a.p, live, per, groups, fw, part);            \
+    if (c.quarter)                                                              \
+      plane_density<T, L, true>(c, c.work_a.p, live, per, groups, fw, part);    \
+    else                                                                        \
+      plane_density<T, L, false>(c, c.work_a.p, live, per, groups, fw, part);   \
     break;
       PWK_FOR_EACH_FFT_SIZE(PWK_CASE)
 #undef PWK_CASE

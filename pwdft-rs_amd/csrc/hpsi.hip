@@ -102,100 +102,84 @@ __global__ void __launch_bounds__(64) k_zfwd(const typename V2t<T>::t* __restric
   }
 }
 
-// LDS plane P[NX][NY+1] (one padding column against bank conflicts on row access)
-template <typename T, int NX, int NY>
-struct Plane {
-  static constexpr int LD = NY + 1;
-  static constexpr size_t bytes = (size_t)NX * LD * sizeof(typename V2t<T>::t);
-};
-
-// the y-lines of the plane's rows that carry sticks: row x1list[r] of P, or (x1list null) row r of
-// a plane that holds only those rows
-template <typename T, int NY, int SIGN>
-__device__ __forceinline__ void plane_rows(typename V2t<T>::t* P, int nx1, const int* __restrict__ x1list) {
-  constexpr int LD = NY + 1;
-  for (int r = threadIdx.x; r < nx1; r += blockDim.x) {
-    typename V2t<T>::t* row = P + (x1list ? x1list[r] : r) * LD;
-    T re[NY], im[NY];
+// H·ψ plane pass: the z-plane i3 of SLOTS bands per workgroup (planes.hpp): y-inverse on the rows with
+// sticks, x-inverse, × V(r), x-forward, y-forward, back to the sticks. The rows without sticks are zero
+// through the y passes and their x output is never gathered: the x-lines read them from the image's
+// zero row and write them to a discard row after it, so the loads and stores need no branch. Bound: the
+// vector arithmetic of the line transforms; the traffic is the stick buffer in and out.
+template <typename T, int N>
+__global__ void __launch_bounds__((PlaneShape<T, N>::NT))
+    k_plane_hpsi(typename V2t<T>::t* tbuf, int nb, const T* __restrict__ vr, int S, int nz,
+                 const int* __restrict__ src, int nsrc, int image, const int* __restrict__ st_off, PlaneRows pr,
+                 int nx1, const int* __restrict__ x1list) {
+  using V2 = typename V2t<T>::t;
+  using Sh = PlaneShape<T, N>;
+  constexpr int LD = Sh::LD, NT = Sh::NT, SLOTS = Sh::SLOTS;
+  constexpr int U = 16 / (int)(sizeof(T) / 4);
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
+  V2* P = reinterpret_cast<V2*>(smem_raw);
+  const int i3 = blockIdx.x, b0 = blockIdx.y * SLOTS, nsl = min(SLOTS, nb - b0);
+  const size_t stride = (size_t)nz * S;
+  V2* tp0 = tbuf + (size_t)b0 * stride + (size_t)i3 * S;
+  plane_fill<T, N, NT, U>(P, image, tp0, stride, nsl, src, nsrc);
+  __syncthreads();
+  plane_ylines<T, N, NT, 1>(P, image, nsl, nx1, x1list);
+  __syncthreads();
+  const int slot = threadIdx.x / N, i2 = threadIdx.x - slot * N;
+  if (slot < nsl) {
+    const T* v = vr + (size_t)i3 * N * N + i2;
+    V2* col = P + slot * image + i2;
+    T re[N], im[N];
 #pragma unroll
-    for (int j = 0; j < NY; ++j) {
-      re[j] = row[j].x;
-      im[j] = row[j].y;
+    for (int j = 0; j < N; ++j) {
+      const V2 x = col[plane_row<N>(pr, j, nx1) * LD];
+      re[j] = x.x;
+      im[j] = x.y;
     }
-    fft_dif<T, NY, SIGN>(re, im);
+    fft_dif<T, N, 1>(re, im);
+    T r2[N], m2[N];
 #pragma unroll
-    for (int f = 0; f < NY; ++f) {
-      row[f].x = re[FftOrder<NY>::pos(f)];
-      row[f].y = im[FftOrder<NY>::pos(f)];
+    for (int f = 0; f < N; ++f) {
+      const T vv = v[f * N];
+      r2[f] = re[FftOrder<N>::pos(f)] * vv;
+      m2[f] = im[FftOrder<N>::pos(f)] * vv;
+    }
+    fft_dif<T, N, -1>(r2, m2);
+#pragma unroll
+    for (int f = 0; f < N; ++f) {
+      V2 x;
+      x.x = r2[FftOrder<N>::pos(f)];
+      x.y = m2[FftOrder<N>::pos(f)];
+      col[plane_row<N>(pr, f, nx1 + 1) * LD] = x;
+    }
+  }
+  __syncthreads();
+  plane_ylines<T, N, NT, -1>(P, image, nsl, nx1, x1list);
+  __syncthreads();
+  for (int s0 = threadIdx.x; s0 < S; s0 += U * NT) {
+    int off[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) off[u] = st_off[min(s0 + u * NT, S - 1)];
+    for (int p = 0; p < nsl; ++p) {
+      V2* tp = tp0 + (size_t)p * stride;
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (s0 + u * NT < S) tp[s0 + u * NT] = P[p * image + off[u]];
     }
   }
 }
 
-// H·ψ plane pass: one (z-plane, band) per workgroup. COMPACT: the rows of the plane that carry
-// sticks are the two runs i1 < ra and i1 >= NX - rb (a sphere's columns), and only those
-// nx1 = ra + rb rows are held in LDS, plus a zero row and a discard row. The other rows are zero
-// through the y passes and their x-pass output is never gathered, so the x-lines read them from the
-// zero row and write them to the discard row. Same arithmetic as the whole plane; about half the LDS
-// for a sphere that spans half the axis, so more planes in flight per CU.
-template <typename T, int NX, int NY, bool COMPACT>
-__global__ void __launch_bounds__(64) k_plane_hpsi(typename V2t<T>::t* __restrict__ tbuf, const T* __restrict__ vr,
-                                                   int S, int nz, const int* __restrict__ st_xy,
-                                                   const int* __restrict__ st_x1, int nx1,
-                                                   const int* __restrict__ x1list, int ra, int rb) {
-  extern __shared__ unsigned char smem_raw[];
-  using V2 = typename V2t<T>::t;
-  constexpr int LD = NY + 1;
-  V2* P = reinterpret_cast<V2*>(smem_raw);
-  const int i3 = blockIdx.x, b = blockIdx.y;
-  V2* tp = tbuf + ((size_t)b * nz + i3) * S;
-  const int rows = COMPACT ? nx1 + 2 : NX;
-  for (int i = threadIdx.x; i < rows * LD; i += blockDim.x) {
-    P[i].x = 0;
-    P[i].y = 0;
-  }
-  __syncthreads();
-  for (int s = threadIdx.x; s < S; s += blockDim.x) {
-    const int xy = st_xy[s];
-    P[(COMPACT ? st_x1[s] : xy / NY) * LD + (xy % NY)] = tp[s];
-  }
-  __syncthreads();
-  plane_rows<T, NY, 1>(P, nx1, COMPACT ? nullptr : x1list);
-  __syncthreads();
-  const T* v = vr + (size_t)i3 * NX * NY;
-  // held row of plane row j (COMPACT); a row without sticks reads row nx1 (kept zero) and writes
-  // row nx1 + 1 (discarded), so the loads and stores need no branch
-  auto row = [&](int j, int absent) { return j < ra ? j : (j >= NX - rb ? j - (NX - rb) + ra : absent); };
-  for (int i2 = threadIdx.x; i2 < NY; i2 += blockDim.x) {
-    T re[NX], im[NX];
-#pragma unroll
-    for (int j = 0; j < NX; ++j) {
-      const int r = COMPACT ? row(j, nx1) : j;
-      re[j] = P[r * LD + i2].x;
-      im[j] = P[r * LD + i2].y;
-    }
-    fft_dif<T, NX, 1>(re, im);
-    T r2[NX], m2[NX];
-#pragma unroll
-    for (int f = 0; f < NX; ++f) {
-      T vv = v[f * NY + i2];
-      r2[f] = re[FftOrder<NX>::pos(f)] * vv;
-      m2[f] = im[FftOrder<NX>::pos(f)] * vv;
-    }
-    fft_dif<T, NX, -1>(r2, m2);
-#pragma unroll
-    for (int f = 0; f < NX; ++f) {
-      const int r = COMPACT ? row(f, nx1 + 1) : f;
-      P[r * LD + i2].x = r2[FftOrder<NX>::pos(f)];
-      P[r * LD + i2].y = m2[FftOrder<NX>::pos(f)];
-    }
-  }
-  __syncthreads();
-  plane_rows<T, NY, -1>(P, nx1, COMPACT ? nullptr : x1list);
-  __syncthreads();
-  for (int s = threadIdx.x; s < S; s += blockDim.x) {
-    const int xy = st_xy[s];
-    tp[s] = P[(COMPACT ? st_x1[s] : xy / NY) * LD + (xy % NY)];
-  }
+template <typename T, int N>
+void plane_hpsi(Context& c, typename V2t<T>::t* tbuf, int nb, const T* vr) {
+  using Sh = PlaneShape<T, N>;
+  const int nz = c.dims[2], rows = c.x1_runs ? c.pl_rows + 1 : c.pl_rows, image = rows * Sh::LD;
+  const size_t sh = (size_t)Sh::SLOTS * image * sizeof(typename V2t<T>::t);
+  PWK_REQUIRE(sh <= 160 * 1024, PWK_E_UNSUPPORTED, "plane exceeds the LDS");
+  ensure_lds_limit((const void*)k_plane_hpsi<T, N>, sh);
+  k_plane_hpsi<T, N><<<dim3((unsigned)nz, blocks_for((size_t)nb, Sh::SLOTS)), Sh::NT, sh, c.stream>>>(
+      tbuf, nb, vr, c.nsticks, nz, c.pl_src.as<int>(), c.pl_rows * Sh::LD, image, c.st_off.as<int>(),
+      PlaneRows{c.pl_ra, c.pl_rb}, c.nx1, c.x1_runs ? nullptr : c.x1list.as<int>());
+  PWK_HIP(hipGetLastError());
 }
 
 // V(r) = Re IFFT_unnorm(V_eff(G)) re-ordered to plane-major [i3][i1][i2] (stick path), and in
@@ -356,6 +340,10 @@ template <typename T>
 void zinv_t(Context& c, int nb, const void* psi, typename V2t<T>::t* out, const int* list) {
   using V2 = typename V2t<T>::t;
   PWK_REQUIRE(nb <= 65535, PWK_E_UNSUPPORTED, "too many bands in one launch");
+  if (c.quarter) {
+    sphere_zinv<T>(c, nb, psi, out, list);
+    return;
+  }
   const dim3 gz(blocks_for((size_t)c.nsticks, 64), (unsigned)nb);
   switch (c.dims[2]) {
 #define PWK_CASE(L)                                                                                             \
@@ -376,7 +364,7 @@ void zinv_t(Context& c, int nb, const void* psi, typename V2t<T>::t* out, const 
 template <typename T>
 void hpsi_local(Context& c, const T* kin, int nb, int nbk, const void* psi, void* hpsi) {
   using V2 = typename V2t<T>::t;
-  int nx = c.dims[0], ny = c.dims[1], nz = c.dims[2];
+  int nx = c.dims[0], nz = c.dims[2];
   PWK_REQUIRE(c.have_v, PWK_E_STATE, "V_eff not set (pwk_set_veff)");
   if (!stick_path_ok(c)) {
     hpsi_fullgrid<T>(c, kin, nb, nbk, psi, hpsi);
@@ -392,36 +380,30 @@ void hpsi_local(Context& c, const T* kin, int nb, int nbk, const void* psi, void
     TimedScope ts(c, "hpsi_zinv");
     zinv_t<T>(c, nb, psi, T_, nullptr);
   }
-  dim3 gp((unsigned)nz, (unsigned)nb);
   {
-  TimedScope ts_plane(c, "hpsi_plane");
-  switch (nx) {
-#define PWK_CASE(L)                                                                                      \
-  case L: {                                                                                              \
-    if (c.x1_runs) {                                                                                     \
-      size_t sh = (size_t)(c.nx1 + 2) * (L + 1) * sizeof(V2);                                            \
-      ensure_lds_limit((const void*)k_plane_hpsi<T, L, L, true>, sh);                                   \
-      k_plane_hpsi<T, L, L, true><<<gp, 64, sh, c.stream>>>(T_, vr, c.nsticks, nz, c.st_xy.as<int>(),    \
-                                                            c.st_x1.as<int>(), c.nx1, c.x1list.as<int>(), \
-                                                            c.x1_ra, c.x1_rb);                           \
-    } else {                                                                                             \
-      size_t sh = Plane<T, L, L>::bytes;                                                                 \
-      ensure_lds_limit((const void*)k_plane_hpsi<T, L, L, false>, sh);                                  \
-      k_plane_hpsi<T, L, L, false><<<gp, 64, sh, c.stream>>>(T_, vr, c.nsticks, nz, c.st_xy.as<int>(),   \
-                                                             c.st_x1.as<int>(), c.nx1,                  \
-                                                             c.x1list.as<int>(), 0, 0);                 \
-    }                                                                                                    \
-    break;                                                                                               \
-  }
-    PWK_FOR_EACH_FFT_SIZE(PWK_CASE)
+    TimedScope ts(c, "hpsi_plane");
+    // (the pruned FP64 plane pass of 81 points does not fit the registers)
+    if (c.quarter && !(std::is_same<T, double>::value && nx > 80)) {
+      sphere_plane<T>(c, nb, T_, vr);
+    } else {
+      switch (nx) {
+#define PWK_CASE(L)                    \
+  case L:                              \
+    plane_hpsi<T, L>(c, T_, nb, vr);   \
+    break;
+        PWK_FOR_EACH_FFT_SIZE(PWK_CASE)
 #undef PWK_CASE
-    default:
-      throw Error(PWK_E_UNSUPPORTED, "nx has no compiled kernel");
+        default:
+          throw Error(PWK_E_UNSUPPORTED, "nx has no compiled kernel");
+      }
+    }
   }
-  PWK_HIP(hipGetLastError());
-  }  // the plane scope ends here, before the z-forward launch
   T inv_n = (T)(1.0 / (double)c.N);
   TimedScope ts_zfwd(c, "hpsi_zfwd");
+  if (c.quarter) {
+    sphere_zfwd<T>(c, nb, T_, kin, nbk, psi, hpsi);
+    return;
+  }
   switch (nz) {
 #define PWK_CASE(L)                                                                                     \
   case L:                                                                                               \
@@ -497,6 +479,21 @@ void setup_basis(Context& c, int npw, const int32_t* m) {
     off.push_back((c.x1_runs ? sx1[s] : xy[s] / ny) * ld + xy[s] % ny);
     psrc[(size_t)off.back()] = (int32_t)s;
   }
+  // pruned passes: every index within a quarter of its axis
+  c.quarter = stick_path_ok(c);
+  for (int i = 0; i < npw && c.quarter; ++i)
+    for (int d = 0; d < 3; ++d) c.quarter = c.quarter && std::abs(m[3 * i + d]) <= (c.dims[d] - 1) / 4;
+  std::vector<int32_t> qsrc, qoff;
+  if (c.quarter) {
+    const int pb = (nx - 1) / 4, r = 2 * pb + 1, qld = ny | 1;
+    qsrc.assign((size_t)r * r, -1);
+    for (size_t s = 0; s < xy.size(); ++s) {
+      const int i1 = xy[s] / ny, i2 = xy[s] % ny;
+      const int h1 = i1 <= pb ? i1 : i1 - (nx - r), h2 = i2 <= pb ? i2 : i2 - (ny - r);
+      qsrc[(size_t)h1 * r + h2] = (int32_t)s;
+      qoff.push_back(h1 * qld + i2);
+    }
+  }
   auto up = [&](DevBuf& d, const void* h, size_t bytes) {
     d.ensure(bytes);
     PWK_HIP(hipMemcpyAsync(d.p, h, bytes, hipMemcpyHostToDevice, c.stream));
@@ -510,6 +507,10 @@ void setup_basis(Context& c, int npw, const int32_t* m) {
   up(c.x1list, x1list.data(), x1list.size() * sizeof(int32_t));
   up(c.pl_src, psrc.data(), psrc.size() * sizeof(int32_t));
   up(c.st_off, off.data(), off.size() * sizeof(int32_t));
+  if (c.quarter) {
+    up(c.q_src, qsrc.data(), qsrc.size() * sizeof(int32_t));
+    up(c.q_off, qoff.data(), qoff.size() * sizeof(int32_t));
+  }
   up(c.st_x1, sx1.data(), sx1.size() * sizeof(int32_t));
   c.sync();  // the host tables go out of scope here
 }

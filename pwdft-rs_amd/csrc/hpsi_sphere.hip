@@ -1,0 +1,274 @@
+// Local part of H·ψ and the z-inverse of the density on spheres within a quarter of the axes
+// (planes.hpp, Quarter): the three passes of hpsi.hip with the transforms pruned at compile time.
+//   z-inverse: the sticks of a workgroup (64) are one contiguous range of ψ, which goes through LDS so
+//              that ψ is read coalesced; a lane transforms one stick.
+//   plane:     SLOTS planes per workgroup in LDS: y-inverse, x-inverse, × V(r), x-forward, y-forward.
+//   z-forward: a lane per stick; Hψ = T_kin ψ + (1/N)·(...) is formed in LDS in place of ψ, so that ψ, the
+//              kinetic energies and Hψ are read and written coalesced.
+// Bounds: the plane pass by vector arithmetic, the z passes by the stick buffer's traffic.
+#include <algorithm>
+
+#include "common.hpp"
+#include "fft_sizes.hpp"
+#include "planes.hpp"
+
+namespace pwk {
+
+namespace {
+
+constexpr int ZS = 64;  // sticks (lanes) per workgroup of the z passes
+
+// the basis range of the workgroup's sticks [s0, s1)
+struct StickRange {
+  int w0, n;
+};
+__device__ __forceinline__ StickRange stick_range(int s0, int s1, const int* __restrict__ st_pw0,
+                                                  const int* __restrict__ st_cnt) {
+  const int w0 = st_pw0[s0];
+  return {w0, st_pw0[s1 - 1] + st_cnt[s1 - 1] - w0};
+}
+
+template <typename V, int U>
+__device__ __forceinline__ void range_to_lds(V* dst, const V* __restrict__ src, int n) {
+  for (int e0 = threadIdx.x; e0 < n; e0 += U * ZS) {
+    V v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) v[u] = src[min(e0 + u * ZS, n - 1)];
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (e0 + u * ZS < n) dst[e0 + u * ZS] = v[u];
+  }
+}
+
+template <typename T, int NZ>
+__global__ void __launch_bounds__(ZS) k_zinv_q(const typename V2t<T>::t* __restrict__ psi,
+                                               typename V2t<T>::t* __restrict__ tbuf, int npw, int S,
+                                               const int* __restrict__ st_pw0, const int* __restrict__ st_cnt,
+                                               const int* __restrict__ st_lo, const int* __restrict__ list) {
+  using V2 = typename V2t<T>::t;
+  using Q = Quarter<NZ>;
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
+  V2* L = reinterpret_cast<V2*>(smem_raw);
+  const int s0 = blockIdx.x * ZS, s1 = min(S, s0 + ZS), b = blockIdx.y;
+  const StickRange rg = stick_range(s0, s1, st_pw0, st_cnt);
+  range_to_lds<V2, 8>(L, psi + (size_t)(list ? list[b] : b) * npw + rg.w0, rg.n);
+  const int s = s0 + threadIdx.x;
+  __syncthreads();
+  if (s >= s1) return;
+  const int cnt = st_cnt[s], lo = st_lo[s], o = st_pw0[s] - rg.w0 - lo;
+  T re[NZ], im[NZ];
+#pragma unroll
+  for (int i3 = 0; i3 < NZ; ++i3) {
+    re[i3] = im[i3] = 0;
+    if (Q::has(i3)) {
+      const int n3 = i3 < Q::PA ? i3 : i3 - NZ, j = n3 - lo;
+      const bool in = j >= 0 && j < cnt;
+      const V2 v = L[in ? o + n3 : 0];
+      re[i3] = in ? v.x : (T)0;
+      im[i3] = in ? v.y : (T)0;
+    }
+  }
+  fft_line<T, NZ, 1>(re, im);
+  V2* dst = tbuf + (size_t)b * NZ * S;  // uniform row pointers, one lane offset
+  const unsigned us = (unsigned)s;
+#pragma unroll
+  for (int f = 0; f < NZ; ++f) {
+    V2 v;
+    v.x = re[LineOrder<NZ>::pos(f)];
+    v.y = im[LineOrder<NZ>::pos(f)];
+    (dst + (size_t)f * S)[us] = v;
+  }
+}
+
+template <typename T, int NZ>
+__global__ void __launch_bounds__(ZS) k_zfwd_q(const typename V2t<T>::t* __restrict__ tbuf,
+                                               const typename V2t<T>::t* __restrict__ psi,
+                                               typename V2t<T>::t* __restrict__ hpsi, const T* __restrict__ kin, int npw,
+                                               int S, const int* __restrict__ st_pw0, const int* __restrict__ st_cnt,
+                                               const int* __restrict__ st_lo, T inv_n, int nbk) {
+  using V2 = typename V2t<T>::t;
+  using Q = Quarter<NZ>;
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
+  V2* L = reinterpret_cast<V2*>(smem_raw);
+  T* K = reinterpret_cast<T*>(L + ZS * (Q::R + 1));
+  const int s0 = blockIdx.x * ZS, s1 = min(S, s0 + ZS), b = blockIdx.y;
+  const StickRange rg = stick_range(s0, s1, st_pw0, st_cnt);
+  const int s = min(s0 + (int)threadIdx.x, s1 - 1);  // lanes past the last stick repeat it and store nothing
+  const V2* src = tbuf + (size_t)b * NZ * S;  // uniform row pointers, one lane offset
+  const unsigned us = (unsigned)s;
+  T re[NZ], im[NZ];
+#pragma unroll
+  for (int i3 = 0; i3 < NZ; ++i3) {
+    const V2 v = (src + (size_t)i3 * S)[us];
+    re[i3] = v.x;
+    im[i3] = v.y;
+  }
+  range_to_lds<V2, 8>(L, psi + (size_t)b * npw + rg.w0, rg.n);
+  range_to_lds<T, 8>(K, kin + (size_t)(b / nbk) * npw + rg.w0, rg.n);  // bands of k-point b / nbk
+  __syncthreads();
+  fft_line<T, NZ, -1>(re, im);
+  // a slot of the line that the stick does not reach goes to a discard element of the lane's own: without
+  // a branch, which would draw the transform's last stages into it and double its registers
+  const int cnt = s0 + (int)threadIdx.x < s1 ? st_cnt[s] : 0, lo = st_lo[s], o = st_pw0[s] - rg.w0 - lo;
+  const int none = ZS * Q::R + threadIdx.x;
+#pragma unroll
+  for (int i3 = 0; i3 < NZ; ++i3) {
+    if (!Q::has(i3)) continue;
+    const int n3 = i3 < Q::PA ? i3 : i3 - NZ, j = n3 - lo;
+    const int e = j >= 0 && j < cnt ? o + n3 : none;
+    const V2 ps = L[e];
+    const T tk = K[e];
+    V2 x;
+    x.x = tk * ps.x + re[LineOrder<NZ>::pos(i3)] * inv_n;
+    x.y = tk * ps.y + im[LineOrder<NZ>::pos(i3)] * inv_n;
+    L[e] = x;
+  }
+  __syncthreads();
+  V2* h = hpsi + (size_t)b * npw + rg.w0;
+  for (int e = threadIdx.x; e < rg.n; e += ZS) h[e] = L[e];
+}
+
+template <typename T, int N>
+__global__ void __launch_bounds__((PlaneShape<T, N>::NT))
+    k_plane_q(typename V2t<T>::t* tbuf, int nb, const T* __restrict__ vr, int S, int nz, const int* __restrict__ src,
+              const int* __restrict__ st_off) {
+  using V2 = typename V2t<T>::t;
+  using Sh = PlaneShape<T, N>;
+  using Q = Quarter<N>;
+  constexpr int NT = Sh::NT, SLOTS = Sh::SLOTS, IMG = Q::R * Q::LD;
+  constexpr int U = 16 / (int)(sizeof(T) / 4);
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
+  V2* P = reinterpret_cast<V2*>(smem_raw);
+  const int i3 = blockIdx.x, b0 = blockIdx.y * SLOTS, nsl = min(SLOTS, nb - b0);
+  const size_t stride = (size_t)nz * S;
+  V2* tp0 = tbuf + (size_t)b0 * stride + (size_t)i3 * S;
+  quarter_fill<T, N, NT, U>(P, tp0, stride, nsl, src);
+  __syncthreads();
+  quarter_ylines<T, N, NT, 1>(P, nsl);
+  __syncthreads();
+  const int slot = threadIdx.x / N, i2 = threadIdx.x - slot * N;
+  if (slot < nsl) {
+    const T* v = vr + (size_t)i3 * N * N;
+    const unsigned ui2 = (unsigned)i2;
+    V2* col = P + slot * IMG + i2;
+    T re[N], im[N];
+    quarter_xline<T, N>(col, re, im);
+    T r2[N], m2[N];
+#pragma unroll
+    for (int f = 0; f < N; ++f) {
+      const T vv = (v + f * N)[ui2];
+      r2[f] = re[LineOrder<N>::pos(f)] * vv;
+      m2[f] = im[LineOrder<N>::pos(f)] * vv;
+    }
+    fft_line<T, N, -1>(r2, m2);
+#pragma unroll
+    for (int f = 0; f < N; ++f)
+      if (Q::has(f)) {
+        V2 x;
+        x.x = r2[LineOrder<N>::pos(f)];
+        x.y = m2[LineOrder<N>::pos(f)];
+        col[Q::at(f) * Q::LD] = x;
+      }
+  }
+  __syncthreads();
+  quarter_ylines<T, N, NT, -1>(P, nsl);
+  __syncthreads();
+  for (int e0 = threadIdx.x; e0 < S; e0 += U * NT) {
+    int off[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) off[u] = st_off[min(e0 + u * NT, S - 1)];
+    for (int p = 0; p < nsl; ++p) {
+      V2* tp = tp0 + (size_t)p * stride;
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (e0 + u * NT < S) tp[e0 + u * NT] = P[p * IMG + off[u]];
+    }
+  }
+}
+
+template <typename T, int N>
+void plane_q(Context& c, typename V2t<T>::t* tbuf, int nb, const T* vr) {
+  using Sh = PlaneShape<T, N>;
+  const size_t sh = (size_t)Sh::SLOTS * Quarter<N>::R * Quarter<N>::LD * sizeof(typename V2t<T>::t);
+  ensure_lds_limit((const void*)k_plane_q<T, N>, sh);
+  k_plane_q<T, N><<<dim3((unsigned)c.dims[2], blocks_for((size_t)nb, Sh::SLOTS)), Sh::NT, sh, c.stream>>>(
+      tbuf, nb, vr, c.nsticks, c.dims[2], c.q_src.as<int>(), c.q_off.as<int>());
+}
+
+template <typename T, int N>
+void zfwd_q(Context& c, const typename V2t<T>::t* tbuf, int nb, const T* kin, int nbk, const void* psi, void* hpsi) {
+  using V2 = typename V2t<T>::t;
+  const size_t sh = (size_t)ZS * (Quarter<N>::R + 1) * (sizeof(V2) + sizeof(T));
+  ensure_lds_limit((const void*)k_zfwd_q<T, N>, sh);
+  k_zfwd_q<T, N><<<dim3(blocks_for((size_t)c.nsticks, ZS), (unsigned)nb), ZS, sh, c.stream>>>(
+      tbuf, (const V2*)psi, (V2*)hpsi, kin, c.npw, c.nsticks, c.st_pw0.as<int>(), c.st_cnt.as<int>(),
+      c.st_n3lo.as<int>(), (T)(1.0 / (double)c.N), nbk);
+}
+
+template <typename T, int N>
+void zinv_q(Context& c, int nb, const void* psi, typename V2t<T>::t* tbuf, const int* list) {
+  using V2 = typename V2t<T>::t;
+  const size_t sh = (size_t)ZS * Quarter<N>::R * sizeof(V2);
+  ensure_lds_limit((const void*)k_zinv_q<T, N>, sh);
+  k_zinv_q<T, N><<<dim3(blocks_for((size_t)c.nsticks, ZS), (unsigned)nb), ZS, sh, c.stream>>>(
+      (const V2*)psi, tbuf, c.npw, c.nsticks, c.st_pw0.as<int>(), c.st_cnt.as<int>(), c.st_n3lo.as<int>(), list);
+}
+
+}  // namespace
+
+template <typename T>
+void sphere_zinv(Context& c, int nb, const void* psi, void* out, const int* list) {
+  auto* tbuf = (typename V2t<T>::t*)out;
+  switch (c.dims[2]) {
+#define PWK_CASE(L) \
+  case L:           \
+    zinv_q<T, L>(c, nb, psi, tbuf, list); \
+    break;
+    PWK_FOR_EACH_FFT_SIZE(PWK_CASE)
+#undef PWK_CASE
+    default:
+      throw Error(PWK_E_UNSUPPORTED, "nz has no compiled kernel");
+  }
+  PWK_HIP(hipGetLastError());
+}
+
+template <typename T>
+void sphere_plane(Context& c, int nb, void* buf, const T* vr) {
+  auto* tbuf = (typename V2t<T>::t*)buf;
+  switch (c.dims[0]) {
+#define PWK_CASE(L) \
+  case L:           \
+    plane_q<T, L>(c, tbuf, nb, vr); \
+    break;
+    PWK_FOR_EACH_FFT_SIZE(PWK_CASE)
+#undef PWK_CASE
+    default:
+      throw Error(PWK_E_UNSUPPORTED, "nx has no compiled kernel");
+  }
+  PWK_HIP(hipGetLastError());
+}
+
+template <typename T>
+void sphere_zfwd(Context& c, int nb, const void* buf, const T* kin, int nbk, const void* psi, void* hpsi) {
+  auto* tbuf = (const typename V2t<T>::t*)buf;
+  switch (c.dims[2]) {
+#define PWK_CASE(L) \
+  case L:           \
+    zfwd_q<T, L>(c, tbuf, nb, kin, nbk, psi, hpsi); \
+    break;
+    PWK_FOR_EACH_FFT_SIZE(PWK_CASE)
+#undef PWK_CASE
+    default:
+      throw Error(PWK_E_UNSUPPORTED, "nz has no compiled kernel");
+  }
+  PWK_HIP(hipGetLastError());
+}
+
+template void sphere_zinv<float>(Context&, int, const void*, void*, const int*);
+template void sphere_zinv<double>(Context&, int, const void*, void*, const int*);
+template void sphere_plane<float>(Context&, int, void*, const float*);
+template void sphere_plane<double>(Context&, int, void*, const double*);
+template void sphere_zfwd<float>(Context&, int, const void*, const float*, int, const void*, void*);
+template void sphere_zfwd<double>(Context&, int, const void*, const double*, int, const void*, void*);
+
+}  // namespace pwk

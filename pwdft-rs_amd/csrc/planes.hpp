@@ -13,6 +13,7 @@
 #pragma once
 
 #include "common.hpp"
+#include "fft_pfa.hpp"
 #include "fft_reg.hpp"
 
 namespace pwk {
@@ -64,7 +65,7 @@ __device__ __forceinline__ int plane_row(const PlaneRows& pr, int j, int absent)
 // fills `nsl` images (stride `image` elements) from the stick rows tp0 + p·band_stride; n elements each
 template <typename T, int N, int NT, int U>
 __device__ __forceinline__ void plane_fill(typename V2t<T>::t* P, int image,
-                                           const typename V2t<T>::t* __restrict__ tp0, size_t band_stride, int nsl,
+                                           const typename V2t<T>::t* tp0, size_t band_stride, int nsl,
                                            const int* __restrict__ src, int n) {
   using V2 = typename V2t<T>::t;
   for (int e0 = threadIdx.x; e0 < n; e0 += U * NT) {
@@ -112,6 +113,86 @@ __device__ __forceinline__ void plane_ylines(typename V2t<T>::t* P, int image, i
       row[f].y = im[FftOrder<N>::pos(f)];
     }
   }
+}
+
+// ---- spheres within a quarter of the axes ------------------------------------------------
+// On a grid of at least 4·max|n| + 1 points per axis (ecutrho = 4·ecutwfc, the default) every index that
+// carries plane waves is i < PA or i >= N - PB. Knowing that at compile time, the line transforms load
+// only those inputs and store only those outputs (the arithmetic on the others drops out), the held rows
+// sit at constant offsets and no zero or discard row is needed.
+template <int N>
+struct Quarter {
+  static constexpr int PB = (N - 1) / 4, PA = PB + 1, R = PA + PB;  // held indices
+  static constexpr int LD = N | 1;                                   // odd row stride: no bank conflicts
+  static constexpr bool has(int i) { return i < PA || i >= N - PB; }
+  static constexpr int at(int i) { return i < PA ? i : i - (N - R); }  // held index -> row of the image
+  __host__ __device__ static constexpr int index(int r) { return r < PA ? r : r + (N - R); }
+};
+
+// fills nsl images of R rows: src[r·R + c] is the stick of held row r and held column c, -1 for zero
+template <typename T, int N, int NT, int U>
+__device__ __forceinline__ void quarter_fill(typename V2t<T>::t* P, const typename V2t<T>::t* tp0, size_t band_stride,
+                                             int nsl, const int* __restrict__ src) {
+  using V2 = typename V2t<T>::t;
+  using Q = Quarter<N>;
+  constexpr int n = Q::R * Q::R;
+  for (int e0 = threadIdx.x; e0 < n; e0 += U * NT) {
+    int s[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) s[u] = src[min(e0 + u * NT, n - 1)];
+    for (int p = 0; p < nsl; ++p) {
+      const V2* tp = tp0 + (size_t)p * band_stride;
+      V2 v[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) v[u] = tp[max(s[u], 0)];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int e = e0 + u * NT;
+        if (e < n) {
+          const int r = e / Q::R, c = e - r * Q::R;
+          V2 x;
+          x.x = s[u] >= 0 ? v[u].x : (T)0;
+          x.y = s[u] >= 0 ? v[u].y : (T)0;
+          P[(p * Q::R + r) * Q::LD + Q::index(c)] = x;
+        }
+      }
+    }
+  }
+}
+
+// y-lines of the held rows: inverse (held columns in, all out) or forward (all in, held columns out)
+template <typename T, int N, int NT, int SIGN>
+__device__ __forceinline__ void quarter_ylines(typename V2t<T>::t* P, int nsl) {
+  using Q = Quarter<N>;
+  for (int t = threadIdx.x; t < nsl * Q::R; t += NT) {
+    typename V2t<T>::t* row = P + t * Q::LD;
+    T re[N], im[N];
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      const bool in = SIGN < 0 || Q::has(j);
+      re[j] = in ? row[j].x : (T)0;
+      im[j] = in ? row[j].y : (T)0;
+    }
+    fft_line<T, N, SIGN>(re, im);
+#pragma unroll
+    for (int f = 0; f < N; ++f)
+      if (SIGN > 0 || Q::has(f)) {
+        row[f].x = re[LineOrder<N>::pos(f)];
+        row[f].y = im[LineOrder<N>::pos(f)];
+      }
+  }
+}
+
+// one x-line (column i2 of an image) from the held rows: inverse transform, frequency f at pos(f)
+template <typename T, int N>
+__device__ __forceinline__ void quarter_xline(const typename V2t<T>::t* col, T (&re)[N], T (&im)[N]) {
+  using Q = Quarter<N>;
+#pragma unroll
+  for (int j = 0; j < N; ++j) {
+    re[j] = Q::has(j) ? col[Q::at(j) * Q::LD].x : (T)0;
+    im[j] = Q::has(j) ? col[Q::at(j) * Q::LD].y : (T)0;
+  }
+  fft_line<T, N, 1>(re, im);
 }
 
 }  // namespace pwk

@@ -36,11 +36,14 @@ def to_grid(psi, idx, dims):
     return np.fft.ifftn(g.reshape((len(psi),) + tuple(dims)), axes=(1, 2, 3)) * np.prod(dims)
 
 
-# (grid, sphere radius): 15 with every row carrying sticks and 16 with all but one, 25 and 27 with
-# several planes per workgroup, 45 and 48 around the register limit of the FP64 sums, 64 and 72 with
-# sums in LDS, 81 the longest line
-PLANES = [((15, 15, 18), 7), ((16, 16, 12), 5), ((25, 25, 25), 6), ((27, 27, 27), 13), ((45, 45, 16), 7),
-          ((48, 48, 9), 4), ((60, 60, 10), 4), ((64, 64, 15), 7), ((72, 72, 8), 3), ((81, 81, 72), 3)]
+# (grid, sphere radius). Bases within a quarter of every axis take the pruned passes, the others the
+# general ones: 15 with every row carrying sticks and 16 with all but one, 25 and 27 with several planes
+# per workgroup, 45 and 48 around the register limit of the FP64 sums, 64 and 72 with sums in LDS, 81 the
+# longest line; radii at the quarter (25/6, 45/11, 60/14) and far below it.
+PLANES = [((15, 15, 18), 7), ((16, 16, 12), 5), ((25, 25, 25), 6), ((27, 27, 27), 13), ((27, 27, 32), 6),
+          ((45, 45, 16), 7), ((45, 45, 45), 11), ((48, 48, 9), 4), ((48, 48, 20), 4), ((60, 60, 10), 4),
+          ((60, 60, 60), 14), ((64, 64, 15), 7), ((64, 64, 30), 7), ((72, 72, 8), 3), ((72, 72, 81), 3),
+          ((81, 81, 72), 3), ((81, 81, 12), 5)]
 
 
 @pytest.mark.parametrize("dims,m", PLANES)
@@ -63,5 +66,28 @@ def test_density_planes(gpu, dims, m, prec, tol):
             assert np.abs(got - ref).max() < tol * np.abs(ref).max()
         psi[:] = np.nan  # bands without weight are not read
         assert np.array_equal(gpu.density(psi, np.zeros(nb), rho0, prec), rho0)
+    finally:
+        gpu.set_fused_hpsi(True)
+
+
+@pytest.mark.parametrize("dims,m", PLANES)
+@pytest.mark.parametrize("prec,tol", [("fp64", 1e-14), ("fp32", 4e-6)])
+def test_hpsi_planes(gpu, dims, m, prec, tol):
+    # tolerance relative to the largest |Hψ|: six line transforms of about 6 roundings each (FP32: 36 ·
+    # 6e-8 = 2.2e-6, FP64 36 · 1.1e-16 = 4e-15)
+    gpu.set_fused_hpsi(False)
+    try:
+        miller, idx = setup(gpu, dims, m)
+        rng = np.random.default_rng(32)
+        n = int(np.prod(dims))
+        v = rng.uniform(-13.6, 13.6, dims)
+        gpu.set_veff((np.fft.fftn(v) / n).reshape(-1))
+        for nb in (1, 2, 5):
+            psi = bands(rng, nb, len(miller))
+            print("hpsi planes", dims, m, prec, "bands", nb, flush=True)
+            got = gpu.hpsi(0, psi, prec)
+            w = np.fft.fftn(to_grid(psi, idx, dims) * v, axes=(1, 2, 3)).reshape(nb, -1)[:, idx] / n
+            ref = w + (miller.astype(float) ** 2).sum(1) * psi
+            assert np.abs(got - ref).max() < tol * np.abs(ref).max()
     finally:
         gpu.set_fused_hpsi(True)
