@@ -347,6 +347,10 @@ struct Context {
   DevBuf kin_pack64, kin_pack32, B_pack64, B_pack32, DBH_pack64, DBH_pack32;
   DevBuf band_tab;                  // int32 k-point per band of the last batch
   std::vector<int32_t> band_tab_host;
+  // k × band batches off the small grids: the kinetic diagonal of each band and the projector products,
+  // as uploaded for the last batch
+  DevBuf batch_tab;
+  std::vector<uint64_t> batch_tab_host;
 
   std::vector<double> dens_host;  // weights and list of the last density's live bands
 
@@ -432,7 +436,8 @@ void sphere_zinv(Context& c, int nb, const void* psi, void* out, const int* list
 template <typename T>
 void sphere_plane(Context& c, int nb, void* buf, const T* vr);
 template <typename T>
-void sphere_zfwd(Context& c, int nb, const void* buf, const T* kin, int nbk, const void* psi, void* hpsi);
+void sphere_zfwd(Context& c, int nb, const void* buf, const T* kin, int nbk, const T* const* kin_of,
+                 const void* psi, void* hpsi);
 // density.hip: the band density on square grids of register-length lines (fw on the host)
 void launch_density_sticks(Context& c, int nb, const void* psi, const double* fw_host, void* rho, int precision,
                            bool overwrite);
@@ -485,6 +490,13 @@ void launch_zgemm_mfma(Context& c, int M, int N, int K, const void* A, int lda, 
 void launch_zgemm_mfma_batched(Context& c, int M, int N, int K, const void* A, int lda, long long sA, const void* B,
                                int ldb, long long sB, void* C, int ldc, long long sC, int batch, bool accumulate,
                                int precision);
+// products with their own A (lda shared) and column count: product g is C[:, col..col+n) (+)= A_g·B[:, col..)
+struct GemmGroup {
+  const void* A;
+  int n, col;
+};
+void launch_zgemm_mfma_groups(Context& c, int M, int Nmax, int K, int ngroups, const GemmGroup* groups /* device */,
+                              int lda, const void* B, int ldb, void* C, int ldc, bool accumulate, int precision);
 // eig.hip: lowest nb eigenpairs of nk Hermitian n×n matrices (H overwritten)
 size_t heev_work_doubles(int n, int nb, int nk);
 bool heev_supported(int n, int nb);

@@ -1,16 +1,17 @@
 // Complex GEMM on the matrix cores, column-major: C (+)= A·B, A M×K, B K×N.
 //
-// The complex product is one real product of the embedded matrices
-//   Ã (2M × 2K): [[Re a, -Im a], [Im a, Re a]] per entry,   B̃ (2K × N) = interleaved B,
-//   C̃ (2M × N) = interleaved C,
-// so B and C keep their interleaved (re, im) storage and only A is expanded,
-// in registers on its way into LDS. Block tile: 64 complex rows × 16·NB16
-// columns, 4 waves, each wave 32 real rows × 16·NB16 columns of 16×16 MFMA
-// blocks. K is staged 16 complex (32 real) at a time.
-//   MODE_F32 : v_mfma_f32_16x16x4_f32
-//   MODE_F64 : v_mfma_f64_16x16x4_f64
+// A wave owns 16 complex rows and all columns of its tile. Its complex product is two real products with
+// the same B operand (interleaved re, im along k): the rows of real parts (re, -im, ...) and the rows of
+// imaginary parts (im, re, ...) of A, so a lane holds the real and the imaginary part of each of its C
+// entries. In a 16×16 MFMA step over 32 real k a lane holds row l mod 16 and the 8 real k of group l / 16,
+// which are 4 whole complex entries of A: a lane loads them from global memory into registers (a wave's
+// load is four runs of 16 consecutive rows) and A never passes through LDS. B, which the four waves of a
+// workgroup share, is staged in LDS (split to bf16 on the way in), double-buffered with one barrier per
+// 16 complex k; the loads of the next steps are in flight during the MFMAs of the current one.
+//   MODE_F32 : v_mfma_f32_16x16x4_f32, 8 steps of 4 real k (lane group g supplies k = 8g + step)
+//   MODE_F64 : v_mfma_f64_16x16x4_f64, likewise
 //   MODE_BF16X3 : v_mfma_f32_16x16x32_bf16 on the split x = hi + lo,
-//                 hi = bf16(x), lo = bf16(x - hi); C += Ahi·Bhi + Ahi·Blo + Alo·Bhi (FP32 accumulate)
+//                 hi = bf16(x), lo = bf16(x - hi); C += Alo·Bhi + Ahi·Blo + Ahi·Bhi (FP32 accumulate)
 // Split-K partial sums are reduced in a fixed order (deterministic).
 #include <algorithm>
 #include <type_traits>
@@ -28,9 +29,8 @@ typedef __bf16 bf8v __attribute__((ext_vector_type(8)));
 enum { MODE_F32 = 0, MODE_F64 = 1, MODE_BF16X3 = 2 };
 
 constexpr int BMC = 64;  // complex rows per block
-constexpr int BMR = 128; // real rows per block
-constexpr int BKC = 16;  // complex K per stage
-constexpr int BKR = 32;  // real K per stage
+constexpr int BKC = 16;  // complex K per step
+constexpr int BKR = 32;  // real K per step
 
 template <int MODE>
 struct Traits {
@@ -47,36 +47,80 @@ struct Traits<MODE_F64> {
 
 __device__ __forceinline__ __bf16 to_bf16(float x) { return (__bf16)x; }
 
-// LDS row strides (elements). A rows keep one padding element (the expanded A tile is written
-// column-wise, rows 33 apart spread the lanes over the banks); FP32 B rows are padded to 36
-// floats so each lane's 8 k values are two aligned 16-byte reads (B is written along k, so
-// its stores stay conflict-free); bf16 rows carry eight.
+// LDS row stride of a B column (elements): its 32 real k, padded so that the 16-byte reads of the 16
+// columns of a fragment fall on distinct banks
 template <int MODE>
-struct Lds {
-  static constexpr int AK = (MODE == MODE_BF16X3) ? BKR + 8 : BKR + 1;                                // A [row][k]
-  static constexpr int BK = (MODE == MODE_BF16X3) ? BKR + 8 : (MODE == MODE_F32 ? BKR + 4 : BKR + 1);  // B [col][k]
+constexpr int b_stride() {
+  return MODE == MODE_BF16X3 ? BKR + 8 : MODE == MODE_F32 ? BKR + 4 : BKR + 2;
+}
+
+// a barrier that waits for LDS traffic only: global loads stay in flight across it
+__device__ __forceinline__ void lds_only_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// the A fragments of one step from a lane's 4 complex entries: [0] real rows, [1] imaginary rows
+template <int MODE>
+struct AFrag {
+  using T = typename Traits<MODE>::T;
+  T v[2][8];
+  __device__ __forceinline__ void make(const typename Traits<MODE>::V2 (&a)[4]) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      v[0][2 * k] = a[k].x;
+      v[0][2 * k + 1] = -a[k].y;
+      v[1][2 * k] = a[k].y;
+      v[1][2 * k + 1] = a[k].x;
+    }
+  }
+};
+template <>
+struct AFrag<MODE_BF16X3> {
+  bf8v hi[2], lo[2];
+  __device__ __forceinline__ void make(const float2 (&a)[4]) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const __bf16 hx = to_bf16(a[k].x), hy = to_bf16(a[k].y);
+      const __bf16 lx = to_bf16(a[k].x - (float)hx), ly = to_bf16(a[k].y - (float)hy);
+      hi[0][2 * k] = hx;
+      hi[0][2 * k + 1] = -hy;
+      hi[1][2 * k] = hy;
+      hi[1][2 * k + 1] = hx;
+      lo[0][2 * k] = lx;
+      lo[0][2 * k + 1] = -ly;
+      lo[1][2 * k] = ly;
+      lo[1][2 * k + 1] = lx;
+    }
+  }
 };
 
 template <int MODE, int NB16>
-__global__ void __launch_bounds__(256) k_zgemm_mfma(int M, int N, int K, int kchunk, int nsplit, long long sA,
+constexpr int gemm_wgs_per_cu() {  // by registers: FP64 tiles wider than 64 columns take more than 256
+  return MODE == MODE_F64 && NB16 > 4 ? 1 : 2;
+}
+
+// Bound: the matrix cores; per step a workgroup issues 4·NB16·{6, 16} MFMAs (split-bf16, FP32/FP64).
+template <int MODE, int NB16>
+__global__ void __launch_bounds__(256, (gemm_wgs_per_cu<MODE, NB16>())) k_zgemm_mfma(int M, int N, int K, int kchunk, int nsplit, long long sA,
                                                     long long sB, long long sC,
                                                     const typename Traits<MODE>::V2* __restrict__ A, int lda,
                                                     const typename Traits<MODE>::V2* __restrict__ B, int ldb,
                                                     typename Traits<MODE>::V2* __restrict__ C, int ldc, int accumulate,
-                                                    typename Traits<MODE>::V2* __restrict__ partial) {
-  using T = typename Traits<MODE>::T;
+                                                    typename Traits<MODE>::V2* __restrict__ partial,
+                                                    const GemmGroup* __restrict__ groups) {
   using V2 = typename Traits<MODE>::V2;
+  using T = typename Traits<MODE>::T;
   using acc_t = typename Traits<MODE>::acc_t;
-  constexpr int BN = 16 * NB16;
-  constexpr int AK = Lds<MODE>::AK, BKS = Lds<MODE>::BK;
+  constexpr int BN = 16 * NB16, BKS = b_stride<MODE>();
   constexpr bool SPLIT = MODE == MODE_BF16X3;
   using ldsT = typename std::conditional<SPLIT, __bf16, T>::type;
   constexpr int NPART = SPLIT ? 2 : 1;
-  __shared__ __attribute__((aligned(16))) ldsT As[NPART][BMR * AK];
-  __shared__ __attribute__((aligned(16))) ldsT Bs[NPART][BN * BKS];
+  __shared__ __attribute__((aligned(16))) ldsT Bs[2][NPART][BN * BKS];
 
   const int tid = threadIdx.x;
-  const int lane = tid & 63, w = tid >> 6;
+  const int lane = tid & 63, w = tid >> 6, li = lane & 15, lk = lane >> 4;
   // One-dimensional grid over (row tile, column tile, batch · nsplit + split). Workgroup i runs on
   // XCD i mod 8, and each XCD takes a contiguous range of tiles in an order where neighbours
   // share an operand in that XCD's L2: with split K, the row and column tiles of one K chunk
@@ -86,233 +130,195 @@ __global__ void __launch_bounds__(256) k_zgemm_mfma(int M, int N, int K, int kch
   const int lg = xcd * (total >> 3) + min(xcd, total & 7) + ((int)blockIdx.x >> 3);
   const int bz = lg / plane, rem = lg % plane;
   const int bx = nsplit > 1 ? rem % mt : rem / nt, by = nsplit > 1 ? rem / mt : rem % nt;
-  const int m0 = bx * BMC, n0 = by * BN;
+  const int m0 = bx * BMC + w * 16, n0 = by * BN;
   // bz = batch · nsplit + split
   const int zb = bz / nsplit, zs = bz % nsplit;
-  A += (size_t)zb * sA;
-  B += (size_t)zb * sB;
-  C += (size_t)zb * sC;
-  if (partial) partial += (size_t)zb * nsplit * M * N;
+  if (partial) partial += (size_t)(zb * nsplit + zs) * M * N;
+  if (groups) {  // products of their own A and column count; N is the widest
+    const GemmGroup gr = groups[zb];
+    A = (const V2*)gr.A;
+    B += (size_t)gr.col * ldb;
+    C += (size_t)gr.col * ldc;
+    N = gr.n;
+    if (n0 >= N) return;
+  } else {
+    A += (size_t)zb * sA;
+    B += (size_t)zb * sB;
+    C += (size_t)zb * sC;
+  }
   const int kbeg = zs * kchunk;
   const int kend = min(K, kbeg + kchunk);
 
-  acc_t acc[2][NB16];
+  acc_t acc[NB16][2];
 #pragma unroll
-  for (int rb = 0; rb < 2; ++rb)
+  for (int cb = 0; cb < NB16; ++cb)
 #pragma unroll
-    for (int cb = 0; cb < NB16; ++cb)
+    for (int h = 0; h < 2; ++h)
 #pragma unroll
-      for (int q = 0; q < 4; ++q) acc[rb][cb][q] = 0;
+      for (int q = 0; q < 4; ++q) acc[cb][h][q] = 0;
 
-  // global -> register prefetch of the next K stage overlaps the MFMA work of the current one
-  constexpr int NA = (BMC * BKC) / 256, NBV = (BKC * BN + 255) / 256;
-  V2 ra[NA], rbv[NBV];
-  auto gload = [&](int k0) {
+  // Rows and columns past the matrix repeat its last one (never stored); k past the chunk is zero in A and B.
+  const V2* a_row = A + min(m0 + li, M - 1);
+  constexpr int NBV = (BKC * BN + 255) / 256;
+  V2 ra[2][4], rb[2][NBV];
+  const int kk = tid & (BKC - 1);  // this thread's k within a step of B, for every column it loads
+  const V2* b_col[NBV];
 #pragma unroll
-    for (int e = 0; e < NA; ++e) {
-      const int idx = tid + 256 * e;
-      const int mm = idx & (BMC - 1), kk = idx / BMC;
-      const int gm = m0 + mm, gk = k0 + kk;
-      V2 v;
-      v.x = 0;
-      v.y = 0;
-      if (gm < M && gk < kend) v = A[(size_t)gk * lda + gm];
-      ra[e] = v;
-    }
+  for (int e = 0; e < NBV; ++e) b_col[e] = B + (size_t)min(n0 + min(tid / BKC + 16 * e, BN - 1), N - 1) * ldb;
+  auto load_a = [&](V2(&r)[4], int k0) {
 #pragma unroll
-    for (int e = 0; e < NBV; ++e) {
-      const int idx = tid + 256 * e;
-      V2 v;
-      v.x = 0;
-      v.y = 0;
-      if (idx < BKC * BN) {
-        const int kk = idx % BKC, nn = idx / BKC;
-        const int gk = k0 + kk, gn = n0 + nn;
-        if (gn < N && gk < kend) v = B[(size_t)gn * ldb + gk];
-      }
-      rbv[e] = v;
-    }
+    for (int i = 0; i < 4; ++i) r[i] = a_row[(size_t)min(k0 + 4 * lk + i, kend - 1) * lda];
   };
-  // A tile: 64 complex rows × 16 complex k, expanded to 128 × 32 real; B tile: 16 complex k ×
-  // BN columns, interleaved -> [col][2k+part]
-  auto lstore = [&]() {
+  auto load_b = [&](V2(&r)[NBV], int k0) {
+    const int k = min(k0 + kk, kend - 1);
 #pragma unroll
-    for (int e = 0; e < NA; ++e) {
-      const int idx = tid + 256 * e;
-      const int mm = idx & (BMC - 1), kk = idx / BMC;
-      const V2 v = ra[e];
-      T vals[4] = {v.x, -v.y, v.y, v.x};  // (2m,2k) (2m,2k+1) (2m+1,2k) (2m+1,2k+1)
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        const int r = 2 * mm + (t >> 1), c = 2 * kk + (t & 1);
-        if constexpr (SPLIT) {
-          __bf16 hi = to_bf16(vals[t]);
-          As[0][r * AK + c] = hi;
-          As[1][r * AK + c] = to_bf16(vals[t] - (float)hi);
-        } else {
-          As[0][r * AK + c] = vals[t];
-        }
-      }
-    }
+    for (int e = 0; e < NBV; ++e) r[e] = b_col[e][k];
+  };
+  auto store_b = [&](const V2(&r)[NBV], int buf, int k0) {
+    const bool in = k0 + kk < kend;
 #pragma unroll
     for (int e = 0; e < NBV; ++e) {
-      const int idx = tid + 256 * e;
-      if (idx < BKC * BN) {
-        const int kk = idx % BKC, nn = idx / BKC;
-        const V2 v = rbv[e];
+      const int nn = tid / BKC + 16 * e;
+      {
+        const T x = in ? r[e].x : (T)0, y = in ? r[e].y : (T)0;
+        ldsT* p = &Bs[buf][0][nn * BKS + 2 * kk];
         if constexpr (SPLIT) {
-          __bf16 hx = to_bf16(v.x), hy = to_bf16(v.y);
-          Bs[0][nn * BKS + 2 * kk] = hx;
-          Bs[0][nn * BKS + 2 * kk + 1] = hy;
-          Bs[1][nn * BKS + 2 * kk] = to_bf16(v.x - (float)hx);
-          Bs[1][nn * BKS + 2 * kk + 1] = to_bf16(v.y - (float)hy);
+          const __bf16 hx = to_bf16(x), hy = to_bf16(y);
+          p[0] = hx;
+          p[1] = hy;
+          ldsT* q = &Bs[buf][1][nn * BKS + 2 * kk];
+          q[0] = to_bf16(x - (float)hx);
+          q[1] = to_bf16(y - (float)hy);
         } else {
-          Bs[0][nn * BKS + 2 * kk] = v.x;
-          Bs[0][nn * BKS + 2 * kk + 1] = v.y;
+          p[0] = x;
+          p[1] = y;
         }
       }
     }
   };
-  if (kbeg < kend) gload(kbeg);
-  for (int k0 = kbeg; k0 < kend; k0 += BKC) {
-    lstore();
-    __syncthreads();
-    if (k0 + BKC < kend) gload(k0 + BKC);
-    const int li = lane & 15, lk = lane >> 4;
-    if constexpr (SPLIT) {
-      // one 16x16x32 step covers the 32 real k of the stage; lane holds k = lk*8 .. lk*8+7
+  auto step = [&](V2(&a)[4], V2(&b)[NBV], int k0, int buf) {
+    if (k0 + BKC > kend) {  // the chunk's last, shorter step
 #pragma unroll
-      for (int rb = 0; rb < 2; ++rb) {
-        const int row = w * 32 + rb * 16 + li;
-        bf8v ahi = *reinterpret_cast<const bf8v*>(&As[0][row * AK + lk * 8]);
-        bf8v alo = *reinterpret_cast<const bf8v*>(&As[1][row * AK + lk * 8]);
-#pragma unroll
-        for (int cb = 0; cb < NB16; ++cb) {
-          const int col = cb * 16 + li;
-          bf8v bhi = *reinterpret_cast<const bf8v*>(&Bs[0][col * BKS + lk * 8]);
-          bf8v blo = *reinterpret_cast<const bf8v*>(&Bs[1][col * BKS + lk * 8]);
-          acc[rb][cb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(alo, bhi, acc[rb][cb], 0, 0, 0);
-          acc[rb][cb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ahi, blo, acc[rb][cb], 0, 0, 0);
-          acc[rb][cb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ahi, bhi, acc[rb][cb], 0, 0, 0);
-        }
-      }
-    } else if constexpr (MODE == MODE_F32) {
-      // 8 MFMA k-steps; in step ks lane group lk supplies real k = lk*8 + ks (the sum over the
-      // stage's 32 k values is split differently from the natural order, A and B alike), so
-      // each lane reads its 8 k values of a B column with two 16-byte LDS reads
-      f4v b[NB16][2];
-#pragma unroll
-      for (int cb = 0; cb < NB16; ++cb) {
-        const float* p = &Bs[0][(cb * 16 + li) * BKS + lk * 8];
-        b[cb][0] = *reinterpret_cast<const f4v*>(p);
-        b[cb][1] = *reinterpret_cast<const f4v*>(p + 4);
-      }
-      float a[2][8];
-#pragma unroll
-      for (int rb = 0; rb < 2; ++rb)
-#pragma unroll
-        for (int ks = 0; ks < 8; ++ks) a[rb][ks] = As[0][(w * 32 + rb * 16 + li) * AK + lk * 8 + ks];
-#pragma unroll
-      for (int ks = 0; ks < 8; ++ks) {
-#pragma unroll
-        for (int cb = 0; cb < NB16; ++cb)
-#pragma unroll
-          for (int rb = 0; rb < 2; ++rb)
-            acc[rb][cb] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[rb][ks], b[cb][ks >> 2][ks & 3], acc[rb][cb], 0, 0, 0);
-      }
-    } else {
-#pragma unroll
-      for (int ks = 0; ks < BKR / 4; ++ks) {
-        const int kk = ks * 4 + lk;
-        T a[2];
-#pragma unroll
-        for (int rb = 0; rb < 2; ++rb) a[rb] = As[0][(w * 32 + rb * 16 + li) * AK + kk];
-#pragma unroll
-        for (int cb = 0; cb < NB16; ++cb) {
-          T b = Bs[0][(cb * 16 + li) * BKS + kk];
-#pragma unroll
-          for (int rb = 0; rb < 2; ++rb) acc[rb][cb] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[rb], b, acc[rb][cb], 0, 0, 0);
-        }
-      }
+      for (int i = 0; i < 4; ++i)
+        if (k0 + 4 * lk + i >= kend) a[i].x = a[i].y = 0;
     }
-    __syncthreads();
-  }
-  const int li = lane & 15, lq = lane >> 4;
-  if constexpr (MODE == MODE_F64) {
-    // f64 16x16x4 result layout (measured on gfx950): lane holds real rows lane/16 + 4q,
-    // column lane%16, so a lane holds only real or only imaginary rows; the imaginary
-    // partner of lane l is lane l+16.
+    AFrag<MODE> f;
+    f.make(a);
+    store_b(b, buf, k0);
+    // the loads of the step after next, unconditionally (clamped), so that the waits count them exactly
+    load_b(b, k0 + 2 * BKC);
+    load_a(a, k0 + 2 * BKC);
+    lds_only_barrier();
+    // columns in groups of up to three: enough independent MFMA chains to hide their latency
+    constexpr int G = NB16 % 3 == 0 ? 3 : NB16 % 2 == 0 ? 2 : NB16 == 1 ? 1 : NB16 == 5 ? 5 : 7;
 #pragma unroll
-    for (int rb = 0; rb < 2; ++rb)
+    for (int g = 0; g < NB16; g += G) {
+      if constexpr (SPLIT) {
+        bf8v bhi[G], blo[G];
 #pragma unroll
-      for (int cb = 0; cb < NB16; ++cb) {
-        double partner[4];
+        for (int c = 0; c < G; ++c) {
+          const int o = ((g + c) * 16 + li) * BKS + lk * 8;
+          bhi[c] = *reinterpret_cast<const bf8v*>(&Bs[buf][0][o]);
+          blo[c] = *reinterpret_cast<const bf8v*>(&Bs[buf][1][o]);
+        }
 #pragma unroll
-        for (int q = 0; q < 4; ++q) partner[q] = __shfl_down(acc[rb][cb][q], 16, 64);
-        const int gn = n0 + cb * 16 + li;
-        if ((lq & 1) != 0 || gn >= N) continue;
+        for (int c = 0; c < G; ++c)
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const int gm = m0 + (w * 32 + rb * 16 + lq + 4 * q) / 2;
-          if (gm >= M) continue;
-          V2 o;
-          o.x = acc[rb][cb][q];
-          o.y = partner[q];
-          if (partial) {
-            partial[((size_t)zs * N + gn) * M + gm] = o;
-          } else {
-            V2* c = &C[(size_t)gn * ldc + gm];
-            if (accumulate) {
-              V2 old = *c;
-              o.x += old.x;
-              o.y += old.y;
+          for (int h = 0; h < 2; ++h)
+            acc[g + c][h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f.lo[h], bhi[c], acc[g + c][h], 0, 0, 0);
+#pragma unroll
+        for (int c = 0; c < G; ++c)
+#pragma unroll
+          for (int h = 0; h < 2; ++h)
+            acc[g + c][h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f.hi[h], blo[c], acc[g + c][h], 0, 0, 0);
+#pragma unroll
+        for (int c = 0; c < G; ++c)
+#pragma unroll
+          for (int h = 0; h < 2; ++h)
+            acc[g + c][h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f.hi[h], bhi[c], acc[g + c][h], 0, 0, 0);
+      } else {
+        typedef T v16 __attribute__((ext_vector_type(16 / sizeof(T))));  // 16-byte LDS reads
+        constexpr int V = 16 / (int)sizeof(T);
+        T bv[G][8];
+#pragma unroll
+        for (int c = 0; c < G; ++c)
+#pragma unroll
+          for (int i = 0; i < 8; i += V) {
+            const v16 x = *reinterpret_cast<const v16*>(&Bs[buf][0][((g + c) * 16 + li) * BKS + lk * 8 + i]);
+#pragma unroll
+            for (int j = 0; j < V; ++j) bv[c][i + j] = x[j];
+          }
+#pragma unroll
+        for (int ks = 0; ks < 8; ++ks)
+#pragma unroll
+          for (int c = 0; c < G; ++c)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+              if constexpr (MODE == MODE_F32)
+                acc[g + c][h] = __builtin_amdgcn_mfma_f32_16x16x4f32(f.v[h][ks], bv[c][ks], acc[g + c][h], 0, 0, 0);
+              else
+                acc[g + c][h] = __builtin_amdgcn_mfma_f64_16x16x4f64(f.v[h][ks], bv[c][ks], acc[g + c][h], 0, 0, 0);
             }
-            *c = o;
-          }
-        }
-      }
-    return;
-  }
-  // ---- store: lane holds real rows 4*(lane/16)+q of each 16×16 block, column lane%16
-#pragma unroll
-  for (int rb = 0; rb < 2; ++rb)
-#pragma unroll
-    for (int cb = 0; cb < NB16; ++cb) {
-      const int gn = n0 + cb * 16 + li;
-      if (gn >= N) continue;
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const int gm = m0 + (w * 32 + rb * 16) / 2 + 2 * lq + h;
-        if (gm >= M) continue;
-        V2 o;
-        o.x = acc[rb][cb][2 * h];
-        o.y = acc[rb][cb][2 * h + 1];
-        if (partial) {
-          partial[((size_t)zs * N + gn) * M + gm] = o;
-        } else {
-          V2* c = &C[(size_t)gn * ldc + gm];
-          if (accumulate) {
-            V2 old = *c;
-            o.x += old.x;
-            o.y += old.y;
-          }
-          *c = o;
-        }
       }
     }
+  };
+  if (kbeg < kend) {
+    load_b(rb[0], kbeg);
+    load_a(ra[0], kbeg);
+    load_b(rb[1], kbeg + BKC);
+    load_a(ra[1], kbeg + BKC);
+    // two steps per turn: the registers and the LDS buffers alternate at constant indices (a step past
+    // the chunk adds zeros)
+    for (int k0 = kbeg; k0 < kend; k0 += 2 * BKC) {
+      step(ra[0], rb[0], k0, 0);
+      step(ra[1], rb[1], k0 + BKC, 1);
+    }
+  }
+  // Store. Result rows of a lane: 4·(l/16) + q, or l/16 + 4q in FP64 (measured on gfx950); column l mod 16.
+#pragma unroll
+  for (int cb = 0; cb < NB16; ++cb) {
+    const int gn = n0 + cb * 16 + li;
+    if (gn >= N) continue;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int gm = m0 + (MODE == MODE_F64 ? lk + 4 * q : 4 * lk + q);
+      if (gm >= M) continue;
+      V2 o;
+      o.x = acc[cb][0][q];
+      o.y = acc[cb][1][q];
+      if (partial) {
+        partial[(size_t)gn * M + gm] = o;
+      } else {
+        V2* c = &C[(size_t)gn * ldc + gm];
+        if (accumulate) {
+          const V2 old = *c;
+          o.x += old.x;
+          o.y += old.y;
+        }
+        *c = o;
+      }
+    }
+  }
 }
 
 template <typename V2>
 __global__ void __launch_bounds__(256) k_splitk_sum(int M, int N, int nsplit, const V2* __restrict__ partial,
-                                                    V2* __restrict__ C, int ldc, long long sC, int accumulate) {
+                                                    V2* __restrict__ C, int ldc, long long sC, int accumulate,
+                                                    const GemmGroup* __restrict__ groups) {
   size_t idx = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (idx >= (size_t)M * N) return;
   partial += (size_t)blockIdx.y * nsplit * M * N;
-  C += (size_t)blockIdx.y * sC;
   int gm = (int)(idx % M), gn = (int)(idx / M);
+  if (groups) {
+    if (gn >= groups[blockIdx.y].n) return;
+    C += (size_t)groups[blockIdx.y].col * ldc;
+  } else {
+    C += (size_t)blockIdx.y * sC;
+  }
   V2 s;
   s.x = 0;
   s.y = 0;
+#pragma unroll 8
   for (int z = 0; z < nsplit; ++z) {
     V2 p = partial[(size_t)z * M * N + idx];
     s.x += p.x;
@@ -330,6 +336,7 @@ __global__ void __launch_bounds__(256) k_splitk_sum(int M, int N, int nsplit, co
 struct Batch {
   int count = 1;
   long long sA = 0, sB = 0, sC = 0;  // element strides between consecutive products
+  const GemmGroup* groups = nullptr;  // device; instead of the strides
 };
 
 template <int MODE, int NB16>
@@ -337,7 +344,7 @@ void launch_nb(Context& c, dim3 grid, int M, int N, int K, int kchunk, int nspli
                int lda, const void* B, int ldb, void* C, int ldc, int acc, void* part) {
   using V2 = typename Traits<MODE>::V2;
   k_zgemm_mfma<MODE, NB16><<<grid, 256, 0, c.stream>>>(M, N, K, kchunk, nsplit, bt.sA, bt.sB, bt.sC, (const V2*)A,
-                                                        lda, (const V2*)B, ldb, (V2*)C, ldc, acc, (V2*)part);
+                                                        lda, (const V2*)B, ldb, (V2*)C, ldc, acc, (V2*)part, bt.groups);
 }
 
 template <int MODE>
@@ -345,24 +352,33 @@ void zgemm_mfma_t(Context& c, int M, int N, int K, const void* A, int lda, const
                   bool accumulate, const Batch& bt) {
   using V2 = typename Traits<MODE>::V2;
   const int cus = c.cu_count > 0 ? c.cu_count : 256;
-  int nb16 = std::min(9, (N + 15) / 16);
-  int mt = (M + BMC - 1) / BMC;
-  // fewer tiles than CUs with wide column blocks: halve the block width so that every CU gets
-  // work (the A tile is then read by two column blocks)
-  if ((long)mt * ((N + 16 * nb16 - 1) / (16 * nb16)) * bt.count < cus && nb16 > 4 && (long)mt * bt.count >= cus / 4)
-    nb16 = (nb16 + 1) / 2;
-  int BN = 16 * nb16;
-  int nt = (N + BN - 1) / BN;
-  long tiles = (long)mt * nt * bt.count;
-  int target = 2 * cus;
+  // Column blocks of equal width, at most 144 columns. Among the widths the one whose tiles, dealt to the
+  // CUs, take the fewest MFMA steps on the busiest CU; 1.5 blocks of 16 columns stand for what a tile
+  // costs besides them (loading and converting A): C64 expansion, 108 row tiles × 160 columns in FP64, runs
+  // 216 tiles of 80 columns instead of 432 of 48.
+  const int n16 = (N + 15) / 16, mt = (M + BMC - 1) / BMC;
+  int nb16 = (n16 + (n16 + 8) / 9 - 1) / ((n16 + 8) / 9);
+  auto tiles_of = [&](int w) { return (long)mt * ((n16 + w - 1) / w) * bt.count; };
+  auto cost = [&](int w) { return (double)((tiles_of(w) + cus - 1) / cus) * (w + 1.5); };
+  const bool split = tiles_of(nb16) < cus / 2 && K >= 16 * BKC;
+  if (!split) {
+    int best = nb16;
+    for (int w = nb16; w >= 1; --w)
+      if (cost(w) < cost(best)) best = w;
+    nb16 = best;
+  }
+  const int BN = 16 * nb16, nt = (N + BN - 1) / BN;
+  const long tiles = tiles_of(nb16);
   int nsplit = 1;
   // split K only for K >= 256 (short reductions are cheaper than the extra partial-sum pass) and
   // when the tiles fill less than half the CUs (above that the partial-sum round trip costs
-  // more than the idle CUs), then into chunks of at least 4 stages
-  if (tiles < target / 4 && K >= 16 * BKC)
-    nsplit = (int)std::min<long>((target + tiles - 1) / tiles, std::max(1, K / (4 * BKC)));
+  // more than the idle CUs), into chunks of at least 4 steps and no more workgroups than run at once
+  if (split) {
+    const int per_cu = MODE == MODE_F64 && nb16 > 4 ? 1 : 2;
+    nsplit = (int)std::min<long>(std::max<long>(1, cus * per_cu / tiles), std::max(1, K / (4 * BKC)));
+  }
   int kchunk = (K + nsplit - 1) / nsplit;
-  kchunk = ((kchunk + BKC - 1) / BKC) * BKC;
+  kchunk = ((kchunk + 2 * BKC - 1) / (2 * BKC)) * (2 * BKC);
   nsplit = (K + kchunk - 1) / kchunk;
   PWK_REQUIRE((long)nsplit * bt.count <= 65535, PWK_E_UNSUPPORTED, "GEMM batch too large");
   PWK_REQUIRE((long)mt * nt * nsplit * bt.count <= 0x7fffffffL, PWK_E_UNSUPPORTED, "GEMM grid too large");
@@ -384,7 +400,7 @@ void zgemm_mfma_t(Context& c, int M, int N, int K, const void* A, int lda, const
   if (nsplit > 1) {
     dim3 g(blocks_for((size_t)M * N, 256), (unsigned)bt.count);
     k_splitk_sum<V2><<<g, 256, 0, c.stream>>>(M, N, nsplit, (const V2*)part, (V2*)C, ldc, bt.sC,
-                                              accumulate ? 1 : 0);
+                                              accumulate ? 1 : 0, bt.groups);
     PWK_HIP(hipGetLastError());
   }
 }
@@ -415,6 +431,20 @@ void launch_zgemm_mfma_batched(Context& c, int M, int N, int K, const void* A, i
     zgemm_mfma_t<MODE_BF16X3>(c, M, N, K, A, lda, B, ldb, C, ldc, accumulate, bt);
   else
     zgemm_mfma_t<MODE_F32>(c, M, N, K, A, lda, B, ldb, C, ldc, accumulate, bt);
+}
+
+void launch_zgemm_mfma_groups(Context& c, int M, int Nmax, int K, int ngroups, const GemmGroup* groups, int lda,
+                              const void* B, int ldb, void* C, int ldc, bool accumulate, int precision) {
+  if (M <= 0 || Nmax <= 0 || K <= 0 || ngroups <= 0) return;
+  Batch bt;
+  bt.count = ngroups;
+  bt.groups = groups;
+  if (precision == PWK_FP64)
+    zgemm_mfma_t<MODE_F64>(c, M, Nmax, K, nullptr, lda, B, ldb, C, ldc, accumulate, bt);
+  else if (precision == PWK_SPLIT_BF16)
+    zgemm_mfma_t<MODE_BF16X3>(c, M, Nmax, K, nullptr, lda, B, ldb, C, ldc, accumulate, bt);
+  else
+    zgemm_mfma_t<MODE_F32>(c, M, Nmax, K, nullptr, lda, B, ldb, C, ldc, accumulate, bt);
 }
 
 }  // namespace pwk

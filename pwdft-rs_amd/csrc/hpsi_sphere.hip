@@ -85,7 +85,8 @@ __global__ void __launch_bounds__(ZS) k_zfwd_q(const typename V2t<T>::t* __restr
                                                const typename V2t<T>::t* __restrict__ psi,
                                                typename V2t<T>::t* __restrict__ hpsi, const T* __restrict__ kin, int npw,
                                                int S, const int* __restrict__ st_pw0, const int* __restrict__ st_cnt,
-                                               const int* __restrict__ st_lo, T inv_n, int nbk) {
+                                               const int* __restrict__ st_lo, T inv_n, int nbk,
+                                               const T* const* __restrict__ kin_of) {
   using V2 = typename V2t<T>::t;
   using Q = Quarter<NZ>;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
@@ -104,7 +105,8 @@ __global__ void __launch_bounds__(ZS) k_zfwd_q(const typename V2t<T>::t* __restr
     im[i3] = v.y;
   }
   range_to_lds<V2, 8>(L, psi + (size_t)b * npw + rg.w0, rg.n);
-  range_to_lds<T, 8>(K, kin + (size_t)(b / nbk) * npw + rg.w0, rg.n);  // bands of k-point b / nbk
+  // the band's kinetic diagonal: of its own (k × band batches) or of k-point b / nbk
+  range_to_lds<T, 8>(K, (kin_of ? kin_of[b] : kin + (size_t)(b / nbk) * npw) + rg.w0, rg.n);
   __syncthreads();
   fft_line<T, NZ, -1>(re, im);
   // a slot of the line that the stick does not reach goes to a discard element of the lane's own: without
@@ -196,13 +198,14 @@ void plane_q(Context& c, typename V2t<T>::t* tbuf, int nb, const T* vr) {
 }
 
 template <typename T, int N>
-void zfwd_q(Context& c, const typename V2t<T>::t* tbuf, int nb, const T* kin, int nbk, const void* psi, void* hpsi) {
+void zfwd_q(Context& c, const typename V2t<T>::t* tbuf, int nb, const T* kin, int nbk, const T* const* kin_of,
+            const void* psi, void* hpsi) {
   using V2 = typename V2t<T>::t;
   const size_t sh = (size_t)ZS * (Quarter<N>::R + 1) * (sizeof(V2) + sizeof(T));
   ensure_lds_limit((const void*)k_zfwd_q<T, N>, sh);
   k_zfwd_q<T, N><<<dim3(blocks_for((size_t)c.nsticks, ZS), (unsigned)nb), ZS, sh, c.stream>>>(
       tbuf, (const V2*)psi, (V2*)hpsi, kin, c.npw, c.nsticks, c.st_pw0.as<int>(), c.st_cnt.as<int>(),
-      c.st_n3lo.as<int>(), (T)(1.0 / (double)c.N), nbk);
+      c.st_n3lo.as<int>(), (T)(1.0 / (double)c.N), nbk, kin_of);
 }
 
 template <typename T, int N>
@@ -249,12 +252,13 @@ void sphere_plane(Context& c, int nb, void* buf, const T* vr) {
 }
 
 template <typename T>
-void sphere_zfwd(Context& c, int nb, const void* buf, const T* kin, int nbk, const void* psi, void* hpsi) {
+void sphere_zfwd(Context& c, int nb, const void* buf, const T* kin, int nbk, const T* const* kin_of,
+                 const void* psi, void* hpsi) {
   auto* tbuf = (const typename V2t<T>::t*)buf;
   switch (c.dims[2]) {
 #define PWK_CASE(L) \
   case L:           \
-    zfwd_q<T, L>(c, tbuf, nb, kin, nbk, psi, hpsi); \
+    zfwd_q<T, L>(c, tbuf, nb, kin, nbk, kin_of, psi, hpsi); \
     break;
     PWK_FOR_EACH_FFT_SIZE(PWK_CASE)
 #undef PWK_CASE
@@ -268,7 +272,8 @@ template void sphere_zinv<float>(Context&, int, const void*, void*, const int*);
 template void sphere_zinv<double>(Context&, int, const void*, void*, const int*);
 template void sphere_plane<float>(Context&, int, void*, const float*);
 template void sphere_plane<double>(Context&, int, void*, const double*);
-template void sphere_zfwd<float>(Context&, int, const void*, const float*, int, const void*, void*);
-template void sphere_zfwd<double>(Context&, int, const void*, const double*, int, const void*, void*);
+template void sphere_zfwd<float>(Context&, int, const void*, const float*, int, const float* const*, const void*, void*);
+template void sphere_zfwd<double>(Context&, int, const void*, const double*, int, const double* const*, const void*,
+                                  void*);
 
 }  // namespace pwk

@@ -91,3 +91,66 @@ def test_hpsi_planes(gpu, dims, m, prec, tol):
             assert np.abs(got - ref).max() < tol * np.abs(ref).max()
     finally:
         gpu.set_fused_hpsi(True)
+
+
+@pytest.mark.parametrize("dims,m", [((25, 25, 25), 6), ((27, 27, 27), 9)])
+@pytest.mark.parametrize("prec,tol", [("fp64", 1e-13), ("fp32", 6e-6), ("split_bf16", 2e-5)])
+@pytest.mark.parametrize("channels,counts", [((7, 7, 7), (3, 1, 18)), ((80, 80), (33, 161)), ((5, 0, 5), (2, 2, 2))])
+def test_hpsi_batch_sticks(gpu, dims, m, prec, tol, channels, counts):
+    # k × band batches off the small grids: one launch per pass and grouped projector products when the
+    # entries share a channel count, entry by entry otherwise. Tolerance relative to the largest |Hψ|:
+    # the transforms as above plus sums over npw (projection) and nch terms, √npw ≈ 60 roundings
+    # (FP32 3.6e-6, split-bf16 2^-16 per product: 1.5e-5)
+    miller, idx = setup(gpu, dims, m)
+    npw, n = len(miller), int(np.prod(dims))
+    rng = np.random.default_rng(33)
+    v = rng.uniform(-13.6, 13.6, dims)
+    gpu.set_veff((np.fft.fftn(v) / n).reshape(-1))
+    gpu.set_nk(len(channels))
+    kin, proj = [], []
+    for ik, nch in enumerate(channels):
+        kin.append((miller.astype(float) ** 2).sum(1) * (1 + 0.1 * ik))
+        gpu.set_kinetic(ik, kin[-1])
+        b = (rng.standard_normal((npw, nch)) + 1j * rng.standard_normal((npw, nch))) / np.sqrt(npw)
+        d = rng.standard_normal((nch, npw)) + 1j * rng.standard_normal((nch, npw))
+        proj.append((b, d))
+        gpu.set_nonlocal(ik, b, d)
+    order = list(range(len(channels)))[::-1]  # entries in another order than the k-points
+    nbands = [counts[i] for i in order]
+    psi = bands(rng, sum(nbands), npw)
+    print("hpsi batch", dims, prec, channels, nbands, flush=True)
+    for _ in range(2):  # the second call reuses the tables of the first
+        got = gpu.hpsi_batch(order, nbands, psi, prec)
+    w = np.fft.fftn(to_grid(psi, idx, dims) * v, axes=(1, 2, 3)).reshape(len(psi), -1)[:, idx] / n
+    b0 = 0
+    for ik, nb in zip(order, nbands):
+        p = psi[b0:b0 + nb]
+        w[b0:b0 + nb] += kin[ik] * p + (proj[ik][0] @ (proj[ik][1] @ p.T)).T
+        b0 += nb
+    assert np.abs(got - w).max() < tol * np.abs(w).max()
+    # fewer entries next: the tables change
+    got = gpu.hpsi_batch(order[:1], nbands[:1], psi[:nbands[0]], prec)
+    assert np.abs(got - w[:nbands[0]]).max() < tol * np.abs(w).max()
+
+
+@pytest.mark.parametrize("prec,tol", [("fp64", 1e-13), ("fp32", 2e-5), ("split_bf16", 5e-5)])
+def test_zgemm_column_blocks(gpu, prec, tol):
+    # column counts around one and two blocks of 144, row counts that make few and many tiles, reductions
+    # around the two-step turn of the main loop and around the split-K chunk
+    import torch
+
+    rng = np.random.default_rng(34)
+    dt = torch.complex128 if prec == "fp64" else torch.complex64
+    for (m, n, k) in [(63, 143, 31), (65, 160, 33), (1, 161, 17), (256, 160, 1000), (3000, 80, 48), (512, 144, 2001),
+                      (130, 289, 255), (16, 16, 257)]:
+        A = rng.standard_normal((m, k)) + 1j * rng.standard_normal((m, k))
+        B = rng.standard_normal((k, n)) + 1j * rng.standard_normal((k, n))
+        dA, dB = (torch.from_numpy(np.ascontiguousarray(x.T)).to(dt).cuda() for x in (A, B))
+        dC = torch.full((n, m), float("nan"), dtype=dt).cuda()
+        torch.cuda.synchronize()
+        gpu.zgemm_dev(m, n, k, dA.data_ptr(), m, dB.data_ptr(), k, dC.data_ptr(), m, precision=prec)
+        gpu.sync()
+        ref = A @ B
+        err = np.abs(dC.cpu().numpy().T - ref).max() / np.abs(ref).max()
+        print("zgemm", prec, (m, n, k), f"{err:.2e}", flush=True)
+        assert err < tol, (m, n, k)
