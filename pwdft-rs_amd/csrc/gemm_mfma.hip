@@ -96,14 +96,18 @@ struct AFrag<MODE_BF16X3> {
   }
 };
 
-template <int MODE, int NB16>
-constexpr int gemm_wgs_per_cu() {  // by registers: FP64 tiles wider than 64 columns take more than 256
-  return MODE == MODE_F64 && NB16 > 4 ? 1 : 2;
-}
+// Widest column tile (blocks of 16) and workgroups per CU that split K aims at. Two or three narrow tiles
+// per CU hide each other's loads, conversions and barriers better than one wide tile, and A re-read by the
+// column tiles comes from L2: Si64 split-bf16 512 × 144 × 13133, 3 blocks and 32 chunks 46 us, 9 blocks 53-60;
+// 13133 × 144 × 512 47 against 58; FP64 256 × 160 × 6859, 2 blocks 51 us, 5 blocks 57.
+template <int MODE>
+struct Tile {
+  static constexpr int W = MODE == MODE_F64 ? 2 : 3, PER_CU = MODE == MODE_F64 ? 2 : 3;
+};
 
 // Bound: the matrix cores; per step a workgroup issues 4·NB16·{6, 16} MFMAs (split-bf16, FP32/FP64).
 template <int MODE, int NB16>
-__global__ void __launch_bounds__(256, (gemm_wgs_per_cu<MODE, NB16>())) k_zgemm_mfma(int M, int N, int K, int kchunk, int nsplit, long long sA,
+__global__ void __launch_bounds__(256, 2) k_zgemm_mfma(int M, int N, int K, int kchunk, int nsplit, long long sA,
                                                     long long sB, long long sC,
                                                     const typename Traits<MODE>::V2* __restrict__ A, int lda,
                                                     const typename Traits<MODE>::V2* __restrict__ B, int ldb,
@@ -209,8 +213,8 @@ __global__ void __launch_bounds__(256, (gemm_wgs_per_cu<MODE, NB16>())) k_zgemm_
     load_b(b, k0 + 2 * BKC);
     load_a(a, k0 + 2 * BKC);
     lds_only_barrier();
-    // columns in groups of up to three: enough independent MFMA chains to hide their latency
-    constexpr int G = NB16 % 3 == 0 ? 3 : NB16 % 2 == 0 ? 2 : NB16 == 1 ? 1 : NB16 == 5 ? 5 : 7;
+    // all columns of one product term in turn: independent MFMA chains hide their latency
+    constexpr int G = NB16;
 #pragma unroll
     for (int g = 0; g < NB16; g += G) {
       if constexpr (SPLIT) {
@@ -352,31 +356,29 @@ void zgemm_mfma_t(Context& c, int M, int N, int K, const void* A, int lda, const
                   bool accumulate, const Batch& bt) {
   using V2 = typename Traits<MODE>::V2;
   const int cus = c.cu_count > 0 ? c.cu_count : 256;
-  // Column blocks of equal width, at most 144 columns. Among the widths the one whose tiles, dealt to the
-  // CUs, take the fewest MFMA steps on the busiest CU; 1.5 blocks of 16 columns stand for what a tile
-  // costs besides them (loading and converting A): C64 expansion, 108 row tiles × 160 columns in FP64, runs
-  // 216 tiles of 80 columns instead of 432 of 48.
+  // Column blocks of equal width. Without split K the width whose tiles, dealt to the CUs, take the fewest
+  // steps on the busiest CU (half a block stands for what a tile costs besides its MFMAs), narrower on a tie.
   const int n16 = (N + 15) / 16, mt = (M + BMC - 1) / BMC;
-  int nb16 = (n16 + (n16 + 8) / 9 - 1) / ((n16 + 8) / 9);
+  auto balanced = [&](int w) {
+    const int blocks = (n16 + w - 1) / w;
+    return (n16 + blocks - 1) / blocks;
+  };
   auto tiles_of = [&](int w) { return (long)mt * ((n16 + w - 1) / w) * bt.count; };
-  auto cost = [&](int w) { return (double)((tiles_of(w) + cus - 1) / cus) * (w + 1.5); };
-  const bool split = tiles_of(nb16) < cus / 2 && K >= 16 * BKC;
-  if (!split) {
-    int best = nb16;
-    for (int w = nb16; w >= 1; --w)
-      if (cost(w) < cost(best)) best = w;
-    nb16 = best;
-  }
-  const int BN = 16 * nb16, nt = (N + BN - 1) / BN;
-  const long tiles = tiles_of(nb16);
-  int nsplit = 1;
+  auto cost = [&](int w) { return (double)((tiles_of(w) + cus - 1) / cus) * (w + 0.5); };
+  int nb16 = balanced(Tile<MODE>::W), nsplit = 1;
   // split K only for K >= 256 (short reductions are cheaper than the extra partial-sum pass) and
   // when the tiles fill less than half the CUs (above that the partial-sum round trip costs
-  // more than the idle CUs), into chunks of at least 4 steps and no more workgroups than run at once
-  if (split) {
-    const int per_cu = MODE == MODE_F64 && nb16 > 4 ? 1 : 2;
-    nsplit = (int)std::min<long>(std::max<long>(1, cus * per_cu / tiles), std::max(1, K / (4 * BKC)));
+  // more than the idle CUs), into chunks of at least 4 steps and no more workgroups than run at once;
+  // tiles narrower where even so the CUs are not all busy (64 × 40 × 1921: 10 us instead of 15)
+  if (tiles_of(nb16) < cus / 2 && K >= 16 * BKC) {
+    const int most = std::max(1, K / (4 * BKC));
+    while (nb16 > 1 && tiles_of(nb16) * most < cus) nb16 = balanced(nb16 - 1);
+    nsplit = (int)std::min<long>(std::max<long>(1, cus * Tile<MODE>::PER_CU / tiles_of(nb16)), most);
+  } else {
+    for (int w = Tile<MODE>::W; w >= 1; --w)
+      if (cost(balanced(w)) <= cost(nb16)) nb16 = balanced(w);
   }
+  const int BN = 16 * nb16, nt = (N + BN - 1) / BN;
   int kchunk = (K + nsplit - 1) / nsplit;
   kchunk = ((kchunk + 2 * BKC - 1) / (2 * BKC)) * (2 * BKC);
   nsplit = (K + kchunk - 1) / kchunk;
@@ -390,11 +392,15 @@ void zgemm_mfma_t(Context& c, int M, int N, int K, const void* A, int lda, const
   }
   int acc = (nsplit == 1 && accumulate) ? 1 : 0;
   switch (nb16) {
-#define PWK_NB(X) \
-  case X: launch_nb<MODE, X>(c, grid, M, N, K, kchunk, nsplit, bt, A, lda, B, ldb, C, ldc, acc, part); break;
-    PWK_NB(1) PWK_NB(2) PWK_NB(3) PWK_NB(4) PWK_NB(5) PWK_NB(6) PWK_NB(7) PWK_NB(8)
-#undef PWK_NB
-    default: launch_nb<MODE, 9>(c, grid, M, N, K, kchunk, nsplit, bt, A, lda, B, ldb, C, ldc, acc, part); break;
+    case 1:
+      launch_nb<MODE, 1>(c, grid, M, N, K, kchunk, nsplit, bt, A, lda, B, ldb, C, ldc, acc, part);
+      break;
+    case 2:
+      launch_nb<MODE, 2>(c, grid, M, N, K, kchunk, nsplit, bt, A, lda, B, ldb, C, ldc, acc, part);
+      break;
+    default:
+      launch_nb<MODE, Tile<MODE>::W>(c, grid, M, N, K, kchunk, nsplit, bt, A, lda, B, ldb, C, ldc, acc, part);
+      break;
   }
   PWK_HIP(hipGetLastError());
   if (nsplit > 1) {
