@@ -19,6 +19,8 @@
 // with the matrix and the eigenvectors in LDS (round-robin ordering, n/2
 // disjoint complex rotations per round, at most 30 sweeps).
 // Every loop has a fixed bound; nothing waits on data.
+#include <algorithm>
+
 #include "common.hpp"
 #include "jacobi.hpp"
 
@@ -81,124 +83,19 @@ __device__ double start_entry(int i, int j) {
   return (double)h * (2.0 / 4294967296.0) - 1.0;
 }
 
+// Steps 2-4 on the tridiagonal form (d in LDS, the complex sub-diagonal in ecx): eigenvalues to lam,
+// the phases to dph, eigenvectors of the real tridiagonal to Z. lu holds 6·n·nb doubles (Z first).
 template <int NT>
-__global__ void __launch_bounds__(NT) k_heev(int n, int nb, int a_in_lds, int lu_in_lds, double2* __restrict__ Hb,
-                                             double* __restrict__ work, double* __restrict__ w_out,
-                                             double2* __restrict__ V_out, int* __restrict__ status) {
+__device__ __forceinline__ void tri_pairs(int n, int nb, double* d, double* e, double* e2, double* lam, double* red, double* s_bounds,
+                          const double2* ecx, double2* dph, double* Z) {
   constexpr int EIG_NT = NT;
   constexpr int EIG_WAVES = NT / 64;
-  extern __shared__ unsigned char smem[];
-  double2* v = reinterpret_cast<double2*>(smem);      // n
-  double2* wv = v + n;                                // n
-  double* d = reinterpret_cast<double*>(wv + n);      // n: diagonal of T_r
-  double* e = d + n;                                  // n: sub-diagonal of T_r
-  double* e2 = e + n;                                 // n: e²
-  double* lam = e2 + n;                               // nb: eigenvalues
-  double* red = lam + nb;                             // EIG_WAVES + 2
-  // EIG_WAVES × 64 matvec partials, 16-byte aligned
-  const size_t pp_off = ((size_t)(reinterpret_cast<unsigned char*>(red + EIG_WAVES + 2) - smem) + 15) & ~(size_t)15;
-  double2* pp = reinterpret_cast<double2*>(smem + pp_off);
-  double2* lds_a = pp + 16 * 64;                                          // n·n when a_in_lds
-  double* lds_lu = reinterpret_cast<double*>(lds_a + (a_in_lds ? (size_t)n * n : 0));  // 6·n·nb when lu_in_lds
-  __shared__ double s_bounds[3];
-
-  const int b = blockIdx.x, t = threadIdx.x, lane = t & 63, wave = t >> 6;
-  double2* A = Hb + (size_t)b * n * n;
-  if (a_in_lds) {  // small matrices live in LDS for the whole solve (the input is not written back)
-    for (int i = t; i < n * n; i += EIG_NT) lds_a[i] = A[i];
-    __syncthreads();
-    A = lds_a;
-  }
-  double* base = work + (size_t)b * eig_stride(n, nb);
-  double2* ecx = reinterpret_cast<double2*>(base);    // n
-  double2* dph = ecx + n;                              // n
-  double* Z = lu_in_lds ? lds_lu : reinterpret_cast<double*>(dph + n);  // Z[i*nb + j]
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   double* U0 = Z + (size_t)n * nb;                     // LU factors, interleaved by vector like Z
   double* U1 = U0 + (size_t)n * nb;
   double* U2 = U1 + (size_t)n * nb;
   double* ML = U2 + (size_t)n * nb;
   double* PV = ML + (size_t)n * nb;
-
-  // ---- 1. Householder tridiagonalisation --------------------------------------------
-  for (int k = 0; k + 2 < n; ++k) {
-    const int m = n - k - 1;
-    double2* col = A + (size_t)k * n + k + 1;
-    double part = 0.0;
-    for (int i = t; i < m; i += EIG_NT) part += col[i].x * col[i].x + col[i].y * col[i].y;
-    const double xn = sqrt(block_sum<NT>(part, red));
-    if (xn == 0.0) {
-      for (int i = t; i < m; i += EIG_NT) col[i] = make_double2(0.0, 0.0);  // identity reflector
-      if (t == 0) ecx[k] = make_double2(0.0, 0.0);
-      __syncthreads();
-      continue;
-    }
-    const double2 x0 = col[0];
-    const double ax0 = sqrt(x0.x * x0.x + x0.y * x0.y);
-    const double2 ph = ax0 > 0.0 ? make_double2(x0.x / ax0, x0.y / ax0) : make_double2(1.0, 0.0);
-    const double2 alpha = make_double2(-ph.x * xn, -ph.y * xn);
-    // v = (x - alpha e1) / |x - alpha e1|;  |x - alpha e1|² = 2(|x|² + |x||x0|)
-    const double vn = sqrt(2.0 * (xn * xn + xn * ax0));
-    for (int i = t; i < m; i += EIG_NT) {
-      double2 x = col[i];
-      if (i == 0) {
-        x.x -= alpha.x;
-        x.y -= alpha.y;
-      }
-      v[i] = make_double2(x.x / vn, x.y / vn);
-    }
-    __syncthreads();
-    // p = A_sub v: rows in chunks of 64 lanes, the columns split over the waves, then a
-    // fixed-order sum of the per-wave partials
-    for (int i0 = 0; i0 < m; i0 += 64) {
-      const int i = i0 + lane;
-      double pr = 0.0, pi = 0.0;
-      if (i < m) {
-        const double2* arow = A + (size_t)(k + 1) * n + k + 1 + i;
-        for (int j = wave; j < m; j += EIG_WAVES) {
-          const double2 a = arow[(size_t)j * n];
-          const double2 vj = v[j];
-          pr += a.x * vj.x - a.y * vj.y;
-          pi += a.x * vj.y + a.y * vj.x;
-        }
-      }
-      pp[wave * 64 + lane] = make_double2(pr, pi);
-      __syncthreads();
-      if (wave == 0 && i < m) {
-        double sr = 0.0, si = 0.0;
-        for (int w = 0; w < EIG_WAVES; ++w) {
-          sr += pp[w * 64 + lane].x;
-          si += pp[w * 64 + lane].y;
-        }
-        wv[i] = make_double2(sr, si);
-      }
-      __syncthreads();
-    }
-    part = 0.0;
-    for (int i = t; i < m; i += EIG_NT) part += v[i].x * wv[i].x + v[i].y * wv[i].y;  // v^H p (real)
-    const double K = block_sum<NT>(part, red);
-    for (int i = t; i < m; i += EIG_NT) {
-      wv[i].x -= K * v[i].x;
-      wv[i].y -= K * v[i].y;
-    }
-    __syncthreads();
-    // A_sub -= 2 (v w^H + w v^H)
-    for (int idx = t; idx < m * m; idx += EIG_NT) {
-      const int i = idx % m, j = idx / m;
-      const double2 vi = v[i], wi = wv[i], vj = v[j], wj = wv[j];
-      const double re = (vi.x * wj.x + vi.y * wj.y) + (wi.x * vj.x + wi.y * vj.y);
-      const double im = (vi.y * wj.x - vi.x * wj.y) + (wi.y * vj.x - wi.x * vj.y);
-      double2* a = &A[(size_t)(k + 1 + j) * n + k + 1 + i];
-      a->x -= 2.0 * re;
-      a->y -= 2.0 * im;
-    }
-    __syncthreads();
-    for (int i = t; i < m; i += EIG_NT) col[i] = v[i];
-    if (t == 0) ecx[k] = alpha;
-    __syncthreads();
-  }
-  if (t == 0 && n >= 2) ecx[n - 2] = A[(size_t)(n - 2) * n + n - 1];
-  for (int i = t; i < n; i += EIG_NT) d[i] = A[(size_t)i * n + i].x;
-  __syncthreads();
 
   // ---- 2. real sub-diagonal, phases, Gershgorin bounds -------------------------------
   if (t == 0) {
@@ -373,6 +270,123 @@ __global__ void __launch_bounds__(NT) k_heev(int n, int nb, int a_in_lds, int lu
     for (int r = t; r < n; r += EIG_NT) Z[(size_t)r * nb + j] *= sc;
     __syncthreads();
   }
+}
+
+template <int NT>
+__global__ void __launch_bounds__(NT) k_heev(int n, int nb, int a_in_lds, int lu_in_lds, double2* __restrict__ Hb,
+                                             double* __restrict__ work, double* __restrict__ w_out,
+                                             double2* __restrict__ V_out, int* __restrict__ status) {
+  constexpr int EIG_NT = NT;
+  constexpr int EIG_WAVES = NT / 64;
+  extern __shared__ unsigned char smem[];
+  double2* v = reinterpret_cast<double2*>(smem);      // n
+  double2* wv = v + n;                                // n
+  double* d = reinterpret_cast<double*>(wv + n);      // n: diagonal of T_r
+  double* e = d + n;                                  // n: sub-diagonal of T_r
+  double* e2 = e + n;                                 // n: e²
+  double* lam = e2 + n;                               // nb: eigenvalues
+  double* red = lam + nb;                             // EIG_WAVES + 2
+  // EIG_WAVES × 64 matvec partials, 16-byte aligned
+  const size_t pp_off = ((size_t)(reinterpret_cast<unsigned char*>(red + EIG_WAVES + 2) - smem) + 15) & ~(size_t)15;
+  double2* pp = reinterpret_cast<double2*>(smem + pp_off);
+  double2* lds_a = pp + 16 * 64;                                          // n·n when a_in_lds
+  double* lds_lu = reinterpret_cast<double*>(lds_a + (a_in_lds ? (size_t)n * n : 0));  // 6·n·nb when lu_in_lds
+  __shared__ double s_bounds[3];
+
+  const int b = blockIdx.x, t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  double2* A = Hb + (size_t)b * n * n;
+  if (a_in_lds) {  // small matrices live in LDS for the whole solve (the input is not written back)
+    for (int i = t; i < n * n; i += EIG_NT) lds_a[i] = A[i];
+    __syncthreads();
+    A = lds_a;
+  }
+  double* base = work + (size_t)b * eig_stride(n, nb);
+  double2* ecx = reinterpret_cast<double2*>(base);    // n
+  double2* dph = ecx + n;                              // n
+  double* Z = lu_in_lds ? lds_lu : reinterpret_cast<double*>(dph + n);  // Z[i*nb + j]
+
+  // ---- 1. Householder tridiagonalisation --------------------------------------------
+  for (int k = 0; k + 2 < n; ++k) {
+    const int m = n - k - 1;
+    double2* col = A + (size_t)k * n + k + 1;
+    double part = 0.0;
+    for (int i = t; i < m; i += EIG_NT) part += col[i].x * col[i].x + col[i].y * col[i].y;
+    const double xn = sqrt(block_sum<NT>(part, red));
+    if (xn == 0.0) {
+      for (int i = t; i < m; i += EIG_NT) col[i] = make_double2(0.0, 0.0);  // identity reflector
+      if (t == 0) ecx[k] = make_double2(0.0, 0.0);
+      __syncthreads();
+      continue;
+    }
+    const double2 x0 = col[0];
+    const double ax0 = sqrt(x0.x * x0.x + x0.y * x0.y);
+    const double2 ph = ax0 > 0.0 ? make_double2(x0.x / ax0, x0.y / ax0) : make_double2(1.0, 0.0);
+    const double2 alpha = make_double2(-ph.x * xn, -ph.y * xn);
+    // v = (x - alpha e1) / |x - alpha e1|;  |x - alpha e1|² = 2(|x|² + |x||x0|)
+    const double vn = sqrt(2.0 * (xn * xn + xn * ax0));
+    for (int i = t; i < m; i += EIG_NT) {
+      double2 x = col[i];
+      if (i == 0) {
+        x.x -= alpha.x;
+        x.y -= alpha.y;
+      }
+      v[i] = make_double2(x.x / vn, x.y / vn);
+    }
+    __syncthreads();
+    // p = A_sub v: rows in chunks of 64 lanes, the columns split over the waves, then a
+    // fixed-order sum of the per-wave partials
+    for (int i0 = 0; i0 < m; i0 += 64) {
+      const int i = i0 + lane;
+      double pr = 0.0, pi = 0.0;
+      if (i < m) {
+        const double2* arow = A + (size_t)(k + 1) * n + k + 1 + i;
+        for (int j = wave; j < m; j += EIG_WAVES) {
+          const double2 a = arow[(size_t)j * n];
+          const double2 vj = v[j];
+          pr += a.x * vj.x - a.y * vj.y;
+          pi += a.x * vj.y + a.y * vj.x;
+        }
+      }
+      pp[wave * 64 + lane] = make_double2(pr, pi);
+      __syncthreads();
+      if (wave == 0 && i < m) {
+        double sr = 0.0, si = 0.0;
+        for (int w = 0; w < EIG_WAVES; ++w) {
+          sr += pp[w * 64 + lane].x;
+          si += pp[w * 64 + lane].y;
+        }
+        wv[i] = make_double2(sr, si);
+      }
+      __syncthreads();
+    }
+    part = 0.0;
+    for (int i = t; i < m; i += EIG_NT) part += v[i].x * wv[i].x + v[i].y * wv[i].y;  // v^H p (real)
+    const double K = block_sum<NT>(part, red);
+    for (int i = t; i < m; i += EIG_NT) {
+      wv[i].x -= K * v[i].x;
+      wv[i].y -= K * v[i].y;
+    }
+    __syncthreads();
+    // A_sub -= 2 (v w^H + w v^H)
+    for (int idx = t; idx < m * m; idx += EIG_NT) {
+      const int i = idx % m, j = idx / m;
+      const double2 vi = v[i], wi = wv[i], vj = v[j], wj = wv[j];
+      const double re = (vi.x * wj.x + vi.y * wj.y) + (wi.x * vj.x + wi.y * vj.y);
+      const double im = (vi.y * wj.x - vi.x * wj.y) + (wi.y * vj.x - wi.x * vj.y);
+      double2* a = &A[(size_t)(k + 1 + j) * n + k + 1 + i];
+      a->x -= 2.0 * re;
+      a->y -= 2.0 * im;
+    }
+    __syncthreads();
+    for (int i = t; i < m; i += EIG_NT) col[i] = v[i];
+    if (t == 0) ecx[k] = alpha;
+    __syncthreads();
+  }
+  if (t == 0 && n >= 2) ecx[n - 2] = A[(size_t)(n - 2) * n + n - 1];
+  for (int i = t; i < n; i += EIG_NT) d[i] = A[(size_t)i * n + i].x;
+  __syncthreads();
+
+  tri_pairs<NT>(n, nb, d, e, e2, lam, red, s_bounds, ecx, dph, Z);
 
   // ---- 5. V = Q·D·Z --------------------------------------------------------------------
   double2* V = V_out + (size_t)b * n * nb;
@@ -416,6 +430,276 @@ __global__ void __launch_bounds__(NT) k_heev(int n, int nb, int a_in_lds, int lu
   if (t == 0 && status) status[b] = 0;
 }
 
+// ---- matrices of 65 to 256 rows that do not fit the LDS ---------------------------------------
+// The same steps with the Householder reduction arranged around one pass over the matrix per reflector:
+//  - wave w owns the columns j ≡ w mod 16 and a lane the rows lane + 64r of them for the whole reduction, so
+//    the matrix (in L2) is read and written by the threads that own it and needs no barrier;
+//  - pass k applies the rank-2 update of reflector k - 1 to the columns behind k and multiplies the updated
+//    entries with v_k on the way (rows in registers, the column factors broadcast from LDS); the 16 waves'
+//    partial products go through LDS, and column k + 1 is left there for the next reflector;
+//  - every wave then forms w and the next reflector in its registers, redundantly: wave sums by lane moves,
+//    three barriers per reflector.
+// Back-transformation: one wave per vector, its rows in registers, no barrier.
+// Bound: the L2 traffic of one CU per matrix (2·n³/3·16 bytes) and the chain of reflectors. 8 matrices of
+// 169 rows, 8 pairs: the form above took 5.0 ms with 15 barriers and an integer division per entry and reflector.
+constexpr int ROW_NT = 1024, ROW_WAVES = 16;
+
+template <int CTRL>
+__device__ __forceinline__ double dpp_add(double x) {
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(x), CTRL, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(x), CTRL, 0xf, 0xf, true);
+  return x + __hiloint2double(hi, lo);
+}
+// the sum over a wave, in every lane: within rows of 16 lanes by lane moves, then the four rows
+__device__ __forceinline__ double wave_sum(double x) {
+  x = dpp_add<0xB1>(x);   // quad_perm [1,0,3,2]
+  x = dpp_add<0x4E>(x);   // quad_perm [2,3,0,1]
+  x = dpp_add<0x141>(x);  // row_half_mirror
+  x = dpp_add<0x140>(x);  // row_mirror
+  double s = 0.0;
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+    s += __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(x), 16 * r),
+                          __builtin_amdgcn_readlane(__double2loint(x), 16 * r));
+  return s;
+}
+
+__host__ __device__ inline size_t rows_lds_vectors(int n) { return (size_t)5 * n * sizeof(double2); }
+// LDS of k_heev_rows: vectors v, w, x, column, p (complex) | d, e, e2, lam, red | the waves' partial
+// products, later the tridiagonal's vectors and LU factors when they fit
+inline size_t rows_lds_head(int n, int nb) {
+  return rows_lds_vectors(n) + ((((size_t)3 * n + nb + 32) * sizeof(double) + 15) & ~(size_t)15);
+}
+
+// R = rows per lane
+template <int R>
+__global__ void __launch_bounds__(ROW_NT) k_heev_rows(int n, int nb, int lu_in_lds, double2* __restrict__ Hb,
+                                                      double* __restrict__ work, double* __restrict__ w_out,
+                                                      double2* __restrict__ V_out, int* __restrict__ status) {
+  constexpr int CB = R >= 4 ? 1 : R == 3 ? 2 : 4;  // columns of a wave in flight
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  double2* sv = reinterpret_cast<double2*>(smem);  // reflector k - 1, its w, reflector k
+  double2* sw = sv + n;
+  double2* sx = sw + n;
+  double2* scol = sx + n;  // column k, reflectors up to k - 2 applied
+  double2* sp = scol + n;  // A·v of reflector k - 1
+  double* d = reinterpret_cast<double*>(sp + n);
+  double* e = d + n;
+  double* e2 = e + n;
+  double* lam = e2 + n;
+  double* red = lam + nb;
+  double2* part = reinterpret_cast<double2*>(
+      smem + (((size_t)(reinterpret_cast<unsigned char*>(red + 32) - smem) + 15) & ~(size_t)15));  // [wave][n]
+  __shared__ double s_bounds[3];
+  const int b = blockIdx.x, t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  double2* A = Hb + (size_t)b * n * n;
+  double* base = work + (size_t)b * eig_stride(n, nb);
+  double2* ecx = reinterpret_cast<double2*>(base);
+  double2* dph = ecx + n;
+  double* Z = lu_in_lds ? reinterpret_cast<double*>(part) : reinterpret_cast<double*>(dph + n);
+
+  double2 v[R], w[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) v[r] = w[r] = make_double2(0.0, 0.0);
+  for (int i = t; i < n; i += ROW_NT) {
+    scol[i] = A[i];
+    sp[i] = make_double2(0.0, 0.0);
+  }
+  __syncthreads();
+  for (int k = 0; k + 1 < n; ++k) {
+    // the wave's first columns behind k: loads in flight during the vector phase
+    const int j0 = k + 1 + ((wave - (k + 1)) & (ROW_WAVES - 1));
+    double2 a[CB][R];
+#pragma unroll
+    for (int c = 0; c < CB; ++c)
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        const int j = j0 + ROW_WAVES * c, i = lane + 64 * r;
+        if (j < n && i < n && i > k) a[c][r] = A[(size_t)j * n + i];
+      }
+    // w of reflector k - 1, column k, reflector k (every wave for itself)
+    double2 p[R], x[R];
+    double kk = 0.0;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int i = lane + 64 * r;
+      p[r] = i < n ? sp[i] : make_double2(0.0, 0.0);
+      x[r] = i < n && i >= k ? scol[i] : make_double2(0.0, 0.0);
+      kk += v[r].x * p[r].x + v[r].y * p[r].y;  // v^H p (real)
+    }
+    kk = wave_sum(kk);
+#pragma unroll
+    for (int r = 0; r < R; ++r) w[r] = make_double2(p[r].x - kk * v[r].x, p[r].y - kk * v[r].y);
+    // v_k and w_k of reflector k - 1 at row k, from the lane that holds it
+    double2 vk = make_double2(0.0, 0.0), wk = vk;
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+      if ((k >> 6) == r) {
+        const int l = k & 63;
+        vk.x = __shfl(v[r].x, l, 64);
+        vk.y = __shfl(v[r].y, l, 64);
+        wk.x = __shfl(w[r].x, l, 64);
+        wk.y = __shfl(w[r].y, l, 64);
+      }
+    double xx = 0.0;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int i = lane + 64 * r;
+      const double re = (v[r].x * wk.x + v[r].y * wk.y) + (w[r].x * vk.x + w[r].y * vk.y);
+      const double im = (v[r].y * wk.x - v[r].x * wk.y) + (w[r].y * vk.x - w[r].x * vk.y);
+      x[r].x -= 2.0 * re;
+      x[r].y -= 2.0 * im;
+      if (i > k && i < n) xx += x[r].x * x[r].x + x[r].y * x[r].y;
+      if (i == k && wave == 0) d[k] = x[r].x;
+    }
+    xx = wave_sum(xx);
+    double2 x0 = make_double2(0.0, 0.0);
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+      if (((k + 1) >> 6) == r) {
+        x0.x = __shfl(x[r].x, (k + 1) & 63, 64);
+        x0.y = __shfl(x[r].y, (k + 1) & 63, 64);
+      }
+    // the reflector of the last column is none: its sub-diagonal entry stays as it is
+    const bool last = k + 2 >= n;
+    const double xn = sqrt(xx), ax0 = sqrt(x0.x * x0.x + x0.y * x0.y);
+    const double2 ph = ax0 > 0.0 ? make_double2(x0.x / ax0, x0.y / ax0) : make_double2(1.0, 0.0);
+    const double2 alpha = make_double2(-ph.x * xn, -ph.y * xn);
+    // v = (x - alpha e1) / |x - alpha e1|;  |x - alpha e1|² = 2(|x|² + |x||x0|)
+    const double vn = sqrt(2.0 * (xn * xn + xn * ax0));
+    const double rv = !last && xn > 0.0 ? 1.0 / vn : 0.0;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int i = lane + 64 * r;
+      double2 y = make_double2(0.0, 0.0);
+      if (i > k && i < n && rv > 0.0) {
+        y = x[r];
+        if (i == k + 1) {
+          y.x -= alpha.x;
+          y.y -= alpha.y;
+        }
+        y.x *= rv;
+        y.y *= rv;
+      }
+      x[r] = y;
+      if (wave == 0 && i < n) {
+        sv[i] = v[r];
+        sw[i] = w[r];
+        sx[i] = y;
+        if (i > k && !last) A[(size_t)k * n + i] = y;  // the reflector, for the back-transformation
+      }
+    }
+    if (t == 0) ecx[k] = last ? x0 : alpha;
+    __syncthreads();
+    // pass k
+    double2 q[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) q[r] = make_double2(0.0, 0.0);
+    for (int jb = j0; jb < n; jb += CB * ROW_WAVES) {
+      if (jb != j0) {
+#pragma unroll
+        for (int c = 0; c < CB; ++c)
+#pragma unroll
+          for (int r = 0; r < R; ++r) {
+            const int j = jb + ROW_WAVES * c, i = lane + 64 * r;
+            if (j < n && i < n && i > k) a[c][r] = A[(size_t)j * n + i];
+          }
+      }
+#pragma unroll
+      for (int c = 0; c < CB; ++c) {
+        const int j = jb + ROW_WAVES * c;
+        if (j >= n) break;
+        const double2 vj = sv[j], wj = sw[j], xj = sx[j];
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+          const int i = lane + 64 * r;
+          if (i < n && i > k) {
+            double2 z = a[c][r];
+            const double re = (v[r].x * wj.x + v[r].y * wj.y) + (w[r].x * vj.x + w[r].y * vj.y);
+            const double im = (v[r].y * wj.x - v[r].x * wj.y) + (w[r].y * vj.x - w[r].x * vj.y);
+            z.x -= 2.0 * re;
+            z.y -= 2.0 * im;
+            A[(size_t)j * n + i] = z;
+            if (j == k + 1) scol[i] = z;
+            q[r].x += z.x * xj.x - z.y * xj.y;
+            q[r].y += z.x * xj.y + z.y * xj.x;
+          }
+        }
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int i = lane + 64 * r;
+      if (i < n) part[(size_t)wave * n + i] = q[r];
+      v[r] = x[r];
+    }
+    __syncthreads();
+    if (t < n) {
+      double2 s = make_double2(0.0, 0.0);
+#pragma unroll
+      for (int g = 0; g < ROW_WAVES; ++g) {
+        const double2 y = part[(size_t)g * n + t];
+        s.x += y.x;
+        s.y += y.y;
+      }
+      sp[t] = s;
+    }
+    __syncthreads();
+  }
+  if (t == 0) d[n - 1] = scol[n - 1].x;
+  __syncthreads();
+
+  tri_pairs<ROW_NT>(n, nb, d, e, e2, lam, red, s_bounds, ecx, dph, Z);
+
+  // ---- V = Q·D·Z, a wave per vector ------------------------------------------------------------
+  double2* V = V_out + (size_t)b * n * nb;
+  for (int jj = t; jj < nb; jj += ROW_NT) w_out[(size_t)b * nb + jj] = lam[jj];
+  for (int jj = wave; jj < nb; jj += ROW_WAVES) {
+    double2 y[R], h[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int i = lane + 64 * r;
+      y[r] = h[r] = make_double2(0.0, 0.0);
+      if (i < n) {
+        const double z = Z[(size_t)i * nb + jj];
+        const double2 pz = dph[i];
+        y[r] = make_double2(pz.x * z, pz.y * z);
+      }
+    }
+    auto load = [&](double2(&g)[R], int k) {
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        const int i = lane + 64 * r;
+        g[r] = make_double2(0.0, 0.0);
+        if (k >= 0 && i > k && i < n) g[r] = A[(size_t)k * n + i];
+      }
+    };
+    double2 g[R];
+    load(h, n - 3);
+    for (int k = n - 3; k >= 0; --k) {
+      load(g, k - 1);  // the next reflector, in flight
+      double sr = 0.0, si = 0.0;
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        sr += h[r].x * y[r].x + h[r].y * y[r].y;  // conj(v)·x
+        si += h[r].x * y[r].y - h[r].y * y[r].x;
+      }
+      sr = 2.0 * wave_sum(sr);
+      si = 2.0 * wave_sum(si);
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        y[r].x -= h[r].x * sr - h[r].y * si;
+        y[r].y -= h[r].x * si + h[r].y * sr;
+        h[r] = g[r];
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+      if (lane + 64 * r < n) V[(size_t)jj * n + lane + 64 * r] = y[r];
+  }
+  if (t == 0 && status) status[b] = 0;
+}
+
 // One wavefront per matrix, n <= JMAX: cyclic Jacobi with the matrix and the vectors in LDS.
 __global__ void __launch_bounds__(64) k_jacobi(int n, int nb, const double2* __restrict__ Hb, double* __restrict__ w_out,
                                                double2* __restrict__ V_out) {
@@ -447,6 +731,19 @@ size_t lu_bytes(int n, int nb) { return (size_t)6 * n * nb * sizeof(double); }
 bool a_fits_lds(int n, int nb) { return heev_lds_base(n, nb) + a_bytes(n) <= kLdsCap; }
 bool lu_fits_lds(int n, int nb) {
   return heev_lds_base(n, nb) + (a_fits_lds(n, nb) ? a_bytes(n) : 0) + lu_bytes(n, nb) <= kLdsCap;
+}
+// k_heev_rows: the partial products' area, or the tridiagonal's vectors and factors when they fit
+bool rows_lu_in_lds(int n, int nb) { return rows_lds_head(n, nb) + lu_bytes(n, nb) <= kLdsCap; }
+size_t rows_lds_bytes(int n, int nb) {
+  const size_t part = (size_t)ROW_WAVES * n * sizeof(double2);
+  return rows_lds_head(n, nb) + std::max(part, rows_lu_in_lds(n, nb) ? lu_bytes(n, nb) : (size_t)0);
+}
+template <int R>
+void heev_rows(Context& c, int n, int nb, int nk, void* H, void* work, double* w, void* V, int* status) {
+  const size_t sh = rows_lds_bytes(n, nb);
+  ensure_lds_limit((const void*)k_heev_rows<R>, sh);
+  k_heev_rows<R><<<(unsigned)nk, ROW_NT, sh, c.stream>>>(n, nb, rows_lu_in_lds(n, nb) ? 1 : 0, (double2*)H,
+                                                         (double*)work, w, (double2*)V, status);
 }
 size_t heev_lds_bytes(int n, int nb) {
   return heev_lds_base(n, nb) + (a_fits_lds(n, nb) ? a_bytes(n) : 0) + (lu_fits_lds(n, nb) ? lu_bytes(n, nb) : 0);
@@ -515,6 +812,13 @@ void launch_heev_batched(Context& c, int n, int nb, int nk, void* H, void* work,
     ensure_lds_limit((const void*)k_heev<64>, sh);
     k_heev<64><<<(unsigned)nk, 64, sh, c.stream>>>(n, nb, al, lu, (double2*)H, (double*)work, w, (double2*)V,
                                                    status);
+  } else if (n <= 256 && rows_lds_bytes(n, nb) <= kLdsCap) {
+    if (n <= 128)
+      heev_rows<2>(c, n, nb, nk, H, work, w, V, status);
+    else if (n <= 192)
+      heev_rows<3>(c, n, nb, nk, H, work, w, V, status);
+    else
+      heev_rows<4>(c, n, nb, nk, H, work, w, V, status);
   } else {
     ensure_lds_limit((const void*)k_heev<EIG_NT>, sh);
     k_heev<EIG_NT><<<(unsigned)nk, EIG_NT, sh, c.stream>>>(n, nb, al, lu, (double2*)H, (double*)work, w,
