@@ -20,6 +20,7 @@
 // disjoint complex rotations per round, at most 30 sweeps).
 // Every loop has a fixed bound; nothing waits on data.
 #include <algorithm>
+#include <type_traits>
 
 #include "common.hpp"
 #include "jacobi.hpp"
@@ -58,14 +59,26 @@ __device__ double block_sum(double v, double* red) {
   return red[EIG_WAVES];
 }
 
+// 1/x to the last bit or two: the hardware estimate and two Newton steps, a third of the latency of a
+// division (the Sturm recurrences and the LU sweeps are chains of them)
+__device__ __forceinline__ double recip(double x) {
+  double r = __builtin_amdgcn_rcp(x);
+  r = fma(fma(-x, r, 1.0), r, r);
+  return fma(fma(-x, r, 1.0), r, r);
+}
+
 // Number of eigenvalues of the real symmetric tridiagonal (d, e) below x.
 __device__ int sturm_count(int n, const double* d, const double* e2, double x, double pivmin) {
   int cnt = 0;
   double q = d[0] - x;
   if (fabs(q) < pivmin) q = -pivmin;
   cnt += q < 0.0;
+  double dn = n > 1 ? d[1] - x : 0.0, en = e2[0];
   for (int i = 1; i < n; ++i) {
-    q = d[i] - x - e2[i - 1] / q;
+    const double di = dn, ei = en;
+    dn = d[min(i + 1, n - 1)] - x;  // the next entries, in flight
+    en = e2[i];
+    q = fma(-ei, recip(q), di);
     if (fabs(q) < pivmin) q = -pivmin;
     cnt += q < 0.0;
   }
@@ -98,31 +111,58 @@ __device__ __forceinline__ void tri_pairs(int n, int nb, double* d, double* e, d
   double* PV = ML + (size_t)n * nb;
 
   // ---- 2. real sub-diagonal, phases, Gershgorin bounds -------------------------------
-  if (t == 0) {
-    double2 p = make_double2(1.0, 0.0);
-    dph[0] = p;
-    double lo = 0.0, hi = 0.0, emax2 = 0.0;
-    for (int k = 0; k < n; ++k) {
-      double ab = 0.0;
-      if (k + 1 < n) {
-        const double2 ek = ecx[k];
-        ab = sqrt(ek.x * ek.x + ek.y * ek.y);
-        if (ab > 0.0) p = make_double2((p.x * ek.x - p.y * ek.y) / ab, (p.x * ek.y + p.y * ek.x) / ab);
-        dph[k + 1] = p;
-      }
-      e[k] = ab;
-      e2[k] = ab * ab;
-      emax2 = fmax(emax2, ab * ab);
-      const double r = ab + (k > 0 ? e[k - 1] : 0.0);
-      lo = k == 0 ? d[k] - r : fmin(lo, d[k] - r);
-      hi = k == 0 ? d[k] + r : fmax(hi, d[k] + r);
+  // moduli and unit phases by all threads (the unit phases into Z), then the running product of the
+  // phases by one, which is all that is serial
+  double2* unit = reinterpret_cast<double2*>(Z);
+  for (int k = t; k < n; k += EIG_NT) {
+    double ab = 0.0;
+    double2 u = make_double2(1.0, 0.0);
+    if (k + 1 < n) {
+      const double2 ek = ecx[k];
+      ab = sqrt(ek.x * ek.x + ek.y * ek.y);
+      if (ab > 0.0) u = make_double2(ek.x / ab, ek.y / ab);
     }
+    e[k] = ab;
+    e2[k] = ab * ab;
+    unit[k] = u;
+  }
+  __syncthreads();
+  double lo = 1e308, hi = -1e308;
+  for (int k = t; k < n; k += EIG_NT) {
+    const double r = e[k] + (k > 0 ? e[k - 1] : 0.0);
+    lo = fmin(lo, d[k] - r);
+    hi = fmax(hi, d[k] + r);
+  }
+  for (int off = 32; off > 0; off >>= 1) {
+    lo = fmin(lo, __shfl_down(lo, off, 64));
+    hi = fmax(hi, __shfl_down(hi, off, 64));
+  }
+  if (lane == 0) red[wave] = lo;
+  __syncthreads();
+  if (t == 0) {
+    for (int w = 0; w < EIG_WAVES; ++w) lo = fmin(lo, red[w]);
+    s_bounds[0] = lo;
+  }
+  __syncthreads();
+  if (lane == 0) red[wave] = hi;
+  __syncthreads();
+  if (t == 0) {
+    for (int w = 0; w < EIG_WAVES; ++w) hi = fmax(hi, red[w]);
     const double tnorm = fmax(fabs(lo), fabs(hi));
     const double pad = 2.220446049250313e-16 * tnorm * (double)n + 1e-300;
     s_bounds[0] = lo - pad;
     s_bounds[1] = hi + pad;
     s_bounds[2] = fmax(tnorm, 1e-300);
-    (void)emax2;
+  }
+  if (wave == EIG_WAVES - 1 && lane == 0) {
+    double2 ph = make_double2(1.0, 0.0), u = unit[0];
+    dph[0] = ph;
+    for (int k = 0; k + 1 < n; ++k) {
+      const double2 un = unit[k + 1];  // the next factor, in flight
+      ph = make_double2(ph.x * u.x - ph.y * u.y, ph.x * u.y + ph.y * u.x);
+      dph[k + 1] = ph;
+      u = un;
+    }
   }
   __syncthreads();
   const double tnorm = s_bounds[2];
@@ -170,40 +210,31 @@ __device__ __forceinline__ void tri_pairs(int n, int nb, double* d, double* e, d
   for (int j = t; j < nb; j += EIG_NT) {
     const double lj = lam[j];
     // LU of T_r - lj I with row interchanges (upper factor has two super-diagonals)
+    // U0 holds the pivots' reciprocals; each loop loads the next step's entries before it uses this one's
     double cd = d[0] - lj, cs = n > 1 ? e[0] : 0.0;
+    double sub = cs, an = n > 1 ? d[1] - lj : 0.0, bn = n > 2 ? e[1] : 0.0;
     for (int i = 0; i + 1 < n; ++i) {
-      const double sub = e[i];
-      const double an = d[i + 1] - lj, bn = (i + 2 < n) ? e[i + 1] : 0.0;
-      double u0, u1, u2, ml, pv;
-      if (fabs(cd) >= fabs(sub)) {
-        if (fabs(cd) < tiny) cd = cd < 0.0 ? -tiny : tiny;
-        ml = sub / cd;
-        u0 = cd;
-        u1 = cs;
-        u2 = 0.0;
-        pv = 0.0;
-        cd = an - ml * cs;
-        cs = bn;
-      } else {
-        ml = cd / sub;
-        u0 = sub;
-        u1 = an;
-        u2 = bn;
-        pv = 1.0;
-        cd = cs - ml * an;
-        cs = -ml * bn;
-      }
+      const double dn2 = d[min(i + 2, n - 1)], en1 = e[min(i + 1, n - 1)], en2 = e[min(i + 2, n - 1)];
+      const bool swap = !(fabs(cd) >= fabs(sub));
+      if (!swap && fabs(cd) < tiny) cd = cd < 0.0 ? -tiny : tiny;
+      const double ru = recip(swap ? sub : cd), ml = (swap ? cd : sub) * ru;
       const size_t o = (size_t)i * nb + j;
-      U0[o] = u0;
-      U1[o] = u1;
-      U2[o] = u2;
+      U0[o] = ru;
+      U1[o] = swap ? an : cs;
+      U2[o] = swap ? bn : 0.0;
       ML[o] = ml;
-      PV[o] = pv;
+      PV[o] = swap ? 1.0 : 0.0;
+      const double cd2 = swap ? cs - ml * an : an - ml * cs;
+      cs = swap ? -ml * bn : bn;
+      cd = cd2;
+      sub = en1;
+      an = dn2 - lj;
+      bn = i + 3 < n ? en2 : 0.0;
     }
     if (fabs(cd) < tiny) cd = cd < 0.0 ? -tiny : tiny;
     {
       const size_t o = (size_t)(n - 1) * nb + j;
-      U0[o] = cd;
+      U0[o] = recip(cd);
       U1[o] = 0.0;
       U2[o] = 0.0;
       ML[o] = 0.0;
@@ -220,29 +251,37 @@ __device__ __forceinline__ void tri_pairs(int n, int nb, double* d, double* e, d
       const double sc = 1.0 / sqrt(nrm);
       // forward: row interchanges and multipliers
       double carry = Z[j] * sc;
+      double pv = PV[j], ml = ML[j], zn = Z[(size_t)min(1, n - 1) * nb + j];
       for (int i = 0; i + 1 < n; ++i) {
-        const size_t o = (size_t)i * nb + j;
-        double yn = Z[o + nb] * sc;
-        double yi = carry;
-        if (PV[o] != 0.0) {
-          const double tmp = yi;
-          yi = yn;
-          yn = tmp;
-        }
+        const size_t o = (size_t)i * nb + j, o1 = o + nb, o2 = (size_t)min(i + 2, n - 1) * nb + j;
+        const double pv1 = PV[o1], ml1 = ML[o1], zn1 = Z[o2];
+        const double yn = zn * sc;
+        const bool swap = pv != 0.0;
+        const double yi = swap ? yn : carry;
+        carry = (swap ? carry : yn) - ml * yi;
         Z[o] = yi;
-        carry = yn - ML[o] * yi;
+        pv = pv1;
+        ml = ml1;
+        zn = zn1;
       }
       Z[(size_t)(n - 1) * nb + j] = carry;
       // backward substitution
       double x2 = 0.0, x1 = 0.0;
       nrm = 0.0;
+      size_t ol = (size_t)(n - 1) * nb + j;
+      double zi = carry, r0 = U0[ol], r1 = U1[ol], r2 = U2[ol];
       for (int i = n - 1; i >= 0; --i) {
-        const size_t o = (size_t)i * nb + j;
-        const double xi = (Z[o] - U1[o] * x1 - U2[o] * x2) / U0[o];
+        const size_t o = (size_t)i * nb + j, om = (size_t)max(i - 1, 0) * nb + j;
+        const double zm = Z[om], m0 = U0[om], m1 = U1[om], m2 = U2[om];
+        const double xi = (zi - r1 * x1 - r2 * x2) * r0;
         Z[o] = xi;
         nrm += xi * xi;
         x2 = x1;
         x1 = xi;
+        zi = zm;
+        r0 = m0;
+        r1 = m1;
+        r2 = m2;
       }
       if (!(nrm > 0.0) || !isfinite(nrm)) nrm = 1.0;
     }
@@ -432,17 +471,20 @@ __global__ void __launch_bounds__(NT) k_heev(int n, int nb, int a_in_lds, int lu
 
 // ---- matrices of 65 to 256 rows that do not fit the LDS ---------------------------------------
 // The same steps with the Householder reduction arranged around one pass over the matrix per reflector:
-//  - wave w owns the columns j ≡ w mod 16 and a lane the rows lane + 64r of them for the whole reduction, so
+//  - wave w owns the columns j ≡ w mod 8 and a lane the rows lane + 64r of them for the whole reduction, so
 //    the matrix (in L2) is read and written by the threads that own it and needs no barrier;
 //  - pass k applies the rank-2 update of reflector k - 1 to the columns behind k and multiplies the updated
-//    entries with v_k on the way (rows in registers, the column factors broadcast from LDS); the 16 waves'
+//    entries with v_k on the way (rows in registers, the column factors broadcast from LDS); the eight waves
 //    partial products go through LDS, and column k + 1 is left there for the next reflector;
-//  - every wave then forms w and the next reflector in its registers, redundantly: wave sums by lane moves,
-//    three barriers per reflector.
+//  - one wave then forms w and the next reflector in its registers (wave sums by lane moves; all waves doing so
+//    redundantly took four times as long, they share the vector units) while the others' first loads are
+//    in flight: three barriers per reflector.
 // Back-transformation: one wave per vector, its rows in registers, no barrier.
-// Bound: the L2 traffic of one CU per matrix (2·n³/3·16 bytes) and the chain of reflectors. 8 matrices of
-// 169 rows, 8 pairs: the form above took 5.0 ms with 15 barriers and an integer division per entry and reflector.
-constexpr int ROW_NT = 1024, ROW_WAVES = 16;
+// Bound: the chain of reflectors, each with a pass of about 13k cycles of issue by two waves per SIMD (the
+// loads and stores hide behind it). 8 matrices of 169 rows, 8 pairs: 5.0 ms in the form above (15 barriers and
+// an integer division per entry and reflector), 2.5 with the column factors read from LDS per column, 1.9 by
+// lane moves; 4 or 16 waves per matrix, or more columns in flight, took longer.
+constexpr int ROW_NT = 512, ROW_WAVES = 8, ROW_GROUPS = 2;
 
 template <int CTRL>
 __device__ __forceinline__ double dpp_add(double x) {
@@ -464,11 +506,41 @@ __device__ __forceinline__ double wave_sum(double x) {
   return s;
 }
 
-__host__ __device__ inline size_t rows_lds_vectors(int n) { return (size_t)5 * n * sizeof(double2); }
-// LDS of k_heev_rows: vectors v, w, x, column, p (complex) | d, e, e2, lam, red | the waves' partial
+__host__ __device__ inline size_t rows_lds_vectors(int n) { return (size_t)(4 + ROW_GROUPS) * n * sizeof(double2); }
+// LDS of k_heev_rows: vectors v, w, x, column, p sums (complex) | d, e, e2, lam, red | the waves' partial
 // products, later the tridiagonal's vectors and LU factors when they fit
 inline size_t rows_lds_head(int n, int nb) {
   return rows_lds_vectors(n) + ((((size_t)3 * n + nb + 32) * sizeof(double) + 15) & ~(size_t)15);
+}
+
+constexpr unsigned kNoRow = 0x80000000u;  // an offset past every matrix of 256 rows
+typedef unsigned u4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ double2 buf_load(__amdgpu_buffer_rsrc_t r, unsigned off, int soff) {
+  const u4 v = __builtin_amdgcn_raw_buffer_load_b128(r, off, soff, 0);
+  return make_double2(__hiloint2double((int)v.y, (int)v.x), __hiloint2double((int)v.w, (int)v.z));
+}
+__device__ __forceinline__ void buf_store(__amdgpu_buffer_rsrc_t r, unsigned off, int soff, double2 x) {
+  u4 v;
+  v.x = (unsigned)__double2loint(x.x);
+  v.y = (unsigned)__double2hiint(x.x);
+  v.z = (unsigned)__double2loint(x.y);
+  v.w = (unsigned)__double2hiint(x.y);
+  __builtin_amdgcn_raw_buffer_store_b128(v, r, off, soff, 0);
+}
+
+// the value of lane l (uniform) in every lane
+__device__ __forceinline__ double2 lane_of(const double2& x, int l) {
+  return make_double2(__hiloint2double(__builtin_amdgcn_readlane(__double2hiint(x.x), l),
+                                       __builtin_amdgcn_readlane(__double2loint(x.x), l)),
+                      __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(x.y), l),
+                                       __builtin_amdgcn_readlane(__double2loint(x.y), l)));
+}
+
+// z -= 2(v_i conj(w_j) + w_i conj(v_j)), the factor 2 in w
+__device__ __forceinline__ void rank2(double2& z, const double2& vi, const double2& wi, const double2& vj,
+                                      const double2& wj) {
+  z.x = fma(-vi.x, wj.x, fma(-vi.y, wj.y, fma(-wi.x, vj.x, fma(-wi.y, vj.y, z.x))));
+  z.y = fma(-vi.y, wj.x, fma(vi.x, wj.y, fma(-wi.y, vj.x, fma(wi.x, vj.y, z.y))));
 }
 
 // R = rows per lane
@@ -476,14 +548,14 @@ template <int R>
 __global__ void __launch_bounds__(ROW_NT) k_heev_rows(int n, int nb, int lu_in_lds, double2* __restrict__ Hb,
                                                       double* __restrict__ work, double* __restrict__ w_out,
                                                       double2* __restrict__ V_out, int* __restrict__ status) {
-  constexpr int CB = R >= 4 ? 1 : R == 3 ? 2 : 4;  // columns of a wave in flight
+  constexpr int CB = 1;  // columns of a wave per batch, two batches in flight
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   double2* sv = reinterpret_cast<double2*>(smem);  // reflector k - 1, its w, reflector k
   double2* sw = sv + n;
   double2* sx = sw + n;
   double2* scol = sx + n;  // column k, reflectors up to k - 2 applied
-  double2* sp = scol + n;  // A·v of reflector k - 1
-  double* d = reinterpret_cast<double*>(sp + n);
+  double2* psum = scol + n;  // A·v of reflector k - 1, two partial sums
+  double* d = reinterpret_cast<double*>(psum + ROW_GROUPS * n);
   double* e = d + n;
   double* e2 = e + n;
   double* lam = e2 + n;
@@ -491,158 +563,197 @@ __global__ void __launch_bounds__(ROW_NT) k_heev_rows(int n, int nb, int lu_in_l
   double2* part = reinterpret_cast<double2*>(
       smem + (((size_t)(reinterpret_cast<unsigned char*>(red + 32) - smem) + 15) & ~(size_t)15));  // [wave][n]
   __shared__ double s_bounds[3];
-  const int b = blockIdx.x, t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int b = blockIdx.x, t = threadIdx.x, lane = t & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);  // uniform: column addresses stay in scalar registers
   double2* A = Hb + (size_t)b * n * n;
   double* base = work + (size_t)b * eig_stride(n, nb);
   double2* ecx = reinterpret_cast<double2*>(base);
   double2* dph = ecx + n;
   double* Z = lu_in_lds ? reinterpret_cast<double*>(part) : reinterpret_cast<double*>(dph + n);
 
-  double2 v[R], w[R];
+  const __amdgpu_buffer_rsrc_t Ar = __builtin_amdgcn_make_buffer_rsrc(A, 0, n * n * 16, 0x00027000);
+  double2 x[R];  // wave 0: its rows of the last reflector
 #pragma unroll
-  for (int r = 0; r < R; ++r) v[r] = w[r] = make_double2(0.0, 0.0);
-  for (int i = t; i < n; i += ROW_NT) {
-    scol[i] = A[i];
-    sp[i] = make_double2(0.0, 0.0);
-  }
+  for (int r = 0; r < R; ++r) x[r] = make_double2(0.0, 0.0);
+  for (int i = t; i < n; i += ROW_NT) scol[i] = A[i];
+  for (int i = t; i < ROW_GROUPS * n; i += ROW_NT) psum[i] = make_double2(0.0, 0.0);
   __syncthreads();
   for (int k = 0; k + 1 < n; ++k) {
-    // the wave's first columns behind k: loads in flight during the vector phase
-    const int j0 = k + 1 + ((wave - (k + 1)) & (ROW_WAVES - 1));
-    double2 a[CB][R];
-#pragma unroll
-    for (int c = 0; c < CB; ++c)
-#pragma unroll
-      for (int r = 0; r < R; ++r) {
-        const int j = j0 + ROW_WAVES * c, i = lane + 64 * r;
-        if (j < n && i < n && i > k) a[c][r] = A[(size_t)j * n + i];
-      }
-    // w of reflector k - 1, column k, reflector k (every wave for itself)
-    double2 p[R], x[R];
-    double kk = 0.0;
+    const int j0 = k + 1 + ((wave - (k + 1)) & (ROW_WAVES - 1));  // the wave's first column behind k
+    // A column's rows through buffer accesses: rows that are not behind k get an offset past the buffer, so
+    // their loads give zero and their stores are dropped without a branch, which would hide from the
+    // compiler how many accesses are in flight and make every wait one for all of them.
+    unsigned row[R];
 #pragma unroll
     for (int r = 0; r < R; ++r) {
       const int i = lane + 64 * r;
-      p[r] = i < n ? sp[i] : make_double2(0.0, 0.0);
-      x[r] = i < n && i >= k ? scol[i] : make_double2(0.0, 0.0);
-      kk += v[r].x * p[r].x + v[r].y * p[r].y;  // v^H p (real)
+      row[r] = i > k && i < n ? (unsigned)i * 16u : kNoRow;
     }
-    kk = wave_sum(kk);
-#pragma unroll
-    for (int r = 0; r < R; ++r) w[r] = make_double2(p[r].x - kk * v[r].x, p[r].y - kk * v[r].y);
-    // v_k and w_k of reflector k - 1 at row k, from the lane that holds it
-    double2 vk = make_double2(0.0, 0.0), wk = vk;
-#pragma unroll
-    for (int r = 0; r < R; ++r)
-      if ((k >> 6) == r) {
-        const int l = k & 63;
-        vk.x = __shfl(v[r].x, l, 64);
-        vk.y = __shfl(v[r].y, l, 64);
-        wk.x = __shfl(w[r].x, l, 64);
-        wk.y = __shfl(w[r].y, l, 64);
-      }
-    double xx = 0.0;
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-      const int i = lane + 64 * r;
-      const double re = (v[r].x * wk.x + v[r].y * wk.y) + (w[r].x * vk.x + w[r].y * vk.y);
-      const double im = (v[r].y * wk.x - v[r].x * wk.y) + (w[r].y * vk.x - w[r].x * vk.y);
-      x[r].x -= 2.0 * re;
-      x[r].y -= 2.0 * im;
-      if (i > k && i < n) xx += x[r].x * x[r].x + x[r].y * x[r].y;
-      if (i == k && wave == 0) d[k] = x[r].x;
-    }
-    xx = wave_sum(xx);
-    double2 x0 = make_double2(0.0, 0.0);
-#pragma unroll
-    for (int r = 0; r < R; ++r)
-      if (((k + 1) >> 6) == r) {
-        x0.x = __shfl(x[r].x, (k + 1) & 63, 64);
-        x0.y = __shfl(x[r].y, (k + 1) & 63, 64);
-      }
-    // the reflector of the last column is none: its sub-diagonal entry stays as it is
-    const bool last = k + 2 >= n;
-    const double xn = sqrt(xx), ax0 = sqrt(x0.x * x0.x + x0.y * x0.y);
-    const double2 ph = ax0 > 0.0 ? make_double2(x0.x / ax0, x0.y / ax0) : make_double2(1.0, 0.0);
-    const double2 alpha = make_double2(-ph.x * xn, -ph.y * xn);
-    // v = (x - alpha e1) / |x - alpha e1|;  |x - alpha e1|² = 2(|x|² + |x||x0|)
-    const double vn = sqrt(2.0 * (xn * xn + xn * ax0));
-    const double rv = !last && xn > 0.0 ? 1.0 / vn : 0.0;
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-      const int i = lane + 64 * r;
-      double2 y = make_double2(0.0, 0.0);
-      if (i > k && i < n && rv > 0.0) {
-        y = x[r];
-        if (i == k + 1) {
-          y.x -= alpha.x;
-          y.y -= alpha.y;
-        }
-        y.x *= rv;
-        y.y *= rv;
-      }
-      x[r] = y;
-      if (wave == 0 && i < n) {
-        sv[i] = v[r];
-        sw[i] = w[r];
-        sx[i] = y;
-        if (i > k && !last) A[(size_t)k * n + i] = y;  // the reflector, for the back-transformation
-      }
-    }
-    if (t == 0) ecx[k] = last ? x0 : alpha;
-    __syncthreads();
-    // pass k
-    double2 q[R];
-#pragma unroll
-    for (int r = 0; r < R; ++r) q[r] = make_double2(0.0, 0.0);
-    for (int jb = j0; jb < n; jb += CB * ROW_WAVES) {
-      if (jb != j0) {
-#pragma unroll
-        for (int c = 0; c < CB; ++c)
-#pragma unroll
-          for (int r = 0; r < R; ++r) {
-            const int j = jb + ROW_WAVES * c, i = lane + 64 * r;
-            if (j < n && i < n && i > k) a[c][r] = A[(size_t)j * n + i];
-          }
-      }
+    auto load = [&](double2(&a)[CB][R], int jb) {
 #pragma unroll
       for (int c = 0; c < CB; ++c) {
         const int j = jb + ROW_WAVES * c;
-        if (j >= n) break;
-        const double2 vj = sv[j], wj = sw[j], xj = sx[j];
 #pragma unroll
-        for (int r = 0; r < R; ++r) {
-          const int i = lane + 64 * r;
-          if (i < n && i > k) {
-            double2 z = a[c][r];
-            const double re = (v[r].x * wj.x + v[r].y * wj.y) + (w[r].x * vj.x + w[r].y * vj.y);
-            const double im = (v[r].y * wj.x - v[r].x * wj.y) + (w[r].y * vj.x - w[r].x * vj.y);
-            z.x -= 2.0 * re;
-            z.y -= 2.0 * im;
-            A[(size_t)j * n + i] = z;
-            if (j == k + 1) scol[i] = z;
-            q[r].x += z.x * xj.x - z.y * xj.y;
-            q[r].y += z.x * xj.y + z.y * xj.x;
-          }
+        for (int r = 0; r < R; ++r)
+          if (64 * r + 63 > k) a[c][r] = buf_load(Ar, j < n ? row[r] : kNoRow, min(j, n - 1) * n * 16);
+      }
+    };
+    double2 a0[CB][R], a1[CB][R];
+    load(a0, j0);  // in flight during the vector phase
+    if (wave == 0) {
+      // w of reflector k - 1, column k, reflector k
+      double2 p[R], v[R], w[R];
+      double kk = 0.0;
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        const int i = lane + 64 * r;
+        v[r] = x[r];
+        p[r] = make_double2(0.0, 0.0);
+        x[r] = i < n && i >= k ? scol[i] : make_double2(0.0, 0.0);
+#pragma unroll
+        for (int g = 0; g < ROW_GROUPS; ++g) {
+          const double2 y = psum[g * n + min(i, n - 1)];
+          p[r].x += y.x;
+          p[r].y += y.y;
+        }
+        kk += v[r].x * p[r].x + v[r].y * p[r].y;  // v^H p (real); v is zero past the matrix
+      }
+      kk = wave_sum(kk);
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        w[r] = make_double2(2.0 * (p[r].x - kk * v[r].x), 2.0 * (p[r].y - kk * v[r].y));
+        if (lane + 64 * r < n) {
+          sv[lane + 64 * r] = v[r];
+          sw[lane + 64 * r] = w[r];
         }
       }
+      const double2 vk = sv[k], wk = sw[k];  // (the wave's own stores)
+      double xx = 0.0;
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        const int i = lane + 64 * r;
+        rank2(x[r], v[r], w[r], vk, wk);
+        if (i > k && i < n) xx += x[r].x * x[r].x + x[r].y * x[r].y;
+        if (i == k) d[k] = x[r].x;
+        if (i == k + 1) sx[i] = x[r];
+      }
+      xx = wave_sum(xx);
+      const double2 x0 = sx[k + 1];
+      // the last column has no reflector: its sub-diagonal entry stays as it is
+      const bool last = k + 2 >= n;
+      const double xn = sqrt(xx), ax0 = sqrt(x0.x * x0.x + x0.y * x0.y);
+      const double2 ph = ax0 > 0.0 ? make_double2(x0.x / ax0, x0.y / ax0) : make_double2(1.0, 0.0);
+      const double2 alpha = make_double2(-ph.x * xn, -ph.y * xn);
+      // v = (x - alpha e1) / |x - alpha e1|;  |x - alpha e1|² = 2(|x|² + |x||x0|)
+      const double vn = sqrt(2.0 * (xn * xn + xn * ax0));
+      const double rv = !last && xn > 0.0 ? 1.0 / vn : 0.0;
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        const int i = lane + 64 * r;
+        double2 y = make_double2(0.0, 0.0);
+        if (i > k && i < n && rv > 0.0) {
+          y = x[r];
+          if (i == k + 1) {
+            y.x -= alpha.x;
+            y.y -= alpha.y;
+          }
+          y.x *= rv;
+          y.y *= rv;
+        }
+        x[r] = y;
+        if (i < n) {
+          sx[i] = y;
+          if (i > k && !last) A[(size_t)k * n + i] = y;  // the reflector, for the back-transformation
+        }
+      }
+      if (lane == 0) ecx[k] = last ? x0 : alpha;
     }
+    __syncthreads();
+    // the column factors of this wave's columns, a column per lane (32 at most): a lane move each per use
+    // instead of an LDS read with its latency
+    double2 cv = make_double2(0.0, 0.0), cw = cv, cx = cv;
+    {
+      const int j = j0 + ROW_WAVES * lane;
+      if (j < n) {
+        cv = sv[j];
+        cw = sw[j];
+        cx = sx[j];
+      }
+    }
+    double2 vv[R], ww[R];  // of the rows behind k
 #pragma unroll
     for (int r = 0; r < R; ++r) {
       const int i = lane + 64 * r;
-      if (i < n) part[(size_t)wave * n + i] = q[r];
-      v[r] = x[r];
+      const double2 z = make_double2(0.0, 0.0);
+      vv[r] = i > k && i < n ? sv[i] : z;
+      ww[r] = i > k && i < n ? sw[i] : z;
     }
+    // pass k: the next columns' loads go out before this batch's stores
+    double2 q[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) q[r] = make_double2(0.0, 0.0);
+    // RLO: the first row group with rows behind k (the groups before it are not touched)
+    auto run = [&](auto rlo) {
+      constexpr int RLO = decltype(rlo)::value;
+      auto next = [&](double2(&a)[CB][R], int jb) {
+#pragma unroll
+        for (int c = 0; c < CB; ++c) {
+          const int j = jb + ROW_WAVES * c;
+#pragma unroll
+          for (int r = RLO; r < R; ++r) a[c][r] = buf_load(Ar, j < n ? row[r] : kNoRow, min(j, n - 1) * n * 16);
+        }
+      };
+      auto pass = [&](double2(&a)[CB][R], int jb) {
+#pragma unroll
+        for (int c = 0; c < CB; ++c) {
+          const int j = jb + ROW_WAVES * c, jc = min(j, n - 1), l = min((j - j0) / ROW_WAVES, 63);
+          const double2 vj = lane_of(cv, l), wj = lane_of(cw, l), xj = lane_of(cx, l);
+#pragma unroll
+          for (int r = RLO; r < R; ++r) {
+            double2& z = a[c][r];
+            rank2(z, vv[r], ww[r], vj, wj);
+            buf_store(Ar, j < n ? row[r] : kNoRow, jc * n * 16, z);
+            q[r].x = fma(z.x, xj.x, fma(-z.y, xj.y, q[r].x));
+            q[r].y = fma(z.x, xj.y, fma(z.y, xj.x, q[r].y));
+          }
+          if (j == k + 1) {
+#pragma unroll
+            for (int r = RLO; r < R; ++r)
+              if (lane + 64 * r < n) scol[lane + 64 * r] = a[c][r];
+          }
+        }
+      };
+      constexpr int S = CB * ROW_WAVES;
+      for (int jb = j0; jb < n; jb += 2 * S) {
+        next(a1, jb + S);
+        pass(a0, jb);
+        next(a0, jb + 2 * S);
+        pass(a1, jb + S);
+      }
+    };
+    const int rlo = (k + 1) >> 6;
+    if (rlo == 0)
+      run(std::integral_constant<int, 0>{});
+    else if (rlo == 1)
+      run(std::integral_constant<int, 1>{});
+    else if (R > 2 && rlo == 2)
+      run(std::integral_constant<int, (R > 2 ? 2 : 1)>{});
+    else if (R > 3)
+      run(std::integral_constant<int, (R > 3 ? 3 : 1)>{});
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+      if (lane + 64 * r < n) part[(size_t)wave * n + lane + 64 * r] = q[r];
     __syncthreads();
-    if (t < n) {
+    // the waves' products in two stages: four by four here, the two sums in the vector phase
+    if ((t & 255) < n) {
       double2 s = make_double2(0.0, 0.0);
 #pragma unroll
-      for (int g = 0; g < ROW_WAVES; ++g) {
-        const double2 y = part[(size_t)g * n + t];
+      for (int u = 0; u < ROW_WAVES / ROW_GROUPS; ++u) {
+        const double2 y = part[(size_t)((t >> 8) * (ROW_WAVES / ROW_GROUPS) + u) * n + (t & 255)];
         s.x += y.x;
         s.y += y.y;
       }
-      sp[t] = s;
+      psum[(t >> 8) * n + (t & 255)] = s;
     }
     __syncthreads();
   }
