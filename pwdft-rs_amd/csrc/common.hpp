@@ -543,6 +543,11 @@ bool rr_small_supported(int m);
 // skip (device, may be null): the launch does nothing while *skip is nonzero
 void launch_rr_small(Context& c, int npw, int m, int nres, int nk, const void* Y, const void* HY, void* V,
                      double* lam, double* res, double floor_rel, const int* skip = nullptr);
+// the same over the whole chip (longer vectors), with rr_split_bytes of device workspace; lam and res may be
+// pinned host memory
+size_t rr_split_bytes(int npw, int m, int nk);
+void launch_rr_split(Context& c, int npw, int m, int nres, int nk, const void* Y, const void* HY, void* V, double* lam,
+                     double* res, double floor_rel, void* ws);
 // warm-start Rayleigh-Ritz of nk dense n×n Hamiltonians on n×nb start blocks (Vprev may be
 // null: full solve), residual gate tol per block; w (nk×nb) and V (nk blocks of n×nb) on the
 // device, used_full / max_resid (nk each, host, may be null)

@@ -1313,7 +1313,7 @@ struct Solve {
   int fprec = PWK_FP64;                // precision of the filter's H·ψ
   int degree = 10;
   std::vector<double> ub;              // per-(channel, k) upper bound of the spectrum
-  DevBuf F0, F1, F2, HYf, Y64, HY64, YH, sS, sH, sU, sT, sX, sXH, sW, sC, s_ev, s_lam, s_work, lowest;
+  DevBuf F0, F1, F2, HYf, Y64, HY64, YH, sS, sH, sU, sT, sX, sXH, sW, sC, s_ev, s_lam, s_work, rr_ws, lowest;
   DevBuf kin_all64, kin_all32;              // nk × npw kinetic diagonals
   DevBuf R64, resid;                        // H·V after Rayleigh-Ritz, residual norms
   std::vector<double> resid_host;
@@ -1825,6 +1825,11 @@ void Solve::setup() {
     s_lam.ensure((size_t)2 * nke * nbs * 8);  // Ritz values, then residual norms (fused path)
     pin_rr.ensure((size_t)2 * nke * nbs * 8);
     rr_pinned = pin_rr.as<double>();
+    // Rayleigh-Ritz over the whole chip off the fused small grids (whose passes run batched across requests,
+    // or captured, with the one-workgroup form) from 512 plane waves: 1189 × 32 vectors, 4 k-points 633 us
+    // in one workgroup per k-point
+    if (rr_small_supported(nbs) && npw >= 512 && !hpsi_small_supported(c, PWK_FP64, nch_all))
+      rr_ws.ensure(rr_split_bytes(npw, nbs, nke));
     s_work.ensure(heev_work_doubles(nbs, nbs, nke) * 8);
     projall.ensure((size_t)nk * std::max(1, nch_all) * nbs * 16);
     ev_sub.assign((size_t)ns * nk * nbs, 0.0);
@@ -2008,7 +2013,10 @@ void Solve::rr_launch(const double2* Y, const double2* HY) {
     TimedScope ts(c, "scf_rayleigh_ritz");
     const size_t nkm = (size_t)nke * nbs;
     // Ritz values and residual norms go straight into pinned host memory
-    launch_rr_small(c, npw, nbs, nb, nke, Y, HY, Vc(), rr_pinned, rr_pinned + nkm, 1e-14);
+    if (rr_ws.p)
+      launch_rr_split(c, npw, nbs, nb, nke, Y, HY, Vc(), rr_pinned, rr_pinned + nkm, 1e-14, rr_ws.p);
+    else
+      launch_rr_small(c, npw, nbs, nb, nke, Y, HY, Vc(), rr_pinned, rr_pinned + nkm, 1e-14);
     return;
   }
   rr_general(Y, HY);

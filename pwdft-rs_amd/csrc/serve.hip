@@ -372,12 +372,13 @@ size_t scf_footprint(const pwk_crystal& cr, const pwk_scf_params& p) {
     b += 8 * nke * n * nbs * 16;                                          // filter and Rayleigh-Ritz blocks
     b += 8 * nke * nbs * nbs * 16 + heev_work_doubles((int)nbs, (int)nbs, (int)nke) * 8;
     b += (size_t)nk * std::max<size_t>(1, nch) * nbs * 16 + 3 * nke * n * 16;  // projections, Lanczos
+    b += rr_split_bytes(npw, (int)nbs, (int)nke);
   } else {
     b += (size_t)nk * n * n * 16 + heev_work_doubles(npw, (int)nb, nk) * 8;    // dense H batch, scratch
   }
   b += (size_t)nk * n * nb * 16 + (size_t)nk * std::max<size_t>(1, nch) * nb * 16;  // final expectations
-  // density and H·psi workspaces: stick buffers of the band batch or per-group density partials
-  b += std::max(nke * nbs * (size_t)dims[2] * n * 16, (size_t)128 * N * 8) + ((size_t)64 << 20);
+  // density and H·psi workspaces: stick buffers of the band batch and per-group density partials
+  b += nke * nbs * (size_t)dims[2] * n * 16 + (size_t)129 * N * 8 + ((size_t)64 << 20);
   return b;
 }
 

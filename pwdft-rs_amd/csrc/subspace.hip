@@ -189,20 +189,12 @@ struct RrLds {
   double red[16][MB];
 };
 
+// The Gram products of one block over the rows [row0, row_end): S into J.A and Hs into L.Hs.
 template <int MB>
-__device__ __forceinline__ void rr_small_body(int k, int npw, int m, int nres, const double2* __restrict__ Yb,
-                                              const double2* __restrict__ HYb, double2* __restrict__ Vb,
-                                              double* __restrict__ lam_out, double* __restrict__ res_out,
-                                              double floor_rel, const int* __restrict__ skip) {
-  static_assert(MB == 16 || MB == 32, "blocks of up to 16 or 32 vectors");
-  if (skip && *skip) return;  // a filter pass after the residual gate passed (uniform)
-  extern __shared__ unsigned char smem_raw[];
-  RrLds<MB>& L = *reinterpret_cast<RrLds<MB>*>(smem_raw);
+__device__ __forceinline__ void rr_gram(RrLds<MB>& L, const double2* __restrict__ Y, const double2* __restrict__ HY,
+                                        int npw, int m, int row0, int row_end) {
   JacobiLdsT<MB>& J = L.J;
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-  const double2* Y = Yb + (size_t)k * npw * m;
-  const double2* HY = HYb + (size_t)k * npw * m;
-  double2* V = Vb + (size_t)k * npw * m;
   // S(i, j) = Σ_G conj(Y_i) Y_j and Hs(i, j) = Σ_G conj(Y_i) (HY)_j over row chunks staged in LDS
   // (coalesced loads; the next chunk's loads are issued before this chunk's products). Wave w takes
   // rows [w·RR_ROWS/4, (w+1)·RR_ROWS/4) of every chunk and each lane a BLK × BLK block of entries,
@@ -221,13 +213,13 @@ __device__ __forceinline__ void rr_small_body(int k, int npw, int m, int nres, c
     for (int q = 0; q < LPT; ++q) {
       const int e = t + q * RR_NT;
       const int gg = e % RR_ROWS, i = e / RR_ROWS, g = g0 + gg;
-      const bool in = e < RR_ROWS * m && g < npw;
+      const bool in = e < RR_ROWS * m && g < row_end;
       py[q] = in ? Y[(size_t)i * npw + g] : make_double2(0.0, 0.0);
       ph[q] = in ? HY[(size_t)i * npw + g] : make_double2(0.0, 0.0);
     }
   };
-  load_chunk(0);
-  for (int g0 = 0; g0 < npw; g0 += RR_ROWS) {
+  load_chunk(row0);
+  for (int g0 = row0; g0 < row_end; g0 += RR_ROWS) {
 #pragma unroll
     for (int q = 0; q < LPT; ++q) {
       const int e = t + q * RR_NT;
@@ -237,8 +229,8 @@ __device__ __forceinline__ void rr_small_body(int k, int npw, int m, int nres, c
       }
     }
     __syncthreads();
-    if (g0 + RR_ROWS < npw) load_chunk(g0 + RR_ROWS);
-    const int r0 = wave * WROWS, r1 = min(npw - g0, r0 + WROWS);
+    if (g0 + RR_ROWS < row_end) load_chunk(g0 + RR_ROWS);
+    const int r0 = wave * WROWS, r1 = min(row_end - g0, r0 + WROWS);
     for (int gg = r0; gg < r1; ++gg) {
       double2 a[BLK], b[BLK], h[BLK];
 #pragma unroll
@@ -281,6 +273,13 @@ __device__ __forceinline__ void rr_small_body(int k, int npw, int m, int nres, c
     }
     __syncthreads();
   }
+}
+
+// From the Gram products (J.A, L.Hs) to the combination C (L.C) and the Ritz values (J.A's diagonal in J.order).
+template <int MB>
+__device__ __forceinline__ void rr_mid(RrLds<MB>& L, int m, double floor_rel) {
+  JacobiLdsT<MB>& J = L.J;
+  const int t = threadIdx.x;
   // Hermitian parts (subspace.hip k_hermitize), V = I
   for (int e = t; e < m * m; e += RR_NT) {
     const int i = e % m, j = e / m;
@@ -409,6 +408,25 @@ __device__ __forceinline__ void rr_small_body(int k, int npw, int m, int nres, c
     }
     L.C[i][jj] = make_double2(re, im);
   }
+  __syncthreads();
+}
+
+template <int MB>
+__device__ __forceinline__ void rr_small_body(int k, int npw, int m, int nres, const double2* __restrict__ Yb,
+                                              const double2* __restrict__ HYb, double2* __restrict__ Vb,
+                                              double* __restrict__ lam_out, double* __restrict__ res_out,
+                                              double floor_rel, const int* __restrict__ skip) {
+  static_assert(MB == 16 || MB == 32, "blocks of up to 16 or 32 vectors");
+  if (skip && *skip) return;  // a filter pass after the residual gate passed (uniform)
+  extern __shared__ unsigned char smem_raw[];
+  RrLds<MB>& L = *reinterpret_cast<RrLds<MB>*>(smem_raw);
+  JacobiLdsT<MB>& J = L.J;
+  const int t = threadIdx.x, wave = t >> 6;
+  const double2* Y = Yb + (size_t)k * npw * m;
+  const double2* HY = HYb + (size_t)k * npw * m;
+  double2* V = Vb + (size_t)k * npw * m;
+  rr_gram<MB>(L, Y, HY, npw, m, 0, npw);
+  rr_mid<MB>(L, m, floor_rel);
   if (t < m) lam_out[(size_t)k * m + t] = J.A[J.order[t]][J.order[t]].x;
   __syncthreads();
   double acc[MB];
@@ -461,6 +479,112 @@ __device__ __forceinline__ void rr_small_body(int k, int npw, int m, int nres, c
     double v = 0.0;
     for (int w = 0; w < RR_NT / 64; ++w) v += L.red[w][t];
     res_out[(size_t)k * m + t] = sqrt(v);
+  }
+}
+
+// ---- the same step over the whole chip, for longer vectors --------------------------------------
+// One workgroup per block reads 2·npw·m entries twice: at 1189 plane waves and 32 vectors 633 us, on 4 of
+// 256 CUs for 4 k-points. Here the Gram products and the new vectors with their residuals are spread over
+// row chunks, with the small dense steps between them in one workgroup per block as before; sums over the
+// chunks are taken in chunk order.
+constexpr int RR_GROWS = 64, RR_VROWS = 64;  // rows per workgroup of the Gram and vector launches
+
+// part[block][chunk][S, Hs][m·m]
+template <int MB>
+__global__ void __launch_bounds__(RR_NT) k_rr_gram(int npw, int m, const double2* __restrict__ Yb,
+                                                   const double2* __restrict__ HYb, double2* __restrict__ part) {
+  extern __shared__ unsigned char smem_raw[];
+  RrLds<MB>& L = *reinterpret_cast<RrLds<MB>*>(smem_raw);
+  const int k = blockIdx.y, row0 = blockIdx.x * RR_GROWS;
+  rr_gram<MB>(L, Yb + (size_t)k * npw * m, HYb + (size_t)k * npw * m, npw, m, row0, min(npw, row0 + RR_GROWS));
+  double2* o = part + ((size_t)k * gridDim.x + blockIdx.x) * 2 * m * m;
+  for (int e = threadIdx.x; e < m * m; e += RR_NT) {
+    o[e] = L.J.A[e / m][e % m];
+    o[m * m + e] = L.Hs[e / m][e % m];
+  }
+}
+
+template <int MB>
+__global__ void __launch_bounds__(RR_NT) k_rr_mid(int m, int nchunks, const double2* __restrict__ part,
+                                                  double floor_rel, double2* __restrict__ Cb,
+                                                  double* __restrict__ lam_dev, double* __restrict__ lam_out) {
+  extern __shared__ unsigned char smem_raw[];
+  RrLds<MB>& L = *reinterpret_cast<RrLds<MB>*>(smem_raw);
+  const int k = blockIdx.x;
+  const double2* p = part + (size_t)k * nchunks * 2 * m * m;
+  for (int e = threadIdx.x; e < 2 * m * m; e += RR_NT) {
+    double2 s = make_double2(0.0, 0.0);
+#pragma unroll 8
+    for (int x = 0; x < nchunks; ++x) {
+      const double2 v = p[(size_t)x * 2 * m * m + e];
+      s.x += v.x;
+      s.y += v.y;
+    }
+    const int f = e < m * m ? e : e - m * m;
+    (e < m * m ? L.J.A : L.Hs)[f / m][f % m] = s;
+  }
+  __syncthreads();
+  rr_mid<MB>(L, m, floor_rel);
+  for (int e = threadIdx.x; e < m * m; e += RR_NT) Cb[(size_t)k * m * m + e] = L.C[e / m][e % m];  // [i][jj]
+  if ((int)threadIdx.x < m) {
+    const double l = L.J.A[L.J.order[threadIdx.x]][L.J.order[threadIdx.x]].x;
+    lam_dev[(size_t)k * m + threadIdx.x] = l;
+    lam_out[(size_t)k * m + threadIdx.x] = l;
+  }
+}
+
+// V = Y·C and the residual weights of RR_VROWS rows: a lane per row, wave w the columns 8w .. 8w + 7 of
+// each turn, whose factors C are uniform over the wave (scalar loads). rpart[block][chunk][m].
+__global__ void __launch_bounds__(RR_NT) k_rr_vectors(int npw, int m, int nres, const double2* __restrict__ Yb,
+                                                      const double2* __restrict__ HYb, const double2* __restrict__ Cb,
+                                                      const double* __restrict__ lam, double2* __restrict__ Vb,
+                                                      double* __restrict__ rpart) {
+  constexpr int CB = 8;
+  const int k = blockIdx.y, lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int g = blockIdx.x * RR_VROWS + lane, gr = min(g, npw - 1);
+  const double2* Y = Yb + (size_t)k * npw * m;
+  const double2* HY = HYb + (size_t)k * npw * m;
+  const double2* C = Cb + (size_t)k * m * m;
+  for (int jc = wave * CB; jc < m; jc += CB * (RR_NT / 64)) {
+    double vr[CB], vi[CB], rr[CB], ri[CB];
+#pragma unroll
+    for (int q = 0; q < CB; ++q) vr[q] = vi[q] = rr[q] = ri[q] = 0.0;
+#pragma unroll 4
+    for (int i = 0; i < m; ++i) {
+      const double2 y = Y[(size_t)i * npw + gr], h = HY[(size_t)i * npw + gr];
+#pragma unroll
+      for (int q = 0; q < CB; ++q) {
+        const double2 c = C[i * m + min(jc + q, m - 1)];
+        vr[q] += y.x * c.x - y.y * c.y;
+        vi[q] += y.x * c.y + y.y * c.x;
+        rr[q] += h.x * c.x - h.y * c.y;
+        ri[q] += h.x * c.y + h.y * c.x;
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < CB; ++q) {
+      const int jj = jc + q;
+      if (jj >= m) continue;  // uniform
+      if (g < npw) Vb[((size_t)k * m + jj) * npw + g] = make_double2(vr[q], vi[q]);
+      if (jj >= nres) continue;
+      const double l = lam[(size_t)k * m + jj];
+      const double dx = rr[q] - l * vr[q], dy = ri[q] - l * vi[q];
+      double v = g < npw ? dx * dx + dy * dy : 0.0;
+      for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+      if (lane == 0) rpart[((size_t)k * gridDim.x + blockIdx.x) * m + jj] = v;
+    }
+  }
+}
+
+__global__ void __launch_bounds__(64) k_rr_norms(int m, int nres, int nchunks, const double* __restrict__ rpart,
+                                                 double* __restrict__ res_out) {
+  const int k = blockIdx.x;
+  for (int j = threadIdx.x; j < nres; j += 64) {
+    double s = 0.0;
+#pragma unroll 8
+    for (int x = 0; x < nchunks; ++x) s += rpart[((size_t)k * nchunks + x) * m + j];
+    res_out[(size_t)k * m + j] = sqrt(s);
   }
 }
 
@@ -570,6 +694,37 @@ void launch_rr_small(Context& c, int npw, int m, int nres, int nk, const void* Y
     go(k_rr_small<16>, sizeof(RrLds<16>));
   else
     go(k_rr_small<32>, sizeof(RrLds<32>));
+  PWK_HIP(hipGetLastError());
+}
+
+size_t rr_split_bytes(int npw, int m, int nk) {
+  const size_t g = (npw + RR_GROWS - 1) / RR_GROWS, v = (npw + RR_VROWS - 1) / RR_VROWS;
+  return (size_t)nk * (g * 2 * m * m * sizeof(double2) + (size_t)m * m * sizeof(double2) + (v + 1) * m * sizeof(double));
+}
+
+void launch_rr_split(Context& c, int npw, int m, int nres, int nk, const void* Y, const void* HY, void* V, double* lam,
+                     double* res, double floor_rel, void* ws) {
+  PWK_REQUIRE(rr_small_supported(m) && nres <= m && npw >= m && nk >= 1 && nk <= 65535, PWK_E_INVALID,
+              "bad Rayleigh-Ritz shape");
+  const int g = (npw + RR_GROWS - 1) / RR_GROWS, v = (npw + RR_VROWS - 1) / RR_VROWS;
+  double2* part = (double2*)ws;
+  double2* C = part + (size_t)nk * g * 2 * m * m;
+  double* rpart = (double*)(C + (size_t)nk * m * m);
+  double* lam_dev = rpart + (size_t)nk * v * m;
+  auto go = [&](auto gram, auto mid, size_t sh) {
+    ensure_lds_limit((const void*)gram, sh);
+    ensure_lds_limit((const void*)mid, sh);
+    gram<<<dim3((unsigned)g, (unsigned)nk), RR_NT, sh, c.stream>>>(npw, m, (const double2*)Y, (const double2*)HY, part);
+    mid<<<(unsigned)nk, RR_NT, sh, c.stream>>>(m, g, part, floor_rel, C, lam_dev, lam);
+  };
+  if (m <= 16)
+    go(k_rr_gram<16>, k_rr_mid<16>, sizeof(RrLds<16>));
+  else
+    go(k_rr_gram<32>, k_rr_mid<32>, sizeof(RrLds<32>));
+  k_rr_vectors<<<dim3((unsigned)v, (unsigned)nk), RR_NT, 0, c.stream>>>(npw, m, nres, (const double2*)Y,
+                                                                        (const double2*)HY, C, lam_dev, (double2*)V,
+                                                                        rpart);
+  k_rr_norms<<<(unsigned)nk, 64, 0, c.stream>>>(m, nres, v, rpart, res);
   PWK_HIP(hipGetLastError());
 }
 
