@@ -316,7 +316,8 @@ struct Context {
   int pl_rows = 0, pl_ra = 0, pl_rb = 0;
   DevBuf pl_src;   // int32 pl_rows·(ny + 1)
   DevBuf st_off;   // int32 nsticks
-  // every plane wave within a quarter of each axis (planes.hpp, Quarter): the pruned passes run, with
+  // every plane wave within a quarter of each axis (planes.hpp, Quarter) and every axis a register length:
+  // the pruned passes run (also where nx != ny), with
   // the stick of each held (row, column) and the image element of each stick
   bool quarter = false;
   DevBuf q_src, q_off;
@@ -433,12 +434,18 @@ void launch_zinv(Context& c, int nb, const void* psi, void* out, int precision, 
 // hpsi_sphere.hip: the passes on spheres within a quarter of the axes (c.quarter)
 template <typename T>
 void sphere_zinv(Context& c, int nb, const void* psi, void* out, const int* list);
+// (rows: where nx != ny, sphere_rows_elems entries for the held rows [band][i3][row][i2], which
+// sphere_rows_inverse fills from the sticks)
+size_t sphere_rows_elems(const Context& c, int nb);
 template <typename T>
-void sphere_plane(Context& c, int nb, void* buf, const T* vr);
+void sphere_rows_inverse(Context& c, int nb, void* buf, void* rows);
+template <typename T>
+void sphere_plane(Context& c, int nb, void* buf, const T* vr, void* rows);
 template <typename T>
 void sphere_zfwd(Context& c, int nb, const void* buf, const T* kin, int nbk, const T* const* kin_of,
                  const void* psi, void* hpsi);
-// density.hip: the band density on square grids of register-length lines (fw on the host)
+// density.hip: the band density on square grids of register-length lines and on any with c.quarter (fw on
+// the host)
 void launch_density_sticks(Context& c, int nb, const void* psi, const double* fw_host, void* rho, int precision,
                            bool overwrite);
 void launch_hpsi_multi(Context& c, int nk, int nb, const void* psi, void* hpsi, int precision, const void* kin,

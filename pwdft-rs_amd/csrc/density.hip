@@ -118,6 +118,45 @@ __global__ void __launch_bounds__((DensityShape<T, N>::NT))
   }
 }
 
+// The same for grids with nx != ny, whose y-lines have been taken already (rows[band][i3][held row][i2],
+// sphere_rows_inverse): a lane per (i3, i2) transforms its x-line of every band of the group.
+template <typename T, int NX>
+__global__ void __launch_bounds__(64) k_cols_density(const typename V2t<T>::t* __restrict__ rows, int nb, int per,
+                                                     const double* __restrict__ fw, double* __restrict__ part, int ny,
+                                                     int nz) {
+  using V2 = typename V2t<T>::t;
+  using Q = Quarter<NX>;
+  const int l = blockIdx.x * 64 + threadIdx.x, g = blockIdx.y;
+  if (l >= ny * nz) return;
+  const int i3 = l / ny, i2 = l - i3 * ny;
+  double acc[NX];
+#pragma unroll
+  for (int q = 0; q < NX; ++q) acc[q] = 0.0;
+  const int b_end = min(nb, (g + 1) * per);
+  for (int b = g * per; b < b_end; ++b) {
+    const V2* up = rows + ((size_t)b * nz + i3) * Q::R * ny + i2;
+    const double f = fw[b];
+    T re[NX], im[NX];
+#pragma unroll
+    for (int j = 0; j < NX; ++j) {
+      V2 x;
+      x.x = x.y = 0;
+      if (Q::has(j)) x = up[Q::at(j) * ny];
+      re[j] = x.x;
+      im[j] = x.y;
+    }
+    fft_line<T, NX, 1>(re, im);
+#pragma unroll
+    for (int q = 0; q < NX; ++q) {
+      const double x = (double)re[LineOrder<NX>::pos(q)], y = (double)im[LineOrder<NX>::pos(q)];
+      acc[q] += f * (x * x + y * y);
+    }
+  }
+  double* out = part + ((size_t)g * nz + i3) * NX * ny + i2;
+#pragma unroll
+  for (int q = 0; q < NX; ++q) out[q * ny] = acc[q];
+}
+
 // rho[i1][i2][i3] (+)= Σ_g part[g][i3][i1][i2] in group order; a 32 × 32 (i2, i3) tile per workgroup
 // goes through LDS, so that both sides are read and written along their contiguous axis. Bound: the
 // partials' traffic (groups·N·8 bytes).
@@ -205,20 +244,27 @@ void density_sticks_t(Context& c, int nb, const void* psi, const double* fw_host
     const double* fw = c.work_b.as<double>();
     // about 1024 workgroups (four per CU): more only adds partial sums to store and read, fewer leave
     // CUs idle. Measured with the groups' count that this gives: 60 planes × 144 bands in 16 groups.
-    const int slots = plane_slots<T>(nx);
+    const bool square = nx == ny;
+    const int slots = square ? plane_slots<T>(nx) : 1;
     const int batches = (live + slots - 1) / slots;
-    const int per = std::max(1, (int)(((long)batches * nz + 1023) / 1024));
+    const long wgs = square ? nz : (ny * nz + 63) / 64;  // workgroups per group
+    const int per = std::max(1, (int)((batches * wgs + 1023) / 1024));
     groups = (batches + per - 1) / per;
     // one z-inverse buffer for all live bands, then the groups' partial sums
-    const size_t tb = (((size_t)live * nz * c.nsticks * sizeof(V2)) + 255) & ~(size_t)255;
+    const size_t ns = (size_t)live * nz * c.nsticks, held = square ? 0 : sphere_rows_elems(c, live);
+    const size_t tb = ((ns + held) * sizeof(V2) + 255) & ~(size_t)255;
     c.work_a.ensure(tb + (size_t)groups * c.N * sizeof(double));
     double* part = reinterpret_cast<double*>(c.work_a.as<unsigned char>() + tb);
     launch_zinv(c, live, psi, c.work_a.p, std::is_same<T, double>::value ? PWK_FP64 : PWK_FP32,
                 reinterpret_cast<const int*>(fw + live));
+    V2* rows = c.work_a.as<V2>() + ns;
+    if (!square) sphere_rows_inverse<T>(c, live, c.work_a.p, rows);
     switch (nx) {
 #define PWK_CASE(L)                                                             \
   case L:                                                                       \
-    if (c.quarter)                                                              \
+    if (!square)                                                                \
+      k_cols_density<T, L><<<dim3((unsigned)wgs, (unsigned)groups), 64, 0, c.stream>>>(rows, live, per, fw, part, ny, nz); \
+    else if (c.quarter)                                                              \
       plane_density<T, L, true>(c, c.work_a.p, live, per, groups, fw, part);    \
     else                                                                        \
       plane_density<T, L, false>(c, c.work_a.p, live, per, groups, fw, part);   \
@@ -228,6 +274,7 @@ void density_sticks_t(Context& c, int nb, const void* psi, const double* fw_host
       default:
         throw Error(PWK_E_UNSUPPORTED, "nx has no compiled kernel");
     }
+    PWK_HIP(hipGetLastError());
     const dim3 gs(blocks_for((size_t)ny, 32), blocks_for((size_t)nz, 32), (unsigned)nx);
     k_density_sum<<<gs, 256, 0, c.stream>>>(groups, nx, ny, nz, part, rho, overwrite ? 1 : 0);
     PWK_HIP(hipGetLastError());

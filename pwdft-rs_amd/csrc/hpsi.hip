@@ -204,11 +204,12 @@ __global__ void __launch_bounds__(256) k_vr_reorder(const double2* __restrict__ 
   n32[g] = (float)v;
 }
 
-// ---- full-grid path (grids with nx != ny, or an axis beyond the register lengths) --------
+// ---- full-grid path (an axis beyond the register lengths, or nx != ny with a wide sphere) --------
 // the stick path's plane and z kernels hold whole lines in registers: square planes, every axis
-// one of the register lengths
-bool stick_path_ok(const Context& c) {
-  return c.dims[0] == c.dims[1] && fft_len_compiled(c.dims[0]) && fft_len_compiled(c.dims[2]);
+// one of the register lengths; other grids of register lengths when the pruned passes apply (in FP64 up
+// to x-lines of 64 points: longer ones do not fit the registers of the x passes)
+bool stick_path_ok(const Context& c, bool f64) {
+  return (c.quarter && (c.dims[0] == c.dims[1] || !f64 || c.dims[0] <= 64)) || (c.dims[0] == c.dims[1] && fft_len_compiled(c.dims[0]) && fft_len_compiled(c.dims[2]));
 }
 
 // ψ scattered on the whole grid of each band of a chunk, batched 3D FFTs (one compiled
@@ -369,13 +370,13 @@ void hpsi_local(Context& c, const T* kin, int nb, int nbk, const void* psi, void
   using V2 = typename V2t<T>::t;
   int nx = c.dims[0], nz = c.dims[2];
   PWK_REQUIRE(c.have_v, PWK_E_STATE, "V_eff not set (pwk_set_veff)");
-  if (!stick_path_ok(c)) {
+  if (!stick_path_ok(c, std::is_same<T, double>::value)) {
     hpsi_fullgrid<T>(c, kin, nb, nbk, psi, hpsi);
     return;
   }
   PWK_REQUIRE(nb <= 65535, PWK_E_UNSUPPORTED, "too many bands in one H·psi launch");
-  size_t tb = (size_t)nb * nz * c.nsticks * sizeof(V2);
-  c.work_a.ensure(tb);
+  const size_t ns = (size_t)nb * nz * c.nsticks, rows = nx == c.dims[1] ? 0 : sphere_rows_elems(c, nb);
+  c.work_a.ensure((ns + rows) * sizeof(V2));
   V2* T_ = c.work_a.as<V2>();
   const T* vr = std::is_same<T, double>::value ? (const T*)c.vr64.p : (const T*)c.vr32.p;
   dim3 gz(blocks_for((size_t)c.nsticks, 64), (unsigned)nb);
@@ -386,8 +387,8 @@ void hpsi_local(Context& c, const T* kin, int nb, int nbk, const void* psi, void
   {
     TimedScope ts(c, "hpsi_plane");
     // (the pruned FP64 plane pass of 81 points does not fit the registers)
-    if (c.quarter && !(std::is_same<T, double>::value && nx > 80)) {
-      sphere_plane<T>(c, nb, T_, vr);
+    if (c.quarter && !(std::is_same<T, double>::value && nx > 80 && nx == c.dims[1])) {
+      sphere_plane<T>(c, nb, T_, vr, T_ + ns);
     } else {
       switch (nx) {
 #define PWK_CASE(L)                    \
@@ -483,17 +484,17 @@ void setup_basis(Context& c, int npw, const int32_t* m) {
     psrc[(size_t)off.back()] = (int32_t)s;
   }
   // pruned passes: every index within a quarter of its axis
-  c.quarter = stick_path_ok(c);
+  c.quarter = fft_len_compiled(nx) && fft_len_compiled(ny) && fft_len_compiled(nz);
   for (int i = 0; i < npw && c.quarter; ++i)
     for (int d = 0; d < 3; ++d) c.quarter = c.quarter && std::abs(m[3 * i + d]) <= (c.dims[d] - 1) / 4;
   std::vector<int32_t> qsrc, qoff;
   if (c.quarter) {
-    const int pb = (nx - 1) / 4, r = 2 * pb + 1, qld = ny | 1;
-    qsrc.assign((size_t)r * r, -1);
+    const int px = (nx - 1) / 4, py = (ny - 1) / 4, rx = 2 * px + 1, ry = 2 * py + 1, qld = ny | 1;
+    qsrc.assign((size_t)rx * ry, -1);
     for (size_t s = 0; s < xy.size(); ++s) {
       const int i1 = xy[s] / ny, i2 = xy[s] % ny;
-      const int h1 = i1 <= pb ? i1 : i1 - (nx - r), h2 = i2 <= pb ? i2 : i2 - (ny - r);
-      qsrc[(size_t)h1 * r + h2] = (int32_t)s;
+      const int h1 = i1 <= px ? i1 : i1 - (nx - rx), h2 = i2 <= py ? i2 : i2 - (ny - ry);
+      qsrc[(size_t)h1 * ry + h2] = (int32_t)s;
       qoff.push_back(h1 * qld + i2);
     }
   }
@@ -688,8 +689,9 @@ bool hpsi_batch_sticks(Context& c, int nent, const int32_t* ik, const int32_t* n
   const bool f64 = std::is_same<T, double>::value;
   const int nch = c.k(ik[0]).nch;
   // the stick buffer of the whole batch stays below 4 GiB
-  if (!stick_path_ok(c) || total > 65535 ||
-      total * (size_t)c.dims[2] * (size_t)c.nsticks * sizeof(typename V2t<T>::t) > ((size_t)4 << 30))
+  if (!stick_path_ok(c, f64) || total > 65535 ||
+      (total * (size_t)c.dims[2] * (size_t)c.nsticks +
+       (c.dims[0] == c.dims[1] ? 0 : sphere_rows_elems(c, (int)total))) * sizeof(typename V2t<T>::t) > ((size_t)4 << 30))
     return false;
   int nmax = 0;
   for (int e = 0; e < nent; ++e) {
@@ -793,7 +795,7 @@ void launch_density(Context& c, int nb, const void* psi, const double* fw_host, 
     launch_density_small(c, nb, psi, c.work_b.as<double>(), rho, dprec, overwrite);
     return;
   }
-  if (stick_path_ok(c)) {
+  if (stick_path_ok(c, dprec == PWK_FP64)) {
     launch_density_sticks(c, nb, psi, fw_host, rho, dprec, overwrite);
     return;
   }

@@ -188,6 +188,136 @@ __global__ void __launch_bounds__((PlaneShape<T, N>::NT))
   }
 }
 
+// ---- grids with nx != ny ------------------------------------------------------------------
+// The plane pass in three launches, so that each axis has its own compiled length: y-lines of the held rows
+// (sticks -> U[band][i3][held row][i2]), x-lines with the potential between (a lane per (i3, i2), its line
+// read and written along i2), y-lines back to the sticks. Only the held rows move between the launches.
+// si 50 × 25 × 25, 40 bands FP32: the whole-grid transforms this replaces took nine launches over all points.
+constexpr int RT = 64;
+
+template <typename T, int NY, int SIGN>
+__global__ void __launch_bounds__(RT) k_rows_q(typename V2t<T>::t* __restrict__ tbuf, typename V2t<T>::t* __restrict__ U,
+                                               int S, int nz, int rx, const int* __restrict__ src,
+                                               const int* __restrict__ st_off) {
+  using V2 = typename V2t<T>::t;
+  using Q = Quarter<NY>;
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
+  V2* P = reinterpret_cast<V2*>(smem_raw);  // [held row][LD]
+  const size_t pl = (size_t)blockIdx.y * nz + blockIdx.x;
+  V2* tp = tbuf + pl * S;
+  V2* up = U + pl * rx * NY;
+  if (SIGN > 0) {
+    const int n = rx * Q::R;
+    for (int e0 = threadIdx.x; e0 < n; e0 += 8 * RT) {
+      int s[8];
+      V2 v[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) s[u] = src[min(e0 + u * RT, n - 1)];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) v[u] = tp[max(s[u], 0)];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const int e = e0 + u * RT, r = e / Q::R;
+        V2 x;
+        x.x = s[u] >= 0 ? v[u].x : (T)0;
+        x.y = s[u] >= 0 ? v[u].y : (T)0;
+        if (e < n) P[r * Q::LD + Q::index(e - r * Q::R)] = x;
+      }
+    }
+  } else {
+#pragma unroll 8
+    for (int e = threadIdx.x; e < rx * NY; e += RT) P[e / NY * Q::LD + e % NY] = up[e];
+  }
+  __syncthreads();
+  for (int r = threadIdx.x; r < rx; r += RT) {
+    V2* row = P + r * Q::LD;
+    T re[NY], im[NY];
+#pragma unroll
+    for (int j = 0; j < NY; ++j) {
+      const bool in = SIGN < 0 || Q::has(j);
+      re[j] = in ? row[j].x : (T)0;
+      im[j] = in ? row[j].y : (T)0;
+    }
+    fft_line<T, NY, SIGN>(re, im);
+#pragma unroll
+    for (int f = 0; f < NY; ++f)
+      if (SIGN > 0 || Q::has(f)) {
+        row[f].x = re[LineOrder<NY>::pos(f)];
+        row[f].y = im[LineOrder<NY>::pos(f)];
+      }
+  }
+  __syncthreads();
+  if (SIGN > 0) {
+#pragma unroll 8
+    for (int e = threadIdx.x; e < rx * NY; e += RT) up[e] = P[e / NY * Q::LD + e % NY];
+  } else {
+#pragma unroll 8
+    for (int s = threadIdx.x; s < S; s += RT) tp[s] = P[st_off[s]];
+  }
+}
+
+template <typename T, int NX>
+__global__ void __launch_bounds__(RT) k_cols_q(typename V2t<T>::t* U, const T* __restrict__ vr, int ny, int nz,
+                                               int nlines) {
+  using V2 = typename V2t<T>::t;
+  using Q = Quarter<NX>;
+  const int l = blockIdx.x * RT + threadIdx.x;  // i3·ny + i2
+  if (l >= nlines) return;
+  const int i3 = l / ny, i2 = l - i3 * ny;
+  V2* up = U + ((size_t)blockIdx.y * nz + i3) * Q::R * ny + i2;
+  const T* v = vr + (size_t)i3 * NX * ny + i2;
+  T re[NX], im[NX];
+#pragma unroll
+  for (int j = 0; j < NX; ++j) {
+    V2 x;
+    x.x = x.y = 0;
+    if (Q::has(j)) x = up[Q::at(j) * ny];
+    re[j] = x.x;
+    im[j] = x.y;
+  }
+  fft_line<T, NX, 1>(re, im);
+  T r2[NX], m2[NX];
+#pragma unroll
+  for (int f = 0; f < NX; ++f) {
+    const T vv = v[f * ny];
+    r2[f] = re[LineOrder<NX>::pos(f)] * vv;
+    m2[f] = im[LineOrder<NX>::pos(f)] * vv;
+  }
+  fft_line<T, NX, -1>(r2, m2);
+#pragma unroll
+  for (int f = 0; f < NX; ++f)
+    if (Q::has(f)) {
+      V2 x;
+      x.x = r2[LineOrder<NX>::pos(f)];
+      x.y = m2[LineOrder<NX>::pos(f)];
+      up[Q::at(f) * ny] = x;
+    }
+}
+
+template <typename T, int N, int SIGN>
+void rows_q(Context& c, int nb, typename V2t<T>::t* tbuf, typename V2t<T>::t* U) {
+  const int rx = 2 * ((c.dims[0] - 1) / 4) + 1;
+  const size_t sh = (size_t)rx * Quarter<N>::LD * sizeof(typename V2t<T>::t);
+  ensure_lds_limit((const void*)k_rows_q<T, N, SIGN>, sh);
+  k_rows_q<T, N, SIGN><<<dim3((unsigned)c.dims[2], (unsigned)nb), RT, sh, c.stream>>>(
+      tbuf, U, c.nsticks, c.dims[2], rx, c.q_src.as<int>(), c.q_off.as<int>());
+}
+
+template <typename T, int SIGN>
+void rows_any(Context& c, int nb, typename V2t<T>::t* tbuf, typename V2t<T>::t* U) {
+  switch (c.dims[1]) {
+#define PWK_CASE(L) \
+  case L:           \
+    rows_q<T, L, SIGN>(c, nb, tbuf, U); \
+    break;
+    PWK_FOR_EACH_FFT_SIZE(PWK_CASE)
+#undef PWK_CASE
+    default:
+      throw Error(PWK_E_UNSUPPORTED, "ny has no compiled kernel");
+  }
+  PWK_HIP(hipGetLastError());
+}
+
 template <typename T, int N>
 void plane_q(Context& c, typename V2t<T>::t* tbuf, int nb, const T* vr) {
   using Sh = PlaneShape<T, N>;
@@ -235,9 +365,37 @@ void sphere_zinv(Context& c, int nb, const void* psi, void* out, const int* list
   PWK_HIP(hipGetLastError());
 }
 
+size_t sphere_rows_elems(const Context& c, int nb) {
+  return (size_t)nb * c.dims[2] * (2 * ((c.dims[0] - 1) / 4) + 1) * c.dims[1];
+}
+
 template <typename T>
-void sphere_plane(Context& c, int nb, void* buf, const T* vr) {
+void sphere_rows_inverse(Context& c, int nb, void* buf, void* rows) {
+  rows_any<T, 1>(c, nb, (typename V2t<T>::t*)buf, (typename V2t<T>::t*)rows);
+}
+
+template <typename T>
+void sphere_plane(Context& c, int nb, void* buf, const T* vr, void* rows) {
   auto* tbuf = (typename V2t<T>::t*)buf;
+  if (c.dims[0] != c.dims[1]) {
+    auto* U = (typename V2t<T>::t*)rows;
+    const int nlines = c.dims[1] * c.dims[2];
+    const dim3 g(blocks_for((size_t)nlines, RT), (unsigned)nb);
+    rows_any<T, 1>(c, nb, tbuf, U);
+    switch (c.dims[0]) {
+#define PWK_CASE(L) \
+  case L:           \
+    k_cols_q<T, L><<<g, RT, 0, c.stream>>>(U, vr, c.dims[1], c.dims[2], nlines); \
+    break;
+      PWK_FOR_EACH_FFT_SIZE(PWK_CASE)
+#undef PWK_CASE
+      default:
+        throw Error(PWK_E_UNSUPPORTED, "nx has no compiled kernel");
+    }
+    PWK_HIP(hipGetLastError());
+    rows_any<T, -1>(c, nb, tbuf, U);
+    return;
+  }
   switch (c.dims[0]) {
 #define PWK_CASE(L) \
   case L:           \
@@ -270,8 +428,10 @@ void sphere_zfwd(Context& c, int nb, const void* buf, const T* kin, int nbk, con
 
 template void sphere_zinv<float>(Context&, int, const void*, void*, const int*);
 template void sphere_zinv<double>(Context&, int, const void*, void*, const int*);
-template void sphere_plane<float>(Context&, int, void*, const float*);
-template void sphere_plane<double>(Context&, int, void*, const double*);
+template void sphere_rows_inverse<float>(Context&, int, void*, void*);
+template void sphere_rows_inverse<double>(Context&, int, void*, void*);
+template void sphere_plane<float>(Context&, int, void*, const float*, void*);
+template void sphere_plane<double>(Context&, int, void*, const double*, void*);
 template void sphere_zfwd<float>(Context&, int, const void*, const float*, int, const float* const*, const void*, void*);
 template void sphere_zfwd<double>(Context&, int, const void*, const double*, int, const double* const*, const void*,
                                   void*);

@@ -43,7 +43,9 @@ def to_grid(psi, idx, dims):
 PLANES = [((15, 15, 18), 7), ((16, 16, 12), 5), ((25, 25, 25), 6), ((27, 27, 27), 13), ((27, 27, 32), 6),
           ((45, 45, 16), 7), ((45, 45, 45), 11), ((48, 48, 9), 4), ((48, 48, 20), 4), ((60, 60, 10), 4),
           ((60, 60, 60), 14), ((64, 64, 15), 7), ((64, 64, 30), 7), ((72, 72, 8), 3), ((72, 72, 81), 3),
-          ((81, 81, 72), 3), ((81, 81, 12), 5)]
+          ((81, 81, 72), 3), ((81, 81, 12), 5),
+          # nx != ny: pruned (held rows moved between launches), at the quarter, and the whole-grid transforms
+          ((50, 25, 25), 6), ((25, 50, 27), 6), ((16, 81, 15), 3), ((80, 18, 20), 4), ((20, 25, 15), 7)]
 
 
 @pytest.mark.parametrize("dims,m", PLANES)
@@ -93,7 +95,7 @@ def test_hpsi_planes(gpu, dims, m, prec, tol):
         gpu.set_fused_hpsi(True)
 
 
-@pytest.mark.parametrize("dims,m", [((25, 25, 25), 6), ((27, 27, 27), 9)])
+@pytest.mark.parametrize("dims,m", [((25, 25, 25), 6), ((27, 27, 27), 9), ((27, 25, 32), 6)])
 @pytest.mark.parametrize("prec,tol", [("fp64", 1e-13), ("fp32", 6e-6), ("split_bf16", 2e-5)])
 @pytest.mark.parametrize("channels,counts", [((7, 7, 7), (3, 1, 18)), ((80, 80), (33, 161)), ((5, 0, 5), (2, 2, 2))])
 def test_hpsi_batch_sticks(gpu, dims, m, prec, tol, channels, counts):
