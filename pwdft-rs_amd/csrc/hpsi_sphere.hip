@@ -130,8 +130,10 @@ __global__ void __launch_bounds__(ZS) k_zfwd_q(const typename V2t<T>::t* __restr
   for (int e = threadIdx.x; e < rg.n; e += ZS) h[e] = L[e];
 }
 
+// Up to 81 points in FP32 a line's registers leave room for two waves per SIMD, which 64 points does not
+// get unasked: 64³ × 144 bands 111 us -> 71 us. FP64 lines spill under that bound.
 template <typename T, int N>
-__global__ void __launch_bounds__((PlaneShape<T, N>::NT))
+__global__ void __launch_bounds__((PlaneShape<T, N>::NT), (sizeof(T) == 4 && N <= 81 ? 2 : 1))
     k_plane_q(typename V2t<T>::t* tbuf, int nb, const T* __restrict__ vr, int S, int nz, const int* __restrict__ src,
               const int* __restrict__ st_off) {
   using V2 = typename V2t<T>::t;
