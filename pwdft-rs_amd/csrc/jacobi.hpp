@@ -43,6 +43,28 @@ __device__ inline void jacobi_sum2(double& a, double& b, double* red) {
   __syncthreads();
 }
 
+// J.order from the diagonal of J.A
+template <int JM>
+__device__ __forceinline__ void jacobi_order(int n, JacobiLdsT<JM>& J) {
+  const int t = threadIdx.x;
+  // ascending order by rank (ties by index). The order is total even for a NaN diagonal (NaNs
+  // after every number, among themselves by index), so the ranks are always a permutation and
+  // every entry of J.order is written.
+  if (t < n) {
+    const double di = J.A[t][t].x;
+    const bool ni = di != di;
+    int rank = 0;
+    for (int j = 0; j < n; ++j) {
+      const double dj = J.A[j][j].x;
+      const bool nj = dj != dj;
+      const bool before = (ni || nj) ? (nj == ni ? j < t : ni) : (dj < di || (dj == di && j < t));
+      rank += before ? 1 : 0;
+    }
+    J.order[rank] = t;
+  }
+  __syncthreads();
+}
+
 // Diagonalises J.A (n <= JMAX) in place: on return the diagonal of J.A holds the eigenvalues,
 // J.V = V_in · (product of the rotations), J.order[r] the index of the r-th smallest eigenvalue
 // (ties by index). Sweeps stop when the off-diagonal weight falls below 1e-30 of the total.
@@ -169,22 +191,139 @@ __device__ inline void jacobi_lds(int n, JacobiLdsT<JM>& J) {
       __syncthreads();
     }
   }
-  // ascending order by rank (ties by index). The order is total even for a NaN diagonal (NaNs
-  // after every number, among themselves by index), so the ranks are always a permutation and
-  // every entry of J.order is written.
-  if (t < n) {
-    const double di = J.A[t][t].x;
-    const bool ni = di != di;
-    int rank = 0;
-    for (int j = 0; j < n; ++j) {
-      const double dj = J.A[j][j].x;
-      const bool nj = dj != dj;
-      const bool before = (ni || nj) ? (nj == ni ? j < t : ni) : (dj < di || (dj == di && j < t));
-      rank += before ? 1 : 0;
-    }
-    J.order[rank] = t;
+  jacobi_order(n, J);
+}
+
+// 1/sqrt(x) for normal x > 0: v_rsq_f64 (2^-23) and one step of third order, e³ < 2^-66, so the result
+// carries the rounding of the step alone. The library's function and its sqrt handle denormals and
+// infinities as well, which the rotations never pass; they were half of a rotation's serial chain.
+__device__ __forceinline__ double jacobi_rsqrt(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  const double e = fma(-x * y, y, 1.0);
+  return fma(y * e, fma(0.375, e, 0.5), y);
+}
+
+// The rotation W = [[c, σ], [-conj(σ), c]] of columns (p, q) that makes (Wᴴ·A·W)_pq zero. With
+// d = (A_qq - A_pp)/2 and h = sqrt(d² + |A_pq|²): cos 2θ = |d|/h, so c² = (1 + |d|/h)/2, in [1/2, 1]
+// without cancellation, and σ = sign(d)·A_pq/(2·h·c): two reciprocal square roots on the chain and no
+// separate phase.
+__device__ __forceinline__ void jacobi_rotation(double app, double aqq, double2 apq, double& c, double2& s) {
+  const double g2 = apq.x * apq.x + apq.y * apq.y;
+  c = 1.0;
+  s = make_double2(0.0, 0.0);
+  if (g2 > 1e-300) {  // |A_pq| above 1e-150: no denormal reaches the reciprocal roots
+    const double d = 0.5 * (aqq - app);
+    const double ih = jacobi_rsqrt(fma(d, d, g2));
+    const double c2 = fma(0.5 * fabs(d), ih, 0.5);
+    const double ic = jacobi_rsqrt(c2);
+    c = c2 * ic;
+    const double f = (d >= 0.0 ? 0.5 : -0.5) * ih * ic;
+    s = make_double2(apq.x * f, apq.y * f);
   }
-  __syncthreads();
+}
+
+// (x, y) <- (c·x - conj(s)·y, s·x + c·y): the rotation on two columns
+__device__ __forceinline__ void jacobi_cols(double c, double2 s, double2& x, double2& y) {
+  const double2 u = make_double2(c * x.x - (s.x * y.x + s.y * y.y), c * x.y - (s.x * y.y - s.y * y.x));
+  y = make_double2(c * y.x + (s.x * x.x - s.y * x.y), c * y.y + (s.x * x.y + s.y * x.x));
+  x = u;
+}
+
+// pair k of a round: position 0 stays, positions 1..N-1 have rotated `round` times
+__device__ __forceinline__ void jacobi_pair(int N, int round, int k, int& p, int& q) {
+  const int u = N - 1 - k;
+  // (k - 1 - round) and (u - 1 - round) lie in (-(N - 1), N - 1): one wrap is enough
+  int a = k - 1 - round, b = u - 1 - round;
+  a += (a < 0 ? N - 1 : 0) + 1;
+  b += (b < 0 ? N - 1 : 0) + 1;
+  if (k == 0) a = 0;
+  p = min(a, b);
+  q = max(a, b);
+}
+
+// The same for a workgroup of NT >= (JM/2)² threads, with a second image A2 of A (any contents): a thread
+// per 2 × 2 block (kr, kc), which computes both of its rotations itself and writes the block to the other
+// image, so that a round has one barrier and no rotation goes through LDS. A round is a serial chain (LDS
+// read, two reciprocal roots, the updates, barrier), not work: what is computed twice costs less than the
+// exchange. An odd n is padded with a zero row and column, whose rotations are the identity.
+template <int JM, int NT>
+__device__ inline void jacobi_block(int n, JacobiLdsT<JM>& J, double2 (*A2)[JM + 1]) {
+  constexpr int HB = JM / 2;
+  static_assert(NT >= HB * HB, "a thread per block of two pairs");
+  // rows of V: on threads that hold no block where they are enough, beside the blocks elsewhere
+  constexpr bool APART = NT >= HB * HB + HB * JM;
+  const int t = threadIdx.x, N = n + (n & 1), NP = N / 2;
+  const int kc = t % HB, kr = t / HB;
+  const bool on = kc < NP, blk = on && kr < NP;
+  const int v0 = APART ? kr - HB : kr;
+  if (n < N && t < N) {
+    J.A[n][t] = J.A[t][n] = make_double2(0.0, 0.0);
+    J.V[n][t] = J.V[t][n] = make_double2(0.0, 0.0);
+  }
+  double2(*A)[JM + 1] = J.A;
+  double2(*B)[JM + 1] = A2;
+  for (int sweep = 0; sweep < 30; ++sweep) {
+    double off = 0.0, tot = 0.0;
+    for (int e = t; e < JM * JM; e += NT) {
+      const int r = e / JM, col = e % JM;
+      if (r < n && col < n) {
+        const double2 a = A[r][col];
+        const double m2 = a.x * a.x + a.y * a.y;
+        tot += m2;
+        if (r != col) off += m2;
+      }
+    }
+    jacobi_sum2(off, tot, J.red);
+    if (off <= 1e-30 * tot || off < 1e-300) break;  // block-uniform
+    for (int round = 0; round < N - 1; ++round) {
+      if (on) {
+        int pc, qc;
+        jacobi_pair(N, round, kc, pc, qc);
+        double cc;
+        double2 sc;
+        if (blk) {
+          int pr, qr;
+          jacobi_pair(N, round, kr, pr, qr);
+          double2 a00 = A[pr][pc], a01 = A[pr][qc], a10 = A[qr][pc], a11 = A[qr][qc];
+          const double rp = A[pr][pr].x, rq = A[qr][qr].x;
+          const double2 rpq = A[pr][qr];
+          double cr;
+          double2 sr;
+          jacobi_rotation(A[pc][pc].x, A[qc][qc].x, A[pc][qc], cc, sc);
+          jacobi_rotation(rp, rq, rpq, cr, sr);
+          jacobi_cols(cc, sc, a00, a01);
+          jacobi_cols(cc, sc, a10, a11);
+          sr.y = -sr.y;  // rows: the conjugate rotation
+          jacobi_cols(cr, sr, a00, a10);
+          jacobi_cols(cr, sr, a01, a11);
+          B[pr][pc] = a00;
+          B[pr][qc] = a01;
+          B[qr][pc] = a10;
+          B[qr][qc] = a11;
+        } else {
+          jacobi_rotation(A[pc][pc].x, A[qc][qc].x, A[pc][qc], cc, sc);
+        }
+        // the threads of pair kc share its columns of V by rows
+#pragma unroll
+        for (int r = v0; r < (APART ? v0 + 1 : JM); r += HB)
+          if (r >= 0 && r < n) {
+            double2 x = J.V[r][pc], y = J.V[r][qc];
+            jacobi_cols(cc, sc, x, y);
+            J.V[r][pc] = x;
+            J.V[r][qc] = y;
+          }
+      }
+      __syncthreads();
+      double2(*T)[JM + 1] = A;
+      A = B;
+      B = T;
+    }
+  }
+  if (A != J.A) {  // block-uniform
+    if (t < n) J.A[t][t] = A[t][t];
+    __syncthreads();
+  }
+  jacobi_order(n, J);
 }
 
 }  // namespace pwk

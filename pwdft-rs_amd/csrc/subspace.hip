@@ -276,9 +276,19 @@ __device__ __forceinline__ void rr_gram(RrLds<MB>& L, const double2* __restrict_
 }
 
 // From the Gram products (J.A, L.Hs) to the combination C (L.C) and the Ritz values (J.A's diagonal in J.order).
-template <int MB>
+// SPLIT: as a launch of its own, with the one-barrier Jacobi rounds (C is free while they run). The fused
+// forms keep the rounds that they had: mixed-precision solves of the sizes they serve stop their filter
+// passes on the last bits of the residuals, and their iteration counts moved with the rounding (12 and 17
+// instead of 11 to 15 in a spin-polarised two-atom solve).
+template <int MB, bool SPLIT>
 __device__ __forceinline__ void rr_mid(RrLds<MB>& L, int m, double floor_rel) {
   JacobiLdsT<MB>& J = L.J;
+  auto jacobi = [&]() {
+    if constexpr (SPLIT)
+      jacobi_block<MB, RR_NT>(m, J, L.C);
+    else
+      jacobi_lds(m, J);
+  };
   const int t = threadIdx.x;
   // Hermitian parts (subspace.hip k_hermitize), V = I
   for (int e = t; e < m * m; e += RR_NT) {
@@ -353,7 +363,7 @@ __device__ __forceinline__ void rr_mid(RrLds<MB>& L, int m, double floor_rel) {
       J.V[e % m][e / m] = make_double2(e % m == e / m ? 1.0 : 0.0, 0.0);
     }
     __syncthreads();
-    jacobi_lds(m, J);
+    jacobi();
     const double smax = J.A[J.order[m - 1]][J.order[m - 1]].x;
     for (int e = t; e < m * m; e += RR_NT) {
       const int r = e % m, j = e / m;
@@ -396,7 +406,7 @@ __device__ __forceinline__ void rr_mid(RrLds<MB>& L, int m, double floor_rel) {
     J.V[i][j] = make_double2(i == j ? 1.0 : 0.0, 0.0);
   }
   __syncthreads();
-  jacobi_lds(m, J);
+  jacobi();
   // C[:, jj] = X·W[:, order[jj]] (ascending Ritz values)
   for (int e = t; e < m * m; e += RR_NT) {
     const int i = e % m, jj = e / m, w = J.order[jj];
@@ -426,7 +436,7 @@ __device__ __forceinline__ void rr_small_body(int k, int npw, int m, int nres, c
   const double2* HY = HYb + (size_t)k * npw * m;
   double2* V = Vb + (size_t)k * npw * m;
   rr_gram<MB>(L, Y, HY, npw, m, 0, npw);
-  rr_mid<MB>(L, m, floor_rel);
+  rr_mid<MB, false>(L, m, floor_rel);
   if (t < m) lam_out[(size_t)k * m + t] = J.A[J.order[t]][J.order[t]].x;
   __syncthreads();
   double acc[MB];
@@ -504,6 +514,8 @@ __global__ void __launch_bounds__(RR_NT) k_rr_gram(int npw, int m, const double2
   }
 }
 
+// The small dense steps, one workgroup per k-point: serial chains of barriers (32 columns: 288 us with
+// the fused forms' Jacobi rounds, 217 us with the one-barrier rounds).
 template <int MB>
 __global__ void __launch_bounds__(RR_NT) k_rr_mid(int m, int nchunks, const double2* __restrict__ part,
                                                   double floor_rel, double2* __restrict__ Cb,
@@ -524,7 +536,7 @@ __global__ void __launch_bounds__(RR_NT) k_rr_mid(int m, int nchunks, const doub
     (e < m * m ? L.J.A : L.Hs)[f / m][f % m] = s;
   }
   __syncthreads();
-  rr_mid<MB>(L, m, floor_rel);
+  rr_mid<MB, true>(L, m, floor_rel);
   for (int e = threadIdx.x; e < m * m; e += RR_NT) Cb[(size_t)k * m * m + e] = L.C[e / m][e % m];  // [i][jj]
   if ((int)threadIdx.x < m) {
     const double l = L.J.A[L.J.order[threadIdx.x]][L.J.order[threadIdx.x]].x;
