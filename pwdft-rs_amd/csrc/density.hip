@@ -1,4 +1,4 @@
-// Band density on the sphere-pruned FFT (square grids): ρ(r) += Σ_b fw_b |ψ_b(r)|²
+// Band density on the sphere-pruned FFT: ρ(r) += Σ_b fw_b |ψ_b(r)|²
 // (src/scf/density.rs:59-97).
 //
 // Three launches: the z-inverse of the bands that carry weight (launch_zinv), the plane pass
@@ -34,7 +34,8 @@ using DensityShape = PlaneShape<T, N, !acc_in_regs<T, N>()>;
 // once, at the end.
 // Bound: vector arithmetic of the line transforms (a band's plane enters LDS once and never
 // returns). One workgroup per plane that loops over every band, as before, left 60 of 256 CUs with
-// one wave each.
+// one wave each: 144 FP32 bands on 60³ 1741 us -> 72 us;
+// 540 FP64 bands on 25³, the whole density beside other work, 901 us -> 31 us.
 // QUARTER: a sphere within a quarter of the axes (planes.hpp); otherwise the held rows come from the
 // basis' tables.
 template <typename T, int N, bool QUARTER>
@@ -159,7 +160,7 @@ __global__ void __launch_bounds__(64) k_cols_density(const typename V2t<T>::t* _
 
 // rho[i1][i2][i3] (+)= Σ_g part[g][i3][i1][i2] in group order; a 32 × 32 (i2, i3) tile per workgroup
 // goes through LDS, so that both sides are read and written along their contiguous axis. Bound: the
-// partials' traffic (groups·N·8 bytes).
+// partials' traffic (groups·N·8 bytes; 60³ in 15 groups 26 MB, 8.5 us).
 __global__ void __launch_bounds__(256) k_density_sum(int ngroups, int nx, int ny, int nz, const double* __restrict__ part,
                                                      double* __restrict__ rho, int overwrite) {
   __shared__ double tile[32][33];
@@ -243,7 +244,7 @@ void density_sticks_t(Context& c, int nb, const void* psi, const double* fw_host
     PWK_HIP(hipMemcpyAsync(c.work_b.p, h.data(), h.size() * sizeof(double), hipMemcpyHostToDevice, c.stream));
     const double* fw = c.work_b.as<double>();
     // about 1024 workgroups (four per CU): more only adds partial sums to store and read, fewer leave
-    // CUs idle. Measured with the groups' count that this gives: 60 planes × 144 bands in 16 groups.
+    // CUs idle (60³ × 144 bands: 72 batches × 60 planes in 15 groups).
     const bool square = nx == ny;
     const int slots = square ? plane_slots<T>(nx) : 1;
     const int batches = (live + slots - 1) / slots;

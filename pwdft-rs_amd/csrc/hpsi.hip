@@ -1,4 +1,4 @@
-// Local part of H·ψ and the band density on the sphere-pruned FFT.
+// Local part of H·ψ on the sphere-pruned FFT.
 //
 // The plane-wave sphere occupies S z-sticks (distinct (n1, n2)); the
 // reference enumerates the basis n1 -> n2 -> n3 (src/basis.rs:47-59), so the
@@ -11,8 +11,9 @@
 //              Hψ = T_kin ψ + (1/N)·(...)                  (src/scf/potentials.rs:163-190)
 // which equals the dense fill_hamiltonian_with_v_eff product because the
 // wrapped Miller difference there is a circular convolution.
-// The density reuses k_zinv and a plane kernel that accumulates f·|ψ(r)|²
-// (src/scf/density.rs:59-97).
+// Bases within a quarter of every axis (the default ecutrho = 4·ecutwfc) take the same passes pruned at
+// compile time (hpsi_sphere.hip); the kernels here serve the other bases on nx = ny, and the whole-grid
+// transforms below the rest. The band density (density.hip) shares the z-inverse and the planes' layout.
 #include <algorithm>
 #include <cstring>
 #include <map>
@@ -507,7 +508,6 @@ void setup_basis(Context& c, int npw, const int32_t* m) {
   up(c.st_pw0, pw0.data(), pw0.size() * sizeof(int32_t));
   up(c.st_cnt, cnt.data(), cnt.size() * sizeof(int32_t));
   up(c.st_n3lo, lo.data(), lo.size() * sizeof(int32_t));
-  up(c.st_xy, xy.data(), xy.size() * sizeof(int32_t));
   up(c.x1list, x1list.data(), x1list.size() * sizeof(int32_t));
   up(c.pl_src, psrc.data(), psrc.size() * sizeof(int32_t));
   up(c.st_off, off.data(), off.size() * sizeof(int32_t));
@@ -515,7 +515,6 @@ void setup_basis(Context& c, int npw, const int32_t* m) {
     up(c.q_src, qsrc.data(), qsrc.size() * sizeof(int32_t));
     up(c.q_off, qoff.data(), qoff.size() * sizeof(int32_t));
   }
-  up(c.st_x1, sx1.data(), sx1.size() * sizeof(int32_t));
   c.sync();  // the host tables go out of scope here
 }
 
@@ -682,7 +681,8 @@ namespace {
 // The batch on the stick path: one launch sequence over the bands of all entries, each band with its own
 // kinetic diagonal, and the entries' projector products as one grouped launch each. 27 k-points of about
 // 24 bands (1189 plane waves, 25³) took 162 launches one entry at a time. Returns false when the entries
-// cannot share the launches (channel counts that differ, more bands than one launch takes).
+// cannot share the launches (channel counts that differ, more bands than one launch takes), and while the
+// stream is captured with a table that is not on the device yet.
 template <typename T>
 bool hpsi_batch_sticks(Context& c, int nent, const int32_t* ik, const int32_t* nbands, size_t total, const void* psi,
                        void* hpsi, int precision) {
@@ -711,6 +711,10 @@ bool hpsi_batch_sticks(Context& c, int nent, const int32_t* ik, const int32_t* n
     for (int j = 0; j < nbands[e]; ++j) tab[b++] = (uint64_t)(uintptr_t)(f64 ? kd.kin64.p : kd.kin32.p);
   }
   if (tab != c.batch_tab_host || !c.batch_tab.p) {
+    // a new table waits for its upload, which a stream being captured cannot do
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    PWK_HIP(hipStreamIsCapturing(c.stream, &cap));
+    if (cap != hipStreamCaptureStatusNone) return false;
     c.batch_tab.ensure(tab.size() * sizeof(uint64_t));
     c.batch_tab_host.clear();
     PWK_HIP(hipMemcpyAsync(c.batch_tab.p, tab.data(), tab.size() * sizeof(uint64_t), hipMemcpyHostToDevice, c.stream));

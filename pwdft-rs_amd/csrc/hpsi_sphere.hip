@@ -5,7 +5,8 @@
 //   plane:     SLOTS planes per workgroup in LDS: y-inverse, x-inverse, × V(r), x-forward, y-forward.
 //   z-forward: a lane per stick; Hψ = T_kin ψ + (1/N)·(...) is formed in LDS in place of ψ, so that ψ, the
 //              kinetic energies and Hψ are read and written coalesced.
-// Bounds: the plane pass by vector arithmetic, the z passes by the stick buffer's traffic.
+// Bounds: the plane pass by vector arithmetic, the z passes by the stick buffer's traffic (144 bands on
+// 60³: 49 MB each way, 10 us at the rate of a copy).
 #include <algorithm>
 
 #include "common.hpp"
@@ -40,6 +41,7 @@ __device__ __forceinline__ void range_to_lds(V* dst, const V* __restrict__ src, 
   }
 }
 
+// FP32 60³ × 144 bands 18 us -> 16 us, FP64 45³ × 160 bands 18 us -> 17 us (against k_zinv).
 template <typename T, int NZ>
 __global__ void __launch_bounds__(ZS) k_zinv_q(const typename V2t<T>::t* __restrict__ psi,
                                                typename V2t<T>::t* __restrict__ tbuf, int npw, int S,
@@ -80,6 +82,8 @@ __global__ void __launch_bounds__(ZS) k_zinv_q(const typename V2t<T>::t* __restr
   }
 }
 
+// FP32 60³ × 144 bands 38 us -> 21.6 us, FP64 45³ × 160 bands 36 us -> 30 us (against k_zfwd, which gathers
+// and stores the sphere with strided accesses).
 template <typename T, int NZ>
 __global__ void __launch_bounds__(ZS) k_zfwd_q(const typename V2t<T>::t* __restrict__ tbuf,
                                                const typename V2t<T>::t* __restrict__ psi,
@@ -130,6 +134,9 @@ __global__ void __launch_bounds__(ZS) k_zfwd_q(const typename V2t<T>::t* __restr
   for (int e = threadIdx.x; e < rg.n; e += ZS) h[e] = L[e];
 }
 
+// Against the passes over every held row (126 us with one plane per workgroup, 96 us with two; 59 us of
+// those were the vector instructions alone, which is why half of them are pruned): FP32 60³ × 144 bands
+// 67 us, FP64 45³ × 160 bands 151 us -> 103 us.
 // Up to 81 points in FP32 a line's registers leave room for two waves per SIMD, which 64 points does not
 // get unasked: 64³ × 144 bands 111 us -> 71 us. FP64 lines spill under that bound.
 template <typename T, int N>
@@ -194,7 +201,8 @@ __global__ void __launch_bounds__((PlaneShape<T, N>::NT), (sizeof(T) == 4 && N <
 // The plane pass in three launches, so that each axis has its own compiled length: y-lines of the held rows
 // (sticks -> U[band][i3][held row][i2]), x-lines with the potential between (a lane per (i3, i2), its line
 // read and written along i2), y-lines back to the sticks. Only the held rows move between the launches.
-// si 50 × 25 × 25, 40 bands FP32: the whole-grid transforms this replaces took nine launches over all points.
+// 50 × 25 × 25, 40 bands FP32: a whole H·ψ 60 us -> 25 us; the whole-grid transforms that this replaces took
+// nine launches over all points. Bound: launches and the latency of one short wave each.
 constexpr int RT = 64;
 
 template <typename T, int NY, int SIGN>

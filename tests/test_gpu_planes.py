@@ -135,6 +135,61 @@ def test_hpsi_batch_sticks(gpu, dims, m, prec, tol, channels, counts):
     assert np.abs(got - w[:nbands[0]]).max() < tol * np.abs(w).max()
 
 
+@pytest.mark.parametrize("uploaded", [False, True])
+def test_hpsi_batch_sticks_captured(gpu, uploaded):
+    # a batch captured into a graph: entry by entry where its tables are not on the device yet, grouped
+    # afterwards; replays equal the same launches outside the graph
+    import torch
+
+    miller, _ = setup(gpu, (25, 25, 25), 6)
+    npw, nch = len(miller), 7
+    rng = np.random.default_rng(34)
+    gpu.set_veff((np.fft.fftn(rng.uniform(-13.6, 13.6, (25, 25, 25))) / 25 ** 3).reshape(-1))
+    gpu.set_nk(3)
+    for ik in range(3):
+        gpu.set_kinetic(ik, (miller.astype(float) ** 2).sum(1) * (1 + 0.1 * ik))
+        b = (rng.standard_normal((npw, nch)) + 1j * rng.standard_normal((npw, nch))) / np.sqrt(npw)
+        gpu.set_nonlocal(ik, b, b.conj().T.copy())
+    order, nbands = [2, 0, 1], [5, 3, 4]
+    psi = torch.from_numpy(bands(rng, sum(nbands), npw).astype(np.complex64)).cuda()
+    out = torch.empty_like(psi)
+    torch.cuda.synchronize()
+
+    def entries():
+        b0 = 0
+        for ik, nb in zip(order, nbands):
+            gpu.hpsi_dev(ik, nb, psi[b0].data_ptr(), out[b0].data_ptr(), "fp32")
+            b0 += nb
+
+    def batch():
+        gpu.hpsi_batch_dev(order, nbands, psi.data_ptr(), out.data_ptr(), "fp32")
+
+    batch()  # workspaces
+    entries()
+    if not uploaded:
+        gpu.hpsi_batch_dev(order[:2], nbands[:2], psi.data_ptr(), out.data_ptr(), "fp32")  # another table
+        entries()
+    else:
+        batch()
+    gpu.sync()
+    want = out.cpu()
+    print("captured batch", uploaded, flush=True)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.stream(torch.cuda.ExternalStream(gpu.stream)):
+        graph.capture_begin(capture_error_mode="thread_local")
+        try:
+            batch()
+        finally:
+            graph.capture_end()
+        for _ in range(3):
+            out.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(out.cpu(), want)
+            batch()
+            gpu.sync()
+
+
 @pytest.mark.parametrize("prec,tol", [("fp64", 1e-13), ("fp32", 2e-5), ("split_bf16", 5e-5)])
 def test_zgemm_column_blocks(gpu, prec, tol):
     # column counts around one and two blocks of 144, row counts that make few and many tiles, reductions
