@@ -72,8 +72,8 @@ __global__ void __launch_bounds__((DensityShape<T, N>::NT))
     else
       plane_ylines<T, N, NT, 1>(P, image, nsl, nx1, x1list);
     __syncthreads();
-    if (slot < nsl) {
-      const double f = fw[b0 + slot];
+    const double f = slot < nsl ? fw[b0 + slot] : 0.0;
+    if (!(f < 1e-15)) {  // src/scf/density.rs:14,72
       const V2* col = P + slot * image + i2;
       T re[N], im[N];
       if constexpr (QUARTER) {
@@ -137,6 +137,7 @@ __global__ void __launch_bounds__(64) k_cols_density(const typename V2t<T>::t* _
   for (int b = g * per; b < b_end; ++b) {
     const V2* up = rows + ((size_t)b * nz + i3) * Q::R * ny + i2;
     const double f = fw[b];
+    if (f < 1e-15) continue;
     T re[NX], im[NX];
 #pragma unroll
     for (int j = 0; j < NX; ++j) {
@@ -225,23 +226,30 @@ int plane_slots(int n) {
 template <typename T>
 void density_sticks_t(Context& c, int nb, const void* psi, const double* fw_host, double* rho, bool overwrite) {
   using V2 = typename V2t<T>::t;
-  // the bands that carry weight (src/scf/density.rs:14,72), their weights first
+  // the bands that carry weight (src/scf/density.rs:14,72), their weights first. While the stream is captured
+  // every band is transformed and the weights are the caller's own at each replay: the kernels skip the
+  // bands without weight.
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  PWK_HIP(hipStreamIsCapturing(c.stream, &cap));
+  const bool captured = cap != hipStreamCaptureStatusNone;
   std::vector<double>& h = c.dens_host;
-  h.clear();
-  for (int b = 0; b < nb; ++b)
-    if (fw_host[b] >= 1e-15) h.push_back(fw_host[b]);
-  const int live = (int)h.size();
-  h.resize((size_t)live + (size_t)(live + 1) / 2);
-  {
+  int live = nb;
+  if (!captured) {
+    h.clear();
+    for (int b = 0; b < nb; ++b)
+      if (!(fw_host[b] < 1e-15)) h.push_back(fw_host[b]);
+    live = (int)h.size();
+    h.resize((size_t)live + (size_t)(live + 1) / 2);
     int32_t* list = reinterpret_cast<int32_t*>(h.data() + live);
     for (int b = 0, i = 0; b < nb; ++b)
-      if (fw_host[b] >= 1e-15) list[i++] = b;
+      if (!(fw_host[b] < 1e-15)) list[i++] = b;
   }
   const int nx = c.dims[0], ny = c.dims[1], nz = c.dims[2];
   int groups = 0;
   if (live > 0) {
-    c.work_b.ensure(h.size() * sizeof(double));
-    PWK_HIP(hipMemcpyAsync(c.work_b.p, h.data(), h.size() * sizeof(double), hipMemcpyHostToDevice, c.stream));
+    const size_t wbytes = (captured ? (size_t)nb : h.size()) * sizeof(double);
+    c.work_b.ensure(wbytes);
+    PWK_HIP(hipMemcpyAsync(c.work_b.p, captured ? fw_host : h.data(), wbytes, hipMemcpyHostToDevice, c.stream));
     const double* fw = c.work_b.as<double>();
     // about 1024 workgroups (four per CU): more only adds partial sums to store and read, fewer leave
     // CUs idle (60³ × 144 bands: 72 batches × 60 planes in 15 groups).
@@ -257,7 +265,7 @@ void density_sticks_t(Context& c, int nb, const void* psi, const double* fw_host
     c.work_a.ensure(tb + (size_t)groups * c.N * sizeof(double));
     double* part = reinterpret_cast<double*>(c.work_a.as<unsigned char>() + tb);
     launch_zinv(c, live, psi, c.work_a.p, std::is_same<T, double>::value ? PWK_FP64 : PWK_FP32,
-                reinterpret_cast<const int*>(fw + live));
+                captured ? nullptr : reinterpret_cast<const int*>(fw + live));
     V2* rows = c.work_a.as<V2>() + ns;
     if (!square) sphere_rows_inverse<T>(c, live, c.work_a.p, rows);
     switch (nx) {

@@ -190,6 +190,40 @@ def test_hpsi_batch_sticks_captured(gpu, uploaded):
             gpu.sync()
 
 
+@pytest.mark.parametrize("dims,m", [((25, 25, 25), 6), ((27, 25, 32), 6), ((27, 27, 27), 13)])
+def test_density_captured(gpu, dims, m):
+    # a captured density reads the caller's weights at each replay, also where a band gains or loses its weight
+    import torch
+
+    miller, _ = setup(gpu, dims, m)
+    rng = np.random.default_rng(35)
+    nb, n = 7, int(np.prod(dims))
+    psi = bands(rng, nb, len(miller))
+    dev = torch.from_numpy(psi).cuda()
+    rho = torch.zeros(n, dtype=torch.float64, device="cuda")
+    fw = rng.uniform(0.1, 2.0, nb)
+    torch.cuda.synchronize()
+    gpu.density_dev(nb, dev.data_ptr(), fw, rho.data_ptr(), "fp64")  # workspaces
+    gpu.sync()
+    print("captured density", dims, m, flush=True)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.stream(torch.cuda.ExternalStream(gpu.stream)):
+        graph.capture_begin(capture_error_mode="thread_local")
+        try:
+            gpu.density_dev(nb, dev.data_ptr(), fw, rho.data_ptr(), "fp64")
+        finally:
+            graph.capture_end()
+        for zero in ([], [2], [0, 6]):
+            fw[:] = rng.uniform(0.1, 2.0, nb)
+            fw[zero] = 0.0
+            rho.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            want = gpu.density(psi, fw, None, "fp64")
+            # sums over other groups of the bands: a rounding per band
+            assert np.abs(rho.cpu().numpy() - want).max() < nb * 2.3e-16 * want.max()
+
+
 @pytest.mark.parametrize("prec,tol", [("fp64", 1e-13), ("fp32", 2e-5), ("split_bf16", 5e-5)])
 def test_zgemm_column_blocks(gpu, prec, tol):
     # column counts around one and two blocks of 144, row counts that make few and many tiles, reductions
