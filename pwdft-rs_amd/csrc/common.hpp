@@ -272,6 +272,41 @@ struct FftPlan {
   int ord = 0, tpb = 64, zlds = 0;
 };
 
+// ---- k × band batches that share their launches --------------------------------------------
+// The entries of a batch travel by value in the kernel arguments, so a captured launch keeps its own and
+// nothing is uploaded; an entry per lane of a wave. (A device table that every batch rewrote was read by the
+// replays of graphs captured with other entries.) Kernels are compiled for them apart: 0.8 KB more of
+// arguments on every launch took a sequence of eight short launches from 25.3 to 28.3 us.
+constexpr int MAX_BATCH_ENTRIES = 64;
+struct NoBatch {
+  static constexpr bool batch = false;
+};
+// bands [end[e - 1], end[e]) have the kinetic diagonal kin[e]
+struct BatchKin {
+  static constexpr bool batch = true;
+  int n = 0;
+  int end[MAX_BATCH_ENTRIES];
+  const void* kin[MAX_BATCH_ENTRIES];
+};
+// product e is C[:, col..col + cols) (+)= A·B[:, col..col + cols) with its own A
+struct GemmGroups {
+  static constexpr bool batch = true;
+  int n = 0;
+  int cols[MAX_BATCH_ENTRIES], col[MAX_BATCH_ENTRIES];
+  const void* A[MAX_BATCH_ENTRIES];
+};
+// the kinetic diagonal of band b: its entry's (found by one load per lane; every lane of the wave calls it),
+// or without entries that of k-point b / nbk
+template <typename T, class Entries>
+__device__ __forceinline__ const T* band_kin(const Entries& entries, const T* kin, int npw, int nbk, int b) {
+  if constexpr (Entries::batch) {
+    const int lane = threadIdx.x & 63;
+    return (const T*)entries.kin[__popcll(__ballot(lane < entries.n && entries.end[lane] <= b))];
+  } else {
+    return kin + (size_t)(b / nbk) * npw;
+  }
+}
+
 // Device state of one calculation.
 struct Context {
   int device = 0;
@@ -346,10 +381,6 @@ struct Context {
   DevBuf kin_pack64, kin_pack32, B_pack64, B_pack32, DBH_pack64, DBH_pack32;
   DevBuf band_tab;                  // int32 k-point per band of the last batch
   std::vector<int32_t> band_tab_host;
-  // k × band batches off the small grids: the kinetic diagonal of each band and the projector products,
-  // as uploaded for the last batch
-  DevBuf batch_tab;
-  std::vector<uint64_t> batch_tab_host;
 
   std::vector<double> dens_host;  // weights and list of the last density's live bands
 
@@ -439,8 +470,8 @@ template <typename T>
 void sphere_rows_inverse(Context& c, int nb, void* buf, void* rows);
 template <typename T>
 void sphere_plane(Context& c, int nb, void* buf, const T* vr, void* rows);
-template <typename T>
-void sphere_zfwd(Context& c, int nb, const void* buf, const T* kin, int nbk, const T* const* kin_of,
+template <typename T, class Entries>
+void sphere_zfwd(Context& c, int nb, const void* buf, const T* kin, int nbk, const Entries& entries,
                  const void* psi, void* hpsi);
 // density.hip: the band density on square grids of register-length lines and on any with c.quarter (fw on
 // the host)
@@ -495,13 +526,9 @@ void launch_zgemm_mfma(Context& c, int M, int N, int K, const void* A, int lda, 
 void launch_zgemm_mfma_batched(Context& c, int M, int N, int K, const void* A, int lda, long long sA, const void* B,
                                int ldb, long long sB, void* C, int ldc, long long sC, int batch, bool accumulate,
                                int precision);
-// products with their own A (lda shared) and column count: product g is C[:, col..col+n) (+)= A_g·B[:, col..)
-struct GemmGroup {
-  const void* A;
-  int n, col;
-};
-void launch_zgemm_mfma_groups(Context& c, int M, int Nmax, int K, int ngroups, const GemmGroup* groups /* device */,
-                              int lda, const void* B, int ldb, void* C, int ldc, bool accumulate, int precision);
+// the products of a batch's entries (groups.n of them, the widest of Nmax columns; A's lda shared)
+void launch_zgemm_mfma_groups(Context& c, int M, int Nmax, int K, const GemmGroups& groups, int lda, const void* B,
+                              int ldb, void* C, int ldc, bool accumulate, int precision);
 // eig.hip: lowest nb eigenpairs of nk Hermitian n×n matrices (H overwritten)
 size_t heev_work_doubles(int n, int nb, int nk);
 bool heev_supported(int n, int nb);

@@ -109,14 +109,14 @@ struct Tile {
 // Against the form with A and B in LDS behind two barriers per step and one wide tile per CU (projection with
 // its partial sums, expansion): split-bf16 512 × 144 × 13133 75 and 79 us -> 51 and 47 us; FP64
 // 256 × 160 × 6859 133 and 90 us -> 57 and 56 us.
-template <int MODE, int NB16>
+template <int MODE, int NB16, class Groups>
 __global__ void __launch_bounds__(256, 2) k_zgemm_mfma(int M, int N, int K, int kchunk, int nsplit, long long sA,
                                                     long long sB, long long sC,
                                                     const typename Traits<MODE>::V2* __restrict__ A, int lda,
                                                     const typename Traits<MODE>::V2* __restrict__ B, int ldb,
                                                     typename Traits<MODE>::V2* __restrict__ C, int ldc, int accumulate,
                                                     typename Traits<MODE>::V2* __restrict__ partial,
-                                                    const GemmGroup* __restrict__ groups) {
+                                                    const Groups groups) {
   using V2 = typename Traits<MODE>::V2;
   using T = typename Traits<MODE>::T;
   using acc_t = typename Traits<MODE>::acc_t;
@@ -141,12 +141,11 @@ __global__ void __launch_bounds__(256, 2) k_zgemm_mfma(int M, int N, int K, int 
   // bz = batch · nsplit + split
   const int zb = bz / nsplit, zs = bz % nsplit;
   if (partial) partial += (size_t)(zb * nsplit + zs) * M * N;
-  if (groups) {  // products of their own A and column count; N is the widest
-    const GemmGroup gr = groups[zb];
-    A = (const V2*)gr.A;
-    B += (size_t)gr.col * ldb;
-    C += (size_t)gr.col * ldc;
-    N = gr.n;
+  if constexpr (Groups::batch) {  // products of their own A and column count; N is the widest
+    A = (const V2*)groups.A[zb];
+    B += (size_t)groups.col[zb] * ldb;
+    C += (size_t)groups.col[zb] * ldc;
+    N = groups.cols[zb];
     if (n0 >= N) return;
   } else {
     A += (size_t)zb * sA;
@@ -308,17 +307,17 @@ __global__ void __launch_bounds__(256, 2) k_zgemm_mfma(int M, int N, int K, int 
   }
 }
 
-template <typename V2>
+template <typename V2, class Groups>
 __global__ void __launch_bounds__(256) k_splitk_sum(int M, int N, int nsplit, const V2* __restrict__ partial,
                                                     V2* __restrict__ C, int ldc, long long sC, int accumulate,
-                                                    const GemmGroup* __restrict__ groups) {
+                                                    const Groups groups) {
   size_t idx = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (idx >= (size_t)M * N) return;
   partial += (size_t)blockIdx.y * nsplit * M * N;
   int gm = (int)(idx % M), gn = (int)(idx / M);
-  if (groups) {
-    if (gn >= groups[blockIdx.y].n) return;
-    C += (size_t)groups[blockIdx.y].col * ldc;
+  if constexpr (Groups::batch) {
+    if (gn >= groups.cols[blockIdx.y]) return;
+    C += (size_t)groups.col[blockIdx.y] * ldc;
   } else {
     C += (size_t)blockIdx.y * sC;
   }
@@ -343,20 +342,19 @@ __global__ void __launch_bounds__(256) k_splitk_sum(int M, int N, int nsplit, co
 struct Batch {
   int count = 1;
   long long sA = 0, sB = 0, sC = 0;  // element strides between consecutive products
-  const GemmGroup* groups = nullptr;  // device; instead of the strides
 };
 
-template <int MODE, int NB16>
+template <int MODE, int NB16, class Groups>
 void launch_nb(Context& c, dim3 grid, int M, int N, int K, int kchunk, int nsplit, const Batch& bt, const void* A,
-               int lda, const void* B, int ldb, void* C, int ldc, int acc, void* part) {
+               int lda, const void* B, int ldb, void* C, int ldc, int acc, void* part, const Groups& groups) {
   using V2 = typename Traits<MODE>::V2;
-  k_zgemm_mfma<MODE, NB16><<<grid, 256, 0, c.stream>>>(M, N, K, kchunk, nsplit, bt.sA, bt.sB, bt.sC, (const V2*)A,
-                                                        lda, (const V2*)B, ldb, (V2*)C, ldc, acc, (V2*)part, bt.groups);
+  k_zgemm_mfma<MODE, NB16, Groups><<<grid, 256, 0, c.stream>>>(M, N, K, kchunk, nsplit, bt.sA, bt.sB, bt.sC, (const V2*)A,
+                                                        lda, (const V2*)B, ldb, (V2*)C, ldc, acc, (V2*)part, groups);
 }
 
-template <int MODE>
+template <int MODE, class Groups>
 void zgemm_mfma_t(Context& c, int M, int N, int K, const void* A, int lda, const void* B, int ldb, void* C, int ldc,
-                  bool accumulate, const Batch& bt) {
+                  bool accumulate, const Batch& bt, const Groups& groups) {
   using V2 = typename Traits<MODE>::V2;
   const int cus = c.cu_count > 0 ? c.cu_count : 256;
   // Column blocks of equal width. Without split K the width whose tiles, dealt to the CUs, take the fewest
@@ -396,20 +394,20 @@ void zgemm_mfma_t(Context& c, int M, int N, int K, const void* A, int lda, const
   int acc = (nsplit == 1 && accumulate) ? 1 : 0;
   switch (nb16) {
     case 1:
-      launch_nb<MODE, 1>(c, grid, M, N, K, kchunk, nsplit, bt, A, lda, B, ldb, C, ldc, acc, part);
+      launch_nb<MODE, 1>(c, grid, M, N, K, kchunk, nsplit, bt, A, lda, B, ldb, C, ldc, acc, part, groups);
       break;
     case 2:
-      launch_nb<MODE, 2>(c, grid, M, N, K, kchunk, nsplit, bt, A, lda, B, ldb, C, ldc, acc, part);
+      launch_nb<MODE, 2>(c, grid, M, N, K, kchunk, nsplit, bt, A, lda, B, ldb, C, ldc, acc, part, groups);
       break;
     default:
-      launch_nb<MODE, Tile<MODE>::W>(c, grid, M, N, K, kchunk, nsplit, bt, A, lda, B, ldb, C, ldc, acc, part);
+      launch_nb<MODE, Tile<MODE>::W>(c, grid, M, N, K, kchunk, nsplit, bt, A, lda, B, ldb, C, ldc, acc, part, groups);
       break;
   }
   PWK_HIP(hipGetLastError());
   if (nsplit > 1) {
     dim3 g(blocks_for((size_t)M * N, 256), (unsigned)bt.count);
-    k_splitk_sum<V2><<<g, 256, 0, c.stream>>>(M, N, nsplit, (const V2*)part, (V2*)C, ldc, bt.sC,
-                                              accumulate ? 1 : 0, bt.groups);
+    k_splitk_sum<V2, Groups><<<g, 256, 0, c.stream>>>(M, N, nsplit, (const V2*)part, (V2*)C, ldc, bt.sC,
+                                              accumulate ? 1 : 0, groups);
     PWK_HIP(hipGetLastError());
   }
 }
@@ -435,25 +433,24 @@ void launch_zgemm_mfma_batched(Context& c, int M, int N, int K, const void* A, i
   bt.sB = sB;
   bt.sC = sC;
   if (precision == PWK_FP64)
-    zgemm_mfma_t<MODE_F64>(c, M, N, K, A, lda, B, ldb, C, ldc, accumulate, bt);
+    zgemm_mfma_t<MODE_F64>(c, M, N, K, A, lda, B, ldb, C, ldc, accumulate, bt, NoBatch{});
   else if (precision == PWK_SPLIT_BF16)
-    zgemm_mfma_t<MODE_BF16X3>(c, M, N, K, A, lda, B, ldb, C, ldc, accumulate, bt);
+    zgemm_mfma_t<MODE_BF16X3>(c, M, N, K, A, lda, B, ldb, C, ldc, accumulate, bt, NoBatch{});
   else
-    zgemm_mfma_t<MODE_F32>(c, M, N, K, A, lda, B, ldb, C, ldc, accumulate, bt);
+    zgemm_mfma_t<MODE_F32>(c, M, N, K, A, lda, B, ldb, C, ldc, accumulate, bt, NoBatch{});
 }
 
-void launch_zgemm_mfma_groups(Context& c, int M, int Nmax, int K, int ngroups, const GemmGroup* groups, int lda,
-                              const void* B, int ldb, void* C, int ldc, bool accumulate, int precision) {
-  if (M <= 0 || Nmax <= 0 || K <= 0 || ngroups <= 0) return;
+void launch_zgemm_mfma_groups(Context& c, int M, int Nmax, int K, const GemmGroups& groups, int lda, const void* B,
+                              int ldb, void* C, int ldc, bool accumulate, int precision) {
+  if (M <= 0 || Nmax <= 0 || K <= 0 || groups.n <= 0) return;
   Batch bt;
-  bt.count = ngroups;
-  bt.groups = groups;
+  bt.count = groups.n;
   if (precision == PWK_FP64)
-    zgemm_mfma_t<MODE_F64>(c, M, Nmax, K, nullptr, lda, B, ldb, C, ldc, accumulate, bt);
+    zgemm_mfma_t<MODE_F64>(c, M, Nmax, K, nullptr, lda, B, ldb, C, ldc, accumulate, bt, groups);
   else if (precision == PWK_SPLIT_BF16)
-    zgemm_mfma_t<MODE_BF16X3>(c, M, Nmax, K, nullptr, lda, B, ldb, C, ldc, accumulate, bt);
+    zgemm_mfma_t<MODE_BF16X3>(c, M, Nmax, K, nullptr, lda, B, ldb, C, ldc, accumulate, bt, groups);
   else
-    zgemm_mfma_t<MODE_F32>(c, M, Nmax, K, nullptr, lda, B, ldb, C, ldc, accumulate, bt);
+    zgemm_mfma_t<MODE_F32>(c, M, Nmax, K, nullptr, lda, B, ldb, C, ldc, accumulate, bt, groups);
 }
 
 }  // namespace pwk

@@ -15,7 +15,6 @@
 // compile time (hpsi_sphere.hip); the kernels here serve the other bases on nx = ny, and the whole-grid
 // transforms below the rest. The band density (density.hip) shares the z-inverse and the planes' layout.
 #include <algorithm>
-#include <cstring>
 #include <map>
 
 #include "common.hpp"
@@ -67,15 +66,16 @@ __global__ void __launch_bounds__(64) k_zinv(const typename V2t<T>::t* __restric
   }
 }
 
-template <typename T, int NZ>
+template <typename T, int NZ, class Entries>
 __global__ void __launch_bounds__(64) k_zfwd(const typename V2t<T>::t* __restrict__ tbuf,
                                              const typename V2t<T>::t* __restrict__ psi,
                                              typename V2t<T>::t* __restrict__ hpsi, const T* __restrict__ kin,
                                              int npw, int S, const int* __restrict__ st_pw0,
                                              const int* __restrict__ st_cnt, const int* __restrict__ st_lo,
-                                             T inv_n, int nbk, const T* const* __restrict__ kin_of) {
+                                             T inv_n, int nbk, const Entries entries) {
   int s = blockIdx.x * 64 + threadIdx.x;
   int b = blockIdx.y;
+  const T* tb = band_kin(entries, kin, npw, nbk, b);
   if (s >= S) return;
   int pw0 = st_pw0[s], cnt = st_cnt[s], lo = st_lo[s];
   const typename V2t<T>::t* src = tbuf + (size_t)b * NZ * S + s;
@@ -89,8 +89,7 @@ __global__ void __launch_bounds__(64) k_zfwd(const typename V2t<T>::t* __restric
   fft_dif<T, NZ, -1>(re, im);
   const typename V2t<T>::t* p = psi + (size_t)b * npw + pw0;
   typename V2t<T>::t* h = hpsi + (size_t)b * npw + pw0;
-  // the band's kinetic diagonal: of its own (k × band batches) or of k-point b / nbk
-  const T* t = (kin_of ? kin_of[b] : kin + (size_t)(b / nbk) * npw) + pw0;
+  const T* t = tb + pw0;
 #pragma unroll
   for (int i3 = 0; i3 < NZ; ++i3) {
     int j = stick_slot(i3, lo, NZ);
@@ -365,9 +364,9 @@ void zinv_t(Context& c, int nb, const void* psi, typename V2t<T>::t* out, const 
 
 // Local part of H·ψ for nb bands; band b uses the kinetic diagonal kin + (b / nbk)·npw,
 // so consecutive groups of nbk bands may belong to different k-points.
-template <typename T>
+template <typename T, class Entries = NoBatch>
 void hpsi_local(Context& c, const T* kin, int nb, int nbk, const void* psi, void* hpsi,
-                const T* const* kin_of = nullptr) {
+                const Entries& entries = Entries()) {
   using V2 = typename V2t<T>::t;
   int nx = c.dims[0], nz = c.dims[2];
   PWK_REQUIRE(c.have_v, PWK_E_STATE, "V_eff not set (pwk_set_veff)");
@@ -406,15 +405,15 @@ void hpsi_local(Context& c, const T* kin, int nb, int nbk, const void* psi, void
   T inv_n = (T)(1.0 / (double)c.N);
   TimedScope ts_zfwd(c, "hpsi_zfwd");
   if (c.quarter) {
-    sphere_zfwd<T>(c, nb, T_, kin, nbk, kin_of, psi, hpsi);
+    sphere_zfwd<T>(c, nb, T_, kin, nbk, entries, psi, hpsi);
     return;
   }
   switch (nz) {
 #define PWK_CASE(L)                                                                                     \
   case L:                                                                                               \
-    k_zfwd<T, L><<<gz, 64, 0, c.stream>>>(T_, (const V2*)psi, (V2*)hpsi, kin, c.npw, c.nsticks,         \
+    k_zfwd<T, L, Entries><<<gz, 64, 0, c.stream>>>(T_, (const V2*)psi, (V2*)hpsi, kin, c.npw, c.nsticks,         \
                                           c.st_pw0.as<int>(), c.st_cnt.as<int>(), c.st_n3lo.as<int>(),  \
-                                          inv_n, nbk, kin_of);                                          \
+                                          inv_n, nbk, entries);                                         \
     break;
     PWK_FOR_EACH_FFT_SIZE(PWK_CASE)
 #undef PWK_CASE
@@ -678,70 +677,66 @@ size_t batch_bands(Context& c, int nent, const int32_t* ik, const int32_t* nband
 
 namespace {
 
-// The batch on the stick path: one launch sequence over the bands of all entries, each band with its own
-// kinetic diagonal, and the entries' projector products as one grouped launch each. 27 k-points of about
-// 24 bands (1189 plane waves, 25³) took 162 launches one entry at a time. Returns false when the entries
-// cannot share the launches (channel counts that differ, more bands than one launch takes), and while the
-// stream is captured with a table that is not on the device yet.
+// The entries [e0, e1) of a batch on the stick path: one launch sequence over the bands of all of them, each
+// with its entry's kinetic diagonal, and the entries' projector products as one grouped launch each.
+// 27 k-points of about 24 bands (1189 plane waves, 25³) took 162 launches one entry at a time.
 template <typename T>
-bool hpsi_batch_sticks(Context& c, int nent, const int32_t* ik, const int32_t* nbands, size_t total, const void* psi,
+void hpsi_batch_sticks(Context& c, int e0, int e1, const int32_t* ik, const int32_t* nbands, const void* psi,
                        void* hpsi, int precision) {
   const bool f64 = std::is_same<T, double>::value;
-  const int nch = c.k(ik[0]).nch;
-  // the stick buffer of the whole batch stays below 4 GiB
-  if (!stick_path_ok(c, f64) || total > 65535 ||
-      (total * (size_t)c.dims[2] * (size_t)c.nsticks +
-       (c.dims[0] == c.dims[1] ? 0 : sphere_rows_elems(c, (int)total))) * sizeof(typename V2t<T>::t) > ((size_t)4 << 30))
-    return false;
-  int nmax = 0;
-  for (int e = 0; e < nent; ++e) {
-    const KData& kd = c.k(ik[e]);
-    if (kd.nch != nch || (nch > 0 && !(f64 ? kd.B64.p && kd.DBH64.p : kd.B32.p && kd.DBH32.p))) return false;
-    nmax = std::max(nmax, (int)nbands[e]);
+  const int nch = c.k(ik[e0]).nch;
+  BatchKin kin;
+  GemmGroups project, expand;
+  kin.n = project.n = expand.n = e1 - e0;
+  int total = 0, nmax = 0;
+  for (int e = 0; e < e1 - e0; ++e) {
+    const KData& kd = c.k(ik[e0 + e]);
+    project.A[e] = f64 ? kd.DBH64.p : kd.DBH32.p;
+    expand.A[e] = f64 ? kd.B64.p : kd.B32.p;
+    project.col[e] = expand.col[e] = total;
+    project.cols[e] = expand.cols[e] = nbands[e0 + e];
+    total += nbands[e0 + e];
+    nmax = std::max(nmax, (int)nbands[e0 + e]);
+    kin.end[e] = total;
+    kin.kin[e] = f64 ? kd.kin64.p : kd.kin32.p;
   }
-  // the table: a kinetic diagonal per band, then the entries of the projections and of the expansions
-  static_assert(sizeof(GemmGroup) == 16, "two words per product");
-  std::vector<uint64_t> tab(total + 4 * (size_t)nent);
-  size_t b = 0;
-  for (int e = 0; e < nent; ++e) {
-    const KData& kd = c.k(ik[e]);
-    const GemmGroup pj{f64 ? kd.DBH64.p : kd.DBH32.p, nbands[e], (int)b}, ex{f64 ? kd.B64.p : kd.B32.p, nbands[e], (int)b};
-    std::memcpy(&tab[total + 2 * (size_t)e], &pj, sizeof pj);
-    std::memcpy(&tab[total + 2 * (size_t)(nent + e)], &ex, sizeof ex);
-    for (int j = 0; j < nbands[e]; ++j) tab[b++] = (uint64_t)(uintptr_t)(f64 ? kd.kin64.p : kd.kin32.p);
-  }
-  if (tab != c.batch_tab_host || !c.batch_tab.p) {
-    // a new table waits for its upload, which a stream being captured cannot do
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    PWK_HIP(hipStreamIsCapturing(c.stream, &cap));
-    if (cap != hipStreamCaptureStatusNone) return false;
-    c.batch_tab.ensure(tab.size() * sizeof(uint64_t));
-    c.batch_tab_host.clear();
-    PWK_HIP(hipMemcpyAsync(c.batch_tab.p, tab.data(), tab.size() * sizeof(uint64_t), hipMemcpyHostToDevice, c.stream));
-    PWK_HIP(hipStreamSynchronize(c.stream));  // the host table goes out of scope
-    c.batch_tab_host = tab;
-  }
-  const uint64_t* dt = c.batch_tab.as<uint64_t>();
-  hpsi_local<T>(c, nullptr, (int)total, 1, psi, hpsi, reinterpret_cast<const T* const*>(dt));
+  hpsi_local<T>(c, nullptr, total, 1, psi, hpsi, kin);
   if (nch > 0) {
     c.proj.ensure((size_t)nch * total * sizeof(typename V2t<T>::t));
-    const auto* pj = reinterpret_cast<const GemmGroup*>(dt + total);
     {
       TimedScope ts(c, "hpsi_nl_project");
-      launch_zgemm_mfma_groups(c, nch, nmax, c.npw, nent, pj, nch, psi, c.npw, c.proj.p, nch, false, precision);
+      launch_zgemm_mfma_groups(c, nch, nmax, c.npw, project, nch, psi, c.npw, c.proj.p, nch, false, precision);
     }
     TimedScope ts(c, "hpsi_nl_expand");
-    launch_zgemm_mfma_groups(c, c.npw, nmax, nch, nent, pj + nent, c.npw, c.proj.p, nch, hpsi, c.npw, true, precision);
+    launch_zgemm_mfma_groups(c, c.npw, nmax, nch, expand, c.npw, c.proj.p, nch, hpsi, c.npw, true, precision);
   }
-  return true;
+}
+
+// The entries from e0 on that share their launches: as many as one launch takes, with one channel count and
+// at most 256 MiB of sticks (a chunk of the whole-grid path; entries beyond it fill the chip by themselves).
+template <typename T>
+int batch_run(Context& c, int nent, int e0, const int32_t* ik, const int32_t* nbands) {
+  const bool f64 = std::is_same<T, double>::value;
+  const size_t per_band = ((size_t)c.dims[2] * c.nsticks + (c.dims[0] == c.dims[1] ? 0 : sphere_rows_elems(c, 1))) *
+                          sizeof(typename V2t<T>::t);
+  const int nch = c.k(ik[e0]).nch;
+  size_t total = 0;
+  int e = e0;
+  for (; e < nent && e - e0 < MAX_BATCH_ENTRIES; ++e) {
+    const KData& kd = c.k(ik[e]);
+    total += (size_t)nbands[e];
+    if (total > 65535 || total * per_band > ((size_t)256 << 20)) break;
+    if (kd.nch != nch || (nch > 0 && !(f64 ? kd.B64.p && kd.DBH64.p : kd.B32.p && kd.DBH32.p))) break;
+  }
+  return std::max(e, e0 + 1);
 }
 
 }  // namespace
 
 // H·ψ of a k × band batch with a band count per entry: entry e holds nbands[e] bands of k-point
 // ik[e], the entries' bands packed back to back in psi and hpsi. On small cubic grids the whole
-// batch is one fused launch that reads each band's k-point from a band table; on the stick path the
-// entries share each launch; elsewhere, or when the k-points' channel counts differ, one H·ψ per entry.
+// batch is one fused launch that reads each band's k-point from a band table; on the stick path entries
+// with the same channel count share each launch; elsewhere one H·ψ per entry.
 void launch_hpsi_batch(Context& c, int nent, const int32_t* ik, const int32_t* nbands, const void* psi, void* hpsi,
                        int precision) {
   c.check_basis();
@@ -767,14 +762,24 @@ void launch_hpsi_batch(Context& c, int nent, const int32_t* ik, const int32_t* n
     return;
   }
   const size_t es = precision == PWK_FP64 ? sizeof(double2) : sizeof(float2);
-  if (nent > 1 && (precision == PWK_SPLIT_BF16 || !hpsi_small_supported(c, precision, nch)) &&
-      (precision == PWK_FP64 ? hpsi_batch_sticks<double>(c, nent, ik, nbands, total, psi, hpsi, precision)
-                             : hpsi_batch_sticks<float>(c, nent, ik, nbands, total, psi, hpsi, precision)))
-    return;
-  size_t off = 0;
-  for (int e = 0; e < nent; ++e) {
-    launch_hpsi(c, ik[e], nbands[e], (const char*)psi + off * es, (char*)hpsi + off * es, precision);
-    off += (size_t)nbands[e] * c.npw;
+  const bool sticks = (precision == PWK_SPLIT_BF16 || !hpsi_small_supported(c, precision, nch)) &&
+                      stick_path_ok(c, precision == PWK_FP64);
+  for (int e = 0; e < nent;) {
+    const char* in = (const char*)psi;
+    char* out = (char*)hpsi;
+    const int end = !sticks ? e + 1
+                    : precision == PWK_FP64 ? batch_run<double>(c, nent, e, ik, nbands)
+                                            : batch_run<float>(c, nent, e, ik, nbands);
+    if (end == e + 1)
+      launch_hpsi(c, ik[e], nbands[e], in, out, precision);
+    else if (precision == PWK_FP64)
+      hpsi_batch_sticks<double>(c, e, end, ik, nbands, in, out, precision);
+    else
+      hpsi_batch_sticks<float>(c, e, end, ik, nbands, in, out, precision);
+    for (; e < end; ++e) {
+      psi = (const char*)psi + (size_t)nbands[e] * c.npw * es;
+      hpsi = (char*)hpsi + (size_t)nbands[e] * c.npw * es;
+    }
   }
 }
 

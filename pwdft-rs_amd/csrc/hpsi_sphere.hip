@@ -84,13 +84,13 @@ __global__ void __launch_bounds__(ZS) k_zinv_q(const typename V2t<T>::t* __restr
 
 // FP32 60³ × 144 bands 38 us -> 21.6 us, FP64 45³ × 160 bands 36 us -> 30 us (against k_zfwd, which gathers
 // and stores the sphere with strided accesses).
-template <typename T, int NZ>
+template <typename T, int NZ, class Entries>
 __global__ void __launch_bounds__(ZS) k_zfwd_q(const typename V2t<T>::t* __restrict__ tbuf,
                                                const typename V2t<T>::t* __restrict__ psi,
                                                typename V2t<T>::t* __restrict__ hpsi, const T* __restrict__ kin, int npw,
                                                int S, const int* __restrict__ st_pw0, const int* __restrict__ st_cnt,
                                                const int* __restrict__ st_lo, T inv_n, int nbk,
-                                               const T* const* __restrict__ kin_of) {
+                                               const Entries entries) {
   using V2 = typename V2t<T>::t;
   using Q = Quarter<NZ>;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
@@ -109,8 +109,7 @@ __global__ void __launch_bounds__(ZS) k_zfwd_q(const typename V2t<T>::t* __restr
     im[i3] = v.y;
   }
   range_to_lds<V2, 8>(L, psi + (size_t)b * npw + rg.w0, rg.n);
-  // the band's kinetic diagonal: of its own (k × band batches) or of k-point b / nbk
-  range_to_lds<T, 8>(K, (kin_of ? kin_of[b] : kin + (size_t)(b / nbk) * npw) + rg.w0, rg.n);
+  range_to_lds<T, 8>(K, band_kin(entries, kin, npw, nbk, b) + rg.w0, rg.n);
   __syncthreads();
   fft_line<T, NZ, -1>(re, im);
   // a slot of the line that the stick does not reach goes to a discard element of the lane's own: without
@@ -337,15 +336,15 @@ void plane_q(Context& c, typename V2t<T>::t* tbuf, int nb, const T* vr) {
       tbuf, nb, vr, c.nsticks, c.dims[2], c.q_src.as<int>(), c.q_off.as<int>());
 }
 
-template <typename T, int N>
-void zfwd_q(Context& c, const typename V2t<T>::t* tbuf, int nb, const T* kin, int nbk, const T* const* kin_of,
+template <typename T, int N, class Entries>
+void zfwd_q(Context& c, const typename V2t<T>::t* tbuf, int nb, const T* kin, int nbk, const Entries& entries,
             const void* psi, void* hpsi) {
   using V2 = typename V2t<T>::t;
   const size_t sh = (size_t)ZS * (Quarter<N>::R + 1) * (sizeof(V2) + sizeof(T));
-  ensure_lds_limit((const void*)k_zfwd_q<T, N>, sh);
-  k_zfwd_q<T, N><<<dim3(blocks_for((size_t)c.nsticks, ZS), (unsigned)nb), ZS, sh, c.stream>>>(
+  ensure_lds_limit((const void*)k_zfwd_q<T, N, Entries>, sh);
+  k_zfwd_q<T, N, Entries><<<dim3(blocks_for((size_t)c.nsticks, ZS), (unsigned)nb), ZS, sh, c.stream>>>(
       tbuf, (const V2*)psi, (V2*)hpsi, kin, c.npw, c.nsticks, c.st_pw0.as<int>(), c.st_cnt.as<int>(),
-      c.st_n3lo.as<int>(), (T)(1.0 / (double)c.N), nbk, kin_of);
+      c.st_n3lo.as<int>(), (T)(1.0 / (double)c.N), nbk, entries);
 }
 
 template <typename T, int N>
@@ -419,14 +418,14 @@ void sphere_plane(Context& c, int nb, void* buf, const T* vr, void* rows) {
   PWK_HIP(hipGetLastError());
 }
 
-template <typename T>
-void sphere_zfwd(Context& c, int nb, const void* buf, const T* kin, int nbk, const T* const* kin_of,
+template <typename T, class Entries>
+void sphere_zfwd(Context& c, int nb, const void* buf, const T* kin, int nbk, const Entries& entries,
                  const void* psi, void* hpsi) {
   auto* tbuf = (const typename V2t<T>::t*)buf;
   switch (c.dims[2]) {
 #define PWK_CASE(L) \
   case L:           \
-    zfwd_q<T, L>(c, tbuf, nb, kin, nbk, kin_of, psi, hpsi); \
+    zfwd_q<T, L>(c, tbuf, nb, kin, nbk, entries, psi, hpsi); \
     break;
     PWK_FOR_EACH_FFT_SIZE(PWK_CASE)
 #undef PWK_CASE
@@ -442,8 +441,9 @@ template void sphere_rows_inverse<float>(Context&, int, void*, void*);
 template void sphere_rows_inverse<double>(Context&, int, void*, void*);
 template void sphere_plane<float>(Context&, int, void*, const float*, void*);
 template void sphere_plane<double>(Context&, int, void*, const double*, void*);
-template void sphere_zfwd<float>(Context&, int, const void*, const float*, int, const float* const*, const void*, void*);
-template void sphere_zfwd<double>(Context&, int, const void*, const double*, int, const double* const*, const void*,
-                                  void*);
+template void sphere_zfwd(Context&, int, const void*, const float*, int, const NoBatch&, const void*, void*);
+template void sphere_zfwd(Context&, int, const void*, const float*, int, const BatchKin&, const void*, void*);
+template void sphere_zfwd(Context&, int, const void*, const double*, int, const NoBatch&, const void*, void*);
+template void sphere_zfwd(Context&, int, const void*, const double*, int, const BatchKin&, const void*, void*);
 
 }  // namespace pwk

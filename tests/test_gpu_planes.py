@@ -97,10 +97,11 @@ def test_hpsi_planes(gpu, dims, m, prec, tol):
 
 @pytest.mark.parametrize("dims,m", [((25, 25, 25), 6), ((27, 27, 27), 9), ((27, 25, 32), 6)])
 @pytest.mark.parametrize("prec,tol", [("fp64", 1e-13), ("fp32", 6e-6), ("split_bf16", 2e-5)])
-@pytest.mark.parametrize("channels,counts", [((7, 7, 7), (3, 1, 18)), ((80, 80), (33, 161)), ((5, 0, 5), (2, 2, 2))])
+@pytest.mark.parametrize("channels,counts", [((7, 7, 7), (3, 1, 18)), ((80, 80), (33, 161)), ((5, 0, 5), (2, 2, 2)),
+                                             ((3, 3, 6, 6, 6), (2, 1, 2, 3, 1)), ((4,) * 66, (1, 2) * 33)])
 def test_hpsi_batch_sticks(gpu, dims, m, prec, tol, channels, counts):
     # k × band batches off the small grids: one launch per pass and grouped projector products when the
-    # entries share a channel count, entry by entry otherwise. Tolerance relative to the largest |Hψ|:
+    # entries share a channel count (64 of them at most), entry by entry otherwise. Tolerance relative to the largest |Hψ|:
     # the transforms as above plus sums over npw (projection) and nch terms, √npw ≈ 60 roundings
     # (FP32 3.6e-6, split-bf16 2^-16 per product: 1.5e-5)
     miller, idx = setup(gpu, dims, m)
@@ -121,7 +122,7 @@ def test_hpsi_batch_sticks(gpu, dims, m, prec, tol, channels, counts):
     nbands = [counts[i] for i in order]
     psi = bands(rng, sum(nbands), npw)
     print("hpsi batch", dims, prec, channels, nbands, flush=True)
-    for _ in range(2):  # the second call reuses the tables of the first
+    for _ in range(2):
         got = gpu.hpsi_batch(order, nbands, psi, prec)
     w = np.fft.fftn(to_grid(psi, idx, dims) * v, axes=(1, 2, 3)).reshape(len(psi), -1)[:, idx] / n
     b0 = 0
@@ -130,50 +131,55 @@ def test_hpsi_batch_sticks(gpu, dims, m, prec, tol, channels, counts):
         w[b0:b0 + nb] += kin[ik] * p + (proj[ik][0] @ (proj[ik][1] @ p.T)).T
         b0 += nb
     assert np.abs(got - w).max() < tol * np.abs(w).max()
-    # fewer entries next: the tables change
+    # fewer entries next
     got = gpu.hpsi_batch(order[:1], nbands[:1], psi[:nbands[0]], prec)
     assert np.abs(got - w[:nbands[0]]).max() < tol * np.abs(w).max()
 
 
-@pytest.mark.parametrize("uploaded", [False, True])
-def test_hpsi_batch_sticks_captured(gpu, uploaded):
-    # a batch captured into a graph: entry by entry where its tables are not on the device yet, grouped
-    # afterwards; replays equal the same launches outside the graph
+# batches run between the replays of one with k-points 2, 0, 1 and 5, 3, 4 bands: fewer entries, the same
+# size with other k-points and counts, more entries, more bands
+OTHERS = [([2, 0], [5, 3]), ([1], [12]), ([0, 1, 2], [4, 5, 3]), ([1, 1, 0, 2, 0], [1, 2, 3, 1, 9])]
+
+
+@pytest.mark.parametrize("dims", [(25, 25, 25), (27, 25, 32)])
+def test_hpsi_batch_sticks_captured(gpu, dims):
+    # replays of a captured batch equal the same batch run directly, whatever other batches (of either
+    # precision) run between them
     import torch
 
-    miller, _ = setup(gpu, (25, 25, 25), 6)
+    miller, _ = setup(gpu, dims, 6)
     npw, nch = len(miller), 7
     rng = np.random.default_rng(34)
-    gpu.set_veff((np.fft.fftn(rng.uniform(-13.6, 13.6, (25, 25, 25))) / 25 ** 3).reshape(-1))
+    gpu.set_veff((np.fft.fftn(rng.uniform(-13.6, 13.6, dims)) / np.prod(dims)).reshape(-1))
     gpu.set_nk(3)
     for ik in range(3):
         gpu.set_kinetic(ik, (miller.astype(float) ** 2).sum(1) * (1 + 0.1 * ik))
         b = (rng.standard_normal((npw, nch)) + 1j * rng.standard_normal((npw, nch))) / np.sqrt(npw)
         gpu.set_nonlocal(ik, b, b.conj().T.copy())
     order, nbands = [2, 0, 1], [5, 3, 4]
-    psi = torch.from_numpy(bands(rng, sum(nbands), npw).astype(np.complex64)).cuda()
-    out = torch.empty_like(psi)
+    most = max(sum(nb) for _, nb in OTHERS)
+    psi = torch.from_numpy(bands(rng, most, npw).astype(np.complex64)).cuda()
+    psi64 = psi.to(torch.complex128)
+    out, other, other64 = torch.empty_like(psi), torch.empty_like(psi), torch.empty_like(psi64)
     torch.cuda.synchronize()
-
-    def entries():
-        b0 = 0
-        for ik, nb in zip(order, nbands):
-            gpu.hpsi_dev(ik, nb, psi[b0].data_ptr(), out[b0].data_ptr(), "fp32")
-            b0 += nb
 
     def batch():
         gpu.hpsi_batch_dev(order, nbands, psi.data_ptr(), out.data_ptr(), "fp32")
 
-    batch()  # workspaces
-    entries()
-    if not uploaded:
-        gpu.hpsi_batch_dev(order[:2], nbands[:2], psi.data_ptr(), out.data_ptr(), "fp32")  # another table
-        entries()
-    else:
-        batch()
+    def others():
+        for ks, nb in OTHERS:
+            gpu.hpsi_batch_dev(ks, nb, psi.data_ptr(), other.data_ptr(), "fp32")
+            yield ks
+            gpu.hpsi_batch_dev(ks, nb, psi64.data_ptr(), other64.data_ptr(), "fp64")
+            yield ks
+
+    list(others())  # workspaces
+    out.zero_()
+    torch.cuda.synchronize()
+    batch()
     gpu.sync()
     want = out.cpu()
-    print("captured batch", uploaded, flush=True)
+    print("captured batch", dims, flush=True)
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.stream(torch.cuda.ExternalStream(gpu.stream)):
         graph.capture_begin(capture_error_mode="thread_local")
@@ -181,13 +187,16 @@ def test_hpsi_batch_sticks_captured(gpu, uploaded):
             batch()
         finally:
             graph.capture_end()
-        for _ in range(3):
+        for ks in others():
+            gpu.sync()
             out.zero_()
             graph.replay()
             torch.cuda.synchronize()
-            assert torch.equal(out.cpu(), want)
-            batch()
-            gpu.sync()
+            assert torch.equal(out.cpu(), want), ks
+        out.zero_()
+        batch()
+        gpu.sync()
+        assert torch.equal(out.cpu(), want)
 
 
 @pytest.mark.parametrize("dims,m", [((25, 25, 25), 6), ((27, 25, 32), 6), ((27, 27, 27), 13)])
