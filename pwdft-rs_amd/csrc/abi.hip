@@ -539,7 +539,7 @@ int pwk_dense_eigh(pwk_ctx* ctx, int n, int nb, int nk, double* h, double* w, do
     dw.ensure(nw * 8);
     dv.ensure(nv * 8);
     PWK_HIP(hipMemcpyAsync(dh.p, h, nh * 8, hipMemcpyHostToDevice, c.stream));
-    c.eig_work.ensure(pwk::heev_work_doubles(n, nb, nk) * 8);
+    c.workspace(c.eig_work, pwk::heev_work_doubles(n, nb, nk) * 8);
     pwk::launch_heev_batched(c, n, nb, nk, dh.p, c.eig_work.p, dw.as<double>(), dv.p, nullptr);
     PWK_HIP(hipMemcpyAsync(h, dh.p, nh * 8, hipMemcpyDeviceToHost, c.stream));
     PWK_HIP(hipMemcpyAsync(w, dw.p, nw * 8, hipMemcpyDeviceToHost, c.stream));
@@ -552,7 +552,7 @@ int pwk_dev_dense_eigh(pwk_ctx* ctx, int n, int nb, int nk, void* h, void* w, vo
   return guarded([&] {
     Context& c = ctx_of(ctx);
     PWK_REQUIRE(h && w && v, PWK_E_INVALID, "null eigensolver buffer");
-    c.eig_work.ensure(pwk::heev_work_doubles(n, nb, nk) * 8);
+    c.workspace(c.eig_work, pwk::heev_work_doubles(n, nb, nk) * 8);
     pwk::launch_heev_batched(c, n, nb, nk, h, c.eig_work.p, (double*)w, v, nullptr);
   });
 }

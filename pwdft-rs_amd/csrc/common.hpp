@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 #include <cstdio>
 #include <map>
@@ -390,6 +391,27 @@ struct Context {
   DevBuf gemm_ws;         // split-K partial sums
   DevBuf eig_work;        // dense eigensolver scratch
   DevBuf host_in, host_out;  // staging for host-pointer entry points
+
+  // Workspaces that captured kernels use outlive their growth: a larger call would free the block under the
+  // graphs that hold its address. Once the stream has been captured a workspace grows by at least half into a
+  // new block, and the old blocks (together at most twice the present one) stay until the context ends.
+  bool graph_seen = false;
+  std::vector<DevBuf> retired;
+  bool capturing() {
+    hipStreamCaptureStatus s = hipStreamCaptureStatusNone;
+    PWK_HIP(hipStreamIsCapturing(stream, &s));
+    if (s != hipStreamCaptureStatusNone) graph_seen = true;
+    return s != hipStreamCaptureStatusNone;
+  }
+  void* workspace(DevBuf& b, size_t bytes) {
+    if (!graph_seen) (void)capturing();
+    if (bytes > b.bytes && b.p && graph_seen) {
+      bytes = std::max(bytes, b.bytes + b.bytes / 2);
+      retired.push_back(std::move(b));
+    }
+    b.ensure(bytes);
+    return b.p;
+  }
 
   Profiler prof;
 

@@ -229,9 +229,7 @@ void density_sticks_t(Context& c, int nb, const void* psi, const double* fw_host
   // the bands that carry weight (src/scf/density.rs:14,72), their weights first. While the stream is captured
   // every band is transformed and the weights are the caller's own at each replay: the kernels skip the
   // bands without weight.
-  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-  PWK_HIP(hipStreamIsCapturing(c.stream, &cap));
-  const bool captured = cap != hipStreamCaptureStatusNone;
+  const bool captured = c.capturing();
   std::vector<double>& h = c.dens_host;
   int live = nb;
   if (!captured) {
@@ -248,7 +246,7 @@ void density_sticks_t(Context& c, int nb, const void* psi, const double* fw_host
   int groups = 0;
   if (live > 0) {
     const size_t wbytes = (captured ? (size_t)nb : h.size()) * sizeof(double);
-    c.work_b.ensure(wbytes);
+    c.workspace(c.work_b, wbytes);
     PWK_HIP(hipMemcpyAsync(c.work_b.p, captured ? fw_host : h.data(), wbytes, hipMemcpyHostToDevice, c.stream));
     const double* fw = c.work_b.as<double>();
     // about 1024 workgroups (four per CU): more only adds partial sums to store and read, fewer leave
@@ -262,7 +260,7 @@ void density_sticks_t(Context& c, int nb, const void* psi, const double* fw_host
     // one z-inverse buffer for all live bands, then the groups' partial sums
     const size_t ns = (size_t)live * nz * c.nsticks, held = square ? 0 : sphere_rows_elems(c, live);
     const size_t tb = ((ns + held) * sizeof(V2) + 255) & ~(size_t)255;
-    c.work_a.ensure(tb + (size_t)groups * c.N * sizeof(double));
+    c.workspace(c.work_a, tb + (size_t)groups * c.N * sizeof(double));
     double* part = reinterpret_cast<double*>(c.work_a.as<unsigned char>() + tb);
     launch_zinv(c, live, psi, c.work_a.p, std::is_same<T, double>::value ? PWK_FP64 : PWK_FP32,
                 captured ? nullptr : reinterpret_cast<const int*>(fw + live));

@@ -388,7 +388,7 @@ void zgemm_mfma_t(Context& c, int M, int N, int K, const void* A, int lda, const
   dim3 grid((unsigned)((long)mt * nt * nsplit * bt.count));
   void* part = nullptr;
   if (nsplit > 1) {
-    c.gemm_ws.ensure((size_t)bt.count * nsplit * M * N * sizeof(V2));
+    c.workspace(c.gemm_ws, (size_t)bt.count * nsplit * M * N * sizeof(V2));
     part = c.gemm_ws.p;
   }
   int acc = (nsplit == 1 && accumulate) ? 1 : 0;

@@ -293,7 +293,7 @@ void hpsi_fullgrid(Context& c, const T* kin, int nb, int nbk, const void* psi, v
   const T* vr = std::is_same<T, double>::value ? (const T*)c.vrn64.p : (const T*)c.vrn32.p;
   const size_t N = c.N;
   const int chunk = grid_chunk<T>(c, nb);
-  c.work_a.ensure((size_t)chunk * N * sizeof(V2));
+  c.workspace(c.work_a, (size_t)chunk * N * sizeof(V2));
   V2* grid = c.work_a.as<V2>();
   TimedScope ts(c, "hpsi_fullgrid");
   for (int b0 = 0; b0 < nb; b0 += chunk) {
@@ -320,8 +320,8 @@ void density_fullgrid(Context& c, int nb, const void* psi, const double* fw_host
   const int prec = std::is_same<T, double>::value ? PWK_FP64 : PWK_FP32;
   const size_t N = c.N;
   const int chunk = grid_chunk<T>(c, nb);
-  c.work_a.ensure((size_t)chunk * N * sizeof(V2));
-  c.work_b.ensure((size_t)nb * sizeof(double));
+  c.workspace(c.work_a, (size_t)chunk * N * sizeof(V2));
+  c.workspace(c.work_b, (size_t)nb * sizeof(double));
   PWK_HIP(hipMemcpyAsync(c.work_b.p, fw_host, (size_t)nb * sizeof(double), hipMemcpyHostToDevice, c.stream));
   V2* grid = c.work_a.as<V2>();
   for (int b0 = 0; b0 < nb; b0 += chunk) {
@@ -376,7 +376,7 @@ void hpsi_local(Context& c, const T* kin, int nb, int nbk, const void* psi, void
   }
   PWK_REQUIRE(nb <= 65535, PWK_E_UNSUPPORTED, "too many bands in one H·psi launch");
   const size_t ns = (size_t)nb * nz * c.nsticks, rows = nx == c.dims[1] ? 0 : sphere_rows_elems(c, nb);
-  c.work_a.ensure((ns + rows) * sizeof(V2));
+  c.workspace(c.work_a, (ns + rows) * sizeof(V2));
   V2* T_ = c.work_a.as<V2>();
   const T* vr = std::is_same<T, double>::value ? (const T*)c.vr64.p : (const T*)c.vr32.p;
   dim3 gz(blocks_for((size_t)c.nsticks, 64), (unsigned)nb);
@@ -539,7 +539,7 @@ void set_veff_device(Context& c, const void* veff_g_dev, int slot, bool need_g) 
   } else {
     PWK_REQUIRE(c.vrn64.bytes >= 2 * n * sizeof(double), PWK_E_STATE, "second V_eff slot not reserved");
   }
-  c.work_b.ensure(n * sizeof(double2));
+  c.workspace(c.work_b, n * sizeof(double2));
   launch_fft3d_copy(c, veff_g_dev, c.work_b.p, +1);
   const size_t o = (size_t)slot * n;
   k_vr_reorder<<<blocks_for(n, 256), 256, 0, c.stream>>>(c.work_b.as<double2>(), c.vr64.as<double>() + o,
@@ -576,7 +576,7 @@ void launch_hpsi(Context& c, int ik, int nb, const void* psi, void* hpsi, int pr
   if (kd.nch > 0) {
     // P = (D·B^H)·ψ  (nch × nb), then Hψ += B·P   (src/potential/nonlocal.rs:432-450)
     size_t es = precision == PWK_FP64 ? sizeof(double2) : sizeof(float2);
-    c.proj.ensure((size_t)kd.nch * nb * es);
+    c.workspace(c.proj, (size_t)kd.nch * nb * es);
     const void* dbh = precision == PWK_FP64 ? kd.DBH64.p : kd.DBH32.p;
     const void* bm = precision == PWK_FP64 ? kd.B64.p : kd.B32.p;
     {
@@ -702,7 +702,7 @@ void hpsi_batch_sticks(Context& c, int e0, int e1, const int32_t* ik, const int3
   }
   hpsi_local<T>(c, nullptr, total, 1, psi, hpsi, kin);
   if (nch > 0) {
-    c.proj.ensure((size_t)nch * total * sizeof(typename V2t<T>::t));
+    c.workspace(c.proj, (size_t)nch * total * sizeof(typename V2t<T>::t));
     {
       TimedScope ts(c, "hpsi_nl_project");
       launch_zgemm_mfma_groups(c, nch, nmax, c.npw, project, nch, psi, c.npw, c.proj.p, nch, false, precision);
@@ -799,7 +799,7 @@ void launch_density(Context& c, int nb, const void* psi, const double* fw_host, 
   PWK_REQUIRE(nb > 0, PWK_E_INVALID, "nb must be positive");
   const int dprec = precision == PWK_FP64 ? PWK_FP64 : PWK_FP32;
   if (density_small_supported(c, dprec)) {
-    c.work_b.ensure((size_t)nb * sizeof(double));
+    c.workspace(c.work_b, (size_t)nb * sizeof(double));
     PWK_HIP(hipMemcpyAsync(c.work_b.p, fw_host, (size_t)nb * sizeof(double), hipMemcpyHostToDevice, c.stream));
     launch_density_small(c, nb, psi, c.work_b.as<double>(), rho, dprec, overwrite);
     return;

@@ -842,7 +842,7 @@ void launch_density_small_t(Context& c, int nb, const void* psi, const double* f
   const size_t sh = small_lds_bytes<T>(n, 0);
   const int gsize = std::max(1, (nb + 127) / 128);  // at most 128 groups, as the reduction takes
   const int ng = (nb + gsize - 1) / gsize;
-  c.work_a.ensure((size_t)ng * c.N * sizeof(double));
+  c.workspace(c.work_a, (size_t)ng * c.N * sizeof(double));
   TimedScope ts(c, "density_small");
   switch (n) {
 #define PWK_CASE(L)                                                                                            \

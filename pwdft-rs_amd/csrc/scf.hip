@@ -1795,7 +1795,7 @@ void Solve::setup() {
   if (p.precision != PWK_FP64) V32.ensure((size_t)ns * nk * npw * nbs * 8);
   if (!chebyshev) {
     Hb.ensure((size_t)nk * npw * npw * 16);
-    c.eig_work.ensure(heev_work_doubles(npw, nb, nk) * 8);
+    c.workspace(c.eig_work, heev_work_doubles(npw, nb, nk) * 8);
   } else {
     PWK_REQUIRE(heev_supported(nbs, nbs), PWK_E_UNSUPPORTED, "too many bands for the subspace eigensolver");
     fprec = p.precision;

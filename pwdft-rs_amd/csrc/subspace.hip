@@ -649,7 +649,7 @@ void subspace_rr(Context& c, int n, int nb, int nk, const void* H, const void* V
     launch_zgemm_mfma_batched(c, nb, nb, n, VH.p, nb, nbk, HV.p, n, nbk, Hs.p, nb, bb, nk, false, PWK_FP64);
     k_lower_to_full<<<dim3(blocks_for((size_t)bb, 256), (unsigned)nk), 256, 0, c.stream>>>(nb, Hs.as<double2>());
     PWK_HIP(hipGetLastError());
-    c.eig_work.ensure(heev_work_doubles(nb, nb, nk) * 8);
+    c.workspace(c.eig_work, heev_work_doubles(nb, nb, nk) * 8);
     launch_heev_batched(c, nb, nb, nk, Hs.p, c.eig_work.p, w, U.p, nullptr);
     launch_zgemm_mfma_batched(c, n, nb, nb, Vprev, n, nbk, U.p, nb, bb, V, n, nbk, nk, false, PWK_FP64);
     launch_zgemm_mfma_batched(c, n, nb, n, H, n, nn, V, n, nbk, HV.p, n, nbk, nk, false, PWK_FP64);
@@ -679,7 +679,7 @@ void subspace_rr(Context& c, int n, int nb, int nk, const void* H, const void* V
     for (int i = 0; i < nf; ++i)
       PWK_HIP(hipMemcpyAsync(hf.as<double2>() + (size_t)i * nn, (const double2*)H + (size_t)redo[(size_t)i] * nn,
                              (size_t)nn * 16, hipMemcpyDeviceToDevice, c.stream));
-    c.eig_work.ensure(heev_work_doubles(n, nb, nf) * 8);
+    c.workspace(c.eig_work, heev_work_doubles(n, nb, nf) * 8);
     launch_heev_batched(c, n, nb, nf, hf.p, c.eig_work.p, wf.as<double>(), vf.p, nullptr);
     for (int i = 0; i < nf; ++i) {
       const int k = redo[(size_t)i];

@@ -254,3 +254,53 @@ def test_zgemm_column_blocks(gpu, prec, tol):
         err = np.abs(dC.cpu().numpy().T - ref).max() / np.abs(ref).max()
         print("zgemm", prec, (m, n, k), f"{err:.2e}", flush=True)
         assert err < tol, (m, n, k)
+
+
+@pytest.mark.parametrize("dims", [(25, 25, 25), (27, 25, 32)])
+def test_captured_workspaces_survive_growth(pwk_mod, gpu, dims):
+    # replays of a captured H·ψ batch and density after larger direct calls, which grow every workspace that
+    # the graph's kernels use
+    import torch
+
+    acc = pwk_mod.GpuAccelerator(0)  # workspaces of its own, as small as the first calls need
+    try:
+        miller, _ = setup(acc, dims, 6)
+        npw, nch, n = len(miller), 40, int(np.prod(dims))
+        rng = np.random.default_rng(36)
+        acc.set_veff((np.fft.fftn(rng.uniform(-13.6, 13.6, dims)) / n).reshape(-1))
+        acc.set_nk(2)
+        for ik in range(2):
+            acc.set_kinetic(ik, (miller.astype(float) ** 2).sum(1) * (1 + 0.1 * ik))
+            b = (rng.standard_normal((npw, nch)) + 1j * rng.standard_normal((npw, nch))) / np.sqrt(npw)
+            acc.set_nonlocal(ik, b, b.conj().T.copy())
+        fw = rng.uniform(0.1, 2.0, 96)
+        psi = torch.from_numpy(bands(rng, 96, npw)).cuda()
+        out, rho = torch.zeros_like(psi), torch.zeros(n, dtype=torch.float64, device="cuda")
+        other, rho2 = torch.zeros_like(psi), torch.zeros_like(rho)
+        torch.cuda.synchronize()
+
+        def calls(nb, h, r):
+            acc.hpsi_batch_dev([1, 0], [nb, nb - 1], psi.data_ptr(), h.data_ptr(), "fp64")
+            acc.density_dev(nb, psi.data_ptr(), fw, r.data_ptr(), "fp64")
+
+        calls(2, out, rho)
+        acc.sync()
+        want = out.cpu(), rho.cpu()
+        print("captured, then larger calls", dims, flush=True)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.stream(torch.cuda.ExternalStream(acc.stream)):
+            graph.capture_begin(capture_error_mode="thread_local")
+            try:
+                calls(2, out, rho)
+            finally:
+                graph.capture_end()
+            for nb in (5, 17, 48):
+                calls(nb, other, rho2)
+                acc.sync()
+                out.zero_()
+                rho.zero_()
+                graph.replay()
+                torch.cuda.synchronize()
+                assert torch.equal(out.cpu(), want[0]) and torch.equal(rho.cpu(), want[1]), nb
+    finally:
+        acc.close()
