@@ -243,24 +243,26 @@ void density_sticks_t(Context& c, int nb, const void* psi, const double* fw_host
       if (!(fw_host[b] < 1e-15)) list[i++] = b;
   }
   const int nx = c.dims[0], ny = c.dims[1], nz = c.dims[2];
-  int groups = 0;
+  // about 1024 workgroups (four per CU): more only adds partial sums to store and read, fewer leave
+  // CUs idle (60³ × 144 bands: 72 batches × 60 planes in 15 groups).
+  const bool square = nx == ny;
+  const int slots = square ? plane_slots<T>(nx) : 1;
+  const long wgs = square ? nz : (ny * nz + 63) / 64;  // workgroups per group
+  // The workspaces are sized for all nb bands, whatever their weights: a captured call transforms every band
+  // and cannot allocate, and its first run outside the graph may have had bands without weight. One z-inverse
+  // buffer, then the groups' partial sums, of which any number of live bands makes at most max_groups.
+  const size_t ns = (size_t)nb * nz * c.nsticks, held = square ? 0 : sphere_rows_elems(c, nb);
+  const size_t tb = ((ns + held) * sizeof(V2) + 255) & ~(size_t)255;
+  const long max_groups = std::min<long>((nb + slots - 1) / slots, (1024 + wgs - 1) / wgs);
+  c.workspace(c.work_a, tb + (size_t)max_groups * c.N * sizeof(double));
+  c.workspace(c.work_b, ((size_t)nb + (size_t)(nb + 1) / 2) * sizeof(double));
   if (live > 0) {
     const size_t wbytes = (captured ? (size_t)nb : h.size()) * sizeof(double);
-    c.workspace(c.work_b, wbytes);
     PWK_HIP(hipMemcpyAsync(c.work_b.p, captured ? fw_host : h.data(), wbytes, hipMemcpyHostToDevice, c.stream));
     const double* fw = c.work_b.as<double>();
-    // about 1024 workgroups (four per CU): more only adds partial sums to store and read, fewer leave
-    // CUs idle (60³ × 144 bands: 72 batches × 60 planes in 15 groups).
-    const bool square = nx == ny;
-    const int slots = square ? plane_slots<T>(nx) : 1;
     const int batches = (live + slots - 1) / slots;
-    const long wgs = square ? nz : (ny * nz + 63) / 64;  // workgroups per group
     const int per = std::max(1, (int)((batches * wgs + 1023) / 1024));
-    groups = (batches + per - 1) / per;
-    // one z-inverse buffer for all live bands, then the groups' partial sums
-    const size_t ns = (size_t)live * nz * c.nsticks, held = square ? 0 : sphere_rows_elems(c, live);
-    const size_t tb = ((ns + held) * sizeof(V2) + 255) & ~(size_t)255;
-    c.workspace(c.work_a, tb + (size_t)groups * c.N * sizeof(double));
+    const int groups = (batches + per - 1) / per;
     double* part = reinterpret_cast<double*>(c.work_a.as<unsigned char>() + tb);
     launch_zinv(c, live, psi, c.work_a.p, std::is_same<T, double>::value ? PWK_FP64 : PWK_FP32,
                 captured ? nullptr : reinterpret_cast<const int*>(fw + live));

@@ -233,6 +233,46 @@ def test_density_captured(gpu, dims, m):
             assert np.abs(rho.cpu().numpy() - want).max() < nb * 2.3e-16 * want.max()
 
 
+@pytest.mark.parametrize("dims,m", [((25, 25, 25), 6), ((27, 25, 32), 6), ((27, 27, 27), 13)])
+@pytest.mark.parametrize("first", [[2, 3, 4, 5, 6], list(range(7))])
+def test_density_captured_after_unoccupied_bands(pwk_mod, gpu, dims, m, first):
+    # the call before the capture has bands without weight (or nothing but such bands); the captured one uses
+    # every band
+    import torch
+
+    acc = pwk_mod.GpuAccelerator(0)  # workspaces as that first call leaves them
+    try:
+        miller, _ = setup(acc, dims, m)
+        rng = np.random.default_rng(37)
+        nb, n = 7, int(np.prod(dims))
+        psi = bands(rng, nb, len(miller))
+        dev = torch.from_numpy(psi).cuda()
+        rho = torch.zeros(n, dtype=torch.float64, device="cuda")
+        fw = rng.uniform(0.1, 2.0, nb)
+        weights = fw.copy()
+        fw[first] = 0.0
+        torch.cuda.synchronize()
+        print("captured density after zero weights", dims, m, first, flush=True)
+        acc.density_dev(nb, dev.data_ptr(), fw, rho.data_ptr(), "fp64")
+        acc.sync()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.stream(torch.cuda.ExternalStream(acc.stream)):
+            graph.capture_begin(capture_error_mode="thread_local")
+            try:
+                acc.density_dev(nb, dev.data_ptr(), fw, rho.data_ptr(), "fp64")
+            finally:
+                graph.capture_end()
+            fw[:] = weights
+            want = acc.density(psi, fw, None, "fp64")
+            for _ in range(3):
+                rho.zero_()
+                graph.replay()
+                torch.cuda.synchronize()
+                assert np.abs(rho.cpu().numpy() - want).max() < nb * 2.3e-16 * want.max()
+    finally:
+        acc.close()
+
+
 @pytest.mark.parametrize("prec,tol", [("fp64", 1e-13), ("fp32", 2e-5), ("split_bf16", 5e-5)])
 def test_zgemm_column_blocks(gpu, prec, tol):
     # column counts around one and two blocks of 144, row counts that make few and many tiles, reductions
