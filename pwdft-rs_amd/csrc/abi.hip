@@ -380,7 +380,6 @@ int pwk_set_basis(pwk_ctx* ctx, int npw, const int32_t* miller) {
     Context& c = ctx_of(ctx);
     pwk::setup_basis(c, npw, miller);
     c.kd.clear();
-    c.pack_valid = false;
   });
 }
 
@@ -389,7 +388,6 @@ int pwk_set_nk(pwk_ctx* ctx, int nk) {
     Context& c = ctx_of(ctx);
     PWK_REQUIRE(nk >= 0, PWK_E_INVALID, "nk must be non-negative");
     c.kd.resize((size_t)nk);
-    c.pack_valid = false;
   });
 }
 
@@ -398,7 +396,6 @@ int pwk_set_kinetic(pwk_ctx* ctx, int ik, const double* t) {
     Context& c = ctx_of(ctx);
     c.check_basis();
     pwk::KData& kd = c.k(ik);
-    c.pack_valid = false;
     kd.kin64.ensure((size_t)c.npw * 8);
     kd.kin32.ensure((size_t)c.npw * 4);
     PWK_HIP(hipMemcpyAsync(kd.kin64.p, t, (size_t)c.npw * 8, hipMemcpyHostToDevice, c.stream));
@@ -433,7 +430,6 @@ int pwk_set_nonlocal(pwk_ctx* ctx, int ik, int nch, const double* B, const doubl
     c.check_basis();
     pwk::KData& kd = c.k(ik);
     PWK_REQUIRE(nch >= 0, PWK_E_INVALID, "nch must be non-negative");
-    c.pack_valid = false;
     kd.nch = nch;
     if (nch == 0) return;
     size_t n = (size_t)c.npw * nch;

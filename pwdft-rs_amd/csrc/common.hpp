@@ -289,6 +289,13 @@ struct BatchKin {
   int end[MAX_BATCH_ENTRIES];
   const void* kin[MAX_BATCH_ENTRIES];
 };
+// the same on the fused small grids, with the projector blocks
+struct BatchSmall {
+  static constexpr bool batch = true;
+  int n = 0;
+  int end[MAX_BATCH_ENTRIES];
+  const void *kin[MAX_BATCH_ENTRIES], *B[MAX_BATCH_ENTRIES], *DBH[MAX_BATCH_ENTRIES];
+};
 // product e is C[:, col..col + cols) (+)= A·B[:, col..col + cols) with its own A
 struct GemmGroups {
   static constexpr bool batch = true;
@@ -296,13 +303,17 @@ struct GemmGroups {
   int cols[MAX_BATCH_ENTRIES], col[MAX_BATCH_ENTRIES];
   const void* A[MAX_BATCH_ENTRIES];
 };
-// the kinetic diagonal of band b: its entry's (found by one load per lane; every lane of the wave calls it),
-// or without entries that of k-point b / nbk
+// the entry of band b (uniform) by one load per lane; every lane of the wave calls it
+template <class Entries>
+__device__ __forceinline__ int batch_entry(const Entries& entries, int b) {
+  const int lane = threadIdx.x & 63;
+  return __popcll(__ballot(lane < entries.n && entries.end[lane] <= b));
+}
+// the kinetic diagonal of band b: its entry's, or without entries that of k-point b / nbk
 template <typename T, class Entries>
 __device__ __forceinline__ const T* band_kin(const Entries& entries, const T* kin, int npw, int nbk, int b) {
   if constexpr (Entries::batch) {
-    const int lane = threadIdx.x & 63;
-    return (const T*)entries.kin[__popcll(__ballot(lane < entries.n && entries.end[lane] <= b))];
+    return (const T*)entries.kin[batch_entry(entries, b)];
   } else {
     return kin + (size_t)(b / nbk) * npw;
   }
@@ -375,13 +386,6 @@ struct Context {
   FftPlan fft_plan;
 
   std::vector<KData> kd;
-  // the kinetic diagonals and projector blocks of all k-points packed k-major (ragged k × band
-  // H·ψ batches on small grids); rebuilt after any change to the per-k data
-  bool pack_valid = false;
-  int pack_nch = 0;
-  DevBuf kin_pack64, kin_pack32, B_pack64, B_pack32, DBH_pack64, DBH_pack32;
-  DevBuf band_tab;                  // int32 k-point per band of the last batch
-  std::vector<int32_t> band_tab_host;
 
   std::vector<double> dens_host;  // weights and list of the last density's live bands
 
@@ -511,11 +515,11 @@ void launch_density_batch(Context& c, int nent, const int32_t* ik, const int32_t
 bool hpsi_small_supported(const Context& c, int precision, int nch);
 // nkv > 0: the band blocks of consecutive groups of nkv k-points use V(r) slot 0, 1, ...
 // (spin channels of LSDA; kinetic and projector blocks are indexed by block mod nkv)
-// band_k (device, nbands entries): k-point block of every band, for ragged k × band batches
 void launch_hpsi_small(Context& c, int nbands, int nbk, const void* psi, void* hpsi, int precision, const void* kin,
                        int nch, const void* B, const void* DBH, const double* coef = nullptr,
-                       const void* X = nullptr, int nkv = 0, const int* band_k = nullptr,
-                       const int* skip = nullptr);
+                       const void* X = nullptr, int nkv = 0, const int* skip = nullptr);
+// the entries of a ragged k × band batch with nch channels each, in one launch
+void launch_hpsi_small_batch(Context& c, const BatchSmall& entries, const void* psi, void* hpsi, int precision, int nch);
 // the whole degree-`degree` Chebyshev filter of nbands bands in one launch on small cubic grids:
 // Yout (FP64) = p(H)·V (FP64) with the recurrence in `precision`; coef (device) holds (α, c, β)
 // per step and band block, coef[(i·nblocks + kb)·3 + j]

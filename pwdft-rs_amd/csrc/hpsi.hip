@@ -619,47 +619,6 @@ void launch_hpsi_multi(Context& c, int nk, int nb, const void* psi, void* hpsi, 
 
 namespace {
 
-// Packs the kinetic diagonals and projector blocks of every k-point k-major into the context's
-// pack buffers (device copies), once per change of the per-k data. False when the k-points do
-// not share one channel count or miss data (the caller then goes k-point by k-point).
-bool pack_kdata(Context& c) {
-  if (c.pack_valid) return true;
-  const int nk = (int)c.kd.size();
-  if (nk == 0) return false;
-  const int nch = c.kd[0].nch;
-  for (const KData& kd : c.kd)
-    if (!kd.have_kin || kd.nch != nch || (nch > 0 && !(kd.B64.p && kd.DBH64.p && kd.B32.p && kd.DBH32.p)))
-      return false;
-  const size_t npw = (size_t)c.npw, blk = npw * (size_t)nch;
-  c.kin_pack64.ensure((size_t)nk * npw * 8);
-  c.kin_pack32.ensure((size_t)nk * npw * 4);
-  if (nch > 0) {
-    c.B_pack64.ensure((size_t)nk * blk * 16);
-    c.DBH_pack64.ensure((size_t)nk * blk * 16);
-    c.B_pack32.ensure((size_t)nk * blk * 8);
-    c.DBH_pack32.ensure((size_t)nk * blk * 8);
-  }
-  for (int k = 0; k < nk; ++k) {
-    const KData& kd = c.kd[(size_t)k];
-    PWK_HIP(hipMemcpyAsync(c.kin_pack64.as<double>() + (size_t)k * npw, kd.kin64.p, npw * 8, hipMemcpyDeviceToDevice,
-                           c.stream));
-    PWK_HIP(hipMemcpyAsync(c.kin_pack32.as<float>() + (size_t)k * npw, kd.kin32.p, npw * 4, hipMemcpyDeviceToDevice,
-                           c.stream));
-    if (nch == 0) continue;
-    PWK_HIP(hipMemcpyAsync(c.B_pack64.as<double2>() + (size_t)k * blk, kd.B64.p, blk * 16, hipMemcpyDeviceToDevice,
-                           c.stream));
-    PWK_HIP(hipMemcpyAsync(c.DBH_pack64.as<double2>() + (size_t)k * blk, kd.DBH64.p, blk * 16,
-                           hipMemcpyDeviceToDevice, c.stream));
-    PWK_HIP(hipMemcpyAsync(c.B_pack32.as<float2>() + (size_t)k * blk, kd.B32.p, blk * 8, hipMemcpyDeviceToDevice,
-                           c.stream));
-    PWK_HIP(hipMemcpyAsync(c.DBH_pack32.as<float2>() + (size_t)k * blk, kd.DBH32.p, blk * 8, hipMemcpyDeviceToDevice,
-                           c.stream));
-  }
-  c.pack_nch = nch;
-  c.pack_valid = true;
-  return true;
-}
-
 size_t batch_bands(Context& c, int nent, const int32_t* ik, const int32_t* nbands) {
   PWK_REQUIRE(nent >= 1 && ik && nbands, PWK_E_INVALID, "empty or null k-point batch");
   size_t total = 0;
@@ -712,20 +671,21 @@ void hpsi_batch_sticks(Context& c, int e0, int e1, const int32_t* ik, const int3
   }
 }
 
-// The entries from e0 on that share their launches: as many as one launch takes, with one channel count and
-// at most 256 MiB of sticks (a chunk of the whole-grid path; entries beyond it fill the chip by themselves).
-template <typename T>
-int batch_run(Context& c, int nent, int e0, const int32_t* ik, const int32_t* nbands) {
-  const bool f64 = std::is_same<T, double>::value;
-  const size_t per_band = ((size_t)c.dims[2] * c.nsticks + (c.dims[0] == c.dims[1] ? 0 : sphere_rows_elems(c, 1))) *
-                          sizeof(typename V2t<T>::t);
+// The entries from e0 on that share their launches: as many as one launch takes, with one channel count, and
+// off the small grids at most 256 MiB of sticks (a chunk of the whole-grid path; entries beyond it fill the
+// chip by themselves).
+int batch_run(Context& c, int nent, int e0, const int32_t* ik, const int32_t* nbands, bool small, bool f64) {
+  const size_t per_band = small ? 0
+                                : ((size_t)c.dims[2] * c.nsticks + (c.dims[0] == c.dims[1] ? 0 : sphere_rows_elems(c, 1))) *
+                                      (f64 ? sizeof(double2) : sizeof(float2));
+  const size_t most = small ? 0x7fffffff : 65535;
   const int nch = c.k(ik[e0]).nch;
   size_t total = 0;
   int e = e0;
   for (; e < nent && e - e0 < MAX_BATCH_ENTRIES; ++e) {
     const KData& kd = c.k(ik[e]);
     total += (size_t)nbands[e];
-    if (total > 65535 || total * per_band > ((size_t)256 << 20)) break;
+    if (total > most || total * per_band > ((size_t)256 << 20)) break;
     if (kd.nch != nch || (nch > 0 && !(f64 ? kd.B64.p && kd.DBH64.p : kd.B32.p && kd.DBH32.p))) break;
   }
   return std::max(e, e0 + 1);
@@ -734,48 +694,37 @@ int batch_run(Context& c, int nent, int e0, const int32_t* ik, const int32_t* nb
 }  // namespace
 
 // H·ψ of a k × band batch with a band count per entry: entry e holds nbands[e] bands of k-point
-// ik[e], the entries' bands packed back to back in psi and hpsi. On small cubic grids the whole
-// batch is one fused launch that reads each band's k-point from a band table; on the stick path entries
-// with the same channel count share each launch; elsewhere one H·ψ per entry.
+// ik[e], the entries' bands packed back to back in psi and hpsi. Consecutive entries with the same channel
+// count share each launch on the stick path, and are one fused launch on small cubic grids; elsewhere one H·ψ
+// per entry.
 void launch_hpsi_batch(Context& c, int nent, const int32_t* ik, const int32_t* nbands, const void* psi, void* hpsi,
                        int precision) {
   c.check_basis();
-  const size_t total = batch_bands(c, nent, ik, nbands);
-  int nch = c.k(ik[0]).nch;
-  if (precision != PWK_SPLIT_BF16 && c.have_v && hpsi_small_supported(c, precision, nch) && pack_kdata(c)) {
-    nch = c.pack_nch;
-    std::vector<int32_t> tab(total);
-    size_t b = 0;
-    for (int e = 0; e < nent; ++e)
-      for (int j = 0; j < nbands[e]; ++j) tab[b++] = ik[e];
-    if (tab != c.band_tab_host) {
-      c.band_tab_host = tab;
-      c.band_tab.ensure(total * sizeof(int32_t));
-      PWK_HIP(hipMemcpyAsync(c.band_tab.p, c.band_tab_host.data(), total * sizeof(int32_t), hipMemcpyHostToDevice,
-                             c.stream));
-      PWK_HIP(hipStreamSynchronize(c.stream));  // the host table may change with the next batch
-    }
-    const bool f64 = precision == PWK_FP64;
-    launch_hpsi_small(c, (int)total, 1, psi, hpsi, precision, f64 ? c.kin_pack64.p : c.kin_pack32.p, nch,
-                      f64 ? c.B_pack64.p : c.B_pack32.p, f64 ? c.DBH_pack64.p : c.DBH_pack32.p, nullptr, nullptr, 0,
-                      c.band_tab.as<int>());
-    return;
-  }
-  const size_t es = precision == PWK_FP64 ? sizeof(double2) : sizeof(float2);
-  const bool sticks = (precision == PWK_SPLIT_BF16 || !hpsi_small_supported(c, precision, nch)) &&
-                      stick_path_ok(c, precision == PWK_FP64);
+  batch_bands(c, nent, ik, nbands);
+  const bool f64 = precision == PWK_FP64;
+  const size_t es = f64 ? sizeof(double2) : sizeof(float2);
   for (int e = 0; e < nent;) {
-    const char* in = (const char*)psi;
-    char* out = (char*)hpsi;
-    const int end = !sticks ? e + 1
-                    : precision == PWK_FP64 ? batch_run<double>(c, nent, e, ik, nbands)
-                                            : batch_run<float>(c, nent, e, ik, nbands);
-    if (end == e + 1)
-      launch_hpsi(c, ik[e], nbands[e], in, out, precision);
-    else if (precision == PWK_FP64)
-      hpsi_batch_sticks<double>(c, e, end, ik, nbands, in, out, precision);
-    else
-      hpsi_batch_sticks<float>(c, e, end, ik, nbands, in, out, precision);
+    const int nch = c.k(ik[e]).nch;
+    const bool small = precision != PWK_SPLIT_BF16 && c.have_v && hpsi_small_supported(c, precision, nch);
+    const int end = small || stick_path_ok(c, f64) ? batch_run(c, nent, e, ik, nbands, small, f64) : e + 1;
+    if (end == e + 1) {
+      launch_hpsi(c, ik[e], nbands[e], psi, hpsi, precision);
+    } else if (small) {
+      BatchSmall entries;
+      entries.n = end - e;
+      for (int i = 0, total = 0; i < end - e; ++i) {
+        const KData& kd = c.k(ik[e + i]);
+        entries.end[i] = total += nbands[e + i];
+        entries.kin[i] = f64 ? kd.kin64.p : kd.kin32.p;
+        entries.B[i] = f64 ? kd.B64.p : kd.B32.p;
+        entries.DBH[i] = f64 ? kd.DBH64.p : kd.DBH32.p;
+      }
+      launch_hpsi_small_batch(c, entries, psi, hpsi, precision, nch);
+    } else if (f64) {
+      hpsi_batch_sticks<double>(c, e, end, ik, nbands, psi, hpsi, precision);
+    } else {
+      hpsi_batch_sticks<float>(c, e, end, ik, nbands, psi, hpsi, precision);
+    }
     for (; e < end; ++e) {
       psi = (const char*)psi + (size_t)nbands[e] * c.npw * es;
       hpsi = (char*)hpsi + (size_t)nbands[e] * c.npw * es;

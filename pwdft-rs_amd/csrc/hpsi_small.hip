@@ -223,8 +223,9 @@ __device__ __forceinline__ void small_ypass(typename V2s<T>::t* G, const LineAct
 // Band b (k-point b / nbk) of psi -> hpsi. vr is V(r) in natural grid order; g2fft the flat
 // grid index of each plane wave; B (npw × nch) and DBH (nch × npw) column-major blocks per k.
 // With coef (α, c, β per k-point) the output is the Chebyshev recurrence step
-// α_k (Hψ − c_k ψ) − β_k X (X may be null) instead of Hψ.
-template <typename T, int N>
+// α_k (Hψ − c_k ψ) − β_k X (X may be null) instead of Hψ. Entries: NoBatch, or the BatchSmall whose entries
+// have their own kin, B and DBH.
+template <typename T, int N, class Entries>
 __device__ __forceinline__ void hpsi_small_body(int bid, int nblocks, const typename V2s<T>::t* __restrict__ psi,
                                                          typename V2s<T>::t* __restrict__ hpsi,
                                                          const T* __restrict__ kin, const T* __restrict__ vr,
@@ -233,8 +234,7 @@ __device__ __forceinline__ void hpsi_small_body(int bid, int nblocks, const type
                                                          const typename V2s<T>::t* __restrict__ DBH, T inv_n,
                                                          const double* __restrict__ coef,
                                                          const typename V2s<T>::t* __restrict__ X, int nkv,
-                                                         const int* __restrict__ band_k,
-                                                         const int* __restrict__ skip) {
+                                                         const int* __restrict__ skip, const Entries& entries) {
   using V2 = typename V2s<T>::t;
   if (skip && *skip) return;  // a filter pass after the residual gate passed (uniform)
   extern __shared__ unsigned char smem_raw[];
@@ -246,14 +246,22 @@ __device__ __forceinline__ void hpsi_small_body(int bid, int nblocks, const type
   // k-point (and its projector blocks) in one XCD's L2
   const int q = nblocks >> 3, r = nblocks & 7, xcd = bid & 7;
   const int b = xcd * q + min(xcd, r) + (bid >> 3), kb = b / nbk;
-  // band block kb: k-point kb mod nkv, V(r) channel kb / nkv (coefficients per block); with a
-  // band table (ragged k × band batches) the k-point of every band is read from it
-  const int k = band_k ? band_k[b] : nkv > 0 ? kb % nkv : kb;
+  // band block kb: k-point kb mod nkv, V(r) channel kb / nkv (coefficients per block)
+  const int k = nkv > 0 ? kb % nkv : kb;
   if (nkv > 0) vr += (size_t)(kb / nkv) * N * N * N;
   const V2* p = psi + (size_t)b * npw;
-  const T* t = kin + (size_t)k * npw;
-  const V2* bk = B + (size_t)k * npw * nch;
-  const V2* dk = DBH + (size_t)k * nch * npw;
+  const T* t;
+  const V2 *bk, *dk;
+  if constexpr (Entries::batch) {
+    const int e = batch_entry(entries, b);
+    t = (const T*)entries.kin[e];
+    bk = (const V2*)entries.B[e];
+    dk = (const V2*)entries.DBH[e];
+  } else {
+    t = kin + (size_t)k * npw;
+    bk = B + (size_t)k * npw * nch;
+    dk = DBH + (size_t)k * nch * npw;
+  }
   const V2* xb = X ? X + (size_t)b * npw : nullptr;
   // operands of the epilogue for this thread's first plane wave, loaded now so that their latency
   // hides behind the transforms (projector rows for up to PF channels)
@@ -577,7 +585,7 @@ __device__ __forceinline__ void cheb_filter_body(int bid, int nblocks, const dou
   for (int g = threadIdx.x; g < npw; g += SMALL_NT) y[g] = make_double2((double)cur[g].x, (double)cur[g].y);
 }
 
-template <typename T, int N>
+template <typename T, int N, class Entries>
 __global__ void __launch_bounds__(SMALL_NT) k_hpsi_small(const typename V2s<T>::t* __restrict__ psi,
                                                          typename V2s<T>::t* __restrict__ hpsi,
                                                          const T* __restrict__ kin, const T* __restrict__ vr,
@@ -586,10 +594,9 @@ __global__ void __launch_bounds__(SMALL_NT) k_hpsi_small(const typename V2s<T>::
                                                          const typename V2s<T>::t* __restrict__ DBH, T inv_n,
                                                          const double* __restrict__ coef,
                                                          const typename V2s<T>::t* __restrict__ X, int nkv,
-                                                         const int* __restrict__ band_k,
-                                                         const int* __restrict__ skip) {
+                                                         const int* __restrict__ skip, const Entries entries) {
   hpsi_small_body<T, N>((int)blockIdx.x, (int)gridDim.x, psi, hpsi, kin, vr, g2fft, npw, nbk, nch, B, DBH, inv_n,
-                        coef, X, nkv, band_k, skip);
+                        coef, X, nkv, skip, entries);
 }
 
 template <typename T, int N>
@@ -627,7 +634,7 @@ __global__ void __launch_bounds__(SMALL_NT) k_hpsi_multi(PassSmallMulti m, int n
   if ((int)blockIdx.x >= q.nbands) return;  // uniform
   hpsi_small_body<T, N>((int)blockIdx.x, q.nbands, (const V2*)q.in, (V2*)q.out, (const T*)q.kin, (const T*)q.vr,
                         q.g2fft, npw, nbk, nch, (const V2*)q.B, (const V2*)q.DBH, inv_n, nullptr, nullptr, q.nkv,
-                        nullptr, q.skip);
+                        q.skip, NoBatch{});
 }
 
 // Band density on small cubic grids: workgroup g takes bands [g·gsize, (g+1)·gsize), runs the
@@ -776,10 +783,10 @@ bool small_len(int n) {
   }
 }
 
-template <typename T>
+template <typename T, class Entries>
 void launch_small_t(Context& c, int nbands, int nbk, const void* psi, void* hpsi, const void* kin, int nch,
-                    const void* B, const void* DBH, const double* coef, const void* X, int nkv, const int* band_k,
-                    const int* skip) {
+                    const void* B, const void* DBH, const double* coef, const void* X, int nkv, const int* skip,
+                    const Entries& entries) {
   using V2 = typename V2s<T>::t;
   const int n = c.dims[0];
   const size_t sh = small_lds_bytes<T>(n, nch);
@@ -789,10 +796,10 @@ void launch_small_t(Context& c, int nbands, int nbk, const void* psi, void* hpsi
   switch (n) {
 #define PWK_CASE(L)                                                                                            \
   case L:                                                                                                      \
-    ensure_lds_limit((const void*)k_hpsi_small<T, L>, sh);                                                    \
-    k_hpsi_small<T, L><<<(unsigned)nbands, SMALL_NT, sh, c.stream>>>(                                          \
+    ensure_lds_limit((const void*)k_hpsi_small<T, L, Entries>, sh);                                           \
+    k_hpsi_small<T, L, Entries><<<(unsigned)nbands, SMALL_NT, sh, c.stream>>>(                                          \
         (const V2*)psi, (V2*)hpsi, (const T*)kin, vr, c.g2fft.as<int>(), c.npw, nbk, nch, (const V2*)B,        \
-        (const V2*)DBH, inv_n, coef, (const V2*)X, nkv, band_k, skip);                                         \
+        (const V2*)DBH, inv_n, coef, (const V2*)X, nkv, skip, entries);                                        \
     break;
     PWK_SMALL_SIZES(PWK_CASE)
 #undef PWK_CASE
@@ -1017,7 +1024,7 @@ void launch_lanczos_small(Context& c, int nke, int nkv, int steps, const double*
 
 void launch_hpsi_small(Context& c, int nbands, int nbk, const void* psi, void* hpsi, int precision, const void* kin,
                        int nch, const void* B, const void* DBH, const double* coef, const void* X, int nkv,
-                       const int* band_k, const int* skip) {
+                       const int* skip) {
   c.check_basis();
   PWK_REQUIRE(c.have_v, PWK_E_STATE, "V_eff not set (pwk_set_veff)");
   PWK_REQUIRE(nbands > 0 && nbk > 0 && nbands % nbk == 0, PWK_E_INVALID, "band counts must be positive");
@@ -1026,11 +1033,21 @@ void launch_hpsi_small(Context& c, int nbands, int nbk, const void* psi, void* h
     const size_t slots = ((size_t)(nbands / nbk) + nkv - 1) / nkv;
     PWK_REQUIRE(c.vrn64.bytes >= slots * c.N * sizeof(double), PWK_E_STATE, "V_eff slots not set");
   }
-  PWK_REQUIRE(!band_k || (!coef && nkv == 0), PWK_E_INVALID, "a band table excludes filter coefficients");
   if (precision == PWK_FP64)
-    launch_small_t<double>(c, nbands, nbk, psi, hpsi, kin, nch, B, DBH, coef, X, nkv, band_k, skip);
+    launch_small_t<double>(c, nbands, nbk, psi, hpsi, kin, nch, B, DBH, coef, X, nkv, skip, NoBatch{});
   else
-    launch_small_t<float>(c, nbands, nbk, psi, hpsi, kin, nch, B, DBH, coef, X, nkv, band_k, skip);
+    launch_small_t<float>(c, nbands, nbk, psi, hpsi, kin, nch, B, DBH, coef, X, nkv, skip, NoBatch{});
+}
+
+void launch_hpsi_small_batch(Context& c, const BatchSmall& entries, const void* psi, void* hpsi, int precision, int nch) {
+  c.check_basis();
+  PWK_REQUIRE(c.have_v, PWK_E_STATE, "V_eff not set (pwk_set_veff)");
+  PWK_REQUIRE(hpsi_small_supported(c, precision, nch), PWK_E_UNSUPPORTED, "grid too large for the fused kernel");
+  const int nbands = entries.end[entries.n - 1];
+  if (precision == PWK_FP64)
+    launch_small_t<double>(c, nbands, 1, psi, hpsi, nullptr, nch, nullptr, nullptr, nullptr, nullptr, 0, nullptr, entries);
+  else
+    launch_small_t<float>(c, nbands, 1, psi, hpsi, nullptr, nch, nullptr, nullptr, nullptr, nullptr, 0, nullptr, entries);
 }
 
 }  // namespace pwk

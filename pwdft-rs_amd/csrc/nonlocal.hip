@@ -279,7 +279,6 @@ void build_nonlocal_batch(Context& c, int ik0, int nkb, const double* kvecs, con
       }
   }
   int nch = (int)ch_atom.size();
-  c.pack_valid = false;
   for (int i = 0; i < nkb; ++i) c.k(ik0 + i).nch = nch;
   if (nch == 0) return;
   hipStream_t st = c.stream;

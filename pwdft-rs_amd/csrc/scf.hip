@@ -1518,7 +1518,6 @@ void Solve::setup() {
   for (int k = 0; k < nk; ++k) wk[(size_t)k] = kpts[(size_t)k].weight;
   c.kd.clear();
   c.kd.resize((size_t)nk);
-  c.pack_valid = false;
 
   // radial tables → V_loc(G), ρ_core(r), start density
   RadialArgs ra{};
@@ -2815,7 +2814,7 @@ void Solve::pass_dev(int fp) {
                            f64 ? Ball64.p : Ball32.p, f64 ? DBHall64.p : DBHall32.p, coef.as<double>(), degree, nkv,
                            flag);
   launch_hpsi_small(c, nke * nbs, nbs, Y64.p, HY64.p, PWK_FP64, kin_all64.p, nch_all, Ball64.p, DBHall64.p, nullptr,
-                    nullptr, nkv, nullptr, flag);
+                    nullptr, nkv, flag);
   launch_rr_small(c, npw, nbs, nb, nke, Y64.p, HY64.p, Vc(), lam_dev.as<double>(), lam_dev.as<double>() + nkm, 1e-14,
                   flag);
   gate_dev(true);

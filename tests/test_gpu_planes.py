@@ -95,13 +95,13 @@ def test_hpsi_planes(gpu, dims, m, prec, tol):
         gpu.set_fused_hpsi(True)
 
 
-@pytest.mark.parametrize("dims,m", [((25, 25, 25), 6), ((27, 27, 27), 9), ((27, 25, 32), 6)])
+@pytest.mark.parametrize("dims,m", [((25, 25, 25), 6), ((27, 27, 27), 9), ((27, 25, 32), 6), ((15, 15, 15), 3)])
 @pytest.mark.parametrize("prec,tol", [("fp64", 1e-13), ("fp32", 6e-6), ("split_bf16", 2e-5)])
 @pytest.mark.parametrize("channels,counts", [((7, 7, 7), (3, 1, 18)), ((80, 80), (33, 161)), ((5, 0, 5), (2, 2, 2)),
                                              ((3, 3, 6, 6, 6), (2, 1, 2, 3, 1)), ((4,) * 66, (1, 2) * 33)])
 def test_hpsi_batch_sticks(gpu, dims, m, prec, tol, channels, counts):
-    # k × band batches off the small grids: one launch per pass and grouped projector products when the
-    # entries share a channel count (64 of them at most), entry by entry otherwise. Tolerance relative to the largest |Hψ|:
+    # k × band batches: one launch per pass and grouped projector products (one fused launch on the small grid)
+    # for up to 64 consecutive entries with one channel count. Tolerance relative to the largest |Hψ|:
     # the transforms as above plus sums over npw (projection) and nch terms, √npw ≈ 60 roundings
     # (FP32 3.6e-6, split-bf16 2^-16 per product: 1.5e-5)
     miller, idx = setup(gpu, dims, m)
@@ -141,13 +141,13 @@ def test_hpsi_batch_sticks(gpu, dims, m, prec, tol, channels, counts):
 OTHERS = [([2, 0], [5, 3]), ([1], [12]), ([0, 1, 2], [4, 5, 3]), ([1, 1, 0, 2, 0], [1, 2, 3, 1, 9])]
 
 
-@pytest.mark.parametrize("dims", [(25, 25, 25), (27, 25, 32)])
-def test_hpsi_batch_sticks_captured(gpu, dims):
+@pytest.mark.parametrize("dims", [(25, 25, 25), (27, 25, 32), (15, 15, 15), (20, 20, 20)])
+def test_hpsi_batch_captured(gpu, dims):
     # replays of a captured batch equal the same batch run directly, whatever other batches (of either
-    # precision) run between them
+    # precision) run between them: on the stick path and on the fused small grids
     import torch
 
-    miller, _ = setup(gpu, dims, 6)
+    miller, _ = setup(gpu, dims, 6 if dims[0] > 20 else 3)
     npw, nch = len(miller), 7
     rng = np.random.default_rng(34)
     gpu.set_veff((np.fft.fftn(rng.uniform(-13.6, 13.6, dims)) / np.prod(dims)).reshape(-1))
