@@ -497,8 +497,11 @@ void sphere_rows_inverse(Context& c, int nb, void* buf, void* rows);
 template <typename T>
 void sphere_plane(Context& c, int nb, void* buf, const T* vr, void* rows);
 template <typename T, class Entries>
-void sphere_zfwd(Context& c, int nb, const void* buf, const T* kin, int nbk, const Entries& entries,
+void sphere_zfwd(Context& c, int nb, const void* buf, const T* kin, int nbk, int b0, const Entries& entries,
                  const void* psi, void* hpsi);
+// bands per launch sequence on the stick path: all of them where nx = ny, else at most 256 MiB of sticks and
+// held rows (es bytes each), the amount that the whole-grid path takes, and no more than one grid holds
+int stick_chunk(const Context& c, int nb, size_t es);
 // density.hip: the band density on square grids of register-length lines and on any with c.quarter (fw on
 // the host)
 void launch_density_sticks(Context& c, int nb, const void* psi, const double* fw_host, void* rho, int precision,

@@ -250,43 +250,50 @@ void density_sticks_t(Context& c, int nb, const void* psi, const double* fw_host
   const long wgs = square ? nz : (ny * nz + 63) / 64;  // workgroups per group
   // The workspaces are sized for all nb bands, whatever their weights: a captured call transforms every band
   // and cannot allocate, and its first run outside the graph may have had bands without weight. One z-inverse
-  // buffer, then the groups' partial sums, of which any number of live bands makes at most max_groups.
-  const size_t ns = (size_t)nb * nz * c.nsticks, held = square ? 0 : sphere_rows_elems(c, nb);
+  // buffer (of a chunk), then the groups' partial sums, of which any number of live bands makes at most
+  // max_groups.
+  const int chunk = stick_chunk(c, nb, sizeof(V2));
+  const size_t ns = (size_t)chunk * nz * c.nsticks, held = square ? 0 : sphere_rows_elems(c, chunk);
   const size_t tb = ((ns + held) * sizeof(V2) + 255) & ~(size_t)255;
-  const long max_groups = std::min<long>((nb + slots - 1) / slots, (1024 + wgs - 1) / wgs);
+  const long max_groups = std::min<long>((chunk + slots - 1) / slots, (1024 + wgs - 1) / wgs);
   c.workspace(c.work_a, tb + (size_t)max_groups * c.N * sizeof(double));
   c.workspace(c.work_b, ((size_t)nb + (size_t)(nb + 1) / 2) * sizeof(double));
   if (live > 0) {
     const size_t wbytes = (captured ? (size_t)nb : h.size()) * sizeof(double);
     PWK_HIP(hipMemcpyAsync(c.work_b.p, captured ? fw_host : h.data(), wbytes, hipMemcpyHostToDevice, c.stream));
-    const double* fw = c.work_b.as<double>();
-    const int batches = (live + slots - 1) / slots;
-    const int per = std::max(1, (int)((batches * wgs + 1023) / 1024));
-    const int groups = (batches + per - 1) / per;
+    const double* weights = c.work_b.as<double>();
     double* part = reinterpret_cast<double*>(c.work_a.as<unsigned char>() + tb);
-    launch_zinv(c, live, psi, c.work_a.p, std::is_same<T, double>::value ? PWK_FP64 : PWK_FP32,
-                captured ? nullptr : reinterpret_cast<const int*>(fw + live));
     V2* rows = c.work_a.as<V2>() + ns;
-    if (!square) sphere_rows_inverse<T>(c, live, c.work_a.p, rows);
-    switch (nx) {
-#define PWK_CASE(L)                                                             \
-  case L:                                                                       \
-    if (!square)                                                                \
-      k_cols_density<T, L><<<dim3((unsigned)wgs, (unsigned)groups), 64, 0, c.stream>>>(rows, live, per, fw, part, ny, nz); \
-    else if (c.quarter)                                                              \
-      plane_density<T, L, true>(c, c.work_a.p, live, per, groups, fw, part);    \
-    else                                                                        \
-      plane_density<T, L, false>(c, c.work_a.p, live, per, groups, fw, part);   \
+    for (int b0 = 0; b0 < live; b0 += chunk) {
+      const int n = std::min(chunk, live - b0);
+      const double* fw = weights + b0;
+      const int batches = (n + slots - 1) / slots;
+      const int per = std::max(1, (int)((batches * wgs + 1023) / 1024));
+      const int groups = (batches + per - 1) / per;
+      launch_zinv(c, n, captured ? (const V2*)psi + (size_t)b0 * c.npw : psi, c.work_a.p,
+                  std::is_same<T, double>::value ? PWK_FP64 : PWK_FP32,
+                  captured ? nullptr : reinterpret_cast<const int*>(weights + live) + b0);
+      if (!square) sphere_rows_inverse<T>(c, n, c.work_a.p, rows);
+      switch (nx) {
+#define PWK_CASE(L)                                                                                                   \
+  case L:                                                                                                             \
+    if (!square)                                                                                                      \
+      k_cols_density<T, L><<<dim3((unsigned)wgs, (unsigned)groups), 64, 0, c.stream>>>(rows, n, per, fw, part, ny, nz); \
+    else if (c.quarter)                                                                                               \
+      plane_density<T, L, true>(c, c.work_a.p, n, per, groups, fw, part);                                             \
+    else                                                                                                              \
+      plane_density<T, L, false>(c, c.work_a.p, n, per, groups, fw, part);                                            \
     break;
-      PWK_FOR_EACH_FFT_SIZE(PWK_CASE)
+        PWK_FOR_EACH_FFT_SIZE(PWK_CASE)
 #undef PWK_CASE
-      default:
-        throw Error(PWK_E_UNSUPPORTED, "nx has no compiled kernel");
+        default:
+          throw Error(PWK_E_UNSUPPORTED, "nx has no compiled kernel");
+      }
+      PWK_HIP(hipGetLastError());
+      const dim3 gs(blocks_for((size_t)ny, 32), blocks_for((size_t)nz, 32), (unsigned)nx);
+      k_density_sum<<<gs, 256, 0, c.stream>>>(groups, nx, ny, nz, part, rho, overwrite && b0 == 0 ? 1 : 0);
+      PWK_HIP(hipGetLastError());
     }
-    PWK_HIP(hipGetLastError());
-    const dim3 gs(blocks_for((size_t)ny, 32), blocks_for((size_t)nz, 32), (unsigned)nx);
-    k_density_sum<<<gs, 256, 0, c.stream>>>(groups, nx, ny, nz, part, rho, overwrite ? 1 : 0);
-    PWK_HIP(hipGetLastError());
   } else if (overwrite) {
     const dim3 gs(blocks_for((size_t)ny, 32), blocks_for((size_t)nz, 32), (unsigned)nx);
     k_density_sum<<<gs, 256, 0, c.stream>>>(0, nx, ny, nz, nullptr, rho, 1);

@@ -374,53 +374,59 @@ void hpsi_local(Context& c, const T* kin, int nb, int nbk, const void* psi, void
     hpsi_fullgrid<T>(c, kin, nb, nbk, psi, hpsi);
     return;
   }
-  PWK_REQUIRE(nb <= 65535, PWK_E_UNSUPPORTED, "too many bands in one H·psi launch");
-  const size_t ns = (size_t)nb * nz * c.nsticks, rows = nx == c.dims[1] ? 0 : sphere_rows_elems(c, nb);
+  const int chunk = stick_chunk(c, nb, sizeof(V2));
+  PWK_REQUIRE(chunk <= 65535, PWK_E_UNSUPPORTED, "too many bands in one H·psi launch");
+  const size_t ns = (size_t)chunk * nz * c.nsticks, rows = nx == c.dims[1] ? 0 : sphere_rows_elems(c, chunk);
   c.workspace(c.work_a, (ns + rows) * sizeof(V2));
   V2* T_ = c.work_a.as<V2>();
   const T* vr = std::is_same<T, double>::value ? (const T*)c.vr64.p : (const T*)c.vr32.p;
-  dim3 gz(blocks_for((size_t)c.nsticks, 64), (unsigned)nb);
-  {
-    TimedScope ts(c, "hpsi_zinv");
-    zinv_t<T>(c, nb, psi, T_, nullptr);
-  }
-  {
-    TimedScope ts(c, "hpsi_plane");
-    // (the pruned FP64 plane pass of 81 points does not fit the registers)
-    if (c.quarter && !(std::is_same<T, double>::value && nx > 80 && nx == c.dims[1])) {
-      sphere_plane<T>(c, nb, T_, vr, T_ + ns);
-    } else {
-      switch (nx) {
+  for (int b0 = 0; b0 < nb; b0 += chunk) {
+    const int nbc = std::min(chunk, nb - b0);
+    const V2* in = (const V2*)psi + (size_t)b0 * c.npw;
+    V2* out = (V2*)hpsi + (size_t)b0 * c.npw;
+    {
+      TimedScope ts(c, "hpsi_zinv");
+      zinv_t<T>(c, nbc, in, T_, nullptr);
+    }
+    {
+      TimedScope ts(c, "hpsi_plane");
+      // (the pruned FP64 plane pass of 81 points does not fit the registers)
+      if (c.quarter && !(std::is_same<T, double>::value && nx > 80 && nx == c.dims[1])) {
+        sphere_plane<T>(c, nbc, T_, vr, T_ + ns);
+      } else {
+        switch (nx) {
 #define PWK_CASE(L)                    \
   case L:                              \
-    plane_hpsi<T, L>(c, T_, nb, vr);   \
+    plane_hpsi<T, L>(c, T_, nbc, vr);  \
     break;
-        PWK_FOR_EACH_FFT_SIZE(PWK_CASE)
+          PWK_FOR_EACH_FFT_SIZE(PWK_CASE)
 #undef PWK_CASE
-        default:
-          throw Error(PWK_E_UNSUPPORTED, "nx has no compiled kernel");
+          default:
+            throw Error(PWK_E_UNSUPPORTED, "nx has no compiled kernel");
+        }
       }
     }
-  }
-  T inv_n = (T)(1.0 / (double)c.N);
-  TimedScope ts_zfwd(c, "hpsi_zfwd");
-  if (c.quarter) {
-    sphere_zfwd<T>(c, nb, T_, kin, nbk, entries, psi, hpsi);
-    return;
-  }
-  switch (nz) {
+    TimedScope ts(c, "hpsi_zfwd");
+    if (c.quarter) {
+      sphere_zfwd<T>(c, nbc, T_, kin, nbk, b0, entries, in, out);
+      continue;
+    }
+    const T inv_n = (T)(1.0 / (double)c.N);
+    const dim3 gz(blocks_for((size_t)c.nsticks, 64), (unsigned)nbc);  // (nx = ny: one chunk)
+    switch (nz) {
 #define PWK_CASE(L)                                                                                     \
   case L:                                                                                               \
-    k_zfwd<T, L, Entries><<<gz, 64, 0, c.stream>>>(T_, (const V2*)psi, (V2*)hpsi, kin, c.npw, c.nsticks,         \
+    k_zfwd<T, L, Entries><<<gz, 64, 0, c.stream>>>(T_, in, out, kin, c.npw, c.nsticks,                  \
                                           c.st_pw0.as<int>(), c.st_cnt.as<int>(), c.st_n3lo.as<int>(),  \
                                           inv_n, nbk, entries);                                         \
     break;
-    PWK_FOR_EACH_FFT_SIZE(PWK_CASE)
+      PWK_FOR_EACH_FFT_SIZE(PWK_CASE)
 #undef PWK_CASE
-    default:
-      throw Error(PWK_E_UNSUPPORTED, "nz has no compiled kernel");
+      default:
+        throw Error(PWK_E_UNSUPPORTED, "nz has no compiled kernel");
+    }
+    PWK_HIP(hipGetLastError());
   }
-  PWK_HIP(hipGetLastError());
 }
 
 inline int wrap(int n, int d) { return ((n % d) + d) % d; }

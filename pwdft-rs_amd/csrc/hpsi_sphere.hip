@@ -89,7 +89,7 @@ __global__ void __launch_bounds__(ZS) k_zfwd_q(const typename V2t<T>::t* __restr
                                                const typename V2t<T>::t* __restrict__ psi,
                                                typename V2t<T>::t* __restrict__ hpsi, const T* __restrict__ kin, int npw,
                                                int S, const int* __restrict__ st_pw0, const int* __restrict__ st_cnt,
-                                               const int* __restrict__ st_lo, T inv_n, int nbk,
+                                               const int* __restrict__ st_lo, T inv_n, int nbk, int b0,
                                                const Entries entries) {
   using V2 = typename V2t<T>::t;
   using Q = Quarter<NZ>;
@@ -109,7 +109,7 @@ __global__ void __launch_bounds__(ZS) k_zfwd_q(const typename V2t<T>::t* __restr
     im[i3] = v.y;
   }
   range_to_lds<V2, 8>(L, psi + (size_t)b * npw + rg.w0, rg.n);
-  range_to_lds<T, 8>(K, band_kin(entries, kin, npw, nbk, b) + rg.w0, rg.n);
+  range_to_lds<T, 8>(K, band_kin(entries, kin, npw, nbk, b0 + b) + rg.w0, rg.n);
   __syncthreads();
   fft_line<T, NZ, -1>(re, im);
   // a slot of the line that the stick does not reach goes to a discard element of the lane's own: without
@@ -337,14 +337,14 @@ void plane_q(Context& c, typename V2t<T>::t* tbuf, int nb, const T* vr) {
 }
 
 template <typename T, int N, class Entries>
-void zfwd_q(Context& c, const typename V2t<T>::t* tbuf, int nb, const T* kin, int nbk, const Entries& entries,
+void zfwd_q(Context& c, const typename V2t<T>::t* tbuf, int nb, const T* kin, int nbk, int b0, const Entries& entries,
             const void* psi, void* hpsi) {
   using V2 = typename V2t<T>::t;
   const size_t sh = (size_t)ZS * (Quarter<N>::R + 1) * (sizeof(V2) + sizeof(T));
   ensure_lds_limit((const void*)k_zfwd_q<T, N, Entries>, sh);
   k_zfwd_q<T, N, Entries><<<dim3(blocks_for((size_t)c.nsticks, ZS), (unsigned)nb), ZS, sh, c.stream>>>(
       tbuf, (const V2*)psi, (V2*)hpsi, kin, c.npw, c.nsticks, c.st_pw0.as<int>(), c.st_cnt.as<int>(),
-      c.st_n3lo.as<int>(), (T)(1.0 / (double)c.N), nbk, entries);
+      c.st_n3lo.as<int>(), (T)(1.0 / (double)c.N), nbk, b0, entries);
 }
 
 template <typename T, int N>
@@ -376,6 +376,12 @@ void sphere_zinv(Context& c, int nb, const void* psi, void* out, const int* list
 
 size_t sphere_rows_elems(const Context& c, int nb) {
   return (size_t)nb * c.dims[2] * (2 * ((c.dims[0] - 1) / 4) + 1) * c.dims[1];
+}
+
+int stick_chunk(const Context& c, int nb, size_t es) {
+  if (c.dims[0] == c.dims[1]) return nb;
+  const size_t per = ((size_t)c.dims[2] * c.nsticks + sphere_rows_elems(c, 1)) * es;
+  return (int)std::max<size_t>(1, std::min<size_t>(std::min<size_t>((size_t)nb, 32768), ((size_t)256 << 20) / per));
 }
 
 template <typename T>
@@ -419,13 +425,13 @@ void sphere_plane(Context& c, int nb, void* buf, const T* vr, void* rows) {
 }
 
 template <typename T, class Entries>
-void sphere_zfwd(Context& c, int nb, const void* buf, const T* kin, int nbk, const Entries& entries,
+void sphere_zfwd(Context& c, int nb, const void* buf, const T* kin, int nbk, int b0, const Entries& entries,
                  const void* psi, void* hpsi) {
   auto* tbuf = (const typename V2t<T>::t*)buf;
   switch (c.dims[2]) {
 #define PWK_CASE(L) \
   case L:           \
-    zfwd_q<T, L>(c, tbuf, nb, kin, nbk, entries, psi, hpsi); \
+    zfwd_q<T, L>(c, tbuf, nb, kin, nbk, b0, entries, psi, hpsi); \
     break;
     PWK_FOR_EACH_FFT_SIZE(PWK_CASE)
 #undef PWK_CASE
@@ -441,9 +447,9 @@ template void sphere_rows_inverse<float>(Context&, int, void*, void*);
 template void sphere_rows_inverse<double>(Context&, int, void*, void*);
 template void sphere_plane<float>(Context&, int, void*, const float*, void*);
 template void sphere_plane<double>(Context&, int, void*, const double*, void*);
-template void sphere_zfwd(Context&, int, const void*, const float*, int, const NoBatch&, const void*, void*);
-template void sphere_zfwd(Context&, int, const void*, const float*, int, const BatchKin&, const void*, void*);
-template void sphere_zfwd(Context&, int, const void*, const double*, int, const NoBatch&, const void*, void*);
-template void sphere_zfwd(Context&, int, const void*, const double*, int, const BatchKin&, const void*, void*);
+template void sphere_zfwd(Context&, int, const void*, const float*, int, int, const NoBatch&, const void*, void*);
+template void sphere_zfwd(Context&, int, const void*, const float*, int, int, const BatchKin&, const void*, void*);
+template void sphere_zfwd(Context&, int, const void*, const double*, int, int, const NoBatch&, const void*, void*);
+template void sphere_zfwd(Context&, int, const void*, const double*, int, int, const BatchKin&, const void*, void*);
 
 }  // namespace pwk

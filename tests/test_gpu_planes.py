@@ -199,6 +199,34 @@ def test_hpsi_batch_captured(gpu, dims):
         assert torch.equal(out.cpu(), want)
 
 
+# more bands than the sticks and held rows of one launch sequence take (256 MiB), and than a launch has rows
+@pytest.mark.parametrize("dims,m,nb", [((27, 25, 32), 6, 2500), ((9, 8, 8), 1, 66000)])
+@pytest.mark.parametrize("prec,tol", [("fp64", 1e-13), ("fp32", 4e-6)])
+def test_unequal_axes_many_bands(gpu, dims, m, nb, prec, tol):
+    # tolerances as for the same passes above (FP64: plus nb·eps / 10 of the sums over the bands)
+    miller, idx = setup(gpu, dims, m)
+    npw, n = len(miller), int(np.prod(dims))
+    rng = np.random.default_rng(38)
+    v = rng.uniform(-13.6, 13.6, dims)
+    gpu.set_veff((np.fft.fftn(v) / n).reshape(-1))
+    psi = bands(rng, nb, npw)
+    fw = rng.uniform(0.1, 2.0, nb)
+    fw[::7] = 0.0
+    rho0 = rng.uniform(0.0, 1e-3, n)
+    print("many bands", dims, nb, prec, flush=True)
+    got = gpu.hpsi(0, psi, prec)
+    rho = gpu.density(psi, fw, rho0, prec)
+    ref, diff, top = rho0.copy(), 0.0, 0.0
+    for b in range(0, nb, 500):
+        g = to_grid(psi[b:b + 500], idx, dims)
+        w = np.fft.fftn(g * v, axes=(1, 2, 3)).reshape(len(g), -1)[:, idx] / n
+        w += (miller.astype(float) ** 2).sum(1) * psi[b:b + 500]
+        diff, top = max(diff, np.abs(got[b:b + 500] - w).max()), max(top, np.abs(w).max())
+        ref += (fw[b:b + 500, None] * np.abs(g.reshape(len(g), -1)) ** 2).sum(0)
+    assert diff < tol * top
+    assert np.abs(rho - ref).max() < (tol + nb * 2.3e-17) * np.abs(ref).max()
+
+
 @pytest.mark.parametrize("dims,m", [((25, 25, 25), 6), ((27, 25, 32), 6), ((27, 27, 27), 13)])
 def test_density_captured(gpu, dims, m):
     # a captured density reads the caller's weights at each replay, also where a band gains or loses its weight
