@@ -127,7 +127,8 @@ __device__ __forceinline__ void tri_pairs(int n, int nb, double* d, double* e, d
     unit[k] = u;
   }
   __syncthreads();
-  double lo = 1e308, hi = -1e308;
+  // (fmin and fmax leave NaNs out: the bounds are NaN, and with them every eigenvalue, if all entries are)
+  double lo = __builtin_nan(""), hi = lo;
   for (int k = t; k < n; k += EIG_NT) {
     const double r = e[k] + (k > 0 ? e[k - 1] : 0.0);
     lo = fmin(lo, d[k] - r);
@@ -469,7 +470,7 @@ __global__ void __launch_bounds__(NT) k_heev(int n, int nb, int a_in_lds, int lu
   if (t == 0 && status) status[b] = 0;
 }
 
-// ---- matrices of 65 to 256 rows that do not fit the LDS ---------------------------------------
+// ---- matrices of 65 to 256 rows ------------------------------------------------------------------
 // The same steps with the Householder reduction arranged around one pass over the matrix per reflector:
 //  - wave w owns the columns j ≡ w mod 8 and a lane the rows lane + 64r of them for the whole reduction, so
 //    the matrix (in L2) is read and written by the threads that own it and needs no barrier;
@@ -483,7 +484,10 @@ __global__ void __launch_bounds__(NT) k_heev(int n, int nb, int a_in_lds, int lu
 // Bound: the chain of reflectors, each with a pass of about 13k cycles of issue by two waves per SIMD (the
 // loads and stores hide behind it). 8 matrices of 169 rows, 8 pairs: 5.0 ms in the form above (15 barriers and
 // an integer division per entry and reflector), 2.5 with the column factors read from LDS per column, 1.9 by
-// lane moves; 4 or 16 waves per matrix, or more columns in flight, took longer.
+// lane moves; 4 or 16 waves per matrix, or more columns in flight, took longer. The form above is slower over
+// the whole range, also where the matrix fits the LDS (up to 90 rows): 65 rows 0.78 -> 0.45 ms, 90 rows 1.58 ->
+// 0.65, 128 rows 2.56 -> 1.00, 256 rows 14.8 -> 3.8 (8 pairs, 1 to 64 matrices), 300 matrices of 65 rows
+// 1.56 -> 0.65, of 144 rows 6.9 -> 3.2.
 constexpr int ROW_NT = 512, ROW_WAVES = 8, ROW_GROUPS = 2;
 
 template <int CTRL>
@@ -646,12 +650,15 @@ __global__ void __launch_bounds__(ROW_NT) k_heev_rows(int n, int nb, int lu_in_l
       const double2 alpha = make_double2(-ph.x * xn, -ph.y * xn);
       // v = (x - alpha e1) / |x - alpha e1|;  |x - alpha e1|² = 2(|x|² + |x||x0|)
       const double vn = sqrt(2.0 * (xn * xn + xn * ax0));
-      const double rv = !last && xn > 0.0 ? 1.0 / vn : 0.0;
+      // a column without weight takes no reflector; one with a NaN or an infinity does, and spreads it over
+      // the matrix as the general form does
+      const bool reflect = !last && xn != 0.0;
+      const double rv = reflect ? 1.0 / vn : 0.0;
 #pragma unroll
       for (int r = 0; r < R; ++r) {
         const int i = lane + 64 * r;
         double2 y = make_double2(0.0, 0.0);
-        if (i > k && i < n && rv > 0.0) {
+        if (i > k && i < n && reflect) {
           y = x[r];
           if (i == k + 1) {
             y.x -= alpha.x;

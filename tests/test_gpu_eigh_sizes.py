@@ -27,3 +27,16 @@ def test_dense_eigh_kernel_sizes(gpu, n):
             assert np.abs(w[i] - np.linalg.eigvalsh(h)[:nb]).max() < 2e-13 * norm
             assert np.linalg.norm(h @ v[i] - v[i] * w[i], axis=0).max() < 1e-11 * norm
             assert np.abs(v[i].conj().T @ v[i] - np.eye(nb)).max() < 1e-10
+
+
+@pytest.mark.parametrize("n", [40, 64, 65, 100, 169, 240, 257])
+@pytest.mark.parametrize("bad", [np.nan, np.inf])
+def test_dense_eigh_passes_nan_on(gpu, n, bad):
+    # a NaN or an infinity in the first column reaches every eigenvalue and vector, whichever kernel runs
+    rng = np.random.default_rng(n)
+    a = rng.standard_normal((n, n)) + 1j * rng.standard_normal((n, n))
+    h = (a + a.conj().T) / 2
+    h[5, 0] = h[0, 5] = bad
+    print("eigh", n, bad, flush=True)
+    w, v = gpu.dense_eigh(h[None], 6)
+    assert np.isnan(w).all() and np.isnan(v).all()
