@@ -1826,8 +1826,12 @@ void Solve::setup() {
     rr_pinned = pin_rr.as<double>();
     // Rayleigh-Ritz over the whole chip off the fused small grids (whose passes run batched across requests,
     // or captured, with the one-workgroup form) from 512 plane waves: 1189 × 32 vectors, 4 k-points 633 us
-    // in one workgroup per k-point
-    if (rr_small_supported(nbs) && npw >= 512 && !hpsi_small_supported(c, PWK_FP64, nch_all))
+    // in one workgroup per k-point, 265 us spread; 537 × 12, 1 k-point 127 and 74 us. Up to 24 vectors only below
+    // two k-points per CU: with more of them the one-workgroup form fills the chip by itself (537 × 16: 216
+    // k-points 166 and 130 us, 512 203 and 202, 729 251 and 275, 1728 563 and 651; 537 × 24, 1728 k-points
+    // 2401 and 2475; 537 × 28, 1728 k-points 3207 and 2930).
+    if (rr_small_supported(nbs) && npw >= 512 && (nke < 2 * c.cu_count || nbs > 24) &&
+        !hpsi_small_supported(c, PWK_FP64, nch_all))
       rr_ws.ensure(rr_split_bytes(npw, nbs, nke));
     s_work.ensure(heev_work_doubles(nbs, nbs, nke) * 8);
     projall.ensure((size_t)nk * std::max(1, nch_all) * nbs * 16);
