@@ -75,7 +75,8 @@ __global__ void __launch_bounds__(64) k_zfwd(const typename V2t<T>::t* __restric
                                              T inv_n, int nbk, const Entries entries) {
   int s = blockIdx.x * 64 + threadIdx.x;
   int b = blockIdx.y;
-  const T* tb = band_kin(entries, kin, npw, nbk, b);
+  int ent = 0;  // the band's entry, by all lanes before any leaves
+  if constexpr (Entries::batch) ent = batch_entry(entries, b);
   if (s >= S) return;
   int pw0 = st_pw0[s], cnt = st_cnt[s], lo = st_lo[s];
   const typename V2t<T>::t* src = tbuf + (size_t)b * NZ * S + s;
@@ -87,9 +88,16 @@ __global__ void __launch_bounds__(64) k_zfwd(const typename V2t<T>::t* __restric
     im[i3] = v.y;
   }
   fft_dif<T, NZ, -1>(re, im);
+  if constexpr (sizeof(T) == 8 && NZ > 50) {
+    // lines that fill the registers are complete here: drawn into the branches below, their last stages keep
+    // twice the registers and spill (60 points 748 bytes a lane; shorter lines gain by the earlier loads)
+#pragma unroll
+    for (int f = 0; f < NZ; ++f) asm volatile("" : "+v"(re[f]), "+v"(im[f]));
+  }
   const typename V2t<T>::t* p = psi + (size_t)b * npw + pw0;
   typename V2t<T>::t* h = hpsi + (size_t)b * npw + pw0;
-  const T* t = tb + pw0;
+  const T* t = kin + (size_t)(b / nbk) * npw + pw0;
+  if constexpr (Entries::batch) t = (const T*)entries.kin[ent] + pw0;
 #pragma unroll
   for (int i3 = 0; i3 < NZ; ++i3) {
     int j = stick_slot(i3, lo, NZ);
