@@ -3,7 +3,7 @@
 //
 // Three launches: the z-inverse of the bands that carry weight (launch_zinv), the plane pass
 // k_plane_density on (z-plane, band group), and k_density_sum, which adds the groups' FP64 partial
-// sums in group order, so the result does not depend on scheduling.
+// sums in group order, so the result does not depend on scheduling; two where a small grid has one group.
 #include <algorithm>
 #include <vector>
 
@@ -37,12 +37,12 @@ using DensityShape = PlaneShape<T, N, !acc_in_regs<T, N>()>;
 // one wave each: 144 FP32 bands on 60³ 1741 us -> 72 us;
 // 540 FP64 bands on 25³, the whole density beside other work, 901 us -> 31 us.
 // QUARTER: a sphere within a quarter of the axes (planes.hpp); otherwise the held rows come from the
-// basis' tables.
-template <typename T, int N, bool QUARTER>
+// basis' tables. DIRECT: the one group adds its sums to ρ itself.
+template <typename T, int N, bool QUARTER, bool DIRECT>
 __global__ void __launch_bounds__((DensityShape<T, N>::NT))
     k_plane_density(const typename V2t<T>::t* __restrict__ tbuf, int nb, int per, const double* __restrict__ fw,
                     double* __restrict__ part, int S, int nz, const int* __restrict__ src, int image,
-                    PlaneRows pr, int nx1, const int* __restrict__ x1list) {
+                    PlaneRows pr, int nx1, const int* __restrict__ x1list, int overwrite) {
   using V2 = typename V2t<T>::t;
   using Sh = DensityShape<T, N>;
   constexpr int LD = Sh::LD, NT = Sh::NT, SLOTS = Sh::SLOTS;
@@ -102,7 +102,8 @@ __global__ void __launch_bounds__((DensityShape<T, N>::NT))
   // add the slots in order and write the plane
   double* sum = REGS ? reinterpret_cast<double*>(smem_raw) : acc_lds;  // [N][N]
   if constexpr (REGS) {
-    for (int p = 0; p < SLOTS; ++p) {
+    const int used = DIRECT ? min(SLOTS, nb) : SLOTS;
+    for (int p = 0; p < used; ++p) {
       if (slot == p) {
 #pragma unroll
         for (int q = 0; q < N; ++q) sum[q * N + i2] = p == 0 ? acc[q] : sum[q * N + i2] + acc[q];
@@ -115,7 +116,12 @@ __global__ void __launch_bounds__((DensityShape<T, N>::NT))
     double s = sum[i];
     if (!REGS)
       for (int p = 1; p < SLOTS; ++p) s += sum[p * N * N + i];
-    out[i] = s;
+    if constexpr (DIRECT) {
+      double* d = &part[(size_t)i * nz + i3];
+      *d = overwrite ? s : *d + s;
+    } else {
+      out[i] = s;
+    }
   }
 }
 
@@ -191,8 +197,9 @@ __global__ void __launch_bounds__(256) k_density_sum(int ngroups, int nx, int ny
   }
 }
 
-template <typename T, int N, bool QUARTER>
-void plane_density(Context& c, const void* tbuf, int nb, int per, int groups, const double* fw, double* part) {
+template <typename T, int N, bool QUARTER, bool DIRECT>
+void plane_density(Context& c, const void* tbuf, int nb, int per, int groups, const double* fw, double* part,
+                   int overwrite) {
   using V2 = typename V2t<T>::t;
   using Sh = DensityShape<T, N>;
   const int image = QUARTER ? Quarter<N>::R * Quarter<N>::LD : c.pl_rows * Sh::LD;
@@ -202,12 +209,31 @@ void plane_density(Context& c, const void* tbuf, int nb, int per, int groups, co
   else
     sh += (size_t)Sh::SLOTS * N * N * sizeof(double);
   PWK_REQUIRE(sh <= 160 * 1024, PWK_E_UNSUPPORTED, "density plane exceeds the LDS");
-  ensure_lds_limit((const void*)k_plane_density<T, N, QUARTER>, sh);
+  ensure_lds_limit((const void*)k_plane_density<T, N, QUARTER, DIRECT>, sh);
   const PlaneRows pr{c.pl_ra, c.pl_rb};
-  k_plane_density<T, N, QUARTER><<<dim3((unsigned)c.dims[2], (unsigned)groups), Sh::NT, sh, c.stream>>>(
+  k_plane_density<T, N, QUARTER, DIRECT><<<dim3((unsigned)c.dims[2], (unsigned)groups), Sh::NT, sh, c.stream>>>(
       (const V2*)tbuf, nb, per, fw, part, c.nsticks, c.dims[2], QUARTER ? c.q_src.as<int>() : c.pl_src.as<int>(), image,
-      pr, c.nx1, c.x1_runs ? nullptr : c.x1list.as<int>());
+      pr, c.nx1, c.x1_runs ? nullptr : c.x1list.as<int>(), overwrite);
   PWK_HIP(hipGetLastError());
+}
+
+constexpr int DIRECT_MAX = 27;  // the longest axis of grids whose one group adds to ρ itself
+template <typename T, int N>
+void plane_density_any(Context& c, int nb, int per, int groups, const double* fw, double* part, double* rho,
+                       int overwrite, bool direct) {
+  if constexpr (N <= DIRECT_MAX) {
+    if (direct) {
+      if (c.quarter)
+        plane_density<T, N, true, true>(c, c.work_a.p, nb, per, 1, fw, rho, overwrite);
+      else
+        plane_density<T, N, false, true>(c, c.work_a.p, nb, per, 1, fw, rho, overwrite);
+      return;
+    }
+  }
+  if (c.quarter)
+    plane_density<T, N, true, false>(c, c.work_a.p, nb, per, groups, fw, part, 0);
+  else
+    plane_density<T, N, false, false>(c, c.work_a.p, nb, per, groups, fw, part, 0);
 }
 
 template <typename T>
@@ -270,6 +296,11 @@ void density_sticks_t(Context& c, int nb, const void* psi, const double* fw_host
       const int batches = (n + slots - 1) / slots;
       const int per = std::max(1, (int)((batches * wgs + 1023) / 1024));
       const int groups = (batches + per - 1) / per;
+      const int ow = overwrite && b0 == 0 ? 1 : 0;
+      // one group on a small grid: the plane pass adds to ρ itself, at strides of nz, and the third launch goes
+      // (15 x 15 x 16, 1 band 16.1 us -> 11.2, 20 x 20 x 24 14.9 -> 11.3; on 32³ 18.5 against 17.8, and
+      // 60³ 45.1 against 29.6)
+      const bool direct = square && groups == 1 && nx <= DIRECT_MAX && c.N <= 20000;
       launch_zinv(c, n, captured ? (const V2*)psi + (size_t)b0 * c.npw : psi, c.work_a.p,
                   std::is_same<T, double>::value ? PWK_FP64 : PWK_FP32,
                   captured ? nullptr : reinterpret_cast<const int*>(weights + live) + b0);
@@ -279,10 +310,8 @@ void density_sticks_t(Context& c, int nb, const void* psi, const double* fw_host
   case L:                                                                                                             \
     if (!square)                                                                                                      \
       k_cols_density<T, L><<<dim3((unsigned)wgs, (unsigned)groups), 64, 0, c.stream>>>(rows, n, per, fw, part, ny, nz); \
-    else if (c.quarter)                                                                                               \
-      plane_density<T, L, true>(c, c.work_a.p, n, per, groups, fw, part);                                             \
     else                                                                                                              \
-      plane_density<T, L, false>(c, c.work_a.p, n, per, groups, fw, part);                                            \
+      plane_density_any<T, L>(c, n, per, groups, fw, part, rho, ow, direct);                                          \
     break;
         PWK_FOR_EACH_FFT_SIZE(PWK_CASE)
 #undef PWK_CASE
@@ -290,8 +319,9 @@ void density_sticks_t(Context& c, int nb, const void* psi, const double* fw_host
           throw Error(PWK_E_UNSUPPORTED, "nx has no compiled kernel");
       }
       PWK_HIP(hipGetLastError());
+      if (direct) continue;
       const dim3 gs(blocks_for((size_t)ny, 32), blocks_for((size_t)nz, 32), (unsigned)nx);
-      k_density_sum<<<gs, 256, 0, c.stream>>>(groups, nx, ny, nz, part, rho, overwrite && b0 == 0 ? 1 : 0);
+      k_density_sum<<<gs, 256, 0, c.stream>>>(groups, nx, ny, nz, part, rho, ow);
       PWK_HIP(hipGetLastError());
     }
   } else if (overwrite) {
