@@ -112,33 +112,32 @@ __global__ void __launch_bounds__(64) k_zfwd(const typename V2t<T>::t* __restric
   }
 }
 
-// H·ψ plane pass: the z-plane i3 of SLOTS bands per workgroup (planes.hpp): y-inverse on the rows with
+// H·ψ plane pass: one z-plane of one band per workgroup (planes.hpp): y-inverse on the rows with
 // sticks, x-inverse, × V(r), x-forward, y-forward, back to the sticks. The rows without sticks are zero
 // through the y passes and their x output is never gathered: the x-lines read them from the image's
 // zero row and write them to a discard row after it, so the loads and stores need no branch. Bound: the
 // vector arithmetic of the line transforms; the traffic is the stick buffer in and out.
+// Several planes per workgroup fill its waves better, but an image of a wide sphere's rows lets fewer waves
+// on a CU and fewer workgroups start: a whole H·ψ with radius 9 on 25³, 16 FP32 bands 22.5 us against 18.8,
+// radius 17 on 45³, 60 bands 77.6 against 60.2, radius 12 on 27³, 140 FP64 bands 73.4 against 63.2.
 template <typename T, int N>
-__global__ void __launch_bounds__((PlaneShape<T, N>::NT))
-    k_plane_hpsi(typename V2t<T>::t* tbuf, int nb, const T* __restrict__ vr, int S, int nz,
-                 const int* __restrict__ src, int nsrc, int image, const int* __restrict__ st_off, PlaneRows pr,
-                 int nx1, const int* __restrict__ x1list) {
+__global__ void __launch_bounds__((PlaneShape<T, N, false, true>::NT))
+    k_plane_hpsi(typename V2t<T>::t* tbuf, const T* __restrict__ vr, int S, int nz, const int* __restrict__ src, int nsrc,
+                 const int* __restrict__ st_off, PlaneRows pr, int nx1, const int* __restrict__ x1list) {
   using V2 = typename V2t<T>::t;
-  using Sh = PlaneShape<T, N>;
-  constexpr int LD = Sh::LD, NT = Sh::NT, SLOTS = Sh::SLOTS;
-  constexpr int U = 16 / (int)(sizeof(T) / 4);
+  constexpr int LD = N + 1, NT = PlaneShape<T, N, false, true>::NT;
+  constexpr int UI = in_flight<T, NT>(N * LD), UO = in_flight<T, NT>(N * N / 2);
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
   V2* P = reinterpret_cast<V2*>(smem_raw);
-  const int i3 = blockIdx.x, b0 = blockIdx.y * SLOTS, nsl = min(SLOTS, nb - b0);
-  const size_t stride = (size_t)nz * S;
-  V2* tp0 = tbuf + (size_t)b0 * stride + (size_t)i3 * S;
-  plane_fill<T, N, NT, U>(P, image, tp0, stride, nsl, src, nsrc);
+  const int i3 = blockIdx.x, b = blockIdx.y, i2 = threadIdx.x;
+  V2* tp = tbuf + ((size_t)b * nz + i3) * S;
+  plane_fill<T, N, NT, UI>(P, 0, tp, 0, 1, src, nsrc);
   __syncthreads();
-  plane_ylines<T, N, NT, 1>(P, image, nsl, nx1, x1list);
+  plane_ylines<T, N, NT, 1>(P, 0, 1, nx1, x1list);
   __syncthreads();
-  const int slot = threadIdx.x / N, i2 = threadIdx.x - slot * N;
-  if (slot < nsl) {
+  if (i2 < N) {
     const T* v = vr + (size_t)i3 * N * N + i2;
-    V2* col = P + slot * image + i2;
+    V2* col = P + i2;
     T re[N], im[N];
 #pragma unroll
     for (int j = 0; j < N; ++j) {
@@ -164,30 +163,26 @@ __global__ void __launch_bounds__((PlaneShape<T, N>::NT))
     }
   }
   __syncthreads();
-  plane_ylines<T, N, NT, -1>(P, image, nsl, nx1, x1list);
+  plane_ylines<T, N, NT, -1>(P, 0, 1, nx1, x1list);
   __syncthreads();
-  for (int s0 = threadIdx.x; s0 < S; s0 += U * NT) {
-    int off[U];
+  for (int s0 = threadIdx.x; s0 < S; s0 += UO * NT) {
+    int off[UO];
 #pragma unroll
-    for (int u = 0; u < U; ++u) off[u] = st_off[min(s0 + u * NT, S - 1)];
-    for (int p = 0; p < nsl; ++p) {
-      V2* tp = tp0 + (size_t)p * stride;
+    for (int u = 0; u < UO; ++u) off[u] = st_off[min(s0 + u * NT, S - 1)];
 #pragma unroll
-      for (int u = 0; u < U; ++u)
-        if (s0 + u * NT < S) tp[s0 + u * NT] = P[p * image + off[u]];
-    }
+    for (int u = 0; u < UO; ++u)
+      if (s0 + u * NT < S) tp[s0 + u * NT] = P[off[u]];
   }
 }
 
 template <typename T, int N>
 void plane_hpsi(Context& c, typename V2t<T>::t* tbuf, int nb, const T* vr) {
-  using Sh = PlaneShape<T, N>;
-  const int nz = c.dims[2], rows = c.x1_runs ? c.pl_rows + 1 : c.pl_rows, image = rows * Sh::LD;
-  const size_t sh = (size_t)Sh::SLOTS * image * sizeof(typename V2t<T>::t);
+  const int nz = c.dims[2], rows = c.x1_runs ? c.pl_rows + 1 : c.pl_rows;
+  const size_t sh = (size_t)rows * (N + 1) * sizeof(typename V2t<T>::t);
   PWK_REQUIRE(sh <= 160 * 1024, PWK_E_UNSUPPORTED, "plane exceeds the LDS");
   ensure_lds_limit((const void*)k_plane_hpsi<T, N>, sh);
-  k_plane_hpsi<T, N><<<dim3((unsigned)nz, blocks_for((size_t)nb, Sh::SLOTS)), Sh::NT, sh, c.stream>>>(
-      tbuf, nb, vr, c.nsticks, nz, c.pl_src.as<int>(), c.pl_rows * Sh::LD, image, c.st_off.as<int>(),
+  k_plane_hpsi<T, N><<<dim3((unsigned)nz, (unsigned)nb), PlaneShape<T, N, false, true>::NT, sh, c.stream>>>(
+      tbuf, vr, c.nsticks, nz, c.pl_src.as<int>(), c.pl_rows * (N + 1), c.st_off.as<int>(),
       PlaneRows{c.pl_ra, c.pl_rb}, c.nx1, c.x1_runs ? nullptr : c.x1list.as<int>());
   PWK_HIP(hipGetLastError());
 }

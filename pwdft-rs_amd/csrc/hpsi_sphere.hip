@@ -138,15 +138,15 @@ __global__ void __launch_bounds__(ZS) k_zfwd_q(const typename V2t<T>::t* __restr
 // 67 us, FP64 45³ × 160 bands 151 us -> 103 us.
 // Up to 81 points in FP32 a line's registers leave room for two waves per SIMD, which 64 points does not
 // get unasked: 64³ × 144 bands 111 us -> 71 us. FP64 lines spill under that bound.
-template <typename T, int N>
-__global__ void __launch_bounds__((PlaneShape<T, N>::NT), (sizeof(T) == 4 && N <= 81 ? 2 : 1))
+template <typename T, int N, bool ONE>
+__global__ void __launch_bounds__((PlaneShape<T, N, false, ONE>::NT), (sizeof(T) == 4 && N <= 81 ? 2 : 1))
     k_plane_q(typename V2t<T>::t* tbuf, int nb, const T* __restrict__ vr, int S, int nz, const int* __restrict__ src,
               const int* __restrict__ st_off) {
   using V2 = typename V2t<T>::t;
-  using Sh = PlaneShape<T, N>;
+  using Sh = PlaneShape<T, N, false, ONE>;
   using Q = Quarter<N>;
   constexpr int NT = Sh::NT, SLOTS = Sh::SLOTS, IMG = Q::R * Q::LD;
-  constexpr int U = 16 / (int)(sizeof(T) / 4);
+  constexpr int U = in_flight<T, NT>(Q::R * Q::R);
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
   V2* P = reinterpret_cast<V2*>(smem_raw);
   const int i3 = blockIdx.x, b0 = blockIdx.y * SLOTS, nsl = min(SLOTS, nb - b0);
@@ -327,13 +327,31 @@ void rows_any(Context& c, int nb, typename V2t<T>::t* tbuf, typename V2t<T>::t* 
   PWK_HIP(hipGetLastError());
 }
 
-template <typename T, int N>
+template <typename T, int N, bool ONE>
 void plane_q(Context& c, typename V2t<T>::t* tbuf, int nb, const T* vr) {
-  using Sh = PlaneShape<T, N>;
+  using Sh = PlaneShape<T, N, false, ONE>;
   const size_t sh = (size_t)Sh::SLOTS * Quarter<N>::R * Quarter<N>::LD * sizeof(typename V2t<T>::t);
-  ensure_lds_limit((const void*)k_plane_q<T, N>, sh);
-  k_plane_q<T, N><<<dim3((unsigned)c.dims[2], blocks_for((size_t)nb, Sh::SLOTS)), Sh::NT, sh, c.stream>>>(
+  ensure_lds_limit((const void*)k_plane_q<T, N, ONE>, sh);
+  k_plane_q<T, N, ONE><<<dim3((unsigned)c.dims[2], blocks_for((size_t)nb, Sh::SLOTS)), Sh::NT, sh, c.stream>>>(
       tbuf, nb, vr, c.nsticks, c.dims[2], c.q_src.as<int>(), c.q_off.as<int>());
+}
+
+// One plane per workgroup where the form with more than two would leave SIMDs without a wave (FP32: fewer
+// waves than the 1024 of the chip; half of that in FP64, whose planes take twice as long): a whole H·ψ of 16
+// FP32 bands on 25³ 18.2 us -> 15.9 us, of 60 19.2 -> 17.2, of 140 22.1 against 23.0; 8 bands on 36³ 21.6 ->
+// 17.9, 140 bands 34.0 against 36.7. A single band has the waves of the larger form to itself (FP64 45³ 26.5
+// against 27.6), and two planes (54 points and more) stay together: 60³ x 1 band 25.8 us against 28.7.
+template <typename T, int N>
+void plane_any(Context& c, typename V2t<T>::t* tbuf, int nb, const T* vr) {
+  using Sh = PlaneShape<T, N>;
+  if constexpr (Sh::SLOTS > 2) {
+    const long waves = (long)c.dims[2] * ((nb + Sh::SLOTS - 1) / Sh::SLOTS) * Sh::W;
+    if (nb > 1 && waves < (sizeof(T) == 4 ? 1024 : 512)) {
+      plane_q<T, N, true>(c, tbuf, nb, vr);
+      return;
+    }
+  }
+  plane_q<T, N, false>(c, tbuf, nb, vr);
 }
 
 template <typename T, int N, class Entries>
@@ -414,7 +432,7 @@ void sphere_plane(Context& c, int nb, void* buf, const T* vr, void* rows) {
   switch (c.dims[0]) {
 #define PWK_CASE(L) \
   case L:           \
-    plane_q<T, L>(c, tbuf, nb, vr); \
+    plane_any<T, L>(c, tbuf, nb, vr); \
     break;
     PWK_FOR_EACH_FFT_SIZE(PWK_CASE)
 #undef PWK_CASE

@@ -3,7 +3,8 @@
 //
 // A workgroup works on SLOTS planes at once (the same i3 of SLOTS bands), so that the y-lines (only
 // the nx1 rows that carry sticks, about half of them) and the x-lines of a plane fill whole waves: a
-// 60-point plane alone has 29 y-lines for 64 lanes, two planes have 58.
+// 60-point plane alone has 29 y-lines for 64 lanes, two planes have 58. Or on one (ONE): H·ψ of wider spheres,
+// and of few planes (hpsi_sphere.hip).
 //
 // A plane's LDS image holds only the rows that carry sticks when these are the two runs i1 < ra and
 // i1 >= nx - rb (a sphere's columns), followed by a zero row that stands for every other row; grids
@@ -34,7 +35,7 @@ struct V2t<float> {
 // run y-lines; the cheapest of 1-4 waves is taken, fewer waves on a tie, whose planes fit 72 KB of
 // LDS (two workgroups per CU) with the rows of a sphere, and the 160 KB of a CU with all rows. ACC:
 // an FP64 sum per point and plane in LDS as well.
-template <typename T, int N, bool ACC = false>
+template <typename T, int N, bool ACC = false, bool ONE = false>
 struct PlaneShape {
   static constexpr int LD = N + 1;  // one element of padding against bank conflicts on row access
   static constexpr int slots(int w) { return 64 * w / N; }
@@ -50,8 +51,15 @@ struct PlaneShape {
       if (lds(v, N / 2 + 3) <= 72 * 1024 && lds(v, N + 2) <= 160 * 1024 && cost(v) < cost(w)) w = v;
     return w;
   }
-  static constexpr int W = best(), NT = 64 * W, SLOTS = slots(W);
+  static constexpr int W = ONE ? (N + 63) / 64 : best(), NT = 64 * W, SLOTS = ONE ? 1 : slots(W);
 };
+
+// loads of a thread in flight while NT threads move n elements: no more than it has, up to 16 (FP64 8)
+template <typename T, int NT>
+constexpr int in_flight(int n) {
+  const int most = 16 / (int)(sizeof(T) / 4), need = (n + NT - 1) / NT;
+  return need < most ? need : most;
+}
 
 // the plane row j in the held image (`absent` for a row without sticks)
 struct PlaneRows {

@@ -84,7 +84,9 @@ def test_hpsi_planes(gpu, dims, m, prec, tol):
         n = int(np.prod(dims))
         v = rng.uniform(-13.6, 13.6, dims)
         gpu.set_veff((np.fft.fftn(v) / n).reshape(-1))
-        for nb in (1, 2, 5):
+        # a few bands, and enough of them for several planes per workgroup, the last one not full
+        many = [245] if dims[0] <= 16 else [107] if dims[0] <= 32 else [74] if dims[0] <= 48 else []
+        for nb in [1, 2, 5] + many:
             psi = bands(rng, nb, len(miller))
             print("hpsi planes", dims, m, prec, "bands", nb, flush=True)
             got = gpu.hpsi(0, psi, prec)
