@@ -275,45 +275,82 @@ struct FftPlan {
 
 // ---- k × band batches that share their launches --------------------------------------------
 // The entries of a batch travel by value in the kernel arguments, so a captured launch keeps its own and
-// nothing is uploaded; an entry per lane of a wave. (A device table that every batch rewrote was read by the
-// replays of graphs captured with other entries.) Kernels are compiled for them apart: 0.8 KB more of
-// arguments on every launch took a sequence of eight short launches from 25.3 to 28.3 us.
-constexpr int MAX_BATCH_ENTRIES = 64;
+// nothing is uploaded. (A device table that every batch rewrote was read by the replays of graphs captured with
+// other entries.) Kernels are compiled for them apart: 0.8 KB more of arguments on every launch took a sequence
+// of eight short launches from 25.3 to 28.3 us.
+// A launch copies all CAP entries, so few of them have kernels of their own.
+constexpr int FEW_BATCH_ENTRIES = 16, MAX_BATCH_ENTRIES = 128;
 struct NoBatch {
   static constexpr bool batch = false;
 };
-// bands [end[e - 1], end[e]) have the kinetic diagonal kin[e]
-struct BatchKin {
+// bands [end[e - 1], end[e]) are entry e's; INT32_MAX from the last entry on
+template <int CAP>
+struct BatchBands {
+  int end[CAP];
+  BatchBands() { std::fill(end, end + CAP, INT32_MAX); }
+};
+// with the kinetic diagonal of each entry
+template <int CAP>
+struct BatchKin : BatchBands<CAP> {
   static constexpr bool batch = true;
-  int n = 0;
-  int end[MAX_BATCH_ENTRIES];
-  const void* kin[MAX_BATCH_ENTRIES];
+  const void* kin[CAP];
 };
 // the same on the fused small grids, with the projector blocks
-struct BatchSmall {
-  static constexpr bool batch = true;
-  int n = 0;
-  int end[MAX_BATCH_ENTRIES];
-  const void *kin[MAX_BATCH_ENTRIES], *B[MAX_BATCH_ENTRIES], *DBH[MAX_BATCH_ENTRIES];
+template <int CAP>
+struct BatchSmall : BatchKin<CAP> {
+  const void *B[CAP], *DBH[CAP];
 };
 // product e is C[:, col..col + cols) (+)= A·B[:, col..col + cols) with its own A
+template <int CAP>
 struct GemmGroups {
   static constexpr bool batch = true;
   int n = 0;
-  int cols[MAX_BATCH_ENTRIES], col[MAX_BATCH_ENTRIES];
-  const void* A[MAX_BATCH_ENTRIES];
+  int cols[CAP], col[CAP];
+  const void* A[CAP];
 };
-// the entry of band b (uniform) by one load per lane; every lane of the wave calls it
-template <class Entries>
-__device__ __forceinline__ int batch_entry(const Entries& entries, int b) {
-  const int lane = threadIdx.x & 63;
-  return __popcll(__ballot(lane < entries.n && entries.end[lane] <= b));
+// An array of the entries over the lanes of a wave; an entry's value (uniform) is taken from its lane, and every
+// lane of the wave takes part. All reads of a kernel's arrays are in flight at once: the arguments are slow to
+// reach, and one read after another took 8 k-points x 16 FP32 bands on 15³ from 10.5 us to 10.7 on one stream (a
+// table in device memory 9.9, with a wait for its upload at every change; on several streams 8.2 to 8.4 us
+// either way).
+template <int CAP, typename V>
+struct OverLanes {
+  static constexpr int PER = (CAP + 63) / 64;
+  V v[PER];
+  __device__ __forceinline__ explicit OverLanes(const V* x) {
+#pragma unroll
+    for (int i = 0; i < PER; ++i) v[i] = x[min(64 * i + (int)(threadIdx.x & 63), CAP - 1)];
+  }
+};
+// the entry of band b
+template <int CAP>
+__device__ __forceinline__ int batch_entry(const OverLanes<CAP, int>& end, int b) {
+  int e = 0;
+#pragma unroll
+  for (int i = 0; i < OverLanes<CAP, int>::PER; ++i)
+    e += __popcll(__ballot(64 * i + (int)(threadIdx.x & 63) < CAP && end.v[i] <= b));
+  return e;
+}
+template <typename T, int CAP>
+__device__ __forceinline__ const T* batch_ptr(const OverLanes<CAP, const void*>& p, int e) {
+  unsigned long long v = (unsigned long long)p.v[0];
+#pragma unroll
+  for (int i = 1; i < OverLanes<CAP, const void*>::PER; ++i) v = (e >> 6) == i ? (unsigned long long)p.v[i] : v;
+  const unsigned lo = __builtin_amdgcn_readlane((int)(unsigned)v, e & 63);
+  const unsigned hi = __builtin_amdgcn_readlane((int)(unsigned)(v >> 32), e & 63);
+  return (const T*)(((unsigned long long)hi << 32) | lo);
+}
+template <typename T, int CAP>
+__device__ __forceinline__ const T* entry_kin(const BatchKin<CAP>& x, int b) {
+  const OverLanes<CAP, int> end(x.end);
+  const OverLanes<CAP, const void*> kin(x.kin);
+  return batch_ptr<T>(kin, batch_entry(end, b));
 }
 // the kinetic diagonal of band b: its entry's, or without entries that of k-point b / nbk
 template <typename T, class Entries>
 __device__ __forceinline__ const T* band_kin(const Entries& entries, const T* kin, int npw, int nbk, int b) {
   if constexpr (Entries::batch) {
-    return (const T*)entries.kin[batch_entry(entries, b)];
+    return entry_kin<T>(entries, b);
   } else {
     return kin + (size_t)(b / nbk) * npw;
   }
@@ -522,7 +559,9 @@ void launch_hpsi_small(Context& c, int nbands, int nbk, const void* psi, void* h
                        int nch, const void* B, const void* DBH, const double* coef = nullptr,
                        const void* X = nullptr, int nkv = 0, const int* skip = nullptr);
 // the entries of a ragged k × band batch with nch channels each, in one launch
-void launch_hpsi_small_batch(Context& c, const BatchSmall& entries, const void* psi, void* hpsi, int precision, int nch);
+template <int CAP>
+void launch_hpsi_small_batch(Context& c, const BatchSmall<CAP>& entries, int nbands, const void* psi, void* hpsi,
+                             int precision, int nch);
 // the whole degree-`degree` Chebyshev filter of nbands bands in one launch on small cubic grids:
 // Yout (FP64) = p(H)·V (FP64) with the recurrence in `precision`; coef (device) holds (α, c, β)
 // per step and band block, coef[(i·nblocks + kb)·3 + j]
@@ -556,7 +595,8 @@ void launch_zgemm_mfma_batched(Context& c, int M, int N, int K, const void* A, i
                                int ldb, long long sB, void* C, int ldc, long long sC, int batch, bool accumulate,
                                int precision);
 // the products of a batch's entries (groups.n of them, the widest of Nmax columns; A's lda shared)
-void launch_zgemm_mfma_groups(Context& c, int M, int Nmax, int K, const GemmGroups& groups, int lda, const void* B,
+template <int CAP>
+void launch_zgemm_mfma_groups(Context& c, int M, int Nmax, int K, const GemmGroups<CAP>& groups, int lda, const void* B,
                               int ldb, void* C, int ldc, bool accumulate, int precision);
 // eig.hip: lowest nb eigenpairs of nk Hermitian n×n matrices (H overwritten)
 size_t heev_work_doubles(int n, int nb, int nk);

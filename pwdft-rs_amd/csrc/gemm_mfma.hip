@@ -440,7 +440,8 @@ void launch_zgemm_mfma_batched(Context& c, int M, int N, int K, const void* A, i
     zgemm_mfma_t<MODE_F32>(c, M, N, K, A, lda, B, ldb, C, ldc, accumulate, bt, NoBatch{});
 }
 
-void launch_zgemm_mfma_groups(Context& c, int M, int Nmax, int K, const GemmGroups& groups, int lda, const void* B,
+template <int CAP>
+void launch_zgemm_mfma_groups(Context& c, int M, int Nmax, int K, const GemmGroups<CAP>& groups, int lda, const void* B,
                               int ldb, void* C, int ldc, bool accumulate, int precision) {
   if (M <= 0 || Nmax <= 0 || K <= 0 || groups.n <= 0) return;
   Batch bt;
@@ -452,5 +453,10 @@ void launch_zgemm_mfma_groups(Context& c, int M, int Nmax, int K, const GemmGrou
   else
     zgemm_mfma_t<MODE_F32>(c, M, Nmax, K, nullptr, lda, B, ldb, C, ldc, accumulate, bt, groups);
 }
+
+template void launch_zgemm_mfma_groups(Context&, int, int, int, const GemmGroups<FEW_BATCH_ENTRIES>&, int, const void*, int,
+                                       void*, int, bool, int);
+template void launch_zgemm_mfma_groups(Context&, int, int, int, const GemmGroups<MAX_BATCH_ENTRIES>&, int, const void*, int,
+                                       void*, int, bool, int);
 
 }  // namespace pwk

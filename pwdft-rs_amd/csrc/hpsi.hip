@@ -75,8 +75,8 @@ __global__ void __launch_bounds__(64) k_zfwd(const typename V2t<T>::t* __restric
                                              T inv_n, int nbk, const Entries entries) {
   int s = blockIdx.x * 64 + threadIdx.x;
   int b = blockIdx.y;
-  int ent = 0;  // the band's entry, by all lanes before any leaves
-  if constexpr (Entries::batch) ent = batch_entry(entries, b);
+  const T* tb = nullptr;  // the entry's kinetic diagonal, by all lanes before any leaves
+  if constexpr (Entries::batch) tb = band_kin(entries, kin, npw, nbk, b);
   if (s >= S) return;
   int pw0 = st_pw0[s], cnt = st_cnt[s], lo = st_lo[s];
   const typename V2t<T>::t* src = tbuf + (size_t)b * NZ * S + s;
@@ -96,8 +96,8 @@ __global__ void __launch_bounds__(64) k_zfwd(const typename V2t<T>::t* __restric
   }
   const typename V2t<T>::t* p = psi + (size_t)b * npw + pw0;
   typename V2t<T>::t* h = hpsi + (size_t)b * npw + pw0;
-  const T* t = kin + (size_t)(b / nbk) * npw + pw0;
-  if constexpr (Entries::batch) t = (const T*)entries.kin[ent] + pw0;
+  if constexpr (!Entries::batch) tb = kin + (size_t)(b / nbk) * npw;
+  const T* t = tb + pw0;
 #pragma unroll
   for (int i3 = 0; i3 < NZ; ++i3) {
     int j = stick_slot(i3, lo, NZ);
@@ -648,14 +648,14 @@ namespace {
 // The entries [e0, e1) of a batch on the stick path: one launch sequence over the bands of all of them, each
 // with its entry's kinetic diagonal, and the entries' projector products as one grouped launch each.
 // 27 k-points of about 24 bands (1189 plane waves, 25³) took 162 launches one entry at a time.
-template <typename T>
+template <typename T, int CAP>
 void hpsi_batch_sticks(Context& c, int e0, int e1, const int32_t* ik, const int32_t* nbands, const void* psi,
                        void* hpsi, int precision) {
   const bool f64 = std::is_same<T, double>::value;
   const int nch = c.k(ik[e0]).nch;
-  BatchKin kin;
-  GemmGroups project, expand;
-  kin.n = project.n = expand.n = e1 - e0;
+  BatchKin<CAP> kin;
+  GemmGroups<CAP> project, expand;
+  project.n = expand.n = e1 - e0;
   int total = 0, nmax = 0;
   for (int e = 0; e < e1 - e0; ++e) {
     const KData& kd = c.k(ik[e0 + e]);
@@ -678,6 +678,34 @@ void hpsi_batch_sticks(Context& c, int e0, int e1, const int32_t* ik, const int3
     TimedScope ts(c, "hpsi_nl_expand");
     launch_zgemm_mfma_groups(c, c.npw, nmax, nch, expand, c.npw, c.proj.p, nch, hpsi, c.npw, true, precision);
   }
+}
+
+// the same in the one launch of the fused small grids
+template <int CAP>
+void hpsi_batch_small(Context& c, int e0, int e1, const int32_t* ik, const int32_t* nbands, const void* psi,
+                      void* hpsi, int precision) {
+  const bool f64 = precision == PWK_FP64;
+  BatchSmall<CAP> entries;
+  int total = 0;
+  for (int e = 0; e < e1 - e0; ++e) {
+    const KData& kd = c.k(ik[e0 + e]);
+    entries.end[e] = total += nbands[e0 + e];
+    entries.kin[e] = f64 ? kd.kin64.p : kd.kin32.p;
+    entries.B[e] = f64 ? kd.B64.p : kd.B32.p;
+    entries.DBH[e] = f64 ? kd.DBH64.p : kd.DBH32.p;
+  }
+  launch_hpsi_small_batch(c, entries, total, psi, hpsi, precision, c.k(ik[e0]).nch);
+}
+
+template <int CAP>
+void hpsi_batch_run(Context& c, int e0, int e1, const int32_t* ik, const int32_t* nbands, const void* psi, void* hpsi,
+                    int precision, bool small) {
+  if (small)
+    hpsi_batch_small<CAP>(c, e0, e1, ik, nbands, psi, hpsi, precision);
+  else if (precision == PWK_FP64)
+    hpsi_batch_sticks<double, CAP>(c, e0, e1, ik, nbands, psi, hpsi, precision);
+  else
+    hpsi_batch_sticks<float, CAP>(c, e0, e1, ik, nbands, psi, hpsi, precision);
 }
 
 // The entries from e0 on that share their launches: as many as one launch takes, with one channel count, and
@@ -718,21 +746,10 @@ void launch_hpsi_batch(Context& c, int nent, const int32_t* ik, const int32_t* n
     const int end = small || stick_path_ok(c, f64) ? batch_run(c, nent, e, ik, nbands, small, f64) : e + 1;
     if (end == e + 1) {
       launch_hpsi(c, ik[e], nbands[e], psi, hpsi, precision);
-    } else if (small) {
-      BatchSmall entries;
-      entries.n = end - e;
-      for (int i = 0, total = 0; i < end - e; ++i) {
-        const KData& kd = c.k(ik[e + i]);
-        entries.end[i] = total += nbands[e + i];
-        entries.kin[i] = f64 ? kd.kin64.p : kd.kin32.p;
-        entries.B[i] = f64 ? kd.B64.p : kd.B32.p;
-        entries.DBH[i] = f64 ? kd.DBH64.p : kd.DBH32.p;
-      }
-      launch_hpsi_small_batch(c, entries, psi, hpsi, precision, nch);
-    } else if (f64) {
-      hpsi_batch_sticks<double>(c, e, end, ik, nbands, psi, hpsi, precision);
+    } else if (end - e <= FEW_BATCH_ENTRIES) {
+      hpsi_batch_run<FEW_BATCH_ENTRIES>(c, e, end, ik, nbands, psi, hpsi, precision, small);
     } else {
-      hpsi_batch_sticks<float>(c, e, end, ik, nbands, psi, hpsi, precision);
+      hpsi_batch_run<MAX_BATCH_ENTRIES>(c, e, end, ik, nbands, psi, hpsi, precision, small);
     }
     for (; e < end; ++e) {
       psi = (const char*)psi + (size_t)nbands[e] * c.npw * es;

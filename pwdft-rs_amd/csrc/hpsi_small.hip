@@ -253,10 +253,13 @@ __device__ __forceinline__ void hpsi_small_body(int bid, int nblocks, const type
   const T* t;
   const V2 *bk, *dk;
   if constexpr (Entries::batch) {
-    const int e = batch_entry(entries, b);
-    t = (const T*)entries.kin[e];
-    bk = (const V2*)entries.B[e];
-    dk = (const V2*)entries.DBH[e];
+    constexpr int CAP = sizeof(entries.end) / sizeof(int);
+    const OverLanes<CAP, int> end(entries.end);
+    const OverLanes<CAP, const void*> pk(entries.kin), pb(entries.B), pd(entries.DBH);
+    const int e = batch_entry(end, b);
+    t = batch_ptr<T>(pk, e);
+    bk = batch_ptr<V2>(pb, e);
+    dk = batch_ptr<V2>(pd, e);
   } else {
     t = kin + (size_t)k * npw;
     bk = B + (size_t)k * npw * nch;
@@ -1039,15 +1042,19 @@ void launch_hpsi_small(Context& c, int nbands, int nbk, const void* psi, void* h
     launch_small_t<float>(c, nbands, nbk, psi, hpsi, kin, nch, B, DBH, coef, X, nkv, skip, NoBatch{});
 }
 
-void launch_hpsi_small_batch(Context& c, const BatchSmall& entries, const void* psi, void* hpsi, int precision, int nch) {
+template <int CAP>
+void launch_hpsi_small_batch(Context& c, const BatchSmall<CAP>& entries, int nbands, const void* psi, void* hpsi,
+                             int precision, int nch) {
   c.check_basis();
   PWK_REQUIRE(c.have_v, PWK_E_STATE, "V_eff not set (pwk_set_veff)");
   PWK_REQUIRE(hpsi_small_supported(c, precision, nch), PWK_E_UNSUPPORTED, "grid too large for the fused kernel");
-  const int nbands = entries.end[entries.n - 1];
   if (precision == PWK_FP64)
     launch_small_t<double>(c, nbands, 1, psi, hpsi, nullptr, nch, nullptr, nullptr, nullptr, nullptr, 0, nullptr, entries);
   else
     launch_small_t<float>(c, nbands, 1, psi, hpsi, nullptr, nch, nullptr, nullptr, nullptr, nullptr, 0, nullptr, entries);
 }
+
+template void launch_hpsi_small_batch(Context&, const BatchSmall<FEW_BATCH_ENTRIES>&, int, const void*, void*, int, int);
+template void launch_hpsi_small_batch(Context&, const BatchSmall<MAX_BATCH_ENTRIES>&, int, const void*, void*, int, int);
 
 }  // namespace pwk

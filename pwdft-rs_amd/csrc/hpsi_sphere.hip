@@ -465,9 +465,14 @@ template void sphere_rows_inverse<float>(Context&, int, void*, void*);
 template void sphere_rows_inverse<double>(Context&, int, void*, void*);
 template void sphere_plane<float>(Context&, int, void*, const float*, void*);
 template void sphere_plane<double>(Context&, int, void*, const double*, void*);
-template void sphere_zfwd(Context&, int, const void*, const float*, int, int, const NoBatch&, const void*, void*);
-template void sphere_zfwd(Context&, int, const void*, const float*, int, int, const BatchKin&, const void*, void*);
-template void sphere_zfwd(Context&, int, const void*, const double*, int, int, const NoBatch&, const void*, void*);
-template void sphere_zfwd(Context&, int, const void*, const double*, int, int, const BatchKin&, const void*, void*);
+#define PWK_INST(T)                                                                                                  \
+  template void sphere_zfwd(Context&, int, const void*, const T*, int, int, const NoBatch&, const void*, void*);      \
+  template void sphere_zfwd(Context&, int, const void*, const T*, int, int, const BatchKin<FEW_BATCH_ENTRIES>&,       \
+                            const void*, void*);                                                                      \
+  template void sphere_zfwd(Context&, int, const void*, const T*, int, int, const BatchKin<MAX_BATCH_ENTRIES>&,       \
+                            const void*, void*);
+PWK_INST(float)
+PWK_INST(double)
+#undef PWK_INST
 
 }  // namespace pwk

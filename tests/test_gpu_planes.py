@@ -100,10 +100,10 @@ def test_hpsi_planes(gpu, dims, m, prec, tol):
 @pytest.mark.parametrize("dims,m", [((25, 25, 25), 6), ((27, 27, 27), 9), ((27, 25, 32), 6), ((15, 15, 15), 3)])
 @pytest.mark.parametrize("prec,tol", [("fp64", 1e-13), ("fp32", 6e-6), ("split_bf16", 2e-5)])
 @pytest.mark.parametrize("channels,counts", [((7, 7, 7), (3, 1, 18)), ((80, 80), (33, 161)), ((5, 0, 5), (2, 2, 2)),
-                                             ((3, 3, 6, 6, 6), (2, 1, 2, 3, 1)), ((4,) * 66, (1, 2) * 33)])
+                                             ((3, 3, 6, 6, 6), (2, 1, 2, 3, 1)), ((4,) * 130, (1, 2) * 65)])
 def test_hpsi_batch_sticks(gpu, dims, m, prec, tol, channels, counts):
     # k × band batches: one launch per pass and grouped projector products (one fused launch on the small grid)
-    # for up to 64 consecutive entries with one channel count. Tolerance relative to the largest |Hψ|:
+    # for up to 128 consecutive entries with one channel count. Tolerance relative to the largest |Hψ|:
     # the transforms as above plus sums over npw (projection) and nch terms, √npw ≈ 60 roundings
     # (FP32 3.6e-6, split-bf16 2^-16 per product: 1.5e-5)
     miller, idx = setup(gpu, dims, m)
