@@ -552,7 +552,6 @@ template <int R>
 __global__ void __launch_bounds__(ROW_NT) k_heev_rows(int n, int nb, int lu_in_lds, double2* __restrict__ Hb,
                                                       double* __restrict__ work, double* __restrict__ w_out,
                                                       double2* __restrict__ V_out, int* __restrict__ status) {
-  constexpr int CB = 1;  // columns of a wave per batch, two batches in flight
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   double2* sv = reinterpret_cast<double2*>(smem);  // reflector k - 1, its w, reflector k
   double2* sw = sv + n;
@@ -593,16 +592,12 @@ __global__ void __launch_bounds__(ROW_NT) k_heev_rows(int n, int nb, int lu_in_l
       const int i = lane + 64 * r;
       row[r] = i > k && i < n ? (unsigned)i * 16u : kNoRow;
     }
-    auto load = [&](double2(&a)[CB][R], int jb) {
+    auto load = [&](double2(&a)[R], int j) {
 #pragma unroll
-      for (int c = 0; c < CB; ++c) {
-        const int j = jb + ROW_WAVES * c;
-#pragma unroll
-        for (int r = 0; r < R; ++r)
-          if (64 * r + 63 > k) a[c][r] = buf_load(Ar, j < n ? row[r] : kNoRow, min(j, n - 1) * n * 16);
-      }
+      for (int r = 0; r < R; ++r)
+        if (64 * r + 63 > k) a[r] = buf_load(Ar, j < n ? row[r] : kNoRow, min(j, n - 1) * n * 16);
     };
-    double2 a0[CB][R], a1[CB][R];
+    double2 a0[R], a1[R];  // two columns in flight
     load(a0, j0);  // in flight during the vector phase
     if (wave == 0) {
       // w of reflector k - 1, column k, reflector k
@@ -702,35 +697,28 @@ __global__ void __launch_bounds__(ROW_NT) k_heev_rows(int n, int nb, int lu_in_l
     // RLO: the first row group with rows behind k (the groups before it are not touched)
     auto run = [&](auto rlo) {
       constexpr int RLO = decltype(rlo)::value;
-      auto next = [&](double2(&a)[CB][R], int jb) {
+      auto next = [&](double2(&a)[R], int j) {
 #pragma unroll
-        for (int c = 0; c < CB; ++c) {
-          const int j = jb + ROW_WAVES * c;
+        for (int r = RLO; r < R; ++r) a[r] = buf_load(Ar, j < n ? row[r] : kNoRow, min(j, n - 1) * n * 16);
+      };
+      auto pass = [&](double2(&a)[R], int j) {
+        const int jc = min(j, n - 1), l = min((j - j0) / ROW_WAVES, 63);
+        const double2 vj = lane_of(cv, l), wj = lane_of(cw, l), xj = lane_of(cx, l);
 #pragma unroll
-          for (int r = RLO; r < R; ++r) a[c][r] = buf_load(Ar, j < n ? row[r] : kNoRow, min(j, n - 1) * n * 16);
+        for (int r = RLO; r < R; ++r) {
+          double2& z = a[r];
+          rank2(z, vv[r], ww[r], vj, wj);
+          buf_store(Ar, j < n ? row[r] : kNoRow, jc * n * 16, z);
+          q[r].x = fma(z.x, xj.x, fma(-z.y, xj.y, q[r].x));
+          q[r].y = fma(z.x, xj.y, fma(z.y, xj.x, q[r].y));
+        }
+        if (j == k + 1) {
+#pragma unroll
+          for (int r = RLO; r < R; ++r)
+            if (lane + 64 * r < n) scol[lane + 64 * r] = a[r];
         }
       };
-      auto pass = [&](double2(&a)[CB][R], int jb) {
-#pragma unroll
-        for (int c = 0; c < CB; ++c) {
-          const int j = jb + ROW_WAVES * c, jc = min(j, n - 1), l = min((j - j0) / ROW_WAVES, 63);
-          const double2 vj = lane_of(cv, l), wj = lane_of(cw, l), xj = lane_of(cx, l);
-#pragma unroll
-          for (int r = RLO; r < R; ++r) {
-            double2& z = a[c][r];
-            rank2(z, vv[r], ww[r], vj, wj);
-            buf_store(Ar, j < n ? row[r] : kNoRow, jc * n * 16, z);
-            q[r].x = fma(z.x, xj.x, fma(-z.y, xj.y, q[r].x));
-            q[r].y = fma(z.x, xj.y, fma(z.y, xj.x, q[r].y));
-          }
-          if (j == k + 1) {
-#pragma unroll
-            for (int r = RLO; r < R; ++r)
-              if (lane + 64 * r < n) scol[lane + 64 * r] = a[c][r];
-          }
-        }
-      };
-      constexpr int S = CB * ROW_WAVES;
+      constexpr int S = ROW_WAVES;
       for (int jb = j0; jb < n; jb += 2 * S) {
         next(a1, jb + S);
         pass(a0, jb);

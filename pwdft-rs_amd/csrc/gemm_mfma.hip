@@ -185,20 +185,18 @@ __global__ void __launch_bounds__(256, 2) k_zgemm_mfma(int M, int N, int K, int 
 #pragma unroll
     for (int e = 0; e < NBV; ++e) {
       const int nn = tid / BKC + 16 * e;
-      {
-        const T x = in ? r[e].x : (T)0, y = in ? r[e].y : (T)0;
-        ldsT* p = &Bs[buf][0][nn * BKS + 2 * kk];
-        if constexpr (SPLIT) {
-          const __bf16 hx = to_bf16(x), hy = to_bf16(y);
-          p[0] = hx;
-          p[1] = hy;
-          ldsT* q = &Bs[buf][1][nn * BKS + 2 * kk];
-          q[0] = to_bf16(x - (float)hx);
-          q[1] = to_bf16(y - (float)hy);
-        } else {
-          p[0] = x;
-          p[1] = y;
-        }
+      const T x = in ? r[e].x : (T)0, y = in ? r[e].y : (T)0;
+      ldsT* p = &Bs[buf][0][nn * BKS + 2 * kk];
+      if constexpr (SPLIT) {
+        const __bf16 hx = to_bf16(x), hy = to_bf16(y);
+        p[0] = hx;
+        p[1] = hy;
+        ldsT* q = &Bs[buf][1][nn * BKS + 2 * kk];
+        q[0] = to_bf16(x - (float)hx);
+        q[1] = to_bf16(y - (float)hy);
+      } else {
+        p[0] = x;
+        p[1] = y;
       }
     }
   };
@@ -216,56 +214,52 @@ __global__ void __launch_bounds__(256, 2) k_zgemm_mfma(int M, int N, int K, int 
     load_a(a, k0 + 2 * BKC);
     lds_only_barrier();
     // all columns of one product term in turn: independent MFMA chains hide their latency
-    constexpr int G = NB16;
+    if constexpr (SPLIT) {
+      bf8v bhi[NB16], blo[NB16];
 #pragma unroll
-    for (int g = 0; g < NB16; g += G) {
-      if constexpr (SPLIT) {
-        bf8v bhi[G], blo[G];
+      for (int c = 0; c < NB16; ++c) {
+        const int o = (c * 16 + li) * BKS + lk * 8;
+        bhi[c] = *reinterpret_cast<const bf8v*>(&Bs[buf][0][o]);
+        blo[c] = *reinterpret_cast<const bf8v*>(&Bs[buf][1][o]);
+      }
 #pragma unroll
-        for (int c = 0; c < G; ++c) {
-          const int o = ((g + c) * 16 + li) * BKS + lk * 8;
-          bhi[c] = *reinterpret_cast<const bf8v*>(&Bs[buf][0][o]);
-          blo[c] = *reinterpret_cast<const bf8v*>(&Bs[buf][1][o]);
+      for (int c = 0; c < NB16; ++c)
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+          acc[c][h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f.lo[h], bhi[c], acc[c][h], 0, 0, 0);
+#pragma unroll
+      for (int c = 0; c < NB16; ++c)
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+          acc[c][h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f.hi[h], blo[c], acc[c][h], 0, 0, 0);
+#pragma unroll
+      for (int c = 0; c < NB16; ++c)
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+          acc[c][h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f.hi[h], bhi[c], acc[c][h], 0, 0, 0);
+    } else {
+      typedef T v16 __attribute__((ext_vector_type(16 / sizeof(T))));  // 16-byte LDS reads
+      constexpr int V = 16 / (int)sizeof(T);
+      T bv[NB16][8];
+#pragma unroll
+      for (int c = 0; c < NB16; ++c)
+#pragma unroll
+        for (int i = 0; i < 8; i += V) {
+          const v16 x = *reinterpret_cast<const v16*>(&Bs[buf][0][(c * 16 + li) * BKS + lk * 8 + i]);
+#pragma unroll
+          for (int j = 0; j < V; ++j) bv[c][i + j] = x[j];
         }
 #pragma unroll
-        for (int c = 0; c < G; ++c)
+      for (int ks = 0; ks < 8; ++ks)
 #pragma unroll
-          for (int h = 0; h < 2; ++h)
-            acc[g + c][h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f.lo[h], bhi[c], acc[g + c][h], 0, 0, 0);
+        for (int c = 0; c < NB16; ++c)
 #pragma unroll
-        for (int c = 0; c < G; ++c)
-#pragma unroll
-          for (int h = 0; h < 2; ++h)
-            acc[g + c][h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f.hi[h], blo[c], acc[g + c][h], 0, 0, 0);
-#pragma unroll
-        for (int c = 0; c < G; ++c)
-#pragma unroll
-          for (int h = 0; h < 2; ++h)
-            acc[g + c][h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f.hi[h], bhi[c], acc[g + c][h], 0, 0, 0);
-      } else {
-        typedef T v16 __attribute__((ext_vector_type(16 / sizeof(T))));  // 16-byte LDS reads
-        constexpr int V = 16 / (int)sizeof(T);
-        T bv[G][8];
-#pragma unroll
-        for (int c = 0; c < G; ++c)
-#pragma unroll
-          for (int i = 0; i < 8; i += V) {
-            const v16 x = *reinterpret_cast<const v16*>(&Bs[buf][0][((g + c) * 16 + li) * BKS + lk * 8 + i]);
-#pragma unroll
-            for (int j = 0; j < V; ++j) bv[c][i + j] = x[j];
+          for (int h = 0; h < 2; ++h) {
+            if constexpr (MODE == MODE_F32)
+              acc[c][h] = __builtin_amdgcn_mfma_f32_16x16x4f32(f.v[h][ks], bv[c][ks], acc[c][h], 0, 0, 0);
+            else
+              acc[c][h] = __builtin_amdgcn_mfma_f64_16x16x4f64(f.v[h][ks], bv[c][ks], acc[c][h], 0, 0, 0);
           }
-#pragma unroll
-        for (int ks = 0; ks < 8; ++ks)
-#pragma unroll
-          for (int c = 0; c < G; ++c)
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-              if constexpr (MODE == MODE_F32)
-                acc[g + c][h] = __builtin_amdgcn_mfma_f32_16x16x4f32(f.v[h][ks], bv[c][ks], acc[g + c][h], 0, 0, 0);
-              else
-                acc[g + c][h] = __builtin_amdgcn_mfma_f64_16x16x4f64(f.v[h][ks], bv[c][ks], acc[g + c][h], 0, 0, 0);
-            }
-      }
     }
   };
   if (kbeg < kend) {
