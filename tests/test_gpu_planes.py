@@ -43,9 +43,11 @@ def to_grid(psi, idx, dims):
 PLANES = [((15, 15, 18), 7), ((16, 16, 12), 5), ((25, 25, 25), 6), ((27, 27, 27), 13), ((27, 27, 32), 6),
           ((45, 45, 16), 7), ((45, 45, 45), 11), ((48, 48, 9), 4), ((48, 48, 20), 4), ((60, 60, 10), 4),
           ((60, 60, 60), 14), ((64, 64, 15), 7), ((64, 64, 30), 7), ((72, 72, 8), 3), ((72, 72, 81), 3),
-          ((81, 81, 72), 3), ((81, 81, 12), 5),
-          # nx != ny: pruned (held rows moved between launches), at the quarter, and the whole-grid transforms
-          ((50, 25, 25), 6), ((25, 50, 27), 6), ((16, 81, 15), 3), ((80, 18, 20), 4), ((20, 25, 15), 7)]
+          ((81, 81, 72), 3), ((81, 81, 12), 5), ((75, 75, 15), 3), ((80, 80, 16), 3), ((80, 80, 30), 9),
+          # nx != ny: pruned (held rows moved between launches), at the quarter, and the whole-grid transforms;
+          # 64 and 72 points along x on both sides of the FP64 limit
+          ((50, 25, 25), 6), ((25, 50, 27), 6), ((16, 81, 15), 3), ((80, 18, 20), 4), ((20, 25, 15), 7),
+          ((54, 30, 20), 4), ((60, 24, 27), 5), ((64, 32, 30), 7), ((72, 36, 30), 7)]
 
 
 @pytest.mark.parametrize("dims,m", PLANES)
@@ -100,7 +102,7 @@ def test_hpsi_planes(gpu, dims, m, prec, tol):
 @pytest.mark.parametrize("dims,m", [((25, 25, 25), 6), ((27, 27, 27), 9), ((27, 25, 32), 6), ((15, 15, 15), 3)])
 @pytest.mark.parametrize("prec,tol", [("fp64", 1e-13), ("fp32", 6e-6), ("split_bf16", 2e-5)])
 @pytest.mark.parametrize("channels,counts", [((7, 7, 7), (3, 1, 18)), ((80, 80), (33, 161)), ((5, 0, 5), (2, 2, 2)),
-                                             ((3, 3, 6, 6, 6), (2, 1, 2, 3, 1)), ((4,) * 130, (1, 2) * 65)])
+                                             ((3, 3, 6, 6, 6), (2, 1, 2, 3, 1)), ((2,) * 17, (1,) * 17), ((4,) * 130, (1, 2) * 65)])
 def test_hpsi_batch_sticks(gpu, dims, m, prec, tol, channels, counts):
     # k × band batches: one launch per pass and grouped projector products (one fused launch on the small grid)
     # for up to 128 consecutive entries with one channel count. Tolerance relative to the largest |Hψ|:
@@ -305,25 +307,29 @@ def test_density_captured_after_unoccupied_bands(pwk_mod, gpu, dims, m, first):
 
 @pytest.mark.parametrize("prec,tol", [("fp64", 1e-13), ("fp32", 2e-5), ("split_bf16", 5e-5)])
 def test_zgemm_column_blocks(gpu, prec, tol):
-    # column counts around one and two blocks of 144, row counts that make few and many tiles, reductions
-    # around the two-step turn of the main loop and around the split-K chunk
+    # column counts around the tiles of 16, 32 and 48 columns (FP64: 32 at most) with and without split K, row
+    # counts that make few and many tiles, reductions around the two-step turn of the main loop and around the
+    # split-K chunk; the product stored, and added to what is there
     import torch
 
     rng = np.random.default_rng(34)
     dt = torch.complex128 if prec == "fp64" else torch.complex64
-    for (m, n, k) in [(63, 143, 31), (65, 160, 33), (1, 161, 17), (256, 160, 1000), (3000, 80, 48), (512, 144, 2001),
-                      (130, 289, 255), (16, 16, 257)]:
+    edges = (1, 15, 16, 17, 31, 32, 33, 47, 48, 49, 96, 97, 161)
+    sizes = [(63, 143, 31), (65, 160, 33), (1, 161, 17), (256, 160, 1000), (3000, 80, 48), (512, 144, 2001), (130, 289, 255),
+             (16, 16, 257)] + [(70, n, 1030) for n in edges] + [(9000, n, 40) for n in edges]
+    for (m, n, k) in sizes:
         A = rng.standard_normal((m, k)) + 1j * rng.standard_normal((m, k))
         B = rng.standard_normal((k, n)) + 1j * rng.standard_normal((k, n))
         dA, dB = (torch.from_numpy(np.ascontiguousarray(x.T)).to(dt).cuda() for x in (A, B))
         dC = torch.full((n, m), float("nan"), dtype=dt).cuda()
         torch.cuda.synchronize()
-        gpu.zgemm_dev(m, n, k, dA.data_ptr(), m, dB.data_ptr(), k, dC.data_ptr(), m, precision=prec)
-        gpu.sync()
         ref = A @ B
-        err = np.abs(dC.cpu().numpy().T - ref).max() / np.abs(ref).max()
-        print("zgemm", prec, (m, n, k), f"{err:.2e}", flush=True)
-        assert err < tol, (m, n, k)
+        for add in (False, True):
+            gpu.zgemm_dev(m, n, k, dA.data_ptr(), m, dB.data_ptr(), k, dC.data_ptr(), m, precision=prec, accumulate=add)
+            gpu.sync()
+            err = np.abs(dC.cpu().numpy().T - (2 if add else 1) * ref).max() / np.abs(ref).max()
+            print("zgemm", prec, (m, n, k), add, f"{err:.2e}", flush=True)
+            assert err < tol, (m, n, k, add)
 
 
 @pytest.mark.parametrize("dims", [(25, 25, 25), (27, 25, 32)])
