@@ -15,12 +15,12 @@
 // compile time (hpsi_sphere.hip); the kernels here serve the other bases on nx = ny, and the whole-grid
 // transforms below the rest. The band density (density.hip) shares the z-inverse and the planes' layout.
 #include <algorithm>
-#include <map>
 
 #include "common.hpp"
 #include "fft_reg.hpp"
 #include "fft_sizes.hpp"
 #include "planes.hpp"
+#include "sticks.hpp"
 
 namespace pwk {
 
@@ -432,96 +432,40 @@ void hpsi_local(Context& c, const T* kin, int nb, int nbk, const void* psi, void
   }
 }
 
-inline int wrap(int n, int d) { return ((n % d) + d) % d; }
-
 }  // namespace
 
 void setup_basis(Context& c, int npw, const int32_t* m) {
   c.check_grid();
   PWK_REQUIRE(npw > 0 && m != nullptr, PWK_E_INVALID, "empty basis");
-  const int nx = c.dims[0], ny = c.dims[1], nz = c.dims[2];
-  std::vector<int32_t> g2fft((size_t)npw), pw0, cnt, lo, xy, sx1;
-  std::map<int, int> x1index;
-  std::map<int, int> seen_xy;
-  for (int i = 0; i < npw; ++i) {
-    const int n1 = m[3 * i], n2 = m[3 * i + 1], n3 = m[3 * i + 2];
-    g2fft[(size_t)i] = (int32_t)(((size_t)wrap(n1, nx) * ny + wrap(n2, ny)) * nz + wrap(n3, nz));
-    bool cont = i > 0 && m[3 * i - 3] == n1 && m[3 * i - 2] == n2 && m[3 * i - 1] + 1 == n3;
-    if (!cont) {
-      int col = wrap(n1, nx) * ny + wrap(n2, ny);
-      PWK_REQUIRE(seen_xy.find(col) == seen_xy.end(), PWK_E_UNSUPPORTED,
-                  "basis is not ordered n1 -> n2 -> n3 or two sticks alias on the grid");
-      seen_xy[col] = (int)pw0.size();
-      pw0.push_back(i);
-      cnt.push_back(0);
-      lo.push_back(n3);
-      xy.push_back(col);
-      int i1 = wrap(n1, nx);
-      if (!x1index.count(i1)) x1index[i1] = 0;
-    }
-    cnt.back() += 1;
-    PWK_REQUIRE(cnt.back() <= nz, PWK_E_UNSUPPORTED, "a z-stick is longer than nz (basis aliases on the grid)");
-  }
-  std::vector<int32_t> x1list;
-  for (auto& kv : x1index) {
-    kv.second = (int)x1list.size();
-    x1list.push_back(kv.first);
-  }
-  for (size_t s = 0; s < xy.size(); ++s) sx1.push_back(x1index[xy[s] / ny]);
+  const char* why = nullptr;
+  const StickTables t = stick_tables(c.dims, npw, m, &why);
+  PWK_REQUIRE(!why, PWK_E_UNSUPPORTED, why);
   c.npw = npw;
-  c.nsticks = (int)pw0.size();
-  c.nx1 = (int)x1list.size();
-  // the stick rows as two runs [0, ra) and [nx - rb, nx) (a sphere's columns): the plane pass
-  // then holds only those rows
-  {
-    int ra = 0;
-    while (ra < c.nx1 && x1list[(size_t)ra] == ra) ++ra;
-    const int rb = c.nx1 - ra;
-    bool runs = ra + rb == c.nx1 && c.nx1 < nx;
-    for (int r = 0; r < rb && runs; ++r) runs = x1list[(size_t)(ra + r)] == nx - rb + r;
-    c.x1_runs = runs;
-    c.x1_ra = runs ? ra : 0;
-    c.x1_rb = runs ? rb : 0;
-  }
-  const int ld = ny + 1;
-  c.pl_rows = c.x1_runs ? c.nx1 + 1 : nx;
-  c.pl_ra = c.x1_runs ? c.x1_ra : nx;
-  c.pl_rb = c.x1_runs ? c.x1_rb : 0;
-  std::vector<int32_t> psrc((size_t)c.pl_rows * ld, -1), off;
-  for (size_t s = 0; s < xy.size(); ++s) {
-    off.push_back((c.x1_runs ? sx1[s] : xy[s] / ny) * ld + xy[s] % ny);
-    psrc[(size_t)off.back()] = (int32_t)s;
-  }
-  // pruned passes: every index within a quarter of its axis
-  c.quarter = fft_len_compiled(nx) && fft_len_compiled(ny) && fft_len_compiled(nz);
-  for (int i = 0; i < npw && c.quarter; ++i)
-    for (int d = 0; d < 3; ++d) c.quarter = c.quarter && std::abs(m[3 * i + d]) <= (c.dims[d] - 1) / 4;
-  std::vector<int32_t> qsrc, qoff;
-  if (c.quarter) {
-    const int px = (nx - 1) / 4, py = (ny - 1) / 4, rx = 2 * px + 1, ry = 2 * py + 1, qld = ny | 1;
-    qsrc.assign((size_t)rx * ry, -1);
-    for (size_t s = 0; s < xy.size(); ++s) {
-      const int i1 = xy[s] / ny, i2 = xy[s] % ny;
-      const int h1 = i1 <= px ? i1 : i1 - (nx - rx), h2 = i2 <= py ? i2 : i2 - (ny - ry);
-      qsrc[(size_t)h1 * ry + h2] = (int32_t)s;
-      qoff.push_back(h1 * qld + i2);
-    }
-  }
+  c.nsticks = (int)t.pw0.size();
+  c.nx1 = (int)t.x1list.size();
+  c.x1_runs = t.x1_runs;
+  c.x1_ra = t.x1_ra;
+  c.x1_rb = t.x1_rb;
+  c.pl_rows = t.pl_rows;
+  c.pl_ra = t.pl_ra;
+  c.pl_rb = t.pl_rb;
+  c.quarter = t.quarter;
   auto up = [&](DevBuf& d, const void* h, size_t bytes) {
     d.ensure(bytes);
     PWK_HIP(hipMemcpyAsync(d.p, h, bytes, hipMemcpyHostToDevice, c.stream));
   };
   up(c.miller, m, (size_t)npw * 3 * sizeof(int32_t));
-  up(c.g2fft, g2fft.data(), g2fft.size() * sizeof(int32_t));
-  up(c.st_pw0, pw0.data(), pw0.size() * sizeof(int32_t));
-  up(c.st_cnt, cnt.data(), cnt.size() * sizeof(int32_t));
-  up(c.st_n3lo, lo.data(), lo.size() * sizeof(int32_t));
-  up(c.x1list, x1list.data(), x1list.size() * sizeof(int32_t));
-  up(c.pl_src, psrc.data(), psrc.size() * sizeof(int32_t));
-  up(c.st_off, off.data(), off.size() * sizeof(int32_t));
+  auto table = [&](DevBuf& d, const std::vector<int32_t>& h) { up(d, h.data(), h.size() * sizeof(int32_t)); };
+  table(c.g2fft, t.g2fft);
+  table(c.st_pw0, t.pw0);
+  table(c.st_cnt, t.cnt);
+  table(c.st_n3lo, t.lo);
+  table(c.x1list, t.x1list);
+  table(c.pl_src, t.pl_src);
+  table(c.st_off, t.st_off);
   if (c.quarter) {
-    up(c.q_src, qsrc.data(), qsrc.size() * sizeof(int32_t));
-    up(c.q_off, qoff.data(), qoff.size() * sizeof(int32_t));
+    table(c.q_src, t.q_src);
+    table(c.q_off, t.q_off);
   }
   c.sync();  // the host tables go out of scope here
 }
