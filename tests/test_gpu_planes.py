@@ -140,13 +140,14 @@ def test_hpsi_batch_sticks(gpu, dims, m, prec, tol, channels, counts):
     assert np.abs(got - w[:nbands[0]]).max() < tol * np.abs(w).max()
 
 
-# batches run between the replays of one with k-points 2, 0, 1 and 5, 3, 4 bands: fewer entries, the same
-# size with other k-points and counts, more entries, more bands
+# batches run between the replays of one with k-points 2, 0, 1 and 5, 3, 4 bands (or 18 entries): fewer
+# entries, the same size with other k-points and counts, more entries, more bands
 OTHERS = [([2, 0], [5, 3]), ([1], [12]), ([0, 1, 2], [4, 5, 3]), ([1, 1, 0, 2, 0], [1, 2, 3, 1, 9])]
 
 
 @pytest.mark.parametrize("dims", [(25, 25, 25), (27, 25, 32), (15, 15, 15), (20, 20, 20)])
-def test_hpsi_batch_captured(gpu, dims):
+@pytest.mark.parametrize("order,nbands", [([2, 0, 1], [5, 3, 4]), ([0, 2, 1] * 6, [1] * 18)])
+def test_hpsi_batch_captured(gpu, dims, order, nbands):
     # replays of a captured batch equal the same batch run directly, whatever other batches (of either
     # precision) run between them: on the stick path and on the fused small grids
     import torch
@@ -160,8 +161,7 @@ def test_hpsi_batch_captured(gpu, dims):
         gpu.set_kinetic(ik, (miller.astype(float) ** 2).sum(1) * (1 + 0.1 * ik))
         b = (rng.standard_normal((npw, nch)) + 1j * rng.standard_normal((npw, nch))) / np.sqrt(npw)
         gpu.set_nonlocal(ik, b, b.conj().T.copy())
-    order, nbands = [2, 0, 1], [5, 3, 4]
-    most = max(sum(nb) for _, nb in OTHERS)
+    most = max([sum(nbands)] + [sum(nb) for _, nb in OTHERS])
     psi = torch.from_numpy(bands(rng, most, npw).astype(np.complex64)).cuda()
     psi64 = psi.to(torch.complex128)
     out, other, other64 = torch.empty_like(psi), torch.empty_like(psi), torch.empty_like(psi64)
